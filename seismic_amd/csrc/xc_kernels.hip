@@ -342,54 +342,57 @@ __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restric
     if constexpr (CT) return twmul<mm, 2 * R, 1>(u);
     else return f2c(pre[mm * 64]);
   };
-  // Z = E + i T D with E = Y + conj(Ym), D = Y - conj(Ym), T = e^{2 pi i k/P}
-  auto zform = [](cf a, cf am, cf t) {
-    const float ex = a.x + am.x, ey = a.y - am.y;
-    const float dx = a.x - am.x, dy = a.y + am.y;
-    return cmk(__builtin_fmaf(-t.x, dy, __builtin_fmaf(-t.y, dx, ex)),
-               __builtin_fmaf(t.x, dx, __builtin_fmaf(-t.y, dy, ey)));
-  };
-  // The mirrored bins go through this wave's LDS buffer: bin k sits at lane
-  // t = k % 64, register k / 64, so written as rows of 64 the bins of a few
-  // consecutive registers form a linear range, and every lane reads its
-  // mirror M - k at one address formula — lane 0, whose mirrors are its own
-  // register R - m (the Nyquist bin for m = 0), needs no special case.  In
-  // chunks of Q low registers m (and their partners R - 1 - m): the Q + 1
-  // registers holding the low ones' mirrors, then the Q + 1 holding the high
-  // ones', 2 (Q + 1) 64-lane rows in the 9-row buffer, before any of the
-  // chunk's values change.  The top row of the first set is the register the
-  // previous chunk turned into Z first, so its original is kept.
-  constexpr int Q = 4;
-  static_assert((R / 2) % Q == 0 && Q + 1 <= kWaveLds / 64, "mirror chunks");
-  cf top = cmk(yN, 0.f);  // original y[R - Q c] (the Nyquist bin for c = 0)
-  sfor<0, R / (2 * Q)>([&](auto cc) {
+  // With E = Y[k] + conj(Y[M-k]), D = Y[k] - conj(Y[M-k]), T = e^{2 pi i k/P}:
+  // Z[k] = E + i T D and, as E and D of the mirrored bin are conj(E) and
+  // -conj(D) and its factor -conj(T), Z[M-k] = conj(E - i T D).  One lane so
+  // computes both bins from one product: 12 operations and one packing factor
+  // for two bins instead of 16 and two (each bin by its own lane): the kernel is
+  // bound by vector issue, and N = 4096, C = 3, P = 4096 went 33.00 -> 32.36 ms,
+  // N = 1501, P = 8192 7.58 -> 7.40 ms, N = 1111, C = 2, P = 3072 2.00 -> 1.94 ms.
+  // Lane t owns bin t + 64 m in register m; the lanes of the low registers
+  // m < R/2 compute.  In chunks of Q low registers m = cQ + q, the registers
+  // R - 1 - m that hold their mirrors are written to this wave's LDS buffer as
+  // a linear range of bins (row r: register a0 + r; the bin above the range,
+  // lane 0 of the next register or the Nyquist bin, as row Q), each lane reads
+  // its mirror M - k at one address formula, writes Z[M-k] back to the same
+  // place, and the owners read it.  Lane 0's lowest bin of a chunk, 64 a0,
+  // mirrors into the next chunk: it stays unchanged and goes along as that
+  // chunk's row Q; after the last chunk it is bin M/2, its own mirror.
+  constexpr int HR = R / 2;
+  constexpr int Q = load_group(HR, 8);
+  static_assert(HR % Q == 0 && Q + 1 <= kWaveLds / 64, "mirror chunks");
+  sfor<0, HR / Q>([&](auto cc) {
     constexpr int c = decltype(cc)::value;
-    constexpr int a0 = R - Q - Q * c;  // first register of the low ones' mirror set
-    constexpr int b0 = Q * c;          // first register of the high ones' mirror set
-    cf am[Q], bm[Q];
+    constexpr int a0 = R - Q - Q * c;  // first register of the chunk's mirrors
+    cf am[Q];
     wave_lds_fence();  // earlier reads of the buffer come first
 #pragma unroll
     for (int r = 0; r < Q; ++r) wl[64 * r + lane] = c2f(y[a0 + r]);
-    wl[64 * Q + lane] = c2f(top);
+    wl[64 * Q + lane] = c == 0 ? make_float2(yN, 0.f) : c2f(y[c == 0 ? 0 : a0 + Q]);
     wave_lds_fence();
-    // low m = b0 + q: mirror M - lane - 64 m is row Q - q, lane offset -lane
 #pragma unroll
     for (int q = 0; q < Q; ++q) am[q] = f2c(wl[64 * (Q - q) - lane]);
-    wave_lds_fence();
-#pragma unroll
-    for (int r = 0; r <= Q; ++r) wl[64 * r + lane] = c2f(y[b0 + r]);
-    wave_lds_fence();
-    // high R - 1 - m: mirror 64 (m + 1) - lane is row q + 1
-#pragma unroll
-    for (int q = 0; q < Q; ++q) bm[q] = f2c(wl[64 * (q + 1) - lane]);
-    top = y[a0];  // the next chunk's top row, about to change below
     sfor<0, Q>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
-      constexpr int m = b0 + q, mh = R - 1 - m;
-      y[m] = zform(y[m], am[q], pre_tw(std::integral_constant<int, m>{}));
-      y[mh] = zform(y[mh], bm[q], pre_tw(std::integral_constant<int, mh>{}));
+      constexpr int m = Q * c + q;
+      const cf t = pre_tw(std::integral_constant<int, m>{});
+      const cf a = y[m], b = am[q];
+      const float ex = a.x + b.x, ey = a.y - b.y, dx = a.x - b.x, dy = a.y + b.y;
+      const float re = __builtin_fmaf(t.x, dy, t.y * dx);   // -Re(i T D)
+      const float im = __builtin_fmaf(t.x, dx, -t.y * dy);  // Im(i T D)
+      y[m] = cmk(ex - re, ey + im);
+      am[q] = cmk(ex + re, im - ey);
     });
+    wave_lds_fence();
+#pragma unroll
+    for (int q = 0; q < Q; ++q) wl[64 * (Q - q) - lane] = c2f(am[q]);
+    wave_lds_fence();
+#pragma unroll
+    for (int r = 0; r < Q; ++r) y[a0 + r] = f2c(wl[64 * r + lane]);
+    if constexpr (c > 0) y[a0 + Q] = f2c(wl[64 * Q + lane]);  // lane 0's bin from this chunk's row Q
   });
+  // bin M/2 (lane 0 of register R/2): E + i T D with Y its own mirror, T = i
+  if (lane == 0) y[HR] = cmk(2.f * y[HR].x, -2.f * y[HR].y);
   wave_lds_fence();  // the FFT's transposes reuse the buffer
   __builtin_amdgcn_s_setprio(0);
   wave_fft<R, 1, CT>(y, tw, wl, lane);

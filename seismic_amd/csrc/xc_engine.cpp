@@ -120,7 +120,7 @@ void plan_free(sxc_plan* p) {
   if (!p) return;
   for (hipEvent_t e : p->events) (void)hipEventDestroy(e);
   void* bufs[] = {p->spec, p->col_spec, p->norms, p->traces, p->work, p->ties, p->tie_count,
-                  p->fwd2, p->inv2, p->post, p->winmask, p->hi, p->lo, p->lag_traces, p->tiles,
+                  p->fwd2, p->inv2, p->post, p->hi, p->lo, p->lag_traces, p->tiles,
                   p->fnorms, p->wide, p->wide_count, p->blk_work, p->grp_count};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -159,45 +159,19 @@ std::vector<float2> wave_tables(int R, int sign) {
   return t;
 }
 
-// Lag held by (lane, slot) after the inverse wave FFT: slot = 2*reg + {re, im},
-// reg = 8s + k holds frequency index q = (lane/8 + 8s) + R*(lane%8 + 8k),
-// i.e. samples 2q and 2q+1 of the period-P correlation.
-int slot_lag_host(int R, int lane, int slot) {
-  const int M = 64 * R;
-  const int reg = slot >> 1;
-  const int q = ((lane >> 3) + 8 * (reg >> 3)) + R * ((lane & 7) + 8 * (reg & 7));
-  const int n = 2 * q + (slot & 1);
-  return n <= M ? n : n - 2 * M;
-}
-
 }  // namespace sxc
-
-// Window lane masks of an FFT-form plan: bit l of mask s is set when slot s
-// of lane l holds a lag inside [lag_lo, lag_hi].
-std::vector<unsigned long long> sxc::window_masks(int R, int lag_lo, int lag_hi) {
-  std::vector<unsigned long long> wm(2 * R, 0ull);
-  for (int s = 0; s < 2 * R; ++s)
-    for (int l = 0; l < 64; ++l) {
-      const int lag = slot_lag_host(R, l, s);
-      if (lag >= lag_lo && lag <= lag_hi) wm[s] |= 1ull << l;
-    }
-  return wm;
-}
 
 static int upload_tables(sxc_plan* p) {
   const int R = p->R, M = p->M, P = p->P;
   std::vector<float2> fw = wave_tables(R, -1), iw = wave_tables(R, +1), post(M + 1);
   for (int k = 0; k <= M; ++k) twiddle(k, P, -1, &post[k].x, &post[k].y);
-  std::vector<unsigned long long> wm = window_masks(R, p->d.lag_lo, p->d.lag_hi);
   int rc;
   if ((rc = dev_alloc(&p->fwd2, fw.size(), "twiddles"))) return rc;
   if ((rc = dev_alloc(&p->inv2, iw.size(), "twiddles"))) return rc;
   if ((rc = dev_alloc(&p->post, post.size(), "twiddles"))) return rc;
-  if ((rc = dev_alloc(&p->winmask, wm.size(), "window masks"))) return rc;
   HIP_CHECK(hipMemcpy(p->fwd2, fw.data(), fw.size() * sizeof(float2), hipMemcpyHostToDevice));
   HIP_CHECK(hipMemcpy(p->inv2, iw.data(), iw.size() * sizeof(float2), hipMemcpyHostToDevice));
   HIP_CHECK(hipMemcpy(p->post, post.data(), post.size() * sizeof(float2), hipMemcpyHostToDevice));
-  HIP_CHECK(hipMemcpy(p->winmask, wm.data(), wm.size() * sizeof(unsigned long long), hipMemcpyHostToDevice));
   return SXC_OK;
 }
 
@@ -315,7 +289,6 @@ int sxc::lag_plan_resolve_wide(sxc_plan* p, float* vp, int* lp, float* vn, int* 
   ra.threshold = d.threshold;
   ra.tie_tol = 2e-6f;  // the FFT form's band: its FP32 values are within 5e-7 of FP64
   ra.tw = p->inv2;
-  ra.winmask = p->winmask;
   ra.vpos = vp;
   ra.lpos = lp;
   ra.vneg = vn;
@@ -867,7 +840,6 @@ int fft_stage_pairs(sxc_plan* p, bool reversed, const int2* work, int n_work, fl
   pa.threshold = d.threshold;
   pa.tie_tol = p->tie_tol;
   pa.tw = p->inv2;
-  pa.winmask = p->winmask;
   pa.vpos = d_vals_pos;
   pa.lpos = d_lags_pos;
   pa.vneg = d_vals_neg;
@@ -913,7 +885,6 @@ int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   ra.threshold = d.threshold;
   ra.tie_tol = p->tie_tol;
   ra.tw = p->inv2;
-  ra.winmask = p->winmask;
   ra.vpos = d_vals_pos;
   ra.lpos = d_lags_pos;
   ra.vneg = d_vals_neg;

@@ -49,7 +49,6 @@ struct PairArgs {
   float threshold;
   float tie_tol;
   const float2* tw;       // inverse twiddle tables (TwLayout, then TwLayoutCT)
-  const unsigned long long* winmask;  // [2R] lane masks of in-window slots
   float* vpos;
   int* lpos;
   float* vneg;
@@ -78,7 +77,6 @@ struct ResolveArgs {
   float threshold;
   float tie_tol;
   const float2* tw;
-  const unsigned long long* winmask;
   float* vpos;
   int* lpos;
   float* vneg;

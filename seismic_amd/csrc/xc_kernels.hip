@@ -408,17 +408,57 @@ __host__ __device__ __forceinline__ int slot_lag(int lane, int slot) {
   return n <= M ? n : n - 2 * M;
 }
 
-// Zero every value whose lag is outside the window.  winmask[s] has bit l
-// set when slot s of lane l is inside; it is wave-uniform, so it is read with
-// scalar loads and applied with one select per value.
-template <int R>
-__device__ __forceinline__ void apply_window(cf (&y)[R], const unsigned long long* __restrict__ winmask,
-                                             int lane) {
-  sfor<0, R>([&](auto rc) {
-    constexpr int r = decltype(rc)::value;
-    const unsigned long long m0 = winmask[2 * r], m1 = winmask[2 * r + 1];
-    y[r].x = ((m0 >> lane) & 1ull) ? y[r].x : 0.f;
-    y[r].y = ((m1 >> lane) & 1ull) ? y[r].y : 0.f;
+// Registers a window can touch.  Register 8s + k of the transform's output
+// holds, over the lanes and s, the run of 16 R lags from 16 R k on (k < 4) or
+// 16 R (k - 8) (k >= 4).  A kernel built for G = 1 or 2 serves windows inside
+// the 2G runs around lag 0 (k < G and k >= 8 - G): the other registers are
+// neither scanned nor, as the compiler drops them, computed in the last
+// radix-8 pass.  G = 4 serves every window, G = 0 scans every lag unmasked.
+template <int R, int G>
+constexpr int win_regs() { return G == 0 ? R : R / 8 * 2 * G; }
+template <int R, int G>
+constexpr int win_reg(int i) {  // i-th such register
+  if (G == 0) return i;
+  const int s = i / (2 * G), q = i % (2 * G);
+  return 8 * s + (q < G ? q : 8 - 2 * G + q);
+}
+
+// In-window bit of every value (2 i + {0: x, 1: y}) of a lane's win_regs, built
+// once per workgroup and applied with two operations per value (bit field
+// extract, and).
+template <int R, int G>
+struct WinBits {
+  static constexpr int kWords = (2 * win_regs<R, G>() + 31) / 32;
+  unsigned w[kWords];
+};
+template <int R, int G>
+__device__ __forceinline__ void win_bits(WinBits<R, G>& wb, int lane, int lo, int hi) {
+  constexpr int M = 64 * R;
+  const unsigned span = (unsigned)(hi - lo);
+  const int base = 2 * ((lane >> 3) + R * (lane & 7)) - lo;  // lag - lo of (lane, register 0)
+#pragma unroll
+  for (int w = 0; w < WinBits<R, G>::kWords; ++w) wb.w[w] = 0u;
+  sfor<0, 2 * win_regs<R, G>()>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int reg = win_reg<R, G>(i >> 1), s = reg >> 3, k = reg & 7;
+    constexpr int off = 2 * (8 * s + 8 * R * k) + (i & 1) - (k >= 4 ? 2 * M : 0);
+    bool in = (unsigned)(base + off) <= span;
+    if constexpr (k == 4 && s == 0 && (i & 1) == 0) in = in || (lane == 0 && hi >= M);  // lag M, not -M
+    wb.w[i >> 5] |= in ? 1u << (i & 31) : 0u;
+  });
+}
+// Zero every value whose lag is outside the window.
+template <int R, int G>
+__device__ __forceinline__ void apply_window(cf (&y)[R], const WinBits<R, G>& wb) {
+  sfor<0, win_regs<R, G>()>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int r = win_reg<R, G>(i);
+    auto keep = [&](float v, int bit) {
+      const int m = (int)(wb.w[bit >> 5] << (31 - (bit & 31))) >> 31;
+      return __int_as_float(__float_as_int(v) & m);
+    };
+    y[r].x = keep(y[r].x, 2 * i);
+    y[r].y = keep(y[r].y, 2 * i + 1);
   });
 }
 
@@ -460,28 +500,35 @@ __device__ __forceinline__ void wave_maxmin(float& mx, float& mn) {
 
 // Reference scan rule over the wave's values: strict > (<) starting from
 // (0, lag 0), first occurrence.  Pass 1 keeps the max (min) of each group of
-// four registers (8 values) and reduces them to the exact extrema (DPP wave
+// four registers (8 values; two registers for G = 1) and reduces them to the exact extrema (DPP wave
 // reduction); pass 2 ballots each group maximum (minimum) against extremum
 // -/+ tol, and only for the rare groups where that ballot is non-zero
-// ballots the group's eight values separately: the ballot counts are summed
+// ballots the group's values separately: the ballot counts are summed
 // on the scalar unit, and the last slot whose ballot is non-zero (with its
 // lane mask) locates the extremum.  More than one value within tol flags a
 // near tie, which the FP64 resolver settles.
-template <int R>
+template <int R, int G>
 __device__ __forceinline__ void scan_wave(const cf (&y)[R], int lane, float tol, float thr,
                                           Best& pos, Best& neg, bool& tie_p, bool& tie_n) {
-  static_assert(R % 4 == 0, "groups of four registers");
-  constexpr int G = R / 4;
-  float gp[G], gn[G];
+  constexpr int N = win_regs<R, G>(), S = G == 1 ? 2 : 4;  // registers scanned, and per group
+  static_assert(N % S == 0, "whole groups of registers");
+  constexpr int NG = N / S;
+  float gp[NG], gn[NG];
   float mx = 0.f, mn = 0.f;
-  sfor<0, G>([&](auto gc) {
+  sfor<0, NG>([&](auto gc) {
     constexpr int g = decltype(gc)::value;
-    const cf a = y[4 * g], b = y[4 * g + 1], c = y[4 * g + 2], d = y[4 * g + 3];
     // chained so that each three-operand max (min) takes two new values
-    gp[g] = fmaxf(fmaxf(fmaxf(fmaxf(fmaxf(fmaxf(fmaxf(a.x, a.y), b.x), b.y), c.x), c.y), d.x), d.y);
-    gn[g] = fminf(fminf(fminf(fminf(fminf(fminf(fminf(a.x, a.y), b.x), b.y), c.x), c.y), d.x), d.y);
-    mx = fmaxf(mx, gp[g]);
-    mn = fminf(mn, gn[g]);
+    float hi = y[win_reg<R, G>(S * g)].x, lo = hi;
+    sfor<1, 2 * S>([&](auto qc) {
+      constexpr int q = decltype(qc)::value, r = win_reg<R, G>(S * g + (q >> 1));
+      const float v = (q & 1) ? y[r].y : y[r].x;
+      hi = fmaxf(hi, v);
+      lo = fminf(lo, v);
+    });
+    gp[g] = hi;
+    gn[g] = lo;
+    mx = fmaxf(mx, hi);
+    mn = fminf(mn, lo);
   });
   wave_maxmin(mx, mn);
   const bool want_p = mx > thr && mx > 0.f;
@@ -490,24 +537,24 @@ __device__ __forceinline__ void scan_wave(const cf (&y)[R], int lane, float tol,
   int cnt_p = 0, cnt_n = 0, slot_p = -1, slot_n = -1;
   unsigned long long msk_p = 0, msk_n = 0;
   if (want_p || want_n) {
-    sfor<0, G>([&](auto gc) {
+    sfor<0, NG>([&](auto gc) {
       constexpr int g = decltype(gc)::value;
       if (__ballot(gp[g] >= cp)) {
-        sfor<0, 8>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          const float v = (q & 1) ? y[4 * g + (q >> 1)].y : y[4 * g + (q >> 1)].x;
+        sfor<0, 2 * S>([&](auto qc) {
+          constexpr int q = decltype(qc)::value, r = win_reg<R, G>(S * g + (q >> 1));
+          const float v = (q & 1) ? y[r].y : y[r].x;
           const unsigned long long b = __ballot(v >= cp);
           cnt_p += __popcll(b);
-          if (b) { slot_p = 8 * g + q; msk_p = b; }
+          if (b) { slot_p = 2 * r + (q & 1); msk_p = b; }
         });
       }
       if (__ballot(gn[g] <= cn)) {
-        sfor<0, 8>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          const float v = (q & 1) ? y[4 * g + (q >> 1)].y : y[4 * g + (q >> 1)].x;
+        sfor<0, 2 * S>([&](auto qc) {
+          constexpr int q = decltype(qc)::value, r = win_reg<R, G>(S * g + (q >> 1));
+          const float v = (q & 1) ? y[r].y : y[r].x;
           const unsigned long long b = __ballot(v <= cn);
           cnt_n += __popcll(b);
-          if (b) { slot_n = 8 * g + q; msk_n = b; }
+          if (b) { slot_n = 2 * r + (q & 1); msk_n = b; }
         });
       }
     });
@@ -532,7 +579,8 @@ __device__ __forceinline__ long long packed_index(int i, int j, int n) {
 // e.g. P = 8192 with 5 channels) every wave reads them from global memory.
 // CT: compact twiddle tables (9 KB instead of 66 KB at P = 8192, one extra
 // complex multiply per twiddle; fewer LDS reads per pair).
-template <int R, bool FULL, int kWaves, bool XI_LDS, bool CT>
+// G: the registers scanned (win_regs).
+template <int R, int G, int kWaves, bool XI_LDS, bool CT>
 __global__ __launch_bounds__(kWaves * 64, (R > 32 ? 1 : 2)) void k_pairs(PairArgs a) {
   constexpr int M = 64 * R;
   constexpr int kTab = CT ? TwLayoutCT<R>::kInv : TwLayout<R>::kInv;
@@ -547,6 +595,8 @@ __global__ __launch_bounds__(kWaves * 64, (R > 32 ? 1 : 2)) void k_pairs(PairArg
   float2* wl = xi_lds + (XI_LDS ? a.n_channels * xs : 0) + wv * kWaveLds;
 
   stage_twiddles<R>(twl, a.tw + (CT ? TwLayout<R>::kInv : 0), kTab, threadIdx.x, blockDim.x);
+  WinBits<R, G> wb;
+  if constexpr (G > 0) win_bits<R, G>(wb, lane, a.lag_lo, a.lag_hi);
 
   // XCD-aware walk: workgroups are dispatched round-robin over the 8 XCDs,
   // so XCD x = blockIdx % 8 takes its own contiguous eighth of the
@@ -579,10 +629,10 @@ __global__ __launch_bounds__(kWaves * 64, (R > 32 ? 1 : 2)) void k_pairs(PairArg
       // loads in flight) and the 12-wave budget
       pair_inverse<R, !XI_LDS, CT, (kWaves == 16 || (R >= 48 && (!XI_LDS || kWaves == 12))) ? 16 : 32>(
           y, XI_LDS ? xi_lds : src, xs, xj, a.spec_stride, a.n_channels, twl, wl, lane);
-      if constexpr (!FULL) apply_window<R>(y, a.winmask, lane);
+      if constexpr (G > 0) apply_window<R, G>(y, wb);
       Best pos, neg;
       bool tp, tn;
-      scan_wave<R>(y, lane, a.tie_tol, a.threshold, pos, neg, tp, tn);
+      scan_wave<R, G>(y, lane, a.tie_tol, a.threshold, pos, neg, tp, tn);
       if (lane == 0) {
         const long long idx = dense ? (long long)i * a.dense_cols + j : packed_index(i, j, a.n_events);
         const bool kp = pos.v > a.threshold, kn = neg.v < -a.threshold;
@@ -684,7 +734,11 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
     pair_inverse<R, true, true>(y, a.spec + (long long)i * a.n_channels * a.spec_stride, (int)a.spec_stride,
                           cols + (long long)j * a.n_channels * a.spec_stride, a.spec_stride,
                           a.n_channels, twl, wl, lane);
-    apply_window<R>(y, a.winmask, lane);
+    {
+      WinBits<R, 4> wb;
+      win_bits<R, 4>(wb, lane, a.lag_lo, a.lag_hi);
+      apply_window<R, 4>(y, wb);
+    }
     const long long idx = a.out_ld ? (long long)(i - a.out_row0) * a.out_ld + (j - a.out_col0)
                                    : packed_index(i, j, a.n_events);
     // candidate slots of both sides first (one ballot per slot, kept in this
@@ -810,23 +864,44 @@ hipError_t launch_forward_r(const ForwardArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int R, bool FULL, int W, bool XI_LDS, bool CT>
+template <int R, int G, int W, bool XI_LDS, bool CT>
 static hipError_t launch_pairs_rfw(const PairArgs& a, int grid, hipStream_t st) {
   size_t lds = pair_lds_bytes(R, XI_LDS ? a.n_channels : 0, W, CT);
   static_assert(TwLayout<R>::kInv == 128 * R + 64, "twiddle layout");
   static_assert(TwLayoutCT<R>::kInv == 640 + 8 * R, "compact twiddle layout");
-  hipError_t e = hipFuncSetAttribute((const void*)k_pairs<R, FULL, W, XI_LDS, CT>,
+  hipError_t e = hipFuncSetAttribute((const void*)k_pairs<R, G, W, XI_LDS, CT>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_pairs<R, FULL, W, XI_LDS, CT>), dim3(grid), dim3(W * 64), lds, st, a);
+  hipLaunchKernelGGL((k_pairs<R, G, W, XI_LDS, CT>), dim3(grid), dim3(W * 64), lds, st, a);
   return hipGetLastError();
 }
 
-template <int R, bool FULL>
-static hipError_t launch_pairs_rf(const PairArgs& a, int grid, hipStream_t st) {
+// Narrow windows (G = 1, 2) where the variant is the one that serves most
+// shapes (kNarrow); every window otherwise.
+template <int R, int W, bool XI_LDS, bool CT, bool kNarrow>
+static hipError_t launch_pairs_rw(int groups, const PairArgs& a, int grid, hipStream_t st) {
+  if (groups == 0) return launch_pairs_rfw<R, 0, W, XI_LDS, CT>(a, grid, st);
+  if constexpr (kNarrow) {
+    if (groups == 1) return launch_pairs_rfw<R, 1, W, XI_LDS, CT>(a, grid, st);
+    if (groups == 2) return launch_pairs_rfw<R, 2, W, XI_LDS, CT>(a, grid, st);
+  }
+  return launch_pairs_rfw<R, 4, W, XI_LDS, CT>(a, grid, st);
+}
+
+template <int R>
+hipError_t launch_pairs_r(bool full, const PairArgs& a, int grid, hipStream_t st) {
+  // Runs of 16 R lags the window reaches into on either side of lag 0: the
+  // narrowest build that holds them (win_regs).  Measured at N = 3001, C = 3,
+  // P = 4096: +-512 (G = 2) 20.2 ms -> 18.0
+  // with every value masked by a per-slot lane mask before; N = 3000, C = 3,
+  // P = 2048, every overlapping lag (G = 4) 10.8 -> 9.4.
+  constexpr int kRun = 16 * R;
+  const int runs = (a.lag_hi >= 0 ? a.lag_hi / kRun + 1 : 0), below = (a.lag_lo < 0 ? (-a.lag_lo + kRun - 1) / kRun : 0);
+  const int need = runs > below ? runs : below;
+  const int groups = full ? 0 : (need <= 1 ? 1 : (need == 2 ? 2 : 4));
   // Compact twiddle tables throughout (fewer LDS reads per pair for a few
   // more multiplies: measured 1-1.3% faster at P <= 4096, 22% at P = 6144).
-  // Up to P = 4096, 16 waves (4 per SIMD; 125 VGPRs at P = 4096 with
+  // Up to P = 4096, 16 waves (4 per SIMD; 123 VGPRs at P = 4096 with
   // channel loads in groups of 16 bins) when the staged row spectra fit the
   // 160 KiB of a CU; else 12 waves (3 per SIMD) when they fit, else 8; rows
   // from global memory when none fits.  P = 8192 always runs 8 waves: its 128
@@ -834,18 +909,15 @@ static hipError_t launch_pairs_rf(const PairArgs& a, int grid, hipStream_t st) {
   constexpr size_t kLds = 160 * 1024;
   const int C = a.n_channels;
   if constexpr (R <= 32) {
-    if (pair_lds_bytes(R, C, 16, true) <= kLds) return launch_pairs_rfw<R, FULL, 16, true, true>(a, grid, st);
+    if (pair_lds_bytes(R, C, 16, true) <= kLds) return launch_pairs_rw<R, 16, true, true, true>(groups, a, grid, st);
   }
   if constexpr (R <= 48) {
-    if (pair_lds_bytes(R, C, 12, true) <= kLds) return launch_pairs_rfw<R, FULL, 12, true, true>(a, grid, st);
+    if (pair_lds_bytes(R, C, 12, true) <= kLds)
+      return launch_pairs_rw<R, 12, true, true, (R > 32)>(groups, a, grid, st);
   }
-  if (pair_lds_bytes(R, C, 8, true) <= kLds) return launch_pairs_rfw<R, FULL, 8, true, true>(a, grid, st);
-  return launch_pairs_rfw<R, FULL, 8, false, false>(a, grid, st);
-}
-
-template <int R>
-hipError_t launch_pairs_r(bool full, const PairArgs& a, int grid, hipStream_t st) {
-  return full ? launch_pairs_rf<R, true>(a, grid, st) : launch_pairs_rf<R, false>(a, grid, st);
+  if (pair_lds_bytes(R, C, 8, true) <= kLds)
+    return launch_pairs_rw<R, 8, true, true, (R > 48)>(groups, a, grid, st);
+  return launch_pairs_rw<R, 8, false, false, false>(groups, a, grid, st);
 }
 
 template <int R>

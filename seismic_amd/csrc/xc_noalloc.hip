@@ -5,7 +5,7 @@
 // hipMalloc -- code under HIP graph capture, tight serving loops, harnesses
 // that forbid allocation -- and runs exactly the kernels of sxc_plan_execute
 // with the same launch shapes.  Their workspace (spectra, norms, demeaned
-// traces, work list, window masks, near-tie records and counter, and the
+// traces, work list, near-tie records and counter, and the
 // twiddle tables of every FFT period) lives in one file-scope device array,
 // `scratch`, of kScratchBytes per GPU, held until the process ends.
 //
@@ -48,23 +48,6 @@ __global__ __launch_bounds__(256) void k_fill_work(int2* work, int n, int chunk)
   const int j0 = (int)(c * chunk);
   const int j1 = min(n, j0 + chunk);
   for (int i = threadIdx.x; i < j1; i += blockDim.x) work[off + i] = make_int2(i, max(i, j0));
-}
-
-// Bit l of mask s: slot s of lane l after the inverse wave FFT of R values per
-// lane holds a lag in [lo, hi] (slot = 2 reg + {re, im}; reg = 8 s8 + k holds
-// frequency index q = (l / 8 + 8 s8) + R (l % 8 + 8 k), samples 2q and 2q + 1).
-__global__ void k_fill_winmask(unsigned long long* wm, int R, int lo, int hi) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= 2 * R) return;
-  const int M = 64 * R, reg = s >> 1;
-  unsigned long long m = 0ull;
-  for (int l = 0; l < 64; ++l) {
-    const int q = ((l >> 3) + 8 * (reg >> 3)) + R * ((l & 7) + 8 * (reg & 7));
-    const int n = 2 * q + (s & 1);
-    const int lag = n <= M ? n : n - 2 * M;
-    if (lag >= lo && lag <= hi) m |= 1ull << l;
-  }
-  wm[s] = m;
 }
 
 struct TableOffsets {
@@ -176,8 +159,6 @@ extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* 
   off = align256(off + (size_t)p.tie_cap * sizeof(int4));
   const size_t o_count = off;
   off = align256(off + sizeof(unsigned));
-  const size_t o_mask = off;
-  off = align256(off + (size_t)2 * p.R * sizeof(unsigned long long));
   if (off > kScratchBytes) {
     set_error("this job needs %zu bytes of workspace; the no-allocation entry point holds at most %zu "
               "(%zu after the twiddle tables): use sxc_plan_execute",
@@ -191,19 +172,16 @@ extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* 
   p.work = (int2*)(b + o_work);
   p.ties = (int4*)(b + o_ties);
   p.tie_count = (unsigned*)(b + o_count);
-  p.winmask = (unsigned long long*)(b + o_mask);
   p.fwd2 = (float2*)(b + ds->tab[p.R].fwd);
   p.inv2 = (float2*)(b + ds->tab[p.R].inv);
   p.post = (float2*)(b + ds->tab[p.R].post);
   p.device = dev;
   hipStream_t st = (hipStream_t)stream;
   p.last_stream = st;
-  // the work list and window masks of this call (the previous call's contents
-  // are stale); the tie counter is cleared by the execute itself
+  // the work list of this call (the previous call's contents are stale); the
+  // tie counter is cleared by the execute itself
   const int n_chunks = (desc->n_events + p.chunk - 1) / p.chunk;
   hipLaunchKernelGGL(k_fill_work, dim3(n_chunks), dim3(256), 0, st, p.work, desc->n_events, p.chunk);
-  hipLaunchKernelGGL(k_fill_winmask, dim3((2 * p.R + 63) / 64), dim3(64), 0, st, p.winmask, p.R, desc->lag_lo,
-                     desc->lag_hi);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("scratch set-up launches failed: %s", hipGetErrorString(e));

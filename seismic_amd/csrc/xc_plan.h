@@ -48,7 +48,6 @@ struct sxc_plan {
   int4* ties = nullptr;
   unsigned* tie_count = nullptr;
   float2 *fwd2 = nullptr, *inv2 = nullptr, *post = nullptr;
-  unsigned long long* winmask = nullptr;
   hipStream_t last_stream = nullptr;
   int device = 0;
   // lag-window form
@@ -96,8 +95,6 @@ int fft_plan_forward_events(sxc_plan* p, int e0, int e1, const float* d_traces, 
 int fft_plan_group(sxc_plan* p, int g, const float* d_traces, const float* d_rev, long long trace_stride,
                    int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg,
                    hipStream_t st);
-// lane masks of the in-window slots of the inverse wave FFT of R values per lane
-std::vector<unsigned long long> window_masks(int R, int lag_lo, int lag_hi);
 }  // namespace sxc
 // lag-window forms: planes, norms, FP32 traces, triangle tile list, tie records
 int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out);

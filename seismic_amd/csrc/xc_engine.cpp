@@ -716,6 +716,13 @@ const char* seismic_last_error(void) { return last_error(); }
 
 }  // extern "C"
 
+// Work items (row, column chunk) of the packed triangle, chunk-major: chunk c
+// holds min(N, chunk (c + 1)) rows.
+static long long triangle_items(long long n, long long chunk) {
+  const long long q = n / chunk, r = n % chunk;
+  return chunk * (q * (q + 1) / 2) + (r ? n : 0);
+}
+
 // Geometry of an FFT-form plan (no device memory): period, strides, pair and
 // work-item counts, near-tie band and record capacity.
 void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sxc_plan* p) {
@@ -731,11 +738,8 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sx
   // with the FP64 winner (a flipped winner has an FP32 gap below 2x the error)
   p->tie_tol = desc.tie_tol > 0.f ? desc.tie_tol : 2e-6f;
   p->tie_cap = (int)std::min<long long>(p->n_pairs, tie_cap_max);
-  // work items (row, 64-column chunk), chunk-major: chunk c holds min(N, 64 (c + 1)) rows
-  long long items = 0;
-  for (long long j1 = p->chunk; j1 - p->chunk < desc.n_events; j1 += p->chunk)
-    items += std::min<long long>(j1, desc.n_events);
-  p->n_work = (int)items;
+  if (!p->chunk) p->chunk = pair_chunk(p->R, desc.n_channels, [&](int c) { return triangle_items(desc.n_events, c); });
+  p->n_work = (int)triangle_items(desc.n_events, p->chunk);
 }
 
 extern "C" {
@@ -805,6 +809,7 @@ int fft_stage_forward(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   fa.spec_stride = p->spec_stride;
   fa.tw = p->fwd2;
   fa.post_tw = p->post;
+  fa.zero = p->tie_count;
   HIP_CHECK(launch_forward(p->R, fa, st));
   if (d_rev) {
     ForwardArgs ra = fa;
@@ -818,7 +823,6 @@ int fft_stage_forward(sxc_plan* p, const float* d_traces, const float* d_rev, lo
     ra.norms_in = p->norms;
     HIP_CHECK(launch_forward(p->R, ra, st));
   }
-  HIP_CHECK(launch_fill_u32(p->tie_count, 0u, 1, st));
   return SXC_OK;
 }
 
@@ -847,15 +851,14 @@ int fft_stage_pairs(sxc_plan* p, bool reversed, const int2* work, int n_work, fl
   pa.ties = p->ties;
   pa.tie_count = p->tie_count;
   pa.tie_cap = p->tie_cap;
-  // a multiple of 8 (one share per XCD) whenever there are 8 items or more
-  const int grid = n_work >= 4096 ? 4096 : (n_work >= 8 ? n_work / 8 * 8 : n_work);
-  if (grid > 0) HIP_CHECK(launch_pairs(p->R, p->full, pa, grid, st));
+  if (n_work > 0) HIP_CHECK(launch_pairs(p->R, p->full, pa, pair_grid(n_work), st));
   return SXC_OK;
 }
 
-// The FP64 resolver over the near-tie records from *tie_begin (null: all).
+// The FP64 resolver over the near-tie records from *tie_begin (null: all) of
+// up to n_pairs pairs.
 int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
-                      const unsigned* tie_begin, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
+                      long long n_pairs, const unsigned* tie_begin, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
                       int* d_lags_neg, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   ResolveArgs ra{};
@@ -893,7 +896,7 @@ int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   ra.tie_count = p->tie_count;
   ra.tie_begin = tie_begin;
   ra.tie_cap = p->tie_cap;
-  HIP_CHECK(launch_resolve(p->R, ra, 8192, st));
+  HIP_CHECK(launch_resolve(p->R, ra, resolve_grid(n_pairs), st));
   return SXC_OK;
 }
 }  // namespace
@@ -917,7 +920,7 @@ int sxc::fft_plan_execute(sxc_plan* p, const float* d_traces, const float* d_rev
                             d_lags_neg, st)))
     return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[2], st));
-  if ((rc = fft_stage_resolve(p, d_traces, d_rev, trace_stride, in_len, nullptr, d_vals_pos, d_lags_pos,
+  if ((rc = fft_stage_resolve(p, d_traces, d_rev, trace_stride, in_len, p->n_pairs, nullptr, d_vals_pos, d_lags_pos,
                               d_vals_neg, d_lags_neg, st)))
     return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[3], st));
@@ -1018,7 +1021,7 @@ int sxc::fft_plan_group(sxc_plan* p, int g, const float* d_traces, const float* 
   if ((rc = fft_stage_pairs(p, d_rev != nullptr, p->blk_work + i0, i1 - i0, d_vals_pos, d_lags_pos, d_vals_neg,
                             d_lags_neg, st)))
     return rc;
-  return fft_stage_resolve(p, d_traces, d_rev, trace_stride, in_len, p->grp_count + g, d_vals_pos, d_lags_pos,
+  return fft_stage_resolve(p, d_traces, d_rev, trace_stride, in_len, (long long)(i1 - i0) * p->chunk, p->grp_count + g, d_vals_pos, d_lags_pos,
                            d_vals_neg, d_lags_neg, st);
 }
 

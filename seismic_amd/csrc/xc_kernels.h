@@ -32,6 +32,7 @@ struct ForwardArgs {
   int reversed;
   int rev_shift;
   const double* norms_in;
+  unsigned* zero;         // optional: set to 0 (the near-tie counter of the execute this launch begins)
 };
 
 struct PairArgs {
@@ -42,8 +43,10 @@ struct PairArgs {
   int dense_cols;         // 0: packed upper triangle; > 0: out[i * dense_cols + j], all (i, j)
   int pos_only;           // 1: write only vpos / lpos
   int n_channels;
-  const int2* work;       // (row i, first column) per work item
+  const int2* work;       // (row i, first column) per work item; null (rectangular mode): item e is row
+                          // e % n_rows and column chunk e / n_rows
   int n_work;
+  int n_rows;             // rectangular mode without a work list: rows
   int chunk;              // columns per work item
   int lag_lo, lag_hi;     // scanned lags, inclusive
   float threshold;
@@ -131,8 +134,85 @@ hipError_t launch_hist_threshold(const HistArgs& a, hipStream_t st);
 
 // twiddle tables (full: 128R + 64, compact: 640 + 8R) + staged row spectra +
 // one transpose buffer per wave
-inline size_t pair_lds_bytes(int R, int n_channels, int waves, bool compact = false) {
+constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
+constexpr size_t pair_lds_bytes(int R, int n_channels, int waves, bool compact = false) {
   return (size_t)((compact ? 640 + 8 * R : 128 * R + 64) + n_channels * (64 * R + 1) + waves * 576) * 8;
+}
+
+// Workgroup shapes of a period in order of preference: W waves, S waves per
+// SIMD in all, so 4 S / W workgroups share a CU and its 160 KiB of LDS (tables,
+// staged rows and one buffer per wave each).  The first that fits the job's
+// channels is used.  Compact twiddle tables throughout (fewer LDS reads per
+// pair for a few more multiplies: measured 1-1.3% faster at P <= 4096, 22% at
+// P = 6144).
+//   S: as many waves as the registers allow without spilling the transform
+//   (P = 2048 at S = 6 spills 32 bytes per lane and still gains): short
+//   transforms wait on LDS and memory more than they issue.
+//   W: several small workgroups per CU rather than one of 16 waves, so that one
+//   computes while another waits at the barrier that restages its row.
+// N = 1500, full lags, one 16-wave workgroup -> the shape below: P = 1024,
+// C = 1..4: 1.07 -> 0.80, 1.25 -> 0.95, 1.46 -> 1.15, 1.70 -> 1.42 ms; P = 2048:
+// 1.71 -> 1.46, 2.02 -> 1.77, 2.41 -> 2.21, 2.89 -> 2.70; P = 3072, C = 1..3:
+// 2.52 -> 2.29, 3.00 -> 2.74, 3.51 -> 3.40; P = 4096, C = 1, 2: 3.24 -> 2.95,
+// 3.97 -> 3.90; one 12-wave workgroup -> 3 of 4: P = 5120, C = 1 4.26 -> 4.20,
+// P = 6144 5.11 -> 5.00.  W is a multiple of 4: 6, 10 or 14 waves load the four
+// SIMDs unevenly and the next workgroup no longer fits (P = 1024 with 14: 1.12).
+// P = 8192 runs 8 waves: its 128 spectrum registers per lane need 256 VGPRs.
+struct PairShape {
+  int waves, per_simd;  // W, S; 0: no further shape
+};
+constexpr PairShape pair_shape(int R, int i) {
+  constexpr PairShape k8[] = {{8, 6}, {12, 6}, {8, 4}, {0, 0}, {0, 0}};
+  constexpr PairShape k16[] = {{8, 6}, {12, 6}, {8, 4}, {16, 4}, {0, 0}};
+  constexpr PairShape k24[] = {{8, 4}, {16, 4}, {12, 3}, {0, 0}, {0, 0}};
+  constexpr PairShape k32[] = {{8, 4}, {16, 4}, {12, 3}, {8, 2}, {0, 0}};
+  constexpr PairShape k48[] = {{4, 3}, {12, 3}, {8, 2}, {0, 0}, {0, 0}};  // and R = 40
+  constexpr PairShape k64[] = {{8, 2}, {0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  return R == 8 ? k8[i] : R == 16 ? k16[i] : R == 24 ? k24[i] : R == 32 ? k32[i] : R == 64 ? k64[i] : k48[i];
+}
+constexpr bool pair_shape_fits(int R, int n_channels, PairShape k) {
+  return (size_t)(4 * k.per_simd / k.waves) * pair_lds_bytes(R, n_channels, k.waves, true) <= kLdsBytes;
+}
+constexpr PairShape kGlobalRows = {8, 2};  // rows read from global memory: the rest
+inline PairShape pair_shape_for(int R, int n_channels) {
+  for (int i = 0; pair_shape(R, i).waves > 0; ++i)
+    if (pair_shape_fits(R, n_channels, pair_shape(R, i))) return pair_shape(R, i);
+  return kGlobalRows;
+}
+
+// Columns per work item: 64 keep one chunk's column spectra in an XCD's L2 over
+// its rows, but a small job is then a few workgroups of many serial pairs.  A
+// wave's share of the job, in pairs, is about the workgroups' turns on the
+// 256 CUs times the columns of an item each wave takes, plus half a pair per
+// turn for staging the row; the chunk with the smallest is taken, a smaller one
+// only for a gain of 3%.  items(c): work items with chunks of c columns.
+// With 64 columns always -> this rule (and the shapes above): N = 200, C = 3,
+// P = 2048, +-100 137 -> 102 us; N = 64, C = 3, P = 4096 123 -> 82; one 4096-sample
+// query against 4096 x 3 x 2048 catalog events (P = 5120) 99 -> 48 in the pair
+// kernel.
+template <typename Items>
+inline int pair_chunk(int R, int n_channels, Items items) {
+  const PairShape k = pair_shape_for(R, n_channels);
+  const long long slots = 256 * 4 * k.per_simd / k.waves;
+  int best = 64;
+  double cost = 0.0;
+  for (int c : {64, 32, 16, 8}) {
+    const double t = (double)((items(c) + slots - 1) / slots) * ((c + k.waves - 1) / k.waves + 0.5);
+    if (c == 64 || t < 0.97 * cost) {
+      best = c;
+      cost = t;
+    }
+  }
+  return best;
+}
+// Workgroups of a pair launch: a multiple of 8 (one share per XCD).
+inline int pair_grid(int n_work) { return n_work >= 4096 ? 4096 : (n_work + 7) / 8 * 8; }
+// Workgroups of a resolver launch over the records of up to n_pairs pairs: one
+// wave each, 8192 at most; a small job's grid is kept small, since a launch of
+// 8192 that find no record takes 17 us.
+inline int resolve_grid(long long n_pairs) {
+  const long long few = n_pairs < 256 ? n_pairs : 256, g = n_pairs / 8 > few ? n_pairs / 8 : few;
+  return (int)(g >= 8192 ? 8192 : (g + 7) / 8 * 8);
 }
 
 }  // namespace sxc

@@ -229,6 +229,7 @@ __global__ __launch_bounds__(64 * fwd_waves<R>()) void k_forward(ForwardArgs a) 
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float2* wl = smem + TwLayout<R>::kFft + wv * fwd_wave_buf<R>();  // this wave's transposes, then Z
   float2* zl = wl;
+  if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0u;
   stage_twiddles<R>(twl, a.tw, TwLayout<R>::kFft, threadIdx.x, 64 * W);
   __syncthreads();
   for (int row = blockIdx.x * W + wv; row < a.n_rows; row += gridDim.x * W) {
@@ -579,9 +580,10 @@ __device__ __forceinline__ long long packed_index(int i, int j, int n) {
 // e.g. P = 8192 with 5 channels) every wave reads them from global memory.
 // CT: compact twiddle tables (9 KB instead of 66 KB at P = 8192, one extra
 // complex multiply per twiddle; fewer LDS reads per pair).
-// G: the registers scanned (win_regs).
-template <int R, int G, int kWaves, bool XI_LDS, bool CT>
-__global__ __launch_bounds__(kWaves * 64, (R > 32 ? 1 : 2)) void k_pairs(PairArgs a) {
+// G: the registers scanned (win_regs).  kPerSimd: waves per SIMD the register
+// budget leaves room for.
+template <int R, int G, int kWaves, int kPerSimd, bool XI_LDS, bool CT>
+__global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
   constexpr int M = 64 * R;
   constexpr int kTab = CT ? TwLayoutCT<R>::kInv : TwLayout<R>::kInv;
   extern __shared__ float2 smem[];
@@ -601,12 +603,12 @@ __global__ __launch_bounds__(kWaves * 64, (R > 32 ? 1 : 2)) void k_pairs(PairArg
   // XCD-aware walk: workgroups are dispatched round-robin over the 8 XCDs,
   // so XCD x = blockIdx % 8 takes its own contiguous eighth of the
   // chunk-major work list and keeps one column chunk hot in its L2.
-  const int n_xcd = (gridDim.x % 8 == 0) ? 8 : 1;  // the host sizes the grid to a multiple of 8
+  const int n_xcd = (gridDim.x % 8 == 0) ? 8 : 1;  // pair_grid: a multiple of 8
   const int xcd = blockIdx.x % n_xcd, local = blockIdx.x / n_xcd, n_local = gridDim.x / n_xcd;
   const int seg = (a.n_work + n_xcd - 1) / n_xcd;
   const int seg_end = min(a.n_work, (xcd + 1) * seg);
   for (int item = xcd * seg + local; item < seg_end; item += n_local) {
-    const int2 wk = a.work[item];
+    const int2 wk = a.work ? a.work[item] : make_int2(item % a.n_rows, item / a.n_rows * a.chunk);
     const int i = wk.x;
     const int jb = wk.y;
     const int je = min((jb / a.chunk + 1) * a.chunk, a.n_events);  // end of jb's column chunk
@@ -624,10 +626,10 @@ __global__ __launch_bounds__(kWaves * 64, (R > 32 ? 1 : 2)) void k_pairs(PairArg
     for (int j = (dense ? jb : max(jb, i)) + wv; j < je; j += kWaves) {
       cf y[R];
       const float2* xj = cols + (long long)j * a.n_channels * a.spec_stride;
-      // smaller load groups where registers are short: the 16-wave budget
-      // (128 VGPRs), and at P >= 6144 rows from global memory (twice the
-      // loads in flight) and the 12-wave budget
-      pair_inverse<R, !XI_LDS, CT, (kWaves == 16 || (R >= 48 && (!XI_LDS || kWaves == 12))) ? 16 : 32>(
+      // smaller load groups where registers are short: the budget of 4 waves
+      // per SIMD (128 VGPRs), and at P >= 6144 rows from global memory (twice
+      // the loads in flight) and the budget of 3
+      pair_inverse<R, !XI_LDS, CT, (kPerSimd >= 4 || (R >= 48 && (!XI_LDS || kPerSimd == 3))) ? 16 : 32>(
           y, XI_LDS ? xi_lds : src, xs, xj, a.spec_stride, a.n_channels, twl, wl, lane);
       if constexpr (G > 0) apply_window<R, G>(y, wb);
       Best pos, neg;
@@ -864,28 +866,44 @@ hipError_t launch_forward_r(const ForwardArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int R, int G, int W, bool XI_LDS, bool CT>
+template <int R, int G, int W, int S, bool XI_LDS, bool CT>
 static hipError_t launch_pairs_rfw(const PairArgs& a, int grid, hipStream_t st) {
   size_t lds = pair_lds_bytes(R, XI_LDS ? a.n_channels : 0, W, CT);
   static_assert(TwLayout<R>::kInv == 128 * R + 64, "twiddle layout");
   static_assert(TwLayoutCT<R>::kInv == 640 + 8 * R, "compact twiddle layout");
-  hipError_t e = hipFuncSetAttribute((const void*)k_pairs<R, G, W, XI_LDS, CT>,
+  hipError_t e = hipFuncSetAttribute((const void*)k_pairs<R, G, W, S, XI_LDS, CT>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_pairs<R, G, W, XI_LDS, CT>), dim3(grid), dim3(W * 64), lds, st, a);
+  hipLaunchKernelGGL((k_pairs<R, G, W, S, XI_LDS, CT>), dim3(grid), dim3(W * 64), lds, st, a);
   return hipGetLastError();
 }
 
-// Narrow windows (G = 1, 2) where the variant is the one that serves most
-// shapes (kNarrow); every window otherwise.
-template <int R, int W, bool XI_LDS, bool CT, bool kNarrow>
+// Narrow windows (G = 1, 2) where the build is kept (kNarrow); every window
+// otherwise.
+template <int R, int W, int S, bool XI_LDS, bool CT, bool kNarrow>
 static hipError_t launch_pairs_rw(int groups, const PairArgs& a, int grid, hipStream_t st) {
-  if (groups == 0) return launch_pairs_rfw<R, 0, W, XI_LDS, CT>(a, grid, st);
+  if (groups == 0) return launch_pairs_rfw<R, 0, W, S, XI_LDS, CT>(a, grid, st);
   if constexpr (kNarrow) {
-    if (groups == 1) return launch_pairs_rfw<R, 1, W, XI_LDS, CT>(a, grid, st);
-    if (groups == 2) return launch_pairs_rfw<R, 2, W, XI_LDS, CT>(a, grid, st);
+    if (groups == 1) return launch_pairs_rfw<R, 1, W, S, XI_LDS, CT>(a, grid, st);
+    if (groups == 2) return launch_pairs_rfw<R, 2, W, S, XI_LDS, CT>(a, grid, st);
   }
-  return launch_pairs_rfw<R, 4, W, XI_LDS, CT>(a, grid, st);
+  return launch_pairs_rfw<R, 4, W, S, XI_LDS, CT>(a, grid, st);
+}
+
+// Narrow-window builds go with the shapes of up to four channels; rows from
+// global memory when no shape fits.
+template <int R, int I>
+static hipError_t launch_pairs_fit(int groups, const PairArgs& a, int grid, hipStream_t st) {
+  constexpr PairShape k = pair_shape(R, I);
+  if constexpr (k.waves > 0) {
+    constexpr bool kNarrow = I == 0 || !pair_shape_fits(R, 4, pair_shape(R, I - (I > 0)));
+    if (pair_shape_fits(R, a.n_channels, k))
+      return launch_pairs_rw<R, k.waves, k.per_simd, true, true, kNarrow>(groups, a, grid, st);
+    return launch_pairs_fit<R, I + 1>(groups, a, grid, st);
+  } else if constexpr (!pair_shape_fits(R, 8, pair_shape(R, I - 1))) {
+    return launch_pairs_rw<R, kGlobalRows.waves, kGlobalRows.per_simd, false, false, false>(groups, a, grid, st);
+  }
+  return hipErrorInvalidValue;  // not reached: the last shape holds 8 channels, a plan's most
 }
 
 template <int R>
@@ -899,25 +917,7 @@ hipError_t launch_pairs_r(bool full, const PairArgs& a, int grid, hipStream_t st
   const int runs = (a.lag_hi >= 0 ? a.lag_hi / kRun + 1 : 0), below = (a.lag_lo < 0 ? (-a.lag_lo + kRun - 1) / kRun : 0);
   const int need = runs > below ? runs : below;
   const int groups = full ? 0 : (need <= 1 ? 1 : (need == 2 ? 2 : 4));
-  // Compact twiddle tables throughout (fewer LDS reads per pair for a few
-  // more multiplies: measured 1-1.3% faster at P <= 4096, 22% at P = 6144).
-  // Up to P = 4096, 16 waves (4 per SIMD; 123 VGPRs at P = 4096 with
-  // channel loads in groups of 16 bins) when the staged row spectra fit the
-  // 160 KiB of a CU; else 12 waves (3 per SIMD) when they fit, else 8; rows
-  // from global memory when none fits.  P = 8192 always runs 8 waves: its 128
-  // spectrum registers per lane need the 256-VGPR budget.
-  constexpr size_t kLds = 160 * 1024;
-  const int C = a.n_channels;
-  if constexpr (R <= 32) {
-    if (pair_lds_bytes(R, C, 16, true) <= kLds) return launch_pairs_rw<R, 16, true, true, true>(groups, a, grid, st);
-  }
-  if constexpr (R <= 48) {
-    if (pair_lds_bytes(R, C, 12, true) <= kLds)
-      return launch_pairs_rw<R, 12, true, true, (R > 32)>(groups, a, grid, st);
-  }
-  if (pair_lds_bytes(R, C, 8, true) <= kLds)
-    return launch_pairs_rw<R, 8, true, true, (R > 48)>(groups, a, grid, st);
-  return launch_pairs_rw<R, 8, false, false, false>(groups, a, grid, st);
+  return launch_pairs_fit<R, 0>(groups, a, grid, st);
 }
 
 template <int R>

@@ -36,13 +36,14 @@ constexpr long long kNoallocTieCap = 1LL << 20;  // near-tie records (16 B each)
 constexpr int kMaxDevices = 64;
 constexpr int kRadices[] = {8, 16, 24, 32, 40, 48, 64};
 
-// Work items (row i, first column) of the 64-column chunk c = blockIdx.x, in
-// the chunk-major order of the plan's host-built list: chunk c holds rows
-// 0 .. min(N, 64 (c + 1)) - 1, and chunks before it min(N, 64 (c' + 1)) each,
-// i.e. 32 c (c + 1) items while 64 (c' + 1) <= N, then N per chunk.
+// Work items (row i, first column) of column chunk c = blockIdx.x, in the
+// chunk-major order of the plan's host-built list: with K columns per chunk,
+// chunk c holds rows 0 .. min(N, K (c + 1)) - 1, and chunks before it
+// min(N, K (c' + 1)) each, i.e. K/2 c (c + 1) items while K (c' + 1) <= N, then
+// N per chunk.
 __global__ __launch_bounds__(256) void k_fill_work(int2* work, int n, int chunk) {
   const long long c = blockIdx.x;
-  const long long q = n / chunk;  // chunks whose 64 (c' + 1) <= N
+  const long long q = n / chunk;  // chunks whose K (c' + 1) <= N
   const long long half = chunk / 2;
   const long long off = c <= q ? half * c * (c + 1) : half * q * (q + 1) + (c - q) * n;
   const int j0 = (int)(c * chunk);
@@ -117,21 +118,13 @@ int scratch_for_device(int dev, DeviceScratch** out) {
 
 using namespace sxc;
 
-extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* d_traces, long long trace_stride,
-                                        int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
-                                        int* d_lags_neg, void* stream) {
-  clear_error();
-  if (!desc || !d_traces || !d_vals_pos || !d_lags_pos || !d_vals_neg || !d_lags_neg) {
-    set_error("null argument");
-    return SXC_ERR_INVALID;
-  }
-  int rc = validate_desc(*desc);
-  if (rc) return rc;
-  if (desc->form != SXC_FORM_FFT_F32) {
-    set_error("the no-allocation entry point runs the FFT form only");
-    return SXC_ERR_INVALID;
-  }
+// chunk: columns per work item, 0: the plan's choice.
+static int execute_noalloc(const sxc_plan_desc* desc, int chunk, const float* d_traces, long long trace_stride,
+                           int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg,
+                           void* stream) {
+  int rc;
   sxc_plan p;
+  p.chunk = chunk;
   fft_plan_geometry(*desc, kNoallocTieCap, &p);
   if (in_len < 1 || in_len > p.P || trace_stride < in_len) {
     set_error("in_len %d must be in [1, P=%d] and <= trace_stride %lld", in_len, p.P, trace_stride);
@@ -159,6 +152,10 @@ extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* 
   off = align256(off + (size_t)p.tie_cap * sizeof(int4));
   const size_t o_count = off;
   off = align256(off + sizeof(unsigned));
+  // a job at the limit keeps the shortest work list
+  if (off > kScratchBytes && p.chunk < 64)
+    return execute_noalloc(desc, 64, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
+                           stream);
   if (off > kScratchBytes) {
     set_error("this job needs %zu bytes of workspace; the no-allocation entry point holds at most %zu "
               "(%zu after the twiddle tables): use sxc_plan_execute",
@@ -189,4 +186,22 @@ extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* 
   }
   return fft_plan_execute(&p, d_traces, nullptr, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg,
                           d_lags_neg, st);
+}
+
+extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* d_traces, long long trace_stride,
+                                        int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
+                                        int* d_lags_neg, void* stream) {
+  clear_error();
+  if (!desc || !d_traces || !d_vals_pos || !d_lags_pos || !d_vals_neg || !d_lags_neg) {
+    set_error("null argument");
+    return SXC_ERR_INVALID;
+  }
+  int rc = validate_desc(*desc);
+  if (rc) return rc;
+  if (desc->form != SXC_FORM_FFT_F32) {
+    set_error("the no-allocation entry point runs the FFT form only");
+    return SXC_ERR_INVALID;
+  }
+  return execute_noalloc(desc, 0, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
+                         stream);
 }

@@ -37,7 +37,7 @@ struct sxc_plan {
   bool full = false;
   long long spec_stride = 0;  // float2 per (event, channel) row
   long long n_pairs = 0;
-  int n_work = 0, chunk = 64, tie_cap = 0;  // chunk: columns per work item
+  int n_work = 0, chunk = 0, tie_cap = 0;  // chunk: columns per work item (0: chosen by fft_plan_geometry)
   float tie_tol = 1e-5f;
   // device workspace
   float2* spec = nullptr;

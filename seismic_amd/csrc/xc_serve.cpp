@@ -153,11 +153,9 @@ struct Slot {
   float* d_kv = nullptr;       // [B][kTopkMaxSlices * k] top-k candidates per column slice
   int* d_kl = nullptr;
   int* d_ki = nullptr;
-  int2* d_work = nullptr;      // [B * n_chunks]
   unsigned* d_tie = nullptr;
   float* h_traces = nullptr;   // pinned staging
   int* h_len = nullptr;
-  int2* h_work = nullptr;
   float* h_tv = nullptr;
   int* h_tl = nullptr;
   int* h_ti = nullptr;
@@ -170,8 +168,6 @@ using namespace sxc;
 
 struct sxc_server {
   sxc_server_desc d{};
-  int chunk = 64;
-  int n_chunks = 0;
   long long spec_stride_max = 0;
   std::map<int, Tables> tables;          // by period
   std::map<int, float2*> cat_spec;       // catalog spectra by period
@@ -206,22 +202,21 @@ namespace {
 
 void slot_free(Slot* s) {
   void* dev[] = {s->d_traces, s->d_len, s->d_spec, s->d_norms, s->d_sv, s->d_sl,
-                 s->d_tv, s->d_tl, s->d_ti, s->d_kv, s->d_kl, s->d_ki, s->d_work, s->d_tie};
+                 s->d_tv, s->d_tl, s->d_ti, s->d_kv, s->d_kl, s->d_ki, s->d_tie};
   for (void* p : dev)
     if (p) (void)hipFree(p);
-  void* host[] = {s->h_traces, s->h_len, s->h_work, s->h_tv, s->h_tl, s->h_ti};
+  void* host[] = {s->h_traces, s->h_len, s->h_tv, s->h_tl, s->h_ti};
   for (void* p : host)
     if (p) (void)hipHostFree(p);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   *s = Slot{};
 }
 
-unsigned long long slot_bytes(const sxc_server_desc& d, long long spec_stride_max, int n_chunks) {
+unsigned long long slot_bytes(const sxc_server_desc& d, long long spec_stride_max) {
   const unsigned long long B = d.max_batch_events, C = d.n_channels;
   return B * C * (unsigned long long)d.max_query_len * 4 + B * 4 + B * C * spec_stride_max * 8 +
          B * C * 8 + B * (unsigned long long)d.n_catalog * 8 + B * d.top_k * 12 +
-         B * kTopkMaxSlices * d.top_k * 12 +
-         B * (unsigned long long)n_chunks * 8 + 64;
+         B * kTopkMaxSlices * d.top_k * 12 + 64;
 }
 
 int slot_create(sxc_server* S, Slot* s) {
@@ -240,11 +235,9 @@ int slot_create(sxc_server* S, Slot* s) {
   SRV_CHECK(hipMalloc((void**)&s->d_kv, B * kTopkMaxSlices * d.top_k * sizeof(float)));
   SRV_CHECK(hipMalloc((void**)&s->d_kl, B * kTopkMaxSlices * d.top_k * sizeof(int)));
   SRV_CHECK(hipMalloc((void**)&s->d_ki, B * kTopkMaxSlices * d.top_k * sizeof(int)));
-  SRV_CHECK(hipMalloc((void**)&s->d_work, B * S->n_chunks * sizeof(int2)));
   SRV_CHECK(hipMalloc((void**)&s->d_tie, sizeof(unsigned)));
   SRV_CHECK(hipHostMalloc((void**)&s->h_traces, B * C * d.max_query_len * sizeof(float), hipHostMallocDefault));
   SRV_CHECK(hipHostMalloc((void**)&s->h_len, B * sizeof(int), hipHostMallocDefault));
-  SRV_CHECK(hipHostMalloc((void**)&s->h_work, B * S->n_chunks * sizeof(int2), hipHostMallocDefault));
   SRV_CHECK(hipHostMalloc((void**)&s->h_tv, B * d.top_k * sizeof(float), hipHostMallocDefault));
   SRV_CHECK(hipHostMalloc((void**)&s->h_tl, B * d.top_k * sizeof(int), hipHostMallocDefault));
   SRV_CHECK(hipHostMalloc((void**)&s->h_ti, B * d.top_k * sizeof(int), hipHostMallocDefault));
@@ -262,15 +255,6 @@ int run_batch(sxc_server* S, Slot* s, const std::vector<std::pair<int, int>>& gr
   SRV_CHECK(hipMemcpyAsync(s->d_traces, s->h_traces, (size_t)n_total * C * Lq * sizeof(float),
                            hipMemcpyHostToDevice, s->stream));
   SRV_CHECK(hipMemcpyAsync(s->d_len, s->h_len, (size_t)n_total * sizeof(int), hipMemcpyHostToDevice, s->stream));
-  // work lists for every group (chunk-major, rows relative to the group), staged together
-  int w_off = 0;
-  std::vector<int> w_first;
-  for (auto& g : groups) {
-    w_first.push_back(w_off);
-    for (int c = 0; c < S->n_chunks; ++c)
-      for (int q = 0; q < g.second; ++q) s->h_work[w_off++] = make_int2(q, c * S->chunk);
-  }
-  SRV_CHECK(hipMemcpyAsync(s->d_work, s->h_work, (size_t)w_off * sizeof(int2), hipMemcpyHostToDevice, s->stream));
   for (size_t gi = 0; gi < groups.size(); ++gi) {
     const int first = groups[gi].first, cnt = groups[gi].second;
     if (cnt == 0) continue;
@@ -301,9 +285,11 @@ int run_batch(sxc_server* S, Slot* s, const std::vector<std::pair<int, int>>& gr
     pa.dense_cols = d.n_catalog;
     pa.pos_only = 1;
     pa.n_channels = C;
-    pa.work = s->d_work + w_first[gi];
-    pa.n_work = cnt * S->n_chunks;
-    pa.chunk = S->chunk;
+    // items: every row of the group against one chunk of the catalog, chunk-major
+    auto items = [&](long long c) { return cnt * ((d.n_catalog + c - 1) / c); };
+    pa.chunk = pair_chunk(T.R, C, items);
+    pa.n_work = (int)items(pa.chunk);
+    pa.n_rows = cnt;
     pa.lag_lo = -P / 2 + 1;
     pa.lag_hi = P / 2;
     pa.threshold = -INFINITY;  // keep every pair's maximum for the ranking
@@ -313,8 +299,7 @@ int run_batch(sxc_server* S, Slot* s, const std::vector<std::pair<int, int>>& gr
     pa.lpos = s->d_sl + (size_t)first * d.n_catalog;
     pa.tie_count = s->d_tie;
     pa.tie_cap = 0;  // serving ranks by FP32 values; no FP64 tie records
-    const int grid = pa.n_work >= 4096 ? 4096 : (pa.n_work >= 8 ? pa.n_work / 8 * 8 : pa.n_work);
-    SRV_CHECK(launch_pairs(T.R, true, pa, grid, s->stream));
+    SRV_CHECK(launch_pairs(T.R, true, pa, pair_grid(pa.n_work), s->stream));
     // top-k: a few rows would leave most CUs idle, so each row's columns are
     // split over slices (about 512 workgroups, at least 2048 columns each)
     const int slices = std::max(1, std::min({kTopkMaxSlices, (512 + cnt - 1) / cnt, d.n_catalog / 2048}));
@@ -516,8 +501,7 @@ int sxc_server_create(const sxc_server_desc* desc, const float* catalog, sxc_ser
     return SXC_ERR_INVALID;
   }
   // memory-based admission: every slot reserves one full batch
-  const int n_chunks = (d.n_catalog + 64 - 1) / 64;
-  const unsigned long long per_slot = slot_bytes(d, pmax / 2 + 32, n_chunks);
+  const unsigned long long per_slot = slot_bytes(d, pmax / 2 + 32);
   int n_slots = d.n_slots;
   if (d.mem_budget > 0) n_slots = (int)std::min<unsigned long long>(n_slots, d.mem_budget / per_slot);
   if (n_slots < 1) {
@@ -526,8 +510,6 @@ int sxc_server_create(const sxc_server_desc* desc, const float* catalog, sxc_ser
   }
   sxc_server* S = new sxc_server();
   S->d = d;
-  S->chunk = 64;
-  S->n_chunks = n_chunks;
   S->spec_stride_max = pmax / 2 + 32;
   if (hipGetDevice(&S->device) != hipSuccess) { set_error("no HIP device"); delete S; return SXC_ERR_HIP; }
   S->d.n_slots = n_slots;
@@ -699,7 +681,7 @@ int sxc_server_stats(sxc_server* S, sxc_serve_stats* out) {
   out->mean_requests_per_batch = S->batches ? (double)S->batched_requests / (double)S->batches : 0.0;
   const double span = S->any_submit ? std::chrono::duration<double>(S->t_last_done - S->t_first_submit).count() : 0.0;
   out->events_per_s = span > 0 ? (double)S->events_done / span : 0.0;
-  out->slot_bytes = slot_bytes(S->d, S->spec_stride_max, S->n_chunks);
+  out->slot_bytes = slot_bytes(S->d, S->spec_stride_max);
   out->offered = S->offered;
   out->rejected = S->rejected;
   out->budget_ms = S->budget_ms;

@@ -38,3 +38,18 @@ def test_windows_at_run_edges(oracle, P, C):
         assert np.abs(vp - ref["pos"]).max() <= 1e-5 and np.abs(vn - ref["neg"]).max() <= 1e-5
         sp, sn = ref["gap_pos"] >= 1e-12, ref["gap_neg"] >= 1e-12
         assert np.array_equal(lp[sp], ref["lag_pos"][sp]) and np.array_equal(ln[sn], ref["lag_neg"][sn])
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 17, 31, 33, 64, 65, 130, 257, 420])
+def test_small_jobs_every_column_chunk(oracle, n):
+    """Event counts at and around the multiples of 8, 16, 32 and 64 columns
+    that a small job's work items take: every pair of the triangle."""
+    C, L, P, lo, hi = 1 + n % 3, 300, 1024, -20, 23
+    ev, _ = synth.make_events(n, C, L, seed=500 + n)
+    print(f"case small job N={n} C={C}", flush=True)
+    vp, lp, vn, ln = engine.allpairs_host(ev, P, lo, hi)
+    pi, pj = oracle.packed_pairs(n)
+    ref = oracle.pairs_f64(ev, pi, pj, lo, hi, P=P, circular=True)
+    assert np.abs(vp - ref["pos"]).max() <= 1e-5 and np.abs(vn - ref["neg"]).max() <= 1e-5
+    sp, sn = ref["gap_pos"] >= 1e-12, ref["gap_neg"] >= 1e-12
+    assert np.array_equal(lp[sp], ref["lag_pos"][sp]) and np.array_equal(ln[sn], ref["lag_neg"][sn])

@@ -318,10 +318,21 @@ struct TwLayoutCT {
   static constexpr int kInv = kPreL + 64;
 };
 
-template <int R>
-__device__ __forceinline__ void stage_twiddles(float2* lds_tw, const float2* __restrict__ tab,
-                                               int n, int tid, int nthreads) {
-  for (int k = tid; k < n; k += nthreads) lds_tw[k] = tab[k];
+// Copies N table entries (N even, both sides 16-byte aligned) with T threads,
+// every load of a thread in flight before the first store: one memory round
+// trip (a loop made N / T of them, 14 for the 64-thread resolver at P = 4096).
+template <int N, int T>
+__device__ __forceinline__ void stage_twiddles(float2* lds_tw, const float2* __restrict__ tab, int tid) {
+  static_assert(N % 2 == 0, "whole float4");
+  constexpr int n4 = N / 2, per = (n4 + T - 1) / T;
+  const float4* src = reinterpret_cast<const float4*>(tab);
+  float4* dst = reinterpret_cast<float4*>(lds_tw);
+  float4 v[per];
+#pragma unroll
+  for (int u = 0; u < per; ++u) v[u] = src[min(tid + u * T, n4 - 1)];
+#pragma unroll
+  for (int u = 0; u < per; ++u)
+    if (tid + u * T < n4) dst[tid + u * T] = v[u];
 }
 
 // The four-step wave FFT (see file comment).  `lds` is this wave's private

@@ -193,16 +193,7 @@ __device__ __forceinline__ void forward_row(const ForwardArgs& a, int row, const
   wave_lds_fence();
 
   float2* out = a.spec + (long long)row * a.spec_stride;
-  // X[k] = (Z[k] + conj Z[M-k])/2 - i/2 exp(-2 pi i k/P) (Z[k] - conj Z[M-k])
-  for (int k = lane; k <= M; k += 64) {
-    cf z = f2c(zl[k < M ? k : 0]);       // Z[M] = Z[0]
-    cf zm = f2c(zl[k > 0 ? M - k : 0]);
-    zm.y = -zm.y;
-    cf e = cmk(0.5f * (z.x + zm.x), 0.5f * (z.y + zm.y));
-    cf dd = csub(z, zm);
-    cf od = cmk(0.5f * dd.y, -0.5f * dd.x);  // -i/2 * dd
-    cf t = f2c(a.post_tw[k]);
-    cf X = cadd(e, cmul(od, t));
+  auto emit = [&](int k, cf X) {
     if (a.reversed) {
       // X * exp(+2 pi i q / P), q = k * rev_shift mod P, from the table of
       // exp(-2 pi i k / P), k <= M: conj(post[q]) for q <= M, post[P - q] above
@@ -214,7 +205,38 @@ __device__ __forceinline__ void forward_row(const ForwardArgs& a, int row, const
     }
     if (k == 0 || k == M) X.y = 0.f;
     out[k] = make_float2(X.x * scale, X.y * scale);
+  };
+  // X[k] = E + O e^{-2 pi i k/P} and, E and O of the mirrored bin being
+  // conjugates, X[M-k] = conj(E - O e^{-2 pi i k/P}), with
+  // E = (Z[k] + conj Z[M-k])/2, O = -i/2 (Z[k] - conj Z[M-k]), Z[M] = Z[0]
+  auto convert = [&](int k, float2 t) {
+    const cf z = f2c(zl[k]);
+    cf zm = f2c(zl[k > 0 ? M - k : 0]);
+    zm.y = -zm.y;
+    const cf e = cmk(0.5f * (z.x + zm.x), 0.5f * (z.y + zm.y));
+    const cf dd = csub(z, zm);
+    const cf od = cmul(cmk(0.5f * dd.y, -0.5f * dd.x), f2c(t));
+    emit(k, cadd(e, od));
+    if (2 * k != M) emit(M - k, cmk(e.x - od.x, od.y - e.y));
+  };
+  // the post-twiddles of the next four steps are requested before the stores of
+  // this four (which the compiler cannot move loads across)
+  constexpr int kStep = 4;
+  static_assert((R / 2) % kStep == 0, "whole steps");
+  float2 tw[kStep];
+#pragma unroll
+  for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[lane + 64 * u];
+#pragma unroll 1
+  for (int k0 = lane; k0 < M / 2; k0 += 64 * kStep) {
+    float2 t[kStep];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) t[u] = tw[u];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[min(k0 + 64 * (kStep + u), M)];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) convert(k0 + 64 * u, t[u]);
   }
+  if (lane == 0) convert(M / 2, a.post_tw[M / 2]);
 }
 
 
@@ -223,14 +245,14 @@ __global__ __launch_bounds__(64 * fwd_waves<R>()) void k_forward(ForwardArgs a) 
   constexpr int M = 64 * R;
   constexpr int P = 2 * M;
   constexpr int W = fwd_waves<R>();
-  extern __shared__ float2 smem[];
+  extern __shared__ __align__(16) float2 smem[];
   float2* twl = smem;  // twiddle tables
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float2* wl = smem + TwLayout<R>::kFft + wv * fwd_wave_buf<R>();  // this wave's transposes, then Z
   float2* zl = wl;
   if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0u;
-  stage_twiddles<R>(twl, a.tw, TwLayout<R>::kFft, threadIdx.x, 64 * W);
+  stage_twiddles<TwLayout<R>::kFft, 64 * W>(twl, a.tw, threadIdx.x);
   __syncthreads();
   for (int row = blockIdx.x * W + wv; row < a.n_rows; row += gridDim.x * W) {
     forward_row<R>(a, row, twl, wl, zl, lane);
@@ -586,7 +608,7 @@ template <int R, int G, int kWaves, int kPerSimd, bool XI_LDS, bool CT>
 __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
   constexpr int M = 64 * R;
   constexpr int kTab = CT ? TwLayoutCT<R>::kInv : TwLayout<R>::kInv;
-  extern __shared__ float2 smem[];
+  extern __shared__ __align__(16) float2 smem[];
   const int lane = threadIdx.x & 63;
   // wave index as a scalar: column indices and spectrum addresses then stay
   // in scalar registers (loads use a scalar base and a per-lane offset)
@@ -596,7 +618,7 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
   float2* xi_lds = smem + kTab;
   float2* wl = xi_lds + (XI_LDS ? a.n_channels * xs : 0) + wv * kWaveLds;
 
-  stage_twiddles<R>(twl, a.tw + (CT ? TwLayout<R>::kInv : 0), kTab, threadIdx.x, blockDim.x);
+  stage_twiddles<kTab, 64 * kWaves>(twl, a.tw + (CT ? TwLayout<R>::kInv : 0), threadIdx.x);
   WinBits<R, G> wb;
   if constexpr (G > 0) win_bits<R, G>(wb, lane, a.lag_lo, a.lag_hi);
 
@@ -607,18 +629,32 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
   const int xcd = blockIdx.x % n_xcd, local = blockIdx.x / n_xcd, n_local = gridDim.x / n_xcd;
   const int seg = (a.n_work + n_xcd - 1) / n_xcd;
   const int seg_end = min(a.n_work, (xcd + 1) * seg);
-  for (int item = xcd * seg + local; item < seg_end; item += n_local) {
-    const int2 wk = a.work ? a.work[item] : make_int2(item % a.n_rows, item / a.n_rows * a.chunk);
+  auto fetch = [&](int e) -> int2 {
+    return a.work ? a.work[e] : make_int2(e % a.n_rows, e / a.n_rows * a.chunk);
+  };
+  int item = xcd * seg + local;
+  int2 wk = item < seg_end ? fetch(item) : make_int2(0, 0);
+  for (; item < seg_end; item += n_local) {
     const int i = wk.x;
     const int jb = wk.y;
+    if (item + n_local < seg_end) wk = fetch(item + n_local);  // early: its load is done by the next turn
     const int je = min((jb / a.chunk + 1) * a.chunk, a.n_events);  // end of jb's column chunk
     const bool dense = a.dense_cols > 0;
     const float2* src = a.spec + (long long)i * a.n_channels * a.spec_stride;
     if constexpr (XI_LDS) {
+      // a channel's loads are all in flight before its first store
+      constexpr int T = 64 * kWaves, kPer = (M + T - 1) / T;
       __syncthreads();
-      for (int c = 0; c < a.n_channels; ++c)
-        for (int k = threadIdx.x; k <= M; k += blockDim.x)
-          xi_lds[c * xs + k] = src[c * a.spec_stride + k];
+      for (int c = 0; c < a.n_channels; ++c) {
+        const float2* sc = src + c * a.spec_stride;
+        float2 v[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) v[u] = sc[min((int)threadIdx.x + u * T, M)];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+          if (M % T == 0 || (int)threadIdx.x + u * T < M) xi_lds[c * xs + threadIdx.x + u * T] = v[u];
+      }
+      if ((int)threadIdx.x < a.n_channels) xi_lds[threadIdx.x * xs + M] = src[threadIdx.x * a.spec_stride + M];
       __syncthreads();
     }
 
@@ -670,34 +706,44 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
 //                 own sum for reversed rows (Correlation_in_OMP/
 //                 correlation_c.cpp:270, :63, :102-103): its lag-l value is
 //                 corr_t[L - 1 + l], this sum at shift_q = L - 1 + l.
-// Each ti sample is read once for all NQ, their loads are issued together,
-// and two sets of partial sums per lane keep the FP64 FMA chains short.  The
-// results are wave-uniform.
+// Each ti sample is read once for all NQ, the loads of 8 steps (4 for
+// four lags) are issued together (a record is a serial chain: one memory round
+// trip per 512 or 256 samples instead of one per 128), and two sets of partial sums per lane keep the FP64
+// FMA chains short.  The results are wave-uniform.
 template <int NQ>
 __device__ __forceinline__ void corrn_f64(const float* __restrict__ ti, int len_i, const float* __restrict__ tj,
                                           int len_j, int P, const int (&shift)[4], bool conv, int lane,
                                           double (&out)[4]) {
+  constexpr int U = NQ > 2 ? 4 : 8;  // 64-sample steps whose loads are in flight together
   double sa[NQ], sb[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) sa[q] = sb[q] = 0.0;
-  auto step = [&](int n, double (&acc)[NQ]) {
-    const bool in = n < len_i;
-    const double x = (double)ti[in ? n : 0];
-    float b[NQ];
-    bool ok[NQ];
+  for (int n0 = lane; n0 < len_i; n0 += 64 * U) {
+    float x[U], b[U][NQ];
+    bool ok[U][NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      int u = conv ? shift[q] - n : n - shift[q];  // n, shift in [0, P): one wrap suffices
-      u += u < 0 ? P : 0;
-      ok[q] = in && u < len_j;
-      b[q] = tj[ok[q] ? u : 0];  // always in bounds
+    for (int s = 0; s < U; ++s) {
+      const int n = n0 + 64 * s;
+      const bool in = n < len_i;
+      x[s] = ti[in ? n : 0];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        int u = conv ? shift[q] - n : n - shift[q];  // n, shift in [0, P): one wrap suffices
+        u += u < 0 ? P : 0;
+        ok[s][q] = in && u < len_j;
+        b[s][q] = tj[ok[s][q] ? u : 0];  // always in bounds
+      }
     }
+    asm volatile("" ::: "memory");
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[q] += ok[q] ? x * (double)b[q] : 0.0;
-  };
-  for (int n = lane; n < len_i; n += 128) {
-    step(n, sa);
-    step(n + 64, sb);
+    for (int s = 0; s < U; ++s) {
+      const double xs = (double)x[s];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        double& acc = (s & 1) ? sb[q] : sa[q];
+        acc += ok[s][q] ? xs * (double)b[s][q] : 0.0;
+      }
+    }
   }
 #pragma unroll
   for (int q = 0; q < NQ; ++q) out[q] = wave_sum_f64(sa[q] + sb[q]);
@@ -707,7 +753,7 @@ template <int R>
 __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
   constexpr int M = 64 * R;
   constexpr int P = 2 * M;
-  extern __shared__ float2 smem[];
+  extern __shared__ __align__(16) float2 smem[];
   const int lane = threadIdx.x;
   // records [begin, end): tie_begin, when set, holds the count before the
   // pair launches whose records this launch resolves (the launch groups of
@@ -726,7 +772,7 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
   // compact tables (as the pair kernel): 11.8 KB of LDS at P = 4096
   float2* twl = smem;
   float2* wl = smem + TwLayoutCT<R>::kInv;
-  stage_twiddles<R>(twl, a.tw + TwLayout<R>::kInv, TwLayoutCT<R>::kInv, lane, 64);
+  stage_twiddles<TwLayoutCT<R>::kInv, 64>(twl, a.tw + TwLayout<R>::kInv, lane);
   for (unsigned rec = rec0; rec < seg_end; rec += n_local) {
     const int4 t = a.ties[begin + rec];
     const int i = t.x, j = t.y, side = t.z;
@@ -821,16 +867,23 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
         }
         nb = 0;
       };
-      for (int s = 0; s < 2 * R; ++s) {
-        const unsigned long long ms = cmask[sd * 2 * R + s];
-        unsigned long long mask =
-            ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(ms >> 32)) << 32) |
-            (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)ms);
-        while (mask) {
-          const int src = __ffsll((long long)mask) - 1;
-          mask &= mask - 1;
-          batch[nb++] = slot_lag<R>(src, s);
-          if (nb == 4) flush();
+      // 64 slots' masks at a time, one per lane; only slots with a candidate are
+      // visited (reading each slot's mask in turn was 2R LDS round trips)
+      for (int s0 = 0; s0 < 2 * R; s0 += 64) {
+        const unsigned long long ms = s0 + lane < 2 * R ? cmask[sd * 2 * R + s0 + lane] : 0ull;
+        unsigned long long hit = __ballot(ms != 0ull);
+        while (hit) {
+          const int u = __ffsll((long long)hit) - 1;
+          hit &= hit - 1;
+          unsigned long long mask =
+              ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(ms >> 32), u) << 32) |
+              (unsigned)__builtin_amdgcn_readlane((int)(unsigned)ms, u);
+          while (mask) {
+            const int src = __ffsll((long long)mask) - 1;
+            mask &= mask - 1;
+            batch[nb++] = slot_lag<R>(src, s0 + u);
+            if (nb == 4) flush();
+          }
         }
       }
       flush();

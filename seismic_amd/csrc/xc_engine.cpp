@@ -120,7 +120,7 @@ void plan_free(sxc_plan* p) {
   if (!p) return;
   for (hipEvent_t e : p->events) (void)hipEventDestroy(e);
   void* bufs[] = {p->spec, p->col_spec, p->norms, p->traces, p->work, p->ties, p->tie_count,
-                  p->fwd2, p->inv2, p->post, p->hi, p->lo, p->lag_traces, p->tiles,
+                  p->fwd2, p->narrow.fwd2, p->hi, p->lo, p->lag_traces, p->tiles,
                   p->fnorms, p->wide, p->wide_count, p->blk_work, p->grp_count};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -161,17 +161,23 @@ std::vector<float2> wave_tables(int R, int sign) {
 
 }  // namespace sxc
 
-static int upload_tables(sxc_plan* p) {
-  const int R = p->R, M = p->M, P = p->P;
-  std::vector<float2> fw = wave_tables(R, -1), iw = wave_tables(R, +1), post(M + 1);
-  for (int k = 0; k <= M; ++k) twiddle(k, P, -1, &post[k].x, &post[k].y);
+// The tables of one period, P = 128 R: one allocation (*fwd2) and one copy.
+static int upload_tables(int R, float2** fwd2, float2** inv2, float2** d_post) {
+  const int M = 64 * R, P = 2 * M;
+  std::vector<float2> t = wave_tables(R, -1), iw = wave_tables(R, +1);
+  auto pad = [&] { t.resize((t.size() + 31) / 32 * 32); };  // 256-byte aligned parts
+  pad();
+  const size_t o_inv = t.size();
+  t.insert(t.end(), iw.begin(), iw.end());
+  pad();
+  const size_t o_post = t.size();
+  t.resize(o_post + M + 1);
+  for (int k = 0; k <= M; ++k) twiddle(k, P, -1, &t[o_post + k].x, &t[o_post + k].y);
   int rc;
-  if ((rc = dev_alloc(&p->fwd2, fw.size(), "twiddles"))) return rc;
-  if ((rc = dev_alloc(&p->inv2, iw.size(), "twiddles"))) return rc;
-  if ((rc = dev_alloc(&p->post, post.size(), "twiddles"))) return rc;
-  HIP_CHECK(hipMemcpy(p->fwd2, fw.data(), fw.size() * sizeof(float2), hipMemcpyHostToDevice));
-  HIP_CHECK(hipMemcpy(p->inv2, iw.data(), iw.size() * sizeof(float2), hipMemcpyHostToDevice));
-  HIP_CHECK(hipMemcpy(p->post, post.data(), post.size() * sizeof(float2), hipMemcpyHostToDevice));
+  if ((rc = dev_alloc(fwd2, t.size(), "twiddles"))) return rc;
+  *inv2 = *fwd2 + o_inv;
+  *d_post = *fwd2 + o_post;
+  HIP_CHECK(hipMemcpy(*fwd2, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice));
   return SXC_OK;
 }
 
@@ -246,7 +252,7 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
     if ((rc = dev_alloc(&p->fnorms, (size_t)rows, "norms"))) return fail(rc);
     if ((rc = dev_alloc(&p->wide, (size_t)p->tie_cap, "near-tie records"))) return fail(rc);
     if ((rc = dev_alloc(&p->wide_count, 1, "near-tie counter"))) return fail(rc);
-    if ((rc = upload_tables(p))) return fail(rc);
+    if ((rc = upload_tables(p->R, &p->fwd2, &p->inv2, &p->post))) return fail(rc);
   }
   *out = p;
   return SXC_OK;
@@ -738,7 +744,23 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sx
   // with the FP64 winner (a flipped winner has an FP32 gap below 2x the error)
   p->tie_tol = desc.tie_tol > 0.f ? desc.tie_tol : 2e-6f;
   p->tie_cap = (int)std::min<long long>(p->n_pairs, tie_cap_max);
-  if (!p->chunk) p->chunk = pair_chunk(p->R, desc.n_channels, [&](int c) { return triangle_items(desc.n_events, c); });
+  // The period of executes on traces of L samples: a circular correlation of
+  // traces zero beyond L equals the linear one on the whole window when the
+  // period is at least L + max |lag|, so a window far below P needs less than
+  // P.  Every period is faster than the next (N = 1500, C = 1: P = 1024 0.8 ms,
+  // 2048 1.5, 3072 2.3, 4096 2.9, 5120 4.2, 6144 4.9, 8192 7.2); N = 3001,
+  // C = 3, L = 2048, P = 4096, +-512 runs at 3072: 17.7 -> 13.4 ms.
+  const int reach = std::max(std::abs(desc.lag_lo), std::abs(desc.lag_hi));
+  for (int P : {1024, 2048, 3072, 4096, 5120, 6144})
+    if (P < p->P && P >= desc.trace_len + reach && desc.lag_lo > -P / 2 && desc.lag_hi <= P / 2) {
+      p->narrow.P = P;
+      p->narrow.M = P / 2;
+      p->narrow.R = P / 128;
+      p->narrow.spec_stride = P / 2 + 32;
+      break;
+    }
+  if (!p->chunk)
+    p->chunk = pair_chunk(p->narrow.P ? p->narrow.R : p->R, desc.n_channels, [&](int c) { return triangle_items(desc.n_events, c); });
   p->n_work = (int)triangle_items(desc.n_events, p->chunk);
 }
 
@@ -768,7 +790,9 @@ int sxc_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   }
   if ((rc = dev_alloc(&p->ties, (size_t)p->tie_cap, "near-tie records"))) return fail(rc);
   if ((rc = dev_alloc(&p->tie_count, 1, "near-tie counter"))) return fail(rc);
-  if ((rc = upload_tables(p))) return fail(rc);
+  if ((rc = upload_tables(p->R, &p->fwd2, &p->inv2, &p->post))) return fail(rc);
+  FftGeom& g = p->narrow;
+  if (g.P && (rc = upload_tables(g.R, &g.fwd2, &g.inv2, &g.post))) return fail(rc);
   *out = p;
   return SXC_OK;
 }
@@ -780,18 +804,39 @@ int sxc_plan_destroy(sxc_plan* plan) {
 
 }  // extern "C"
 
-// FFT form.  d_rev == nullptr: column spectra are the row spectra (lag l of
-// pair (i, j) is sum_n x_i[n] x_j[n - l], circular mod P).  d_rev != nullptr:
-// the reference's formulation X_i R_j with the caller's reversed rows
-// (Correlation_in_OMP/correlation_c.cpp:43-45, :270) -- their spectra,
-// rotated by L - 1, become the column spectra, so lag l reads the reference's
-// corr_t[L - 1 + l] whatever length each event really has.
+sxc::FftGeom sxc::fft_geom(const sxc_plan* p, int in_len, bool reversed) {
+  FftGeom g;
+  g.R = p->R;
+  g.M = p->M;
+  g.P = p->P;
+  g.spec_stride = p->spec_stride;
+  g.fwd2 = p->fwd2;
+  g.inv2 = p->inv2;
+  g.post = p->post;
+  g.full = p->full;
+  if (reversed) return g;  // the rows' own lengths set the lags there
+  // samples of a row that can be non-zero (demeaning fills up to L)
+  const int ext = p->d.demean ? std::max(in_len, p->d.trace_len) : in_len;
+  const int reach = std::max(std::abs(p->d.lag_lo), std::abs(p->d.lag_hi));
+  if (p->narrow.P && ext + reach <= p->narrow.P) g = p->narrow;
+  // A window over every lag at which two rows can overlap is scanned without
+  // masks (N = 1111, C = 2, P = 3072: 1.66 -> 1.56 ms): the other lags hold
+  // rounding around an exact 0 (below 5e-7).  Where such a value is the
+  // extremum it is within the band of 0, so the pair is recorded and the
+  // resolver, which looks at the window alone, settles it; hence the default
+  // band at least and room for every record.
+  if (ext + reach <= g.P && p->d.lag_lo <= 1 - ext && p->d.lag_hi >= ext - 1 && p->tie_tol >= 2e-6f &&
+      p->tie_cap >= p->n_pairs)
+    g.full = true;
+  return g;
+}
+
 namespace {
 using namespace sxc;
 
 // The three stages of an FFT-form execute, asynchronous on st.
 // Forward (and reversed-row) R2C of every row, and the near-tie counter reset.
-int fft_stage_forward(sxc_plan* p, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
+int fft_stage_forward(sxc_plan* p, const FftGeom& g, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
                       hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   ForwardArgs fa{};
@@ -804,13 +849,13 @@ int fft_stage_forward(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   fa.demean = d.demean;
   fa.norms = p->norms;
   fa.out_traces = p->traces;
-  fa.out_stride = p->P;
+  fa.out_stride = g.P;
   fa.spec = p->spec;
-  fa.spec_stride = p->spec_stride;
-  fa.tw = p->fwd2;
-  fa.post_tw = p->post;
+  fa.spec_stride = g.spec_stride;
+  fa.tw = g.fwd2;
+  fa.post_tw = g.post;
   fa.zero = p->tie_count;
-  HIP_CHECK(launch_forward(p->R, fa, st));
+  HIP_CHECK(launch_forward(g.R, fa, st));
   if (d_rev) {
     ForwardArgs ra = fa;
     ra.in = d_rev;
@@ -821,19 +866,19 @@ int fft_stage_forward(sxc_plan* p, const float* d_traces, const float* d_rev, lo
     ra.reversed = 1;
     ra.rev_shift = d.trace_len - 1;
     ra.norms_in = p->norms;
-    HIP_CHECK(launch_forward(p->R, ra, st));
+    HIP_CHECK(launch_forward(g.R, ra, st));
   }
   return SXC_OK;
 }
 
 // The pair kernel over work items [work, work + n_work).
-int fft_stage_pairs(sxc_plan* p, bool reversed, const int2* work, int n_work, float* d_vals_pos, int* d_lags_pos,
+int fft_stage_pairs(sxc_plan* p, const FftGeom& g, bool reversed, const int2* work, int n_work, float* d_vals_pos, int* d_lags_pos,
                     float* d_vals_neg, int* d_lags_neg, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   PairArgs pa{};
   pa.spec = p->spec;
   pa.col_spec = reversed ? p->col_spec : nullptr;
-  pa.spec_stride = p->spec_stride;
+  pa.spec_stride = g.spec_stride;
   pa.n_events = d.n_events;
   pa.n_channels = d.n_channels;
   pa.work = work;
@@ -843,7 +888,7 @@ int fft_stage_pairs(sxc_plan* p, bool reversed, const int2* work, int n_work, fl
   pa.lag_hi = d.lag_hi;
   pa.threshold = d.threshold;
   pa.tie_tol = p->tie_tol;
-  pa.tw = p->inv2;
+  pa.tw = g.inv2;
   pa.vpos = d_vals_pos;
   pa.lpos = d_lags_pos;
   pa.vneg = d_vals_neg;
@@ -851,19 +896,19 @@ int fft_stage_pairs(sxc_plan* p, bool reversed, const int2* work, int n_work, fl
   pa.ties = p->ties;
   pa.tie_count = p->tie_count;
   pa.tie_cap = p->tie_cap;
-  if (n_work > 0) HIP_CHECK(launch_pairs(p->R, p->full, pa, pair_grid(n_work), st));
+  if (n_work > 0) HIP_CHECK(launch_pairs(g.R, g.full, pa, pair_grid(n_work), st));
   return SXC_OK;
 }
 
 // The FP64 resolver over the near-tie records from *tie_begin (null: all) of
 // up to n_pairs pairs.
-int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
+int fft_stage_resolve(sxc_plan* p, const FftGeom& g, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
                       long long n_pairs, const unsigned* tie_begin, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
                       int* d_lags_neg, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   ResolveArgs ra{};
   ra.spec = p->spec;
-  ra.spec_stride = p->spec_stride;
+  ra.spec_stride = g.spec_stride;
   if (d_rev) {
     ra.col_spec = p->col_spec;
     ra.rev_traces = d_rev;
@@ -876,8 +921,8 @@ int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   ra.norms = p->norms;
   if (p->traces) {
     ra.traces = p->traces;
-    ra.tr_stride = p->P;
-    ra.tr_len = p->P;
+    ra.tr_stride = g.P;
+    ra.tr_len = g.P;
   } else {
     ra.traces = d_traces;
     ra.tr_stride = trace_stride;
@@ -887,7 +932,7 @@ int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   ra.lag_hi = d.lag_hi;
   ra.threshold = d.threshold;
   ra.tie_tol = p->tie_tol;
-  ra.tw = p->inv2;
+  ra.tw = g.inv2;
   ra.vpos = d_vals_pos;
   ra.lpos = d_lags_pos;
   ra.vneg = d_vals_neg;
@@ -896,7 +941,7 @@ int fft_stage_resolve(sxc_plan* p, const float* d_traces, const float* d_rev, lo
   ra.tie_count = p->tie_count;
   ra.tie_begin = tie_begin;
   ra.tie_cap = p->tie_cap;
-  HIP_CHECK(launch_resolve(p->R, ra, resolve_grid(n_pairs), st));
+  HIP_CHECK(launch_resolve(g.R, ra, resolve_grid(n_pairs), st));
   return SXC_OK;
 }
 }  // namespace
@@ -912,15 +957,16 @@ int sxc::fft_plan_execute(sxc_plan* p, const float* d_traces, const float* d_rev
                           hipStream_t st) {
   hipEvent_t* ev = nullptr;
   if (p->timing && p->timed < (int)p->events.size() / 4) ev = &p->events[4 * p->timed++];
+  const FftGeom g = fft_geom(p, in_len, d_rev != nullptr);
   int rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[0], st));
-  if ((rc = fft_stage_forward(p, d_traces, d_rev, trace_stride, in_len, st))) return rc;
+  if ((rc = fft_stage_forward(p, g, d_traces, d_rev, trace_stride, in_len, st))) return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[1], st));
-  if ((rc = fft_stage_pairs(p, d_rev != nullptr, p->work, p->n_work, d_vals_pos, d_lags_pos, d_vals_neg,
+  if ((rc = fft_stage_pairs(p, g, d_rev != nullptr, p->work, p->n_work, d_vals_pos, d_lags_pos, d_vals_neg,
                             d_lags_neg, st)))
     return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[2], st));
-  if ((rc = fft_stage_resolve(p, d_traces, d_rev, trace_stride, in_len, p->n_pairs, nullptr, d_vals_pos, d_lags_pos,
+  if ((rc = fft_stage_resolve(p, g, d_traces, d_rev, trace_stride, in_len, p->n_pairs, nullptr, d_vals_pos, d_lags_pos,
                               d_vals_neg, d_lags_neg, st)))
     return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[3], st));
@@ -977,6 +1023,7 @@ int sxc::fft_plan_blocks(sxc_plan* p, int B) {
 int sxc::fft_plan_forward_events(sxc_plan* p, int e0, int e1, const float* d_traces, const float* d_rev,
                                  long long trace_stride, int in_len, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
+  const FftGeom g = fft_geom(p, in_len, d_rev != nullptr);
   const long long r0 = (long long)e0 * d.n_channels;
   ForwardArgs fa{};
   fa.in = d_traces + r0 * trace_stride;
@@ -987,25 +1034,25 @@ int sxc::fft_plan_forward_events(sxc_plan* p, int e0, int e1, const float* d_tra
   fa.n_channels = d.n_channels;
   fa.demean = d.demean;
   fa.norms = p->norms + r0;
-  fa.out_traces = p->traces ? p->traces + r0 * p->P : nullptr;
-  fa.out_stride = p->P;
-  fa.spec = p->spec + r0 * p->spec_stride;
-  fa.spec_stride = p->spec_stride;
-  fa.tw = p->fwd2;
-  fa.post_tw = p->post;
+  fa.out_traces = p->traces ? p->traces + r0 * g.P : nullptr;
+  fa.out_stride = g.P;
+  fa.spec = p->spec + r0 * g.spec_stride;
+  fa.spec_stride = g.spec_stride;
+  fa.tw = g.fwd2;
+  fa.post_tw = g.post;
   if (fa.n_rows <= 0) return SXC_OK;
-  HIP_CHECK(launch_forward(p->R, fa, st));
+  HIP_CHECK(launch_forward(g.R, fa, st));
   if (d_rev) {
     ForwardArgs ra = fa;
     ra.in = d_rev + r0 * trace_stride;
     ra.demean = 0;
     ra.norms = nullptr;
     ra.out_traces = nullptr;
-    ra.spec = p->col_spec + r0 * p->spec_stride;
+    ra.spec = p->col_spec + r0 * g.spec_stride;
     ra.reversed = 1;
     ra.rev_shift = d.trace_len - 1;
     ra.norms_in = p->norms + r0;
-    HIP_CHECK(launch_forward(p->R, ra, st));
+    HIP_CHECK(launch_forward(g.R, ra, st));
   }
   return SXC_OK;
 }
@@ -1017,11 +1064,12 @@ int sxc::fft_plan_group(sxc_plan* p, int g, const float* d_traces, const float* 
                         hipStream_t st) {
   HIP_CHECK(hipMemcpyAsync(p->grp_count + g, p->tie_count, sizeof(unsigned), hipMemcpyDeviceToDevice, st));
   const int i0 = p->grp_item[g], i1 = p->grp_item[g + 1];
+  const FftGeom geom = fft_geom(p, in_len, d_rev != nullptr);
   int rc;
-  if ((rc = fft_stage_pairs(p, d_rev != nullptr, p->blk_work + i0, i1 - i0, d_vals_pos, d_lags_pos, d_vals_neg,
+  if ((rc = fft_stage_pairs(p, geom, d_rev != nullptr, p->blk_work + i0, i1 - i0, d_vals_pos, d_lags_pos, d_vals_neg,
                             d_lags_neg, st)))
     return rc;
-  return fft_stage_resolve(p, d_traces, d_rev, trace_stride, in_len, (long long)(i1 - i0) * p->chunk, p->grp_count + g, d_vals_pos, d_lags_pos,
+  return fft_stage_resolve(p, geom, d_traces, d_rev, trace_stride, in_len, (long long)(i1 - i0) * p->chunk, p->grp_count + g, d_vals_pos, d_lags_pos,
                            d_vals_neg, d_lags_neg, st);
 }
 

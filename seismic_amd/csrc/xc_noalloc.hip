@@ -172,6 +172,11 @@ static int execute_noalloc(const sxc_plan_desc* desc, int chunk, const float* d_
   p.fwd2 = (float2*)(b + ds->tab[p.R].fwd);
   p.inv2 = (float2*)(b + ds->tab[p.R].inv);
   p.post = (float2*)(b + ds->tab[p.R].post);
+  if (p.narrow.P) {
+    p.narrow.fwd2 = (float2*)(b + ds->tab[p.narrow.R].fwd);
+    p.narrow.inv2 = (float2*)(b + ds->tab[p.narrow.R].inv);
+    p.narrow.post = (float2*)(b + ds->tab[p.narrow.R].post);
+  }
   p.device = dev;
   hipStream_t st = (hipStream_t)stream;
   p.last_stream = st;

@@ -31,11 +31,24 @@ inline int dev_alloc(T** p, size_t count, const char* what) {
 }
 }  // namespace sxc
 
+namespace sxc {
+// An FFT period and its device tables.
+struct FftGeom {
+  int R = 0, M = 0, P = 0;
+  long long spec_stride = 0;  // float2 per (event, channel) row
+  float2 *fwd2 = nullptr, *inv2 = nullptr, *post = nullptr;
+  bool full = false;          // the pair kernel scans every lag unmasked
+};
+}  // namespace sxc
+
 struct sxc_plan {
   sxc_plan_desc d;
   int R = 0, M = 0, P = 0;
   bool full = false;
   long long spec_stride = 0;  // float2 per (event, channel) row
+  // FFT form: the period of executes on traces short enough that it gives the
+  // same correlations over the window (fft_geom); P = 0: none below P
+  sxc::FftGeom narrow;
   long long n_pairs = 0;
   int n_work = 0, chunk = 0, tie_cap = 0;  // chunk: columns per work item (0: chosen by fft_plan_geometry)
   float tie_tol = 1e-5f;
@@ -78,6 +91,9 @@ void plan_free(sxc_plan* p);
 namespace sxc {
 // FFT form: fills the plan's geometry (no device memory).
 void fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sxc_plan* p);
+// FFT form: the period an execute on rows of in_len samples runs at, and
+// whether it scans every lag.
+FftGeom fft_geom(const sxc_plan* p, int in_len, bool reversed);
 // FFT form: launches forward (and reversed-row) R2C, the pair kernel and the
 // FP64 resolver on the plan's workspace (asynchronous on st).
 int fft_plan_execute(sxc_plan* p, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,

@@ -79,10 +79,9 @@ int validate_desc(const sxc_plan_desc& d) {
       return SXC_ERR_INVALID;
     }
     if (!(d.threshold == d.threshold)) { set_error("threshold is NaN"); return SXC_ERR_INVALID; }
-    // whole blocks of kLagBlock lags from lag_first (== 1 mod 8, <= lag_lo) must fit kLagMaxSpan
     long long lf = d.lag_lo;
     while (((lf - 1) % 8 + 8) % 8 != 0) --lf;
-    const long long span = (d.lag_hi - lf + 1 + kLagBlock - 1) / kLagBlock * kLagBlock;
+    const long long span = (d.lag_hi - lf + 1 + 15) / 16 * 16;
     if (span > kLagMaxSpan) {
       set_error("lag window [%d, %d] spans more than %d lags (the lag forms' limit)", d.lag_lo, d.lag_hi,
                 kLagMaxSpan - 16);
@@ -120,7 +119,7 @@ void plan_free(sxc_plan* p) {
   if (!p) return;
   for (hipEvent_t e : p->events) (void)hipEventDestroy(e);
   void* bufs[] = {p->spec, p->col_spec, p->norms, p->traces, p->work, p->ties, p->tie_count,
-                  p->fwd2, p->narrow.fwd2, p->hi, p->lo, p->lag_traces, p->tiles,
+                  p->fwd2, p->narrow.fwd2, p->h_hi, p->lag_traces, p->tiles,
                   p->fnorms, p->wide, p->wide_count, p->blk_work, p->grp_count};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -194,24 +193,19 @@ static std::vector<int2> build_work(int n, int chunk) {
   return w;
 }
 
-// Lag-window form: zero-padded bf16 (hi, lo) or fp16 planes of every trace,
-// 32 x 32 pair tiles of the upper triangle, blocks of kLagBlock lags.
+// Lag-window form: the row and column operands of every trace as bf16 (hi, lo)
+// or fp16, 32 x 32 pair tiles of the upper triangle, blocks of kLagBlock lags.
 int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   sxc_plan* p = new sxc_plan();
   p->d = *desc;
   p->lag = true;
   const int L = desc->trace_len;
   p->l16 = (L + 15) / 16 * 16;
-  // lag_first == 1 (mod 8) keeps every A and B window 16-byte aligned:
-  // the B window of block lb starts at p0 + n0 + 8h - lb - (kLagBlock - 1).
-  int lf = desc->lag_lo;
-  while (((lf - 1) % 8 + 8) % 8 != 0) --lf;
-  p->lag_first = lf;
-  p->n_blocks = (desc->lag_hi - lf + 1 + kLagBlock - 1) / kLagBlock;
-  const int last = lf + kLagBlock * p->n_blocks - 1;
-  // lowest B index: p0 - last >= 0; highest: p0 + l16 - lf + 8 (24-element windows)
-  p->p0 = std::max(0, (last + 7) / 8 * 8);
-  p->ls = (std::max(p->p0 + p->l16, p->p0 + p->l16 - lf + 9) + 7) / 8 * 8;
+  p->lag_first = desc->lag_lo;
+  p->n_blocks = (desc->lag_hi - desc->lag_lo + 1 + kLagBlock - 1) / kLagBlock;
+  // samples lag_first .. l16 + the last block's last lag; operand loads past a
+  // row's end return 0
+  p->hs = p->l16 + kLagBlock * p->n_blocks;
   p->n_pairs = (long long)desc->n_events * (desc->n_events + 1) / 2;
   // default bands: at least twice the largest coefficient error against FP64
   // measured for the form (bf16x3 4.8e-6, fp16 1.1e-4)
@@ -222,9 +216,17 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   const long long rows = (long long)desc->n_events * desc->n_channels;
   auto fail = [&](int code) { plan_free(p); return code; };
   int rc;
-  if ((rc = dev_alloc(&p->hi, (size_t)(rows * p->ls), "trace planes"))) return fail(rc);
-  if (desc->form == SXC_FORM_LAG_BF16X3 && (rc = dev_alloc(&p->lo, (size_t)(rows * p->ls), "trace planes")))
-    return fail(rc);
+  const size_t h_elems = (size_t)rows * 2 * p->hs;
+  const size_t b_elems = (size_t)((desc->n_events + 31) / 32 * 32) * desc->n_channels * p->l16;
+  // one allocation (h_hi): row operands, then column operands, 256-byte aligned
+  const size_t h_size = (h_elems + 127) / 128 * 128, b_size = (b_elems + 127) / 128 * 128;
+  const bool two = desc->form == SXC_FORM_LAG_BF16X3;
+  if ((rc = dev_alloc(&p->h_hi, (h_size + b_size) * (two ? 2 : 1), "trace operands"))) return fail(rc);
+  p->b_hi = p->h_hi + h_size;
+  if (two) {
+    p->h_lo = p->b_hi + b_size;
+    p->b_lo = p->h_lo + h_size;
+  }
   if ((rc = dev_alloc(&p->norms, (size_t)rows, "norms"))) return fail(rc);
   if ((rc = dev_alloc(&p->lag_traces, (size_t)(rows * L), "FP32 traces"))) return fail(rc);
   const int T = (desc->n_events + 31) / 32;
@@ -277,8 +279,8 @@ int sxc::lag_plan_spectra(sxc_plan* p, hipStream_t st) {
   return SXC_OK;
 }
 
-int sxc::lag_plan_resolve_wide(sxc_plan* p, float* vp, int* lp, float* vn, int* ln, long long out_ld, int out_row0,
-                               int out_col0, hipStream_t st) {
+int sxc::lag_plan_resolve_wide(sxc_plan* p, long long n_pairs, float* vp, int* lp, float* vn, int* ln,
+                               long long out_ld, int out_row0, int out_col0, hipStream_t st) {
   if (!p->P) return SXC_OK;
   const sxc_plan_desc& d = p->d;
   ResolveArgs ra{};
@@ -305,7 +307,7 @@ int sxc::lag_plan_resolve_wide(sxc_plan* p, float* vp, int* lp, float* vn, int* 
   ra.out_ld = out_ld;
   ra.out_row0 = out_row0;
   ra.out_col0 = out_col0;
-  HIP_CHECK(launch_resolve(p->R, ra, 8192, st));
+  HIP_CHECK(launch_resolve(p->R, ra, resolve_grid(n_pairs), st));
   return SXC_OK;
 }
 
@@ -321,14 +323,41 @@ int lag_plan_prep(sxc_plan* p, const float* d_traces, long long trace_stride, in
   pa.n_channels = d.n_channels;
   pa.demean = d.demean;
   pa.fp16 = d.form == SXC_FORM_LAG_FP16;
-  pa.p0 = p->p0;
-  pa.ls = p->ls;
-  pa.hi = p->hi;
-  pa.lo = p->lo;
+  pa.lag_first = p->lag_first;
+  pa.hs = p->hs;
+  pa.l16 = p->l16;
+  pa.h_hi = p->h_hi;
+  pa.h_lo = p->h_lo;
+  pa.b_hi = p->b_hi;
+  pa.b_lo = p->b_lo;
+  pa.zero0 = p->tie_count;
+  pa.zero1 = p->wide_count;
   pa.norms = p->norms;
   pa.traces_out = p->lag_traces;
   HIP_CHECK(launch_lag_prep(pa, st));
   return SXC_OK;
+}
+
+sxc::LagPairArgs sxc::lag_pair_args(const sxc_plan* p) {
+  LagPairArgs ka{};
+  ka.h_hi = p->h_hi;
+  ka.h_lo = p->h_lo;
+  ka.b_hi = p->b_hi;
+  ka.b_lo = p->b_lo;
+  ka.hs = p->hs;
+  ka.n_events = p->d.n_events;
+  ka.n_channels = p->d.n_channels;
+  ka.L = p->d.trace_len;
+  ka.l16 = p->l16;
+  ka.lag_hi = p->d.lag_hi;
+  ka.lag_first = p->lag_first;
+  ka.n_blocks = p->n_blocks;
+  ka.threshold = p->d.threshold;
+  ka.tie_tol = p->tie_tol;
+  ka.ties = p->ties;
+  ka.tie_count = p->tie_count;
+  ka.tie_cap = p->tie_cap;
+  return ka;
 }
 
 static int lag_plan_execute(sxc_plan* p, const float* d_traces, long long trace_stride, int in_len,
@@ -340,33 +369,15 @@ static int lag_plan_execute(sxc_plan* p, const float* d_traces, long long trace_
   int rc = lag_plan_prep(p, d_traces, trace_stride, in_len, st);
   if (rc) return rc;
   if ((rc = lag_plan_spectra(p, st))) return rc;
-  HIP_CHECK(launch_fill_u32(p->tie_count, 0u, 1, st));
-  if (p->wide_count) HIP_CHECK(launch_fill_u32(p->wide_count, 0u, 1, st));
   if (ev) HIP_CHECK(hipEventRecord(ev[1], st));
-  LagPairArgs ka{};
-  ka.hi = p->hi;
-  ka.lo = p->lo;
-  ka.ls = p->ls;
-  ka.n_events = d.n_events;
-  ka.n_channels = d.n_channels;
-  ka.l16 = p->l16;
-  ka.p0 = p->p0;
-  ka.lag_lo = d.lag_lo;
-  ka.lag_hi = d.lag_hi;
-  ka.lag_first = p->lag_first;
-  ka.n_blocks = p->n_blocks;
+  LagPairArgs ka = lag_pair_args(p);
   ka.tiles = p->tiles;
   ka.n_tiles = p->n_tiles;
-  ka.threshold = d.threshold;
-  ka.tie_tol = p->tie_tol;
   ka.vpos = vp;
   ka.lpos = lp;
   ka.vneg = vn;
   ka.lneg = ln;
-  ka.ties = p->ties;
-  ka.tie_count = p->tie_count;
-  ka.tie_cap = p->tie_cap;
-  HIP_CHECK(launch_lag_pairs(d.form == SXC_FORM_LAG_BF16X3, ka, p->n_tiles, st));
+  HIP_CHECK(launch_lag_pairs(d.form == SXC_FORM_LAG_BF16X3, ka, st));
   if (ev) HIP_CHECK(hipEventRecord(ev[2], st));
   LagResolveArgs ra{};
   ra.traces = p->lag_traces;
@@ -388,8 +399,8 @@ static int lag_plan_execute(sxc_plan* p, const float* d_traces, long long trace_
   ra.wide = p->wide;
   ra.wide_count = p->wide_count;
   ra.wide_cap = p->tie_cap;
-  HIP_CHECK(launch_lag_resolve(ra, 8192, st));
-  if ((rc = lag_plan_resolve_wide(p, vp, lp, vn, ln, 0, 0, 0, st))) return rc;
+  HIP_CHECK(launch_lag_resolve(ra, resolve_grid(p->n_pairs), st));
+  if ((rc = lag_plan_resolve_wide(p, p->n_pairs, vp, lp, vn, ln, 0, 0, 0, st))) return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[3], st));
   return SXC_OK;
 }
@@ -442,7 +453,8 @@ static size_t plan_device_bytes(const sxc_plan* p) {
   if (p->traces) b += rows * (size_t)p->P * sizeof(float);
   b += (size_t)p->n_work * sizeof(int2) * (p->blk_work ? 2 : 1) +
        (size_t)p->tie_cap * sizeof(int4) * (p->lag ? 3 : 1);
-  if (p->lag) b += rows * (size_t)p->ls * 2 * (p->lo ? 2 : 1) + rows * (size_t)p->d.trace_len * sizeof(float);
+  if (p->lag)
+    b += rows * ((size_t)p->hs * 2 + p->l16) * 2 * (p->h_lo ? 2 : 1) + rows * (size_t)p->d.trace_len * sizeof(float);
   return b;
 }
 

@@ -4,9 +4,9 @@
 
 namespace sxc {
 
-constexpr int kLagBlock = 16;  // lags per block (one accumulator tile each)
-// The tile kernel keeps lags as 16-bit offsets from the first lag of block 0,
-// so a plan's window spans at most this many lags (whole blocks).
+constexpr int kLagBlock = 32;  // lags per block (one accumulator tile each)
+// A plan's window spans at most this many lags, counted in whole blocks of 16
+// from the last lag at or below its first that is 1 modulo 8.
 constexpr int kLagMaxSpan = 65536;
 
 struct LagPrepArgs {
@@ -18,24 +18,28 @@ struct LagPrepArgs {
   int n_channels;
   int demean;
   int fp16;                 // 1: FP16 plane only; 0: bf16 hi and lo planes
-  int p0;                   // zero samples before each trace in the planes
-  int ls;                   // plane row length (multiple of 8)
-  unsigned short* hi;       // [n_rows][ls]
-  unsigned short* lo;       // [n_rows][ls] or null
+  int lag_first;            // row operand: element q is sample q + lag_first
+  int hs;                   // row operand length (a multiple of 8)
+  int l16;                  // trace length rounded up to 16
+  unsigned short* h_hi;     // [n_rows][2][hs], the second copy one sample on
+  unsigned short* h_lo;     // or null (fp16)
+  unsigned short* b_hi;     // column operand [event / 32][channel][sample / 8][event % 32][8]
+  unsigned short* b_lo;     // or null
+  unsigned* zero0;          // optional counters to clear
+  unsigned* zero1;
   double* norms;            // [n_rows]
   float* traces_out;        // [n_rows][L] FP32 copy (demeaned) for the FP64 resolver
 };
 
 struct LagPairArgs {
-  const unsigned short* hi;
-  const unsigned short* lo;
-  long long ls;
+  const unsigned short *h_hi, *h_lo, *b_hi, *b_lo;  // operands (LagPrepArgs)
+  int hs;
   int n_events, n_channels;
-  int l16;                  // trace length rounded up to 16
-  int p0;
-  int lag_lo, lag_hi;       // scanned lags (inclusive)
-  int lag_first;            // first lag of block 0 (== 1 mod 8, <= lag_lo)
+  int L, l16;               // trace length, and rounded up to 16
+  int lag_hi;               // last scanned lag
+  int lag_first;            // first scanned lag
   int n_blocks;             // blocks of kLagBlock lags
+  int n_ranges, n_long, split;  // set by launch_lag_pairs
   const int2* tiles;        // (row tile, column tile), column >= row
   int n_tiles;
   int tile_row0, tile_col0; // added to every tile entry (block runs)
@@ -90,7 +94,7 @@ struct PackBlockArgs {
 };
 
 hipError_t launch_lag_prep(const LagPrepArgs& a, hipStream_t st);
-hipError_t launch_lag_pairs(bool bf16x3, const LagPairArgs& a, int grid, hipStream_t st);
+hipError_t launch_lag_pairs(bool bf16x3, LagPairArgs a, hipStream_t st);
 hipError_t launch_lag_resolve(const LagResolveArgs& a, int grid, hipStream_t st);
 hipError_t launch_pack_block(const PackBlockArgs& a, hipStream_t st);
 

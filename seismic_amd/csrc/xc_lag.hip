@@ -1,16 +1,19 @@
 // Lag-window form on MFMA (gfx950): the correlation over a bounded window of
-// lags as a lag-blocked dense product.
+// lags as dense products.
 //
-// For pairs (i, j) in a 32 x 32 tile and a block of kLagBlock (16) consecutive lags
-// l = lb + d, the coefficient c_ij(l) = sum_c sum_n xh_ic[n] xh_jc[n - l]
-// (xh = x / (|x| sqrt(C)), linear correlation, zero outside [0, L)) is a
-// 32 x 32 x K product per lag with K running over all samples and channels:
-//   A (32 x 16) = row traces xh_i[n0 .. n0+16)       (held per K step)
-//   B (16 x 32) = column traces xh_j[n0 - l .. )      (a shifted window)
-// on v_mfma_f32_32x32x16_{bf16,f16}.  Each lane loads one 24-element window
-// of its column trace per K step and forms the 16 shifted fragments with
-// v_alignbyte (odd shifts) or plain register selection (even shifts).  The
-// 16 lag accumulators (32 x 32 FP32 each) live in the accumulation registers.
+// The coefficient c_ij(l) = sum_c sum_n xh_ic[n] xh_jc[n - l]
+// (xh = x / (|x| sqrt(C)), linear correlation, zero outside [0, L)) is, with
+// n = k + l, sum_k xh_i[k + l] xh_j[k].  For one row event i, 32 column events j
+// and a block of kLagBlock (32) consecutive lags it is a 32 x 32 x K product
+// with K running over samples and channels:
+//   A (32 x 16): row r = lag lb + lag(r), A[r][k] = xh_i[k + lb + lag(r)] (a
+//                Hankel matrix with its even rows first: lag(r) = 2 (r % 16) + r / 16)
+//   B (16 x 32): column = event j, B[k][j] = xh_j[k]
+// on v_mfma_f32_32x32x16_{bf16,f16}.  A depends on k + lb only, so the A operand
+// of lag block b at step s is that of block b + 1 one step (32 samples)
+// earlier: a wave holds NB blocks' accumulators and a ring of A operands, and a
+// step of NB products needs one new A and one B operand, both loaded as they
+// are used -- no operand is assembled from others.
 //
 // Precision forms
 //   bf16x3: xh = hi + lo with hi = bf16(xh), lo = bf16(xh - hi); the product
@@ -48,9 +51,37 @@ __device__ __forceinline__ float bf16_to_f32(unsigned short h) { return __uint_a
 // ----------------------------------------------------------------------------
 // prep: one workgroup per (event, channel) row
 // ----------------------------------------------------------------------------
+// Column operand of a row: blocked [event / 32][channel][sample / 8][event % 32][8],
+// so the 64 lanes of an operand load read 1 KiB in one piece.
+template <typename Part>
+__device__ __forceinline__ void store_columns(const LagPrepArgs& a, int row, Part&& part) {
+  const int ev = row / a.n_channels, c = row - ev * a.n_channels, n8 = a.l16 / 8;
+  const long long base = ((long long)(ev / 32) * a.n_channels + c) * n8 * 32 + ev % 32;
+  for (int g = threadIdx.x; g < n8; g += 256) {
+    u32x4 hv, lv;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      unsigned short h[2], l[2];
+      part(8 * g + 2 * w, h[0], l[0]);
+      part(8 * g + 2 * w + 1, h[1], l[1]);
+      hv[w] = h[0] | (unsigned)h[1] << 16;
+      lv[w] = l[0] | (unsigned)l[1] << 16;
+    }
+    reinterpret_cast<u32x4*>(a.b_hi)[base + 32ll * g] = hv;
+    if (a.b_lo) reinterpret_cast<u32x4*>(a.b_lo)[base + 32ll * g] = lv;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
   const int row = blockIdx.x;
-  if (row >= a.n_rows) return;
+  if (row == 0 && threadIdx.x == 0) {
+    if (a.zero0) *a.zero0 = 0u;
+    if (a.zero1) *a.zero1 = 0u;
+  }
+  if (row >= a.n_rows) {  // the last column tile's empty events
+    store_columns(a, row, [](int, unsigned short& h, unsigned short& l) { h = l = 0; });
+    return;
+  }
   const float* x = a.in + (long long)row * a.in_stride;
   __shared__ double red[256];
   double s1 = 0.0;
@@ -78,301 +109,423 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
   const double E = red[0];
   if (threadIdx.x == 0) a.norms[row] = sqrt(E);
   const double scale = E > 0.0 ? 1.0 / sqrt(E * (double)a.n_channels) : 0.0;
-  unsigned short* hi = a.hi + (long long)row * a.ls;
-  unsigned short* lo = a.lo ? a.lo + (long long)row * a.ls : nullptr;
-  float* tr = a.traces_out ? a.traces_out + (long long)row * a.L : nullptr;
-  for (int s = threadIdx.x; s < a.ls; s += 256) {
-    const int n = s - a.p0;
+  // sample n of the scaled trace as its 16-bit hi and lo parts
+  auto part = [&](int n, unsigned short& h, unsigned short& l) {
     float v = 0.f;
     if (n >= 0 && n < a.L && n < a.in_len) {
       const float u = a.demean ? (float)((double)x[n] - mean) : x[n];
-      if (tr) tr[n] = u;
       v = (float)((double)u * scale);
-    } else if (tr && n >= 0 && n < a.L) {
-      tr[n] = 0.f;
     }
     if (a.fp16) {
-      hi[s] = __builtin_bit_cast(unsigned short, (_Float16)v);
+      h = __builtin_bit_cast(unsigned short, (_Float16)v);
+      l = 0;
     } else {
-      const unsigned short h = f32_to_bf16_rne(v);
-      hi[s] = h;
-      if (lo) lo[s] = f32_to_bf16_rne(v - bf16_to_f32(h));
+      h = f32_to_bf16_rne(v);
+      l = f32_to_bf16_rne(v - bf16_to_f32(h));
+    }
+  };
+  // row operand: element q of copy 0 is sample q + lag_first, of copy 1 the next
+  unsigned* h0 = reinterpret_cast<unsigned*>(a.h_hi + (long long)row * 2 * a.hs);
+  unsigned* l0 = a.h_lo ? reinterpret_cast<unsigned*>(a.h_lo + (long long)row * 2 * a.hs) : nullptr;
+  for (int q = threadIdx.x; q < a.hs / 2; q += 256) {
+    unsigned short h[3], l[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) part(2 * q + u + a.lag_first, h[u], l[u]);
+    h0[q] = h[0] | (unsigned)h[1] << 16;
+    h0[a.hs / 2 + q] = h[1] | (unsigned)h[2] << 16;
+    if (l0) {
+      l0[q] = l[0] | (unsigned)l[1] << 16;
+      l0[a.hs / 2 + q] = l[1] | (unsigned)l[2] << 16;
+    }
+  }
+  store_columns(a, row, part);
+  if (a.traces_out) {
+    float* tr = a.traces_out + (long long)row * a.L;
+    for (int n = threadIdx.x; n < a.L; n += 256) {
+      const float v = n < a.in_len ? x[n] : 0.f;
+      tr[n] = a.demean && n < a.in_len ? (float)((double)v - mean) : v;
     }
   }
 }
 
 // ----------------------------------------------------------------------------
-// tile kernel: one workgroup (4 waves) per 32 x 32 tile of pairs
+// pair kernel
 // ----------------------------------------------------------------------------
 // MFMA 32x32x16 operand layout: lane l supplies A[l % 32][8*(l/32) + e] and
 // B[8*(l/32) + e][l % 32], e < 8; result register r of lane l holds
 // D[8*(r/4) + 4*(l/32) + r%4][l % 32].
-__device__ __forceinline__ int mfma_row(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+//
+// Lag within a block of register r: the registers' rows 8 (r/4) + 4 h + r%4 hold
+// even lags for r < 8 and the odd ones after them for r >= 8.  Operand loads
+// move 64 bytes per cycle when four neighbouring lanes read one 64-byte piece;
+// with rows in lag order neighbours alternated between the two copies a row
+// operand is stored in (36 instead of about 22 cycles per load: N = 3000,
+// L = 2048, +-20:
+// fp16 2.48 -> 2.05 ms, bf16x3 3.46 -> 2.98).
+__device__ __forceinline__ constexpr int lag_in_block(int h, int r) {
+  return 2 * (8 * ((r & 7) >> 2) + 4 * h + (r & 3)) + (r >> 3);
+}
+// Registers in increasing lag order: order(r) = 2 (r % 8) + r / 8, and back.
+__device__ __forceinline__ constexpr int lag_order(int r) { return 2 * (r & 7) + (r >> 3); }
+__device__ __forceinline__ constexpr int order_lag(int h, int o) { return lag_in_block(h, (o >> 1) + 8 * (o & 1)); }
 
-template <int B, int E, typename F>
-__device__ __forceinline__ void sfor_lag(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    sfor_lag<B + 1, E>(f);
-  }
+// Operand rows go through buffer resources (scalar base and offset, one lane
+// offset, constants as immediates); reads past a row's end return 0.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const unsigned short* base, long long elems) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(2 * elems), 0x00020000);
+}
+__device__ __forceinline__ u32x4 plane_load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
-// One K step's operands for this lane: A (row) 8 samples and the B (column)
-// window of 24 samples, hi and (bf16x3) lo planes.
-struct StepData {
-  u32x4 ah, al;
-  u32x4 bh[3], bl[3];
+// v_med3 on integers (the compiler forms it from four instructions' worth of
+// min and max only when it can see the order of two operands).
+__device__ __forceinline__ int med3_i(int a, int b, int c) {
+  int d;
+  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
+__device__ __forceinline__ unsigned med3_u(unsigned a, unsigned b, unsigned c) {
+  unsigned d;
+  asm("v_med3_u32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
+
+// Running state of a lane's pair on one side, over the lags the lane has seen:
+// the extremum (exact) and the three best keys, largest first, with the lag
+// blocks of the first two.  A key is a value's bits with the low four replaced
+// by 15 - lag_order(r) of its register r, which orders equal values by lag and
+// carries the lag along: inserting is one max and two med3 per value,
+// with the block noted once per 16 values.  The positive side compares bits as
+// signed integers (non-negative floats in order, negative ones below), the
+// negative side as unsigned ones (the most negative first, positive ones
+// last).  A key differs from its value by less than 16 units in the last place,
+// at most kKeySlack for |value| <= 1.
+constexpr float kKeySlack = 2e-6f;
+template <typename T>
+struct Best3 {
+  T e, k1, k2, k3;
+  int b1, b2;
+};
+__device__ __forceinline__ int top(int a, int b) { return a > b ? a : b; }
+__device__ __forceinline__ unsigned top(unsigned a, unsigned b) { return a > b ? a : b; }
+__device__ __forceinline__ int mid(int a, int b, int c) { return med3_i(a, b, c); }
+__device__ __forceinline__ unsigned mid(unsigned a, unsigned b, unsigned c) { return med3_u(a, b, c); }
+
+template <typename T>
+__device__ __forceinline__ void insert16(Best3<T>& s, const T (&bits)[16], const T (&key)[16], int block) {
+  const T o1 = s.k1, o2 = s.k2;
+#pragma unroll
+  for (int r = 0; r < 16; r += 2) s.e = top(top(s.e, bits[r]), bits[r + 1]);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    s.k3 = mid(s.k2, s.k3, key[r]);
+    s.k2 = mid(s.k1, s.k2, key[r]);
+    s.k1 = top(s.k1, key[r]);
+  }
+  const bool c1 = s.k1 != o1;
+  s.b2 = s.k2 == o2 ? s.b2 : ((c1 && s.k2 == o1) ? s.b1 : block);
+  s.b1 = c1 ? block : s.b1;
+}
+
+// A pair's state on one side with the keys in one (signed) order and the lags
+// as offsets from the first: what lanes and waves merge.
+struct Side {
+  int e, k1, k2, k3, o1, o2;
+};
+__device__ __forceinline__ int key_row(int key, int h) { return order_lag(h, 15 - (key & 15)); }
+__device__ __forceinline__ Side side_of(const Best3<int>& s, int h) {
+  return Side{s.e, s.k1, s.k2, s.k3, 32 * s.b1 + key_row(s.k1, h), 32 * s.b2 + key_row(s.k2, h)};
+}
+__device__ __forceinline__ Side side_of(const Best3<unsigned>& s, int h) {
+  constexpr unsigned f = 0x80000000u;  // unsigned order to signed order
+  return Side{(int)(s.e ^ f), (int)(s.k1 ^ f), (int)(s.k2 ^ f), (int)(s.k3 ^ f),
+              32 * s.b1 + key_row((int)s.k1, h), 32 * s.b2 + key_row((int)s.k2, h)};
+}
+// Merge of two lists over disjoint lags; equal first keys go to the smaller lag.
+__device__ __forceinline__ void merge_side(Side& a, const Side& b) {
+  a.e = top(a.e, b.e);
+  const bool tb = b.k1 > a.k1 || (b.k1 == a.k1 && b.o1 < a.o1);
+  // W: the list whose head wins, O: the other
+  const int w1 = tb ? b.k1 : a.k1, w2 = tb ? b.k2 : a.k2, w3 = tb ? b.k3 : a.k3;
+  const int lw1 = tb ? b.o1 : a.o1, lw2 = tb ? b.o2 : a.o2;
+  const int v1 = tb ? a.k1 : b.k1, v2 = tb ? a.k2 : b.k2, lv1 = tb ? a.o1 : b.o1;
+  const bool v_second = v1 > w2;
+  a.k1 = w1;
+  a.o1 = lw1;
+  a.k2 = v_second ? v1 : w2;
+  a.o2 = v_second ? lv1 : lw2;
+  a.k3 = v_second ? top(w2, v2) : top(w3, v1);
+}
+__device__ __forceinline__ Side shfl_side(const Side& s, int mask) {
+  return Side{__shfl_xor(s.e, mask, 64),  __shfl_xor(s.k1, mask, 64), __shfl_xor(s.k2, mask, 64),
+              __shfl_xor(s.k3, mask, 64), __shfl_xor(s.o1, mask, 64), __shfl_xor(s.o2, mask, 64)};
+}
+
+template <bool BF16X3>
+struct Operand {
+  u32x4 hi;
+};
+template <>
+struct Operand<true> {
+  u32x4 hi, lo;
+};
+template <bool BF16X3>
+struct PlaneRows {
+  __amdgpu_buffer_rsrc_t hi, lo;
+  __device__ __forceinline__ Operand<BF16X3> load(int voff, int soff) const {
+    Operand<BF16X3> o;
+    o.hi = plane_load(hi, voff, soff);
+    if constexpr (BF16X3) o.lo = plane_load(lo, voff, soff);
+    return o;
+  }
 };
 
-// One K step's operands from this lane's row (A) and column window (B)
-// bases, `off` elements into the plane row (the step's channel and sample).
-template <bool BF16X3>
-__device__ __forceinline__ void load_step(StepData& s, const unsigned short* __restrict__ ahi,
-                                          const unsigned short* __restrict__ alo,
-                                          const unsigned short* __restrict__ bhi,
-                                          const unsigned short* __restrict__ blo, int off) {
-  s.ah = *reinterpret_cast<const u32x4*>(ahi + off);
-#pragma unroll
-  for (int q = 0; q < 3; ++q) s.bh[q] = *reinterpret_cast<const u32x4*>(bhi + off + 8 * q);
-  if constexpr (BF16X3) {
-    s.al = *reinterpret_cast<const u32x4*>(alo + off);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) s.bl[q] = *reinterpret_cast<const u32x4*>(blo + off + 8 * q);
+// Steps the operands of a range are loaded ahead: a step's products take
+// 32 NI NBX cycles (three times that for bf16x3) and the SIMD's other wave as
+// much, and about 800 cycles cover a load from L2.  RS ring entries and DB
+// column operands (a divisor of RS, so that both are addressed at compile time
+// in a turn of RS steps) give RS - NBX and DB - 1 steps.
+template <bool BF16X3, int NI, int NBX>
+struct Depth {
+  static constexpr int kSteps = 12 / (NI * NBX * (BF16X3 ? 3 : 1));
+  static constexpr int kAhead = kSteps < 2 ? 2 : (kSteps > 6 ? 6 : kSteps);
+  static constexpr int pick() {  // the DB with the shortest ring
+    int best = kAhead + 1;
+    for (int d = kAhead + 1; d <= kAhead + 3; ++d)
+      if (ring(d) < ring(best)) best = d;
+    return best;
   }
-}
+  static constexpr int ring(int d) { return (NBX + kAhead + d - 1) / d * d; }
+  static constexpr int DB = pick(), RS = ring(DB);
+};
 
-// 12 dwords (24 elements) -> the 4 dwords starting at element O (0 <= O <= 16)
-template <int O>
-__device__ __forceinline__ u32x4 window_frag3(const u32x4 (&w)[3]) {
-  auto word = [&](int k) { return w[k >> 2][k & 3]; };
-  u32x4 r;
-  if constexpr ((O & 1) == 0) {
+// The products of NBX lag blocks from block b0 on, for NI row events, into
+// acc[ni * NB + b]: every channel, the 16-sample chunks [t0, t1) in two passes
+// (even, then odd ones): within a pass the lag blocks' A operands are
+// consecutive ring entries.
+template <bool BF16X3, int NI, int NB, int NBX>
+__device__ __forceinline__ void lag_range(f32x16 (&acc)[NI * NB], const PlaneRows<BF16X3> (&rows)[NI],
+                                          const PlaneRows<BF16X3>& cols, int vh, int vb, const LagPairArgs& a, int b0,
+                                          int t0, int t1) {
+  constexpr int DB = Depth<BF16X3, NI, NBX>::DB, RS = Depth<BF16X3, NI, NBX>::RS;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) r[k] = word(O / 2 + k);
-  } else {
+  for (int u = 0; u < NI * NB; ++u) acc[u] = f32x16{};
+  for (int c = 0; c < a.n_channels; ++c)
+    for (int p = 0; p < 2; ++p) {
+      const int t = t0 + ((p - t0) & 1);  // even and odd by the chunk's number: the order does not depend on t0
+      const int steps = (t1 - t + 1) >> 1;
+      int hb = 4 * c * a.hs + 32 * t + 64 * b0;  // bytes: a row is two copies of hs elements
+      int bb = 1024 * (c * (a.l16 / 16) + t);
+      Operand<BF16X3> ring[NI][RS], col[DB];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) r[k] = __builtin_amdgcn_alignbyte(word((O + 1) / 2 + k), word((O - 1) / 2 + k), 2);
-  }
-  return r;
-}
-
-template <bool BF16X3>
-__device__ __forceinline__ void mfma_step(f32x16 (&acc)[kLagBlock], const StepData& s) {
-  // lag lb + d uses window elements 15 - d .. 22 - d
-  auto step = [&](auto dc) {
-    constexpr int d = decltype(dc)::value;
-    const u32x4 b_h = window_frag3<15 - d>(s.bh);
-    if constexpr (BF16X3) {
-      const u32x4 b_l = window_frag3<15 - d>(s.bl);
-      const bf16x8 A_h = __builtin_bit_cast(bf16x8, s.ah), A_l = __builtin_bit_cast(bf16x8, s.al);
-      const bf16x8 B_h = __builtin_bit_cast(bf16x8, b_h), B_l = __builtin_bit_cast(bf16x8, b_l);
-      acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A_l, B_h, acc[d], 0, 0, 0);
-      acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A_h, B_l, acc[d], 0, 0, 0);
-      acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A_h, B_h, acc[d], 0, 0, 0);
-    } else {
-      const f16x8 A_h = __builtin_bit_cast(f16x8, s.ah), B_h = __builtin_bit_cast(f16x8, b_h);
-      acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A_h, B_h, acc[d], 0, 0, 0);
-    }
-  };
-  sfor_lag<0, kLagBlock>(step);
-}
-
-// All K steps (channels x samples) of one block of kLagBlock lags.  Operands
-// are loaded kDepth steps ahead (a ring of kDepth buffers) so one wave per
-// SIMD keeps the MFMA pipe fed: 2 steps for bf16x3 (48 MFMAs per step), 4 for
-// fp16 (16 MFMAs per step, fewer registers per buffer).  The load cursor (the
-// step's element offset in the plane row) advances by additions only: with
-// one wave per SIMD every scalar instruction takes an issue slot from the
-// MFMAs.
-template <bool BF16X3>
-__device__ __forceinline__ void lag_block(f32x16 (&acc)[kLagBlock], const unsigned short* __restrict__ ahi,
-                                          const unsigned short* __restrict__ alo,
-                                          const unsigned short* __restrict__ bhi,
-                                          const unsigned short* __restrict__ blo, int ls,
-                                          int n_channels, int l16, int p0, int lb, int h) {
-  constexpr int kDepth = BF16X3 ? 2 : 4;
+      for (int v = 0; v < DB - 1; ++v) col[v] = cols.load(vb, bb + 2048 * v);
 #pragma unroll
-  for (int d = 0; d < kLagBlock; ++d) acc[d] = f32x16{};
-  const int total = n_channels * (l16 / 16);  // >= 1
-  // lane bases: A at sample 8h of the step, B window 15 + lb samples earlier
-  ahi += p0 + 8 * h;
-  bhi += p0 + 8 * h - lb - 15;
-  if constexpr (BF16X3) {
-    alo += p0 + 8 * h;
-    blo += p0 + 8 * h - lb - 15;
-  }
-  // cursor: element offset of the next step to load, samples of its channel
-  // before it, and steps left before it stops at the last one (loads past
-  // the end repeat that step: harmless and in bounds)
-  int ld_off = 0, ld_n = 0, ld_left = total - 1;
-  auto advance = [&]() {
-    if (ld_left > 0) {
-      --ld_left;
-      ld_n += 16;
-      const bool wrap = ld_n == l16;
-      ld_off += wrap ? ls - l16 + 16 : 16;
-      ld_n = wrap ? 0 : ld_n;
-    }
-  };
-  StepData buf[kDepth];
+      for (int u = 0; u < RS - 1; ++u)
 #pragma unroll
-  for (int q = 0; q < kDepth; ++q) {
-    load_step<BF16X3>(buf[q], ahi, alo, bhi, blo, ld_off);
-    advance();
-  }
-  for (int st = 0; st < total; st += kDepth) {
+        for (int i = 0; i < NI; ++i) ring[i][u] = rows[i].load(vh + 64 * u, hb);
+      for (int s = 0; s < steps; s += RS, hb += 64 * RS, bb += 2048 * RS) {
 #pragma unroll
-    for (int q = 0; q < kDepth; ++q) {
-      if (st + q < total) {
-        mfma_step<BF16X3>(acc, buf[q]);
-        // scheduling: the operand assembly (v_mov, v_alignbyte) spread
-        // evenly between the MFMAs, so the single wave keeps issuing while
-        // its MFMAs run (fp16 4.6% faster, bf16x3 0.3%; same instructions)
+        for (int q = 0; q < RS; ++q) {
+          if (s + q >= steps) break;
+          col[(q + DB - 1) % DB] = cols.load(vb, bb + 2048 * (q + DB - 1));
 #pragma unroll
-        for (int g = 0; g < (BF16X3 ? 48 : 16); ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-          __builtin_amdgcn_sched_group_barrier(0x002, BF16X3 ? 3 : 5, 0);  // then up to this many VALU
+          for (int i = 0; i < NI; ++i) ring[i][(q + RS - 1) % RS] = rows[i].load(vh + 64 * (q + RS - 1), hb);
+          const Operand<BF16X3>& B = col[q % DB];
+          // the three products block by block, so that products into one
+          // accumulator are NI * NBX apart
+          if constexpr (BF16X3) {
+            const bf16x8 b_h = __builtin_bit_cast(bf16x8, B.hi), b_l = __builtin_bit_cast(bf16x8, B.lo);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int b = 0; b < NBX; ++b)
+                acc[i * NB + b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, ring[i][(q + b) % RS].lo), b_h, acc[i * NB + b], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int b = 0; b < NBX; ++b)
+                acc[i * NB + b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, ring[i][(q + b) % RS].hi), b_l, acc[i * NB + b], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int b = 0; b < NBX; ++b)
+                acc[i * NB + b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, ring[i][(q + b) % RS].hi), b_h, acc[i * NB + b], 0, 0, 0);
+          } else {
+            const f16x8 b_h = __builtin_bit_cast(f16x8, B.hi);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int b = 0; b < NBX; ++b)
+                acc[i * NB + b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                    __builtin_bit_cast(f16x8, ring[i][(q + b) % RS].hi), b_h, acc[i * NB + b], 0, 0, 0);
+          }
         }
       }
-      load_step<BF16X3>(buf[q], ahi, alo, bhi, blo, ld_off);
-      advance();
     }
-  }
 }
 
-// Running per-pair state of one wave, in LDS, lane-contiguous so every
-// access is bank-conflict free: [wave][pair r][...][lane].  Per side the three
-// largest values (pos: p1 >= p2 >= p3; neg: n1 <= n2 <= n3) and the lags of
-// the first two as 16-bit offsets from lag_first, packed into one word.
-struct LagState {
-  float v[4][16][6][64];  // p1 p2 p3 n1 n2 n3
-  unsigned l[4][16][2][64];  // (lp1 | lp2 << 16), (ln1 | ln2 << 16) - lag_first
-};
-
-// Merge of two descending top-3 lists (values a/b, lags of the first two) into
-// the top three of their union; ties of the first place go to the smaller lag
-// (the two lists cover disjoint lag blocks).  The negative side calls it with
-// negated values.
-__device__ __forceinline__ void merge_top3(float& a1, float& a2, float& a3, unsigned& la1, unsigned& la2,
-                                           float b1, float b2, float b3, unsigned lb1, unsigned lb2) {
-  const bool take_b = b1 > a1 || (b1 == a1 && lb1 < la1);
-  // W: the list whose head wins, O: the other
-  const float w1 = take_b ? b1 : a1, w2 = take_b ? b2 : a2, w3 = take_b ? b3 : a3;
-  const unsigned lw1 = take_b ? lb1 : la1, lw2 = take_b ? lb2 : la2;
-  const float o1 = take_b ? a1 : b1, o2 = take_b ? a2 : b2;
-  const unsigned lo1 = take_b ? la1 : lb1;
-  const bool o_second = o1 > w2;
-  a1 = w1;
-  la1 = lw1;
-  a2 = o_second ? o1 : w2;
-  la2 = o_second ? lo1 : lw2;
-  a3 = o_second ? fmaxf(w2, o2) : fmaxf(w3, o1);
-}
-
-template <bool BF16X3>
-__global__ __launch_bounds__(256, 1) void k_lag_pairs(LagPairArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int h = lane >> 5;
-  __shared__ LagState st;
-  for (int item = blockIdx.x; item < a.n_tiles; item += gridDim.x) {
-    const int2 t = a.tiles[item];
-    const int i0 = 32 * (t.x + a.tile_row0), j0 = 32 * (t.y + a.tile_col0);
-    if (i0 >= a.n_events || j0 >= a.n_events) continue;  // ragged last block (workgroup-uniform)
-    // this lane's A row and B column (clamped: rows past N compute values that are never stored)
-    const int ia = min(i0 + (lane & 31), a.n_events - 1);
-    const int jb = min(j0 + (lane & 31), a.n_events - 1);
-    const long long rs = (long long)a.n_channels * a.ls;
-    const unsigned short* ahi = a.hi + ia * rs;
-    const unsigned short* alo = BF16X3 ? a.lo + ia * rs : nullptr;
-    const unsigned short* bhi = a.hi + jb * rs;
-    const unsigned short* blo = BF16X3 ? a.lo + jb * rs : nullptr;
-    __syncthreads();  // the previous tile's merge has read the state
+// A range's values into the pair's state, block by block in increasing lag order.
+template <int NI, int NB, int NBX>
+__device__ __forceinline__ void scan_range(f32x16 (&acc)[NI * NB], int ni, Best3<int>& pos, Best3<unsigned>& neg,
+                                           const LagPairArgs& a, int b0, int h) {
+#pragma unroll
+  for (int b = 0; b < NBX; ++b) {
+    f32x16 v = acc[ni * NB + b];
+    if (b == NBX - 1 && b0 + NBX == a.n_blocks) {  // lags beyond the window's last
+      const int last = a.lag_hi - a.lag_first - 32 * (b0 + b);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] = lag_in_block(h, r) <= last ? v[r] : 0.f;
+    }
+    int bits[16], key[16];
+    unsigned ubits[16], ukey[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      st.v[wv][r][0][lane] = 0.f; st.v[wv][r][1][lane] = -3.0e38f; st.v[wv][r][2][lane] = -3.0e38f;
-      st.v[wv][r][3][lane] = 0.f; st.v[wv][r][4][lane] = 3.0e38f; st.v[wv][r][5][lane] = 3.0e38f;
-      st.l[wv][r][0][lane] = 0u; st.l[wv][r][1][lane] = 0u;
+      bits[r] = __float_as_int(v[r]);
+      key[r] = (bits[r] & ~15) | (15 - lag_order(r));
+      ubits[r] = (unsigned)bits[r];
+      ukey[r] = (unsigned)key[r];
     }
-    for (int b = wv; b < a.n_blocks; b += 4) {
-      const int lb = a.lag_first + kLagBlock * b;
-      f32x16 acc[kLagBlock];
-      lag_block<BF16X3>(acc, ahi, alo, bhi, blo, (int)a.ls, a.n_channels, a.l16, a.p0, lb, h);
-      // top-3 values (top-2 lags) per pair over the block's lags, in increasing lag order
+    insert16(pos, bits, key, b0 + b);
+    insert16(neg, ubits, ukey, b0 + b);
+  }
+}
+
+constexpr int kLagWaves = 8;  // per workgroup, two per SIMD
+struct LagMerge {
+  int v[kLagWaves][12][64];
+};
+
+// Bound by the matrix cores at the clock the power limit leaves: 0.82-0.86 busy
+// at 1.6-1.8 GHz, 1.6 PFLOP/s of bf16 and 1.3 of fp16 issued (a 16384-cubed
+// library matmul reaches 1.31 and 1.25 on the same card); deeper or shallower
+// operand rings, one to three steps ahead, change it by less than 1%.  A kernel
+// whose products were 32 x 32 pairs at one lag, with 24-sample column windows
+// shifted into 16 operands per step (3-4 vector instructions per product, one
+// wave per SIMD) and every range run over all samples, took N = 1500, C = 3,
+// L = 2048, +-512 bf16x3 32.0 ms against 25.2 here, N = 2001, L = 4096, +-512 fp16
+// 17.2 against 12.7, and N = 40..491 up to 16 times as long: its unit of work was
+// a whole 32 x 32 tile.
+//
+// One workgroup per (tile of 32 columns, group of rows of the tile's 32).  Its
+// waves take NI consecutive rows each; when a job has too few rows to fill the
+// chip (split > 1), `split` waves share a row's lag ranges and merge in LDS.
+// Ranges are NB or NB - 1 blocks, a.n_long of the former first.
+template <bool BF16X3, int NI, int NB>
+__global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5, r32 = lane & 31;
+  __shared__ LagMerge mg;
+  const int split = a.split, part = wv % split;
+  const int rows_per_wg = kLagWaves / split * NI, groups = 32 / rows_per_wg;
+  const int n_items = a.n_tiles * groups;
+  // lane offsets in bytes: A row r starts lag(r) samples in, at an even element
+  // of the copy of its parity; B column r32 of the chunk's two groups of 8 samples
+  const int vh = 2 * ((r32 >> 4) * a.hs + 8 * h + 2 * (r32 & 15));
+  const int vb = 16 * (32 * h + r32);
+  // XCD-aware walk: XCD blockIdx % 8 takes its own contiguous eighth of the
+  // items, so the tiles of a row of tiles share their rows' operands in its L2
+  const int n_xcd = (gridDim.x % 8 == 0) ? 8 : 1;
+  const int xcd = blockIdx.x % n_xcd, local = blockIdx.x / n_xcd, n_local = gridDim.x / n_xcd;
+  const int seg = (n_items + n_xcd - 1) / n_xcd, seg_end = min(n_items, (xcd + 1) * seg);
+  for (int item = xcd * seg + local; item < seg_end; item += n_local) {
+    const int2 t = a.tiles[item / groups];
+    const int ib = 32 * (t.x + a.tile_row0) + item % groups * rows_per_wg, j0 = 32 * (t.y + a.tile_col0);
+    if (ib >= a.n_events || j0 >= a.n_events) continue;  // ragged last block (workgroup-uniform)
+    const int i0 = ib + wv / split * NI;  // this wave's first row
+    const bool live = i0 < a.n_events;
+    PlaneRows<BF16X3> rows[NI], cols;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float p1 = st.v[wv][r][0][lane], p2 = st.v[wv][r][1][lane], p3 = st.v[wv][r][2][lane];
-        float n1 = st.v[wv][r][3][lane], n2 = st.v[wv][r][4][lane], n3 = st.v[wv][r][5][lane];
-        const unsigned wp = st.l[wv][r][0][lane], wn = st.l[wv][r][1][lane];
-        unsigned lp1 = wp & 0xffffu, lp2 = wp >> 16, ln1 = wn & 0xffffu, ln2 = wn >> 16;
+    for (int i = 0; i < NI; ++i) {
+      const long long o = (long long)min(i0 + i, a.n_events - 1) * a.n_channels * 2 * a.hs;
+      rows[i].hi = plane_rsrc(a.h_hi + o, 2ll * a.n_channels * a.hs);
+      if constexpr (BF16X3) rows[i].lo = plane_rsrc(a.h_lo + o, 2ll * a.n_channels * a.hs);
+    }
+    const long long bo = (long long)(j0 / 32) * a.n_channels * a.l16 * 32;
+    cols.hi = plane_rsrc(a.b_hi + bo, 32ll * a.n_channels * a.l16);
+    if constexpr (BF16X3) cols.lo = plane_rsrc(a.b_lo + bo, 32ll * a.n_channels * a.l16);
+    Best3<int> pos[NI];
+    Best3<unsigned> neg[NI];
 #pragma unroll
-        for (int d = 0; d < kLagBlock; ++d) {
-          const int lag = lb + d;
-          const unsigned off = (unsigned)(kLagBlock * b + d);
-          const bool in = lag >= a.lag_lo && lag <= a.lag_hi;
-          const float v = in ? acc[d][r] : 0.f;
-          const bool gp = v > p1;
-          const bool sp = !gp && v > p2;
-          p3 = (gp || sp) ? p2 : fmaxf(p3, v);
-          p2 = gp ? p1 : (sp ? v : p2);
-          lp2 = gp ? lp1 : (sp ? off : lp2);
-          p1 = gp ? v : p1;
-          lp1 = gp ? off : lp1;
-          const bool gn = v < n1;
-          const bool sn = !gn && v < n2;
-          n3 = (gn || sn) ? n2 : fminf(n3, v);
-          n2 = gn ? n1 : (sn ? v : n2);
-          ln2 = gn ? ln1 : (sn ? off : ln2);
-          n1 = gn ? v : n1;
-          ln1 = gn ? off : ln1;
+    for (int i = 0; i < NI; ++i) {
+      pos[i] = Best3<int>{0, 0, (int)0x80000000, (int)0x80000000, 0, 0};
+      neg[i] = Best3<unsigned>{0x80000000u, 0x80000000u, 0u, 0u, 0, 0};
+    }
+    if (live)
+      for (int rg = part; rg < a.n_ranges; rg += split) {
+        const bool is_long = rg < a.n_long;
+        const int b0 = is_long ? rg * NB : a.n_long * NB + (rg - a.n_long) * (NB - 1);
+        const int nb = is_long ? NB : NB - 1;
+        // samples k with 0 <= k < L and 0 <= k + l < L for some lag l of the range
+        const int l0 = a.lag_first + 32 * b0, l1 = min(l0 + 32 * nb - 1, a.lag_hi);
+        const int t0 = max(0, -l1) >> 4, t1 = (min(a.L, a.L - l0) + 15) >> 4;
+        f32x16 acc[NI * NB];
+        if (is_long) {
+          lag_range<BF16X3, NI, NB, NB>(acc, rows, cols, vh, vb, a, b0, t0, t1);
+#pragma unroll
+          for (int i = 0; i < NI; ++i) scan_range<NI, NB, NB>(acc, i, pos[i], neg[i], a, b0, h);
+        } else if constexpr (NB > 1) {
+          lag_range<BF16X3, NI, NB, NB - 1>(acc, rows, cols, vh, vb, a, b0, t0, t1);
+#pragma unroll
+          for (int i = 0; i < NI; ++i) scan_range<NI, NB, NB - 1>(acc, i, pos[i], neg[i], a, b0, h);
         }
-        st.v[wv][r][0][lane] = p1; st.v[wv][r][1][lane] = p2; st.v[wv][r][2][lane] = p3;
-        st.v[wv][r][3][lane] = n1; st.v[wv][r][4][lane] = n2; st.v[wv][r][5][lane] = n3;
-        st.l[wv][r][0][lane] = lp1 | (lp2 << 16);
-        st.l[wv][r][1][lane] = ln1 | (ln2 << 16);
       }
-    }
-    // merge the 4 waves' states (lag blocks interleave, so ties go to the smaller lag)
-    __syncthreads();
-    if (wv == 0) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float p1 = st.v[0][r][0][lane], p2 = st.v[0][r][1][lane], p3 = st.v[0][r][2][lane];
-        float n1 = -st.v[0][r][3][lane], n2 = -st.v[0][r][4][lane], n3 = -st.v[0][r][5][lane];
-        unsigned lp1 = st.l[0][r][0][lane] & 0xffffu, lp2 = st.l[0][r][0][lane] >> 16;
-        unsigned ln1 = st.l[0][r][1][lane] & 0xffffu, ln2 = st.l[0][r][1][lane] >> 16;
-        for (int w = 1; w < 4; ++w) {
-          const unsigned qp = st.l[w][r][0][lane], qn = st.l[w][r][1][lane];
-          merge_top3(p1, p2, p3, lp1, lp2, st.v[w][r][0][lane], st.v[w][r][1][lane], st.v[w][r][2][lane],
-                     qp & 0xffffu, qp >> 16);
-          merge_top3(n1, n2, n3, ln1, ln2, -st.v[w][r][3][lane], -st.v[w][r][4][lane], -st.v[w][r][5][lane],
-                     qn & 0xffffu, qn >> 16);
-        }
-        n1 = -n1; n2 = -n2; n3 = -n3;
-        const int i = i0 + mfma_row(lane, r);
-        const int j = j0 + (lane & 31);
-        if (i < a.n_events && j < a.n_events && j >= i) {
-          const long long idx = a.out_ld ? (long long)(i - a.out_row0) * a.out_ld + (j - a.out_col0)
-                                         : (long long)i * a.n_events - (long long)i * (i - 1) / 2 + (j - i);
-          const bool kp = p1 > a.threshold && p1 > 0.f;
-          const bool kn = n1 < -a.threshold && n1 < 0.f;
-          const int glp1 = a.lag_first + (int)lp1, gln1 = a.lag_first + (int)ln1;
-          a.vpos[idx] = kp ? p1 : 0.f;
-          a.lpos[idx] = kp ? glp1 : 0;
-          a.vneg[idx] = kn ? n1 : 0.f;
-          a.lneg[idx] = kn ? gln1 : 0;
-          const bool tp = kp && (p1 - p2 < a.tie_tol || p1 < a.tie_tol);
-          const bool tn = kn && (n2 - n1 < a.tie_tol || -n1 < a.tie_tol);
-          // a third lag within the band: every in-window lag is a candidate
-          const bool wp = tp && (p1 - p3 < a.tie_tol || p1 < a.tie_tol);
-          const bool wn = tn && (n3 - n1 < a.tie_tol || -n1 < a.tie_tol);
-          if (tp || tn) {
-            const unsigned slot = atomicAdd(a.tie_count, 1u);
-            if (slot < (unsigned)a.tie_cap) {
-              a.ties[2 * slot] = make_int4(i, j, (tp ? 1 : 0) | (tn ? 2 : 0) | (wp ? 4 : 0) | (wn ? 8 : 0), 0);
-              a.ties[2 * slot + 1] = make_int4(glp1, a.lag_first + (int)lp2, gln1, a.lag_first + (int)ln2);
-            }
+    for (int i = 0; i < NI; ++i) {
+      Side p = side_of(pos[i], h), n = side_of(neg[i], h);
+      merge_side(p, shfl_side(p, 32));
+      merge_side(n, shfl_side(n, 32));
+      if (split > 1) {
+        __syncthreads();  // the previous merge has been read
+        const int w[12] = {p.e, p.k1, p.k2, p.k3, p.o1, p.o2, n.e, n.k1, n.k2, n.k3, n.o1, n.o2};
+#pragma unroll
+        for (int q = 0; q < 12; ++q) mg.v[wv][q][lane] = w[q];
+        __syncthreads();
+        if (part == 0)
+          for (int o = 1; o < split; ++o) {
+            int u[12];
+#pragma unroll
+            for (int q = 0; q < 12; ++q) u[q] = mg.v[wv + o][q][lane];
+            merge_side(p, Side{u[0], u[1], u[2], u[3], u[4], u[5]});
+            merge_side(n, Side{u[6], u[7], u[8], u[9], u[10], u[11]});
           }
+      }
+      const int ii = i0 + i, j = j0 + r32;
+      const bool out = part == 0 && h == 0 && ii < a.n_events && j < a.n_events && j >= ii;
+      // values in float: the negative side's magnitudes
+      auto mag = [](int k) { return -__uint_as_float((unsigned)k ^ 0x80000000u); };
+      const float p1 = __int_as_float(p.e), n1 = -mag(n.e);
+      const bool kp = p1 > a.threshold && p1 > 0.f;
+      const bool kn = n1 < -a.threshold && n1 < 0.f;
+      const int glp1 = a.lag_first + p.o1, gln1 = a.lag_first + n.o1;
+      const float tol = a.tie_tol + 2.f * kKeySlack;
+      const float q1 = __int_as_float(p.k1), m1 = mag(n.k1);
+      // near ties; wide ones (a third lag in the band): every in-window lag is a candidate
+      const bool tp = out && kp && (q1 - __int_as_float(p.k2) < tol || q1 < tol);
+      const bool tn = out && kn && (m1 - mag(n.k2) < tol || m1 < tol);
+      const bool wp = tp && (q1 - __int_as_float(p.k3) < tol || q1 < tol);
+      const bool wn = tn && (m1 - mag(n.k3) < tol || m1 < tol);
+      if (out) {
+        const long long idx = a.out_ld ? (long long)(ii - a.out_row0) * a.out_ld + (j - a.out_col0)
+                                       : (long long)ii * a.n_events - (long long)ii * (ii - 1) / 2 + (j - ii);
+        a.vpos[idx] = kp ? p1 : 0.f;
+        a.lpos[idx] = kp ? glp1 : 0;
+        a.vneg[idx] = kn ? n1 : 0.f;
+        a.lneg[idx] = kn ? gln1 : 0;
+      }
+      const unsigned long long ties = __ballot(tp || tn);  // one counter update per wave
+      if (ties) {
+        unsigned base = 0;
+        if (lane == 0) base = atomicAdd(a.tie_count, (unsigned)__popcll(ties));
+        base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
+        const unsigned slot = base + (unsigned)__popcll(ties & ((1ull << lane) - 1ull));
+        if ((tp || tn) && slot < (unsigned)a.tie_cap) {
+          a.ties[2 * slot] = make_int4(ii, j, (tp ? 1 : 0) | (tn ? 2 : 0) | (wp ? 4 : 0) | (wn ? 8 : 0), 0);
+          a.ties[2 * slot + 1] = make_int4(glp1, a.lag_first + p.o2, gln1, a.lag_first + n.o2);
         }
       }
     }
@@ -598,17 +751,59 @@ __global__ __launch_bounds__(256) void k_pack_block(PackBlockArgs a) {
 // ----------------------------------------------------------------------------
 hipError_t launch_lag_prep(const LagPrepArgs& a, hipStream_t st) {
   if (a.n_rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_lag_prep, dim3(a.n_rows), dim3(256), 0, st, a);
+  const int events = a.n_rows / a.n_channels, rows = (events + 31) / 32 * 32 * a.n_channels;
+  hipLaunchKernelGGL(k_lag_prep, dim3(rows), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
-hipError_t launch_lag_pairs(bool bf16x3, const LagPairArgs& a, int grid, hipStream_t st) {
-  if (a.n_tiles <= 0 || grid <= 0) return hipSuccess;
-  if (bf16x3)
-    hipLaunchKernelGGL(k_lag_pairs<true>, dim3(grid), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL(k_lag_pairs<false>, dim3(grid), dim3(256), 0, st, a);
+template <bool BF16X3, int NI, int NB>
+static hipError_t launch_lag_pairs_k(const LagPairArgs& a, hipStream_t st) {
+  const int items = a.n_tiles * (32 * a.split / (kLagWaves * NI));
+  const int grid = items < (1 << 20) ? (items + 7) / 8 * 8 : 1 << 20;
+  hipLaunchKernelGGL((k_lag_pairs<BF16X3, NI, NB>), dim3(grid), dim3(64 * kLagWaves), 0, st, a);
   return hipGetLastError();
+}
+
+template <bool BF16X3, int NB>
+static hipError_t launch_lag_pairs_nb(int nb, const LagPairArgs& a, hipStream_t st) {
+  if constexpr (NB > 1)
+    if (nb < NB) return launch_lag_pairs_nb<BF16X3, NB - 1>(nb, a, st);
+  // Few blocks make few products per operand load: two rows per wave then share
+  // a column operand, where a job has rows enough (turns of the 256 CUs, a
+  // two-row turn taking about 1.7 of the others').  N = 3000, L = 2048, one
+  // channel, one row per wave -> two: bf16x3 +-10 2.27 -> 1.84 ms, +-20
+  // 2.98 -> 2.64; fp16 +-50 2.68 -> 2.52, +-20 2.05 -> 2.04 (four rows 2.15), +-10
+  // (one block) 1.94 -> 1.98.
+  constexpr int NI = BF16X3 ? (NB <= 3 ? 2 : 1) : (NB >= 2 && NB <= 4 ? 2 : 1);
+  if constexpr (NI > 1) {
+    const long long wgs = 4ll * a.n_tiles;
+    if (a.n_ranges == 1 && 17 * ((wgs / 2 + 255) / 256) <= 10 * ((wgs + 255) / 256))
+      return launch_lag_pairs_k<BF16X3, NI, NB>(a, st);
+  }
+  return launch_lag_pairs_k<BF16X3, 1, NB>(a, st);
+}
+
+hipError_t launch_lag_pairs(bool bf16x3, LagPairArgs a, hipStream_t st) {
+  if (a.n_tiles <= 0) return hipSuccess;
+  // ranges of at most 7 (bf16x3) or 8 blocks (the registers of two waves per
+  // SIMD), as even as possible
+  const int most = bf16x3 ? 7 : 8;
+  a.n_ranges = (a.n_blocks + most - 1) / most;
+  const int nb = (a.n_blocks + a.n_ranges - 1) / a.n_ranges;
+  a.n_long = a.n_blocks - a.n_ranges * (nb - 1);
+  // Waves sharing a row's ranges: a workgroup of 8 takes 8 / split rows, so
+  // the 256 CUs take ceil(4 split tiles / 256) turns of ceil(ranges / split)
+  // ranges each; the split with the fewest (the smallest of equals) is taken.
+  a.split = 1;
+  long long best = 0;
+  for (int sp = 1; sp <= kLagWaves && sp / 2 < a.n_ranges; sp *= 2) {
+    const long long turns = ((long long)a.n_tiles * 4 * sp + 255) / 256 * ((a.n_ranges + sp - 1) / sp);
+    if (sp == 1 || turns < best) {
+      best = turns;
+      a.split = sp;
+    }
+  }
+  return bf16x3 ? launch_lag_pairs_nb<true, 7>(nb, a, st) : launch_lag_pairs_nb<false, 8>(nb, a, st);
 }
 
 hipError_t launch_pack_block(const PackBlockArgs& a, hipStream_t st) {

@@ -6,6 +6,7 @@
 
 #include "../../include/seismic_xcorr.h"
 #include "xc_engine.h"
+#include "xc_lag.h"
 
 #define HIP_CHECK(expr)                                                              \
   do {                                                                               \
@@ -65,8 +66,8 @@ struct sxc_plan {
   int device = 0;
   // lag-window form
   bool lag = false;
-  int l16 = 0, p0 = 0, ls = 0, lag_first = 0, n_blocks = 0, n_tiles = 0;
-  unsigned short *hi = nullptr, *lo = nullptr;
+  int l16 = 0, hs = 0, lag_first = 0, n_blocks = 0, n_tiles = 0;
+  unsigned short *h_hi = nullptr, *h_lo = nullptr, *b_hi = nullptr, *b_lo = nullptr;  // LagPrepArgs
   float* lag_traces = nullptr;
   int2* tiles = nullptr;
   // lag-window forms: near ties with more than two lags in the band go to the
@@ -115,13 +116,15 @@ int fft_plan_group(sxc_plan* p, int g, const float* d_traces, const float* d_rev
 // lag-window forms: planes, norms, FP32 traces, triangle tile list, tie records
 int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out);
 namespace sxc {
+// lag-window forms: the pair kernel's arguments but for tiles and outputs
+LagPairArgs lag_pair_args(const sxc_plan* p);
 // lag-window forms: spectra of the FP32 traces at the plan's period P (when it has one)
 int lag_plan_spectra(sxc_plan* p, hipStream_t st);
-// lag-window forms: FP64 resolution of the wide near ties (the FFT form's resolver);
-// out_ld != 0 writes a dense block as the tiled runs do
-int lag_plan_resolve_wide(sxc_plan* p, float* vp, int* lp, float* vn, int* ln, long long out_ld, int out_row0,
-                          int out_col0, hipStream_t st);
+// lag-window forms: FP64 resolution of the wide near ties (the FFT form's resolver)
+// of up to n_pairs pairs; out_ld != 0 writes a dense block as the tiled runs do
+int lag_plan_resolve_wide(sxc_plan* p, long long n_pairs, float* vp, int* lp, float* vn, int* ln, long long out_ld,
+                          int out_row0, int out_col0, hipStream_t st);
 }  // namespace sxc
-// lag-window forms: FP64 energy, scaled bf16 hi/lo (or fp16) planes and the
-// FP32 copy of every trace
+// lag-window forms: FP64 energy, scaled bf16 hi/lo (or fp16) operands and the
+// FP32 copy of every trace; clears the near-tie counters
 int lag_plan_prep(sxc_plan* p, const float* d_traces, long long trace_stride, int in_len, hipStream_t st);

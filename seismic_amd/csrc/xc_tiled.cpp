@@ -100,18 +100,7 @@ int enqueue_block(sxc_tiled* t, int b) {
   hipStream_t st = t->s_comp;
   HIP_CHECK(launch_fill_u32(p->tie_count, 0u, 1, st));
   if (p->wide_count) HIP_CHECK(launch_fill_u32(p->wide_count, 0u, 1, st));
-  LagPairArgs ka{};
-  ka.hi = p->hi;
-  ka.lo = p->lo;
-  ka.ls = p->ls;
-  ka.n_events = d.n_events;
-  ka.n_channels = d.n_channels;
-  ka.l16 = p->l16;
-  ka.p0 = p->p0;
-  ka.lag_lo = d.lag_lo;
-  ka.lag_hi = d.lag_hi;
-  ka.lag_first = p->lag_first;
-  ka.n_blocks = p->n_blocks;
+  LagPairArgs ka = lag_pair_args(p);
   const bool diag = bk.x == bk.y;
   ka.tiles = diag ? t->d_tiles_diag : t->d_tiles_full;
   ka.n_tiles = diag ? t->n_diag : t->n_full;
@@ -120,16 +109,11 @@ int enqueue_block(sxc_tiled* t, int b) {
   ka.out_ld = t->block;
   ka.out_row0 = row0;
   ka.out_col0 = col0;
-  ka.threshold = d.threshold;
-  ka.tie_tol = p->tie_tol;
   ka.vpos = t->d_vp;
   ka.lpos = t->d_lp;
   ka.vneg = t->d_vn;
   ka.lneg = t->d_ln;
-  ka.ties = p->ties;
-  ka.tie_count = p->tie_count;
-  ka.tie_cap = p->tie_cap;
-  HIP_CHECK(launch_lag_pairs(d.form == SXC_FORM_LAG_BF16X3, ka, ka.n_tiles, st));
+  HIP_CHECK(launch_lag_pairs(d.form == SXC_FORM_LAG_BF16X3, ka, st));
   LagResolveArgs ra{};
   ra.traces = p->lag_traces;
   ra.tr_stride = d.trace_len;
@@ -153,8 +137,9 @@ int enqueue_block(sxc_tiled* t, int b) {
   ra.wide = p->wide;
   ra.wide_count = p->wide_count;
   ra.wide_cap = p->tie_cap;
-  HIP_CHECK(launch_lag_resolve(ra, 8192, st));
-  int rc = lag_plan_resolve_wide(p, t->d_vp, t->d_lp, t->d_vn, t->d_ln, t->block, row0, col0, st);
+  const long long n_pairs = (long long)rows * cols;
+  HIP_CHECK(launch_lag_resolve(ra, resolve_grid(n_pairs), st));
+  int rc = lag_plan_resolve_wide(p, n_pairs, t->d_vp, t->d_lp, t->d_vn, t->d_ln, t->block, row0, col0, st);
   if (rc) return rc;
   HIP_CHECK(hipMemcpyAsync(t->h_ties + slot, p->tie_count, sizeof(unsigned), hipMemcpyDeviceToHost, st));
   // slot reuse: block b - 2's copy out of this slot must be complete

@@ -1,0 +1,40 @@
+"""The lag-window forms over the shapes of their pair kernel: windows of one
+block of 32 lags, one lag fewer and more, one and several ranges of blocks
+(whole and one block short), one-sided windows (whose ranges skip the samples
+no lag of theirs uses), traces of odd lengths down to fewer samples than a
+product takes, jobs small enough that several waves share a row's ranges and
+large enough that a wave takes two rows.  Every pair against FP64 direct sums.
+
+Bars as for the other lag-form tests: coefficients within 1e-5 (bf16x3) and
+2e-3 (fp16), lags equal wherever the FP64 gap of the two best lags is at least
+1e-12 (values above 1e-3)."""
+import numpy as np
+import pytest
+
+from seismic_amd import engine
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {"bf16x3": (engine.FORM_LAG_BF16X3, 1e-5), "fp16": (engine.FORM_LAG_FP16, 2e-3)}
+
+
+@pytest.mark.parametrize("name", ["bf16x3", "fp16"])
+@pytest.mark.parametrize("n,C,L,lo,hi", [
+    (5, 1, 9, -8, 8), (5, 1, 40, -39, 39), (33, 2, 100, -15, 15), (34, 1, 333, 0, 31), (34, 1, 333, 1, 33),
+    (34, 1, 333, -200, -137), (20, 1, 500, -100, -36), (65, 1, 300, 5, 5), (40, 3, 257, -127, 128),
+    (40, 1, 1000, -300, -43), (40, 1, 1000, -128, 128), (70, 2, 640, 100, 639), (40, 1, 900, -899, 899),
+    (97, 1, 513, -223, 224), (600, 1, 130, -7, 8), (600, 1, 130, -20, 20), (600, 2, 131, -40, 50),
+    (600, 1, 130, -60, 60)])
+def test_lag_windows(oracle, name, n, C, L, lo, hi):
+    form, tol = FORMS[name]
+    rng = np.random.default_rng(n + L + hi)
+    x = rng.standard_normal((n, C, L + 2)).astype(np.float32)
+    x = (x[..., 2:] + x[..., 1:-1] + x[..., :-2]) * np.float32(0.5)  # neighbouring lags correlated
+    print(f"case lag window {name} n={n} C={C} L={L} [{lo}, {hi}]", flush=True)
+    vp, lp, vn, ln = engine.allpairs_host(x, 0, lo, hi, form=form)
+    pi, pj = oracle.packed_pairs(n)
+    ref = oracle.pairs_f64(x, pi, pj, lo, hi, circular=False)
+    assert np.abs(vp - ref["pos"]).max() <= tol and np.abs(vn - ref["neg"]).max() <= tol
+    sp = (ref["pos"] > 1e-3) & (ref["gap_pos"] >= 1e-12)
+    sn = (ref["neg"] < -1e-3) & (ref["gap_neg"] >= 1e-12)
+    assert np.array_equal(lp[sp], ref["lag_pos"][sp]) and np.array_equal(ln[sn], ref["lag_neg"][sn])

@@ -109,10 +109,14 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
   const double E = red[0];
   if (threadIdx.x == 0) a.norms[row] = sqrt(E);
   const double scale = E > 0.0 ? 1.0 / sqrt(E * (double)a.n_channels) : 0.0;
+  // A row with a NaN or infinite sample has no coefficients: NaN throughout, so
+  // that every lag of its pairs is NaN whatever samples a range of lags skips,
+  // and the pairs come out as (0, lag 0) as in the FFT form.
+  const float outside = E <= 1.7e308 ? 0.f : __int_as_float(0x7fc00000);
   // sample n of the scaled trace as its 16-bit hi and lo parts
   auto part = [&](int n, unsigned short& h, unsigned short& l) {
-    float v = 0.f;
-    if (n >= 0 && n < a.L && n < a.in_len) {
+    float v = outside;
+    if (outside == 0.f && n >= 0 && n < a.L && n < a.in_len) {
       const float u = a.demean ? (float)((double)x[n] - mean) : x[n];
       v = (float)((double)u * scale);
     }

@@ -38,3 +38,24 @@ def test_lag_windows(oracle, name, n, C, L, lo, hi):
     sp = (ref["pos"] > 1e-3) & (ref["gap_pos"] >= 1e-12)
     sn = (ref["neg"] < -1e-3) & (ref["gap_neg"] >= 1e-12)
     assert np.array_equal(lp[sp], ref["lag_pos"][sp]) and np.array_equal(ln[sn], ref["lag_neg"][sn])
+
+
+@pytest.mark.parametrize("name", ["bf16x3", "fp16", "fft"])
+@pytest.mark.parametrize("lo,hi,at,bad", [(-40, 40, 3, np.nan), (-299, 299, 150, np.nan), (5, 200, 290, np.inf),
+                                          (-250, -30, 0, -np.inf), (-299, 299, 0, -np.nan)])
+def test_nonfinite_rows(oracle, name, lo, hi, at, bad):
+    """A NaN or infinite sample in one channel of one event: that event's pairs
+    are (0, lag 0), whichever lags reach the sample; the other pairs keep their
+    coefficients."""
+    form, tol = FORMS.get(name, (engine.FORM_FFT_F32, 1e-5))
+    n, C, L, e = 40, 2, 300, 17
+    rng = np.random.default_rng(at + abs(hi))
+    x = rng.standard_normal((n, C, L)).astype(np.float32)
+    pi, pj = oracle.packed_pairs(n)
+    ref = oracle.pairs_f64(x, pi, pj, lo, hi, circular=False)
+    x[e, 1, at] = bad
+    print(f"case nonfinite {name} [{lo}, {hi}] at {at}", flush=True)
+    vp, lp, vn, ln = engine.allpairs_host(x, 1024 if name == "fft" else 0, lo, hi, form=form)
+    hit = (pi == e) | (pj == e)
+    assert not vp[hit].any() and not lp[hit].any() and not vn[hit].any() and not ln[hit].any()
+    assert np.abs(vp - ref["pos"])[~hit].max() <= tol and np.abs(vn - ref["neg"])[~hit].max() <= tol

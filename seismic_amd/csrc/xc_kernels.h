@@ -48,6 +48,7 @@ struct PairArgs {
   int n_work;
   int n_rows;             // rectangular mode without a work list: rows
   int chunk;              // columns per work item
+  int n_lds;              // set by launch_pairs: channels of the row held in LDS when not all fit
   int lag_lo, lag_hi;     // scanned lags, inclusive
   float threshold;
   float tie_tol;
@@ -132,11 +133,10 @@ struct HistArgs {
 };
 hipError_t launch_hist_threshold(const HistArgs& a, hipStream_t st);
 
-// twiddle tables (full: 128R + 64, compact: 640 + 8R) + staged row spectra +
-// one transpose buffer per wave
+// compact twiddle tables + staged row spectra + one transpose buffer per wave
 constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
-constexpr size_t pair_lds_bytes(int R, int n_channels, int waves, bool compact = false) {
-  return (size_t)((compact ? 640 + 8 * R : 128 * R + 64) + n_channels * (64 * R + 1) + waves * 576) * 8;
+constexpr size_t pair_lds_bytes(int R, int n_channels, int waves) {
+  return (size_t)(640 + 8 * R + n_channels * (64 * R + 1) + waves * 576) * 8;
 }
 
 // Workgroup shapes of a period in order of preference: W waves, S waves per
@@ -171,13 +171,16 @@ constexpr PairShape pair_shape(int R, int i) {
   return R == 8 ? k8[i] : R == 16 ? k16[i] : R == 24 ? k24[i] : R == 32 ? k32[i] : R == 64 ? k64[i] : k48[i];
 }
 constexpr bool pair_shape_fits(int R, int n_channels, PairShape k) {
-  return (size_t)(4 * k.per_simd / k.waves) * pair_lds_bytes(R, n_channels, k.waves, true) <= kLdsBytes;
+  return (size_t)(4 * k.per_simd / k.waves) * pair_lds_bytes(R, n_channels, k.waves) <= kLdsBytes;
 }
-constexpr PairShape kGlobalRows = {8, 2};  // rows read from global memory: the rest
+// The last shape serves the rest too, with as many channels in LDS as it holds
+// (with all of them read from memory by every wave, the row's spectra doubled
+// the traffic from L2 that bounds such jobs: N = 1500, P = 4096, C = 8 27.6 -> 12.0
+// ms, P = 6144, C = 5 20.0 -> 12.0, P = 8192, C = 4 24.9 -> 14.3, C = 8 56 -> 33).
 inline PairShape pair_shape_for(int R, int n_channels) {
-  for (int i = 0; pair_shape(R, i).waves > 0; ++i)
-    if (pair_shape_fits(R, n_channels, pair_shape(R, i))) return pair_shape(R, i);
-  return kGlobalRows;
+  int i = 0;
+  while (!pair_shape_fits(R, n_channels, pair_shape(R, i)) && pair_shape(R, i + 1).waves > 0) ++i;
+  return pair_shape(R, i);
 }
 
 // Columns per work item: 64 keep one chunk's column spectra in an XCD's L2 over

@@ -292,20 +292,24 @@ __device__ __forceinline__ float2 spec_load(__amdgpu_buffer_rsrc_t r, int voff, 
   return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
 }
 
-template <int R, bool XI_GLOBAL = false, bool CT = false, int kLoadGroup = 32>
-__device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restrict__ xi,
-                                             int xi_stride, const float2* __restrict__ xj,
+// Channels [0, n_lds) of row i are read from xi_lds (stride M + 1), the others from
+// xi in memory (stride xj_stride).
+enum class RowFrom { kLds, kMemory, kBoth };
+template <int R, RowFrom kRow, int kLoadGroup = 32>
+__device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restrict__ xi_lds, int n_lds,
+                                             const float2* __restrict__ xi, const float2* __restrict__ xj,
                                              long long xj_stride, int nch, const float2* tw,
                                              float2* wl, int lane) {
   constexpr int M = 64 * R;
   float yN = 0.f;
   const __amdgpu_buffer_rsrc_t rj = spec_rsrc(xj, xj_stride, nch, M);
-  const __amdgpu_buffer_rsrc_t ri = spec_rsrc(xi, xi_stride, XI_GLOBAL ? nch : 1, M);
+  const __amdgpu_buffer_rsrc_t ri = spec_rsrc(xi, xj_stride, nch, M);
   // channel 0 initialises the accumulators, channels 1.. add to them
-  auto channel = [&](int c, auto first_c) {
+  auto channel = [&](int c, auto first_c, auto memory_c) {
     constexpr bool kFirst = decltype(first_c)::value;
-    const float2* ai = xi + c * xi_stride;
-    const int soff_j = (int)(8 * c * xj_stride), soff_i = 8 * c * xi_stride;
+    constexpr bool XI_GLOBAL = decltype(memory_c)::value;
+    const float2* ai = XI_GLOBAL ? xi + c * xj_stride : xi_lds + c * (M + 1);
+    const int soff_j = (int)(8 * c * xj_stride);
     // per-lane byte offset, redefined per channel (in the loads' block, with
     // a known range) so the bin offsets stay instruction immediates instead
     // of one hoisted offset register per load
@@ -324,7 +328,7 @@ __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restric
       for (int u = 0; u < kGroup; ++u) Bv[u] = spec_load(rj, vb + 512 * (m0 + u), soff_j);
       if constexpr (XI_GLOBAL) {
 #pragma unroll
-        for (int u = 0; u < kGroup; ++u) Av[u] = spec_load(ri, vb + 512 * (m0 + u), soff_i);
+        for (int u = 0; u < kGroup; ++u) Av[u] = spec_load(ri, vb + 512 * (m0 + u), soff_j);
       }
       asm volatile("" ::: "memory");
 #pragma unroll
@@ -351,20 +355,22 @@ __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restric
   // which keeps the SIMD's waves staggered over the phases instead of all
   // waiting on memory or LDS at once (pair kernel 6% faster at P = 4096).
   __builtin_amdgcn_s_setprio(2);
-  channel(0, std::true_type{});
-  for (int c = 1; c < nch; ++c) channel(c, std::false_type{});
+  if constexpr (kRow == RowFrom::kMemory) {
+    channel(0, std::true_type{}, std::true_type{});
+    for (int c = 1; c < nch; ++c) channel(c, std::false_type{}, std::true_type{});
+  } else {
+    channel(0, std::true_type{}, std::false_type{});
+    for (int c = 1; c < (kRow == RowFrom::kLds ? nch : n_lds); ++c) channel(c, std::false_type{}, std::false_type{});
+    if constexpr (kRow == RowFrom::kBoth)
+      for (int c = n_lds; c < nch; ++c) channel(c, std::false_type{}, std::true_type{});
+  }
   __builtin_amdgcn_s_setprio(1);
   // c2r ignores the imaginary parts of the DC and Nyquist bins
   if (lane == 0) y[0].y = 0.f;
 
-  const float2* pre = tw + TwLayout<R>::kPre + lane;
-  const cf u = CT ? f2c(tw[TwLayoutCT<R>::kPreL + lane]) : cmk(0.f, 0.f);
+  const cf u = f2c(tw[TwLayoutCT<R>::kPreL + lane]);
   // exp(+2 pi i (lane + 64 m) / P)
-  auto pre_tw = [&](auto mc) -> cf {
-    constexpr int mm = decltype(mc)::value;
-    if constexpr (CT) return twmul<mm, 2 * R, 1>(u);
-    else return f2c(pre[mm * 64]);
-  };
+  auto pre_tw = [&](auto mc) -> cf { return twmul<decltype(mc)::value, 2 * R, 1>(u); };
   // With E = Y[k] + conj(Y[M-k]), D = Y[k] - conj(Y[M-k]), T = e^{2 pi i k/P}:
   // Z[k] = E + i T D and, as E and D of the mirrored bin are conj(E) and
   // -conj(D) and its factor -conj(T), Z[M-k] = conj(E - i T D).  One lane so
@@ -418,7 +424,7 @@ __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restric
   if (lane == 0) y[HR] = cmk(2.f * y[HR].x, -2.f * y[HR].y);
   wave_lds_fence();  // the FFT's transposes reuse the buffer
   __builtin_amdgcn_s_setprio(0);
-  wave_fft<R, 1, CT>(y, tw, wl, lane);
+  wave_fft<R, 1, true>(y, tw, wl, lane);
 }
 
 // lag of (lane, slot) where slot = 2*reg + {0: x, 1: y}
@@ -597,28 +603,28 @@ __device__ __forceinline__ long long packed_index(int i, int j, int n) {
 // ----------------------------------------------------------------------------
 // pair kernel: one workgroup (kWaves waves) per work item (row i, column chunk)
 // ----------------------------------------------------------------------------
-// XI_LDS: the row spectra of a work item are staged in LDS (shared by the
-// workgroup's waves); otherwise (when they do not fit next to the tables,
-// e.g. P = 8192 with 5 channels) every wave reads them from global memory.
-// CT: compact twiddle tables (9 KB instead of 66 KB at P = 8192, one extra
-// complex multiply per twiddle; fewer LDS reads per pair).
+// The row spectra of a work item are staged in LDS for the workgroup's waves: all
+// of them (kRow = kLds) or, with many channels at a long period, the first
+// a.n_lds, the rest being read from memory by every wave (kBoth).
+// Compact twiddle tables (9 KB instead of 66 KB at P = 8192, one extra complex
+// multiply per twiddle; fewer LDS reads per pair).
 // G: the registers scanned (win_regs).  kPerSimd: waves per SIMD the register
 // budget leaves room for.
-template <int R, int G, int kWaves, int kPerSimd, bool XI_LDS, bool CT>
+template <int R, int G, int kWaves, int kPerSimd, RowFrom kRow>
 __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
   constexpr int M = 64 * R;
-  constexpr int kTab = CT ? TwLayoutCT<R>::kInv : TwLayout<R>::kInv;
+  constexpr int kTab = TwLayoutCT<R>::kInv;
   extern __shared__ __align__(16) float2 smem[];
   const int lane = threadIdx.x & 63;
   // wave index as a scalar: column indices and spectrum addresses then stay
   // in scalar registers (loads use a scalar base and a per-lane offset)
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int xs = XI_LDS ? M + 1 : (int)a.spec_stride;  // row stride of the row spectra
+  const int n_lds = kRow == RowFrom::kLds ? a.n_channels : a.n_lds;
   float2* twl = smem;
   float2* xi_lds = smem + kTab;
-  float2* wl = xi_lds + (XI_LDS ? a.n_channels * xs : 0) + wv * kWaveLds;
+  float2* wl = xi_lds + n_lds * (M + 1) + wv * kWaveLds;
 
-  stage_twiddles<kTab, 64 * kWaves>(twl, a.tw + (CT ? TwLayout<R>::kInv : 0), threadIdx.x);
+  stage_twiddles<kTab, 64 * kWaves>(twl, a.tw + TwLayout<R>::kInv, threadIdx.x);
   WinBits<R, G> wb;
   if constexpr (G > 0) win_bits<R, G>(wb, lane, a.lag_lo, a.lag_hi);
 
@@ -641,20 +647,20 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
     const int je = min((jb / a.chunk + 1) * a.chunk, a.n_events);  // end of jb's column chunk
     const bool dense = a.dense_cols > 0;
     const float2* src = a.spec + (long long)i * a.n_channels * a.spec_stride;
-    if constexpr (XI_LDS) {
+    {
       // a channel's loads are all in flight before its first store
       constexpr int T = 64 * kWaves, kPer = (M + T - 1) / T;
       __syncthreads();
-      for (int c = 0; c < a.n_channels; ++c) {
+      for (int c = 0; c < n_lds; ++c) {
         const float2* sc = src + c * a.spec_stride;
         float2 v[kPer];
 #pragma unroll
         for (int u = 0; u < kPer; ++u) v[u] = sc[min((int)threadIdx.x + u * T, M)];
 #pragma unroll
         for (int u = 0; u < kPer; ++u)
-          if (M % T == 0 || (int)threadIdx.x + u * T < M) xi_lds[c * xs + threadIdx.x + u * T] = v[u];
+          if (M % T == 0 || (int)threadIdx.x + u * T < M) xi_lds[c * (M + 1) + threadIdx.x + u * T] = v[u];
       }
-      if ((int)threadIdx.x < a.n_channels) xi_lds[threadIdx.x * xs + M] = src[threadIdx.x * a.spec_stride + M];
+      if ((int)threadIdx.x < n_lds) xi_lds[threadIdx.x * (M + 1) + M] = src[threadIdx.x * a.spec_stride + M];
       __syncthreads();
     }
 
@@ -663,10 +669,10 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
       cf y[R];
       const float2* xj = cols + (long long)j * a.n_channels * a.spec_stride;
       // smaller load groups where registers are short: the budget of 4 waves
-      // per SIMD (128 VGPRs), and at P >= 6144 rows from global memory (twice
+      // per SIMD (128 VGPRs), and at P >= 6144 channels from memory (twice
       // the loads in flight) and the budget of 3
-      pair_inverse<R, !XI_LDS, CT, (kPerSimd >= 4 || (R >= 48 && (!XI_LDS || kPerSimd == 3))) ? 16 : 32>(
-          y, XI_LDS ? xi_lds : src, xs, xj, a.spec_stride, a.n_channels, twl, wl, lane);
+      pair_inverse<R, kRow, (kPerSimd >= 4 || (R >= 48 && (kRow != RowFrom::kLds || kPerSimd == 3))) ? 16 : 32>(
+          y, xi_lds, n_lds, src, xj, a.spec_stride, a.n_channels, twl, wl, lane);
       if constexpr (G > 0) apply_window<R, G>(y, wb);
       Best pos, neg;
       bool tp, tn;
@@ -779,9 +785,9 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
     wave_lds_fence();
     cf y[R];
     const float2* cols = a.col_spec ? a.col_spec : a.spec;
-    pair_inverse<R, true, true>(y, a.spec + (long long)i * a.n_channels * a.spec_stride, (int)a.spec_stride,
-                          cols + (long long)j * a.n_channels * a.spec_stride, a.spec_stride,
-                          a.n_channels, twl, wl, lane);
+    pair_inverse<R, RowFrom::kMemory>(y, nullptr, 0, a.spec + (long long)i * a.n_channels * a.spec_stride,
+                                      cols + (long long)j * a.n_channels * a.spec_stride, a.spec_stride, a.n_channels, twl,
+                                      wl, lane);
     {
       WinBits<R, 4> wb;
       win_bits<R, 4>(wb, lane, a.lag_lo, a.lag_hi);
@@ -919,42 +925,46 @@ hipError_t launch_forward_r(const ForwardArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int R, int G, int W, int S, bool XI_LDS, bool CT>
+template <int R, int G, int W, int S, RowFrom kRow>
 static hipError_t launch_pairs_rfw(const PairArgs& a, int grid, hipStream_t st) {
-  size_t lds = pair_lds_bytes(R, XI_LDS ? a.n_channels : 0, W, CT);
-  static_assert(TwLayout<R>::kInv == 128 * R + 64, "twiddle layout");
+  const size_t lds = pair_lds_bytes(R, kRow == RowFrom::kLds ? a.n_channels : a.n_lds, W);
   static_assert(TwLayoutCT<R>::kInv == 640 + 8 * R, "compact twiddle layout");
-  hipError_t e = hipFuncSetAttribute((const void*)k_pairs<R, G, W, S, XI_LDS, CT>,
+  hipError_t e = hipFuncSetAttribute((const void*)k_pairs<R, G, W, S, kRow>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_pairs<R, G, W, S, XI_LDS, CT>), dim3(grid), dim3(W * 64), lds, st, a);
+  hipLaunchKernelGGL((k_pairs<R, G, W, S, kRow>), dim3(grid), dim3(W * 64), lds, st, a);
   return hipGetLastError();
 }
 
 // Narrow windows (G = 1, 2) where the build is kept (kNarrow); every window
 // otherwise.
-template <int R, int W, int S, bool XI_LDS, bool CT, bool kNarrow>
+template <int R, int W, int S, RowFrom kRow, bool kNarrow>
 static hipError_t launch_pairs_rw(int groups, const PairArgs& a, int grid, hipStream_t st) {
-  if (groups == 0) return launch_pairs_rfw<R, 0, W, S, XI_LDS, CT>(a, grid, st);
+  if (groups == 0) return launch_pairs_rfw<R, 0, W, S, kRow>(a, grid, st);
   if constexpr (kNarrow) {
-    if (groups == 1) return launch_pairs_rfw<R, 1, W, S, XI_LDS, CT>(a, grid, st);
-    if (groups == 2) return launch_pairs_rfw<R, 2, W, S, XI_LDS, CT>(a, grid, st);
+    if (groups == 1) return launch_pairs_rfw<R, 1, W, S, kRow>(a, grid, st);
+    if (groups == 2) return launch_pairs_rfw<R, 2, W, S, kRow>(a, grid, st);
   }
-  return launch_pairs_rfw<R, 4, W, S, XI_LDS, CT>(a, grid, st);
+  return launch_pairs_rfw<R, 4, W, S, kRow>(a, grid, st);
 }
 
-// Narrow-window builds go with the shapes of up to four channels; rows from
-// global memory when no shape fits.
+// Narrow-window builds go with the shapes of up to four channels;
+// as many channels in LDS as the last shape holds when none holds all.
 template <int R, int I>
 static hipError_t launch_pairs_fit(int groups, const PairArgs& a, int grid, hipStream_t st) {
   constexpr PairShape k = pair_shape(R, I);
   if constexpr (k.waves > 0) {
     constexpr bool kNarrow = I == 0 || !pair_shape_fits(R, 4, pair_shape(R, I - (I > 0)));
     if (pair_shape_fits(R, a.n_channels, k))
-      return launch_pairs_rw<R, k.waves, k.per_simd, true, true, kNarrow>(groups, a, grid, st);
+      return launch_pairs_rw<R, k.waves, k.per_simd, RowFrom::kLds, kNarrow>(groups, a, grid, st);
     return launch_pairs_fit<R, I + 1>(groups, a, grid, st);
-  } else if constexpr (!pair_shape_fits(R, 8, pair_shape(R, I - 1))) {
-    return launch_pairs_rw<R, kGlobalRows.waves, kGlobalRows.per_simd, false, false, false>(groups, a, grid, st);
+  } else {
+    constexpr PairShape last = pair_shape(R, I - 1);
+    if constexpr (!pair_shape_fits(R, 8, last)) {
+      PairArgs b = a;
+      for (b.n_lds = 1; pair_shape_fits(R, b.n_lds + 1, last);) ++b.n_lds;
+      return launch_pairs_rw<R, last.waves, last.per_simd, RowFrom::kBoth, false>(groups, b, grid, st);
+    }
   }
   return hipErrorInvalidValue;  // not reached: the last shape holds 8 channels, a plan's most
 }

@@ -41,7 +41,8 @@ def _windows(P):
 
 @pytest.mark.parametrize("P,C", [(1024, 1), (1024, 3), (1024, 5), (2048, 1), (2048, 2), (2048, 3), (2048, 5),
                                  (3072, 1), (3072, 4), (3072, 7), (4096, 1), (4096, 3), (4096, 6), (4096, 7),
-                                 (4096, 8), (5120, 1), (5120, 2), (6144, 1), (6144, 2), (8192, 1), (8192, 4)])
+                                 (4096, 8), (5120, 1), (5120, 2), (5120, 6), (6144, 1), (6144, 2), (6144, 8), (8192, 1),
+                                 (8192, 4), (8192, 8)])
 def test_windows_at_run_edges(oracle, P, C):
     n, L = 5, P - 200
     ev, _ = synth.make_events(n, C, L, seed=P + C)

@@ -119,7 +119,7 @@ void plan_free(sxc_plan* p) {
   if (!p) return;
   for (hipEvent_t e : p->events) (void)hipEventDestroy(e);
   void* bufs[] = {p->spec, p->col_spec, p->norms, p->traces, p->work, p->ties, p->tie_count,
-                  p->fwd2, p->narrow.fwd2, p->h_hi, p->lag_traces, p->tiles,
+                  p->fwd2, p->narrow.fwd2, p->cut.fwd2, p->h_hi, p->lag_traces, p->tiles,
                   p->fnorms, p->wide, p->wide_count, p->blk_work, p->grp_count};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -250,7 +250,8 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
     p->M = p->P / 2;
     p->R = p->M / 64;
     p->spec_stride = p->M + 32;
-    if ((rc = dev_alloc(&p->spec, (size_t)(rows * p->spec_stride), "spectra"))) return fail(rc);
+    p->spec_elems = (size_t)(rows * p->spec_stride);
+    if ((rc = dev_alloc(&p->spec, p->spec_elems, "spectra"))) return fail(rc);
     if ((rc = dev_alloc(&p->fnorms, (size_t)rows, "norms"))) return fail(rc);
     if ((rc = dev_alloc(&p->wide, (size_t)p->tie_cap, "near-tie records"))) return fail(rc);
     if ((rc = dev_alloc(&p->wide_count, 1, "near-tie counter"))) return fail(rc);
@@ -286,6 +287,8 @@ int sxc::lag_plan_resolve_wide(sxc_plan* p, long long n_pairs, float* vp, int* l
   ResolveArgs ra{};
   ra.spec = p->spec;
   ra.spec_stride = p->spec_stride;
+  ra.n_spec = d.n_channels;
+  ra.period = p->P;
   ra.n_events = d.n_events;
   ra.n_channels = d.n_channels;
   ra.norms = p->fnorms;
@@ -448,7 +451,8 @@ struct HostJob {
 // Device bytes a plan holds (its large buffers; tables and counters aside).
 static size_t plan_device_bytes(const sxc_plan* p) {
   const size_t rows = (size_t)p->d.n_events * p->d.n_channels;
-  size_t b = rows * (size_t)p->spec_stride * sizeof(float2) * ((p->spec ? 1 : 0) + (p->col_spec ? 1 : 0));
+  size_t b = (p->spec ? p->spec_elems : 0) * sizeof(float2);
+  if (p->col_spec) b += rows * (size_t)p->spec_stride * sizeof(float2);
   b += rows * sizeof(double) * ((p->norms ? 1 : 0) + (p->fnorms ? 1 : 0));
   if (p->traces) b += rows * (size_t)p->P * sizeof(float);
   b += (size_t)p->n_work * sizeof(int2) * (p->blk_work ? 2 : 1) +
@@ -743,7 +747,7 @@ static long long triangle_items(long long n, long long chunk) {
 
 // Geometry of an FFT-form plan (no device memory): period, strides, pair and
 // work-item counts, near-tie band and record capacity.
-void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sxc_plan* p) {
+void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bool may_cut, sxc_plan* p) {
   p->d = desc;
   p->P = desc.padded_size;
   p->M = p->P / 2;
@@ -771,8 +775,42 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sx
       p->narrow.spec_stride = P / 2 + 32;
       break;
     }
+  // Windows far shorter than the traces: with the row cut in segments of
+  // P' - (lags) samples, lag l is the sum over segments of a circular
+  // correlation of period P' (each segment of the row against the samples of the
+  // column that its lags reach), so the segments are as many channels to the pair
+  // kernel, which sums their products and runs one transform of P'.  Taken where
+  // the pair kernel's measured time for that is shorter by 5%.
+  // Rows whole at the caller's period -> here: N =
+  // 1500, C = 1, L = 4096, +-50 9.34 -> 1.70 ms, +-512 9.36 -> 2.70, +-1024 9.32 -> 3.89;
+  // L = 2048, +-100 3.67 -> 1.17; C = 3, L = 2500, +-60 7.23 -> 3.21; N = 16, C = 1,
+  // L = 4096, +-50 114 -> 37 us.
+  const int P1 = p->narrow.P ? p->narrow.P : p->P;  // the period of executes on whole rows
+  if (may_cut && desc.trace_len + reach <= p->P) {
+    double best = 0.95 * pair_cost(P1 / 128, desc.n_channels);
+    for (int P : {1024, 2048, 3072, 4096, 5120}) {
+      const int len = P - std::max(0, desc.lag_hi) - std::max(0, -desc.lag_lo);
+      if (P >= P1 || len < 1 || desc.lag_lo <= -P / 2 || desc.lag_hi > P / 2) continue;
+      const int n_seg = (desc.trace_len + len - 1) / len;
+      if (n_seg < 2 || desc.n_channels * n_seg > 8) continue;  // (n_seg < 2: a lag window that no shorter period holds)
+      const double cost = pair_cost(P / 128, desc.n_channels * n_seg);
+      if (cost >= best) continue;
+      best = cost;
+      FftGeom& g = p->cut;
+      g.P = P;
+      g.M = P / 2;
+      g.R = P / 128;
+      g.spec_stride = P / 2 + 32;
+      g.n_seg = n_seg;
+      g.seg_len = len;
+    }
+  }
+  const long long rows = (long long)desc.n_events * desc.n_channels;
+  p->spec_elems = (size_t)rows * std::max(p->spec_stride, 2 * p->cut.n_seg * p->cut.spec_stride);
+  const FftGeom& g = p->cut.P ? p->cut : p->narrow;
   if (!p->chunk)
-    p->chunk = pair_chunk(p->narrow.P ? p->narrow.R : p->R, desc.n_channels, [&](int c) { return triangle_items(desc.n_events, c); });
+    p->chunk = pair_chunk(g.P ? g.R : p->R, desc.n_channels * std::max(1, g.n_seg),
+                          [&](int c) { return triangle_items(desc.n_events, c); });
   p->n_work = (int)triangle_items(desc.n_events, p->chunk);
 }
 
@@ -786,11 +824,11 @@ int sxc_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   if (rc) return rc;
   if (is_lag_form(desc->form)) return lag_plan_create(desc, out);
   sxc_plan* p = new sxc_plan();
-  fft_plan_geometry(*desc, 1LL << 24, p);
+  fft_plan_geometry(*desc, 1LL << 24, true, p);
   HIP_CHECK(hipGetDevice(&p->device));
   const long long rows = (long long)desc->n_events * desc->n_channels;
   auto fail = [&](int code) { plan_free(p); return code; };
-  if ((rc = dev_alloc(&p->spec, (size_t)(rows * p->spec_stride), "spectra"))) return fail(rc);
+  if ((rc = dev_alloc(&p->spec, p->spec_elems, "spectra"))) return fail(rc);
   if ((rc = dev_alloc(&p->norms, (size_t)rows, "norms"))) return fail(rc);
   if (desc->demean && (rc = dev_alloc(&p->traces, (size_t)(rows * p->P), "demeaned traces"))) return fail(rc);
   std::vector<int2> work = build_work(desc->n_events, p->chunk);
@@ -803,8 +841,8 @@ int sxc_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   if ((rc = dev_alloc(&p->ties, (size_t)p->tie_cap, "near-tie records"))) return fail(rc);
   if ((rc = dev_alloc(&p->tie_count, 1, "near-tie counter"))) return fail(rc);
   if ((rc = upload_tables(p->R, &p->fwd2, &p->inv2, &p->post))) return fail(rc);
-  FftGeom& g = p->narrow;
-  if (g.P && (rc = upload_tables(g.R, &g.fwd2, &g.inv2, &g.post))) return fail(rc);
+  for (FftGeom* g : {&p->narrow, &p->cut})
+    if (g->P && (rc = upload_tables(g->R, &g->fwd2, &g->inv2, &g->post))) return fail(rc);
   *out = p;
   return SXC_OK;
 }
@@ -831,6 +869,11 @@ sxc::FftGeom sxc::fft_geom(const sxc_plan* p, int in_len, bool reversed) {
   const int ext = p->d.demean ? std::max(in_len, p->d.trace_len) : in_len;
   const int reach = std::max(std::abs(p->d.lag_lo), std::abs(p->d.lag_hi));
   if (p->narrow.P && ext + reach <= p->narrow.P) g = p->narrow;
+  if (p->cut.P && ext + reach <= p->P && ext > p->cut.seg_len && ext <= p->cut.n_seg * p->cut.seg_len) {
+    g = p->cut;
+    g.n_seg = (ext + g.seg_len - 1) / g.seg_len;
+    return g;
+  }
   // A window over every lag at which two rows can overlap is scanned without
   // masks (N = 1111, C = 2, P = 3072: 1.66 -> 1.56 ms): the other lags hold
   // rounding around an exact 0 (below 5e-7).  Where such a value is the
@@ -847,37 +890,53 @@ namespace {
 using namespace sxc;
 
 // The three stages of an FFT-form execute, asynchronous on st.
-// Forward (and reversed-row) R2C of every row, and the near-tie counter reset.
-int fft_stage_forward(sxc_plan* p, const FftGeom& g, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
-                      hipStream_t st) {
+// Column spectra of an execute with cut rows: after its row spectra.
+float2* seg_cols(const sxc_plan* p, const FftGeom& g) {
+  return p->spec + (long long)p->d.n_events * p->d.n_channels * g.n_seg * g.spec_stride;
+}
+
+// Forward (and reversed-row) R2C of the rows of events [e0, e1); zero: a counter
+// to clear.
+int fft_stage_forward(sxc_plan* p, const FftGeom& g, int e0, int e1, const float* d_traces, const float* d_rev,
+                      long long trace_stride, int in_len, unsigned* zero, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
+  const long long r0 = (long long)e0 * d.n_channels, s0 = r0 * std::max(1, g.n_seg) * g.spec_stride;
+  const long long tr_stride = g.n_seg ? p->P : g.P;
   ForwardArgs fa{};
-  fa.in = d_traces;
+  fa.in = d_traces + r0 * trace_stride;
   fa.in_stride = trace_stride;
   fa.in_len = in_len;
   fa.L = d.trace_len;
-  fa.n_rows = d.n_events * d.n_channels;
+  fa.n_rows = (e1 - e0) * d.n_channels;
   fa.n_channels = d.n_channels;
   fa.demean = d.demean;
-  fa.norms = p->norms;
-  fa.out_traces = p->traces;
-  fa.out_stride = g.P;
-  fa.spec = p->spec;
+  fa.norms = p->norms + r0;
+  fa.out_traces = p->traces ? p->traces + r0 * tr_stride : nullptr;
+  fa.out_stride = tr_stride;
+  fa.spec = p->spec + s0;
   fa.spec_stride = g.spec_stride;
   fa.tw = g.fwd2;
   fa.post_tw = g.post;
-  fa.zero = p->tie_count;
+  fa.zero = zero;
+  if (g.n_seg) {
+    fa.n_seg = g.n_seg;
+    fa.seg_len = g.seg_len;
+    fa.seg_back = std::max(0, d.lag_hi);
+    fa.seg_ahead = std::max(0, -d.lag_lo);
+    fa.seg_cols = seg_cols(p, g) + s0;
+  }
+  if (fa.n_rows <= 0) return SXC_OK;
   HIP_CHECK(launch_forward(g.R, fa, st));
   if (d_rev) {
     ForwardArgs ra = fa;
-    ra.in = d_rev;
+    ra.in = d_rev + r0 * trace_stride;
     ra.demean = 0;
     ra.norms = nullptr;
     ra.out_traces = nullptr;
-    ra.spec = p->col_spec;
+    ra.spec = p->col_spec + s0;
     ra.reversed = 1;
     ra.rev_shift = d.trace_len - 1;
-    ra.norms_in = p->norms;
+    ra.norms_in = p->norms + r0;
     HIP_CHECK(launch_forward(g.R, ra, st));
   }
   return SXC_OK;
@@ -889,10 +948,10 @@ int fft_stage_pairs(sxc_plan* p, const FftGeom& g, bool reversed, const int2* wo
   const sxc_plan_desc& d = p->d;
   PairArgs pa{};
   pa.spec = p->spec;
-  pa.col_spec = reversed ? p->col_spec : nullptr;
+  pa.col_spec = reversed ? p->col_spec : (g.n_seg ? seg_cols(p, g) : nullptr);
   pa.spec_stride = g.spec_stride;
   pa.n_events = d.n_events;
-  pa.n_channels = d.n_channels;
+  pa.n_channels = d.n_channels * std::max(1, g.n_seg);
   pa.work = work;
   pa.n_work = n_work;
   pa.chunk = p->chunk;
@@ -927,14 +986,18 @@ int fft_stage_resolve(sxc_plan* p, const FftGeom& g, const float* d_traces, cons
     ra.rev_stride = trace_stride;
     ra.rev_len = in_len;
     ra.rev_shift = d.trace_len - 1;
+  } else if (g.n_seg) {
+    ra.col_spec = seg_cols(p, g);
   }
+  ra.n_spec = d.n_channels * std::max(1, g.n_seg);
+  ra.period = g.n_seg ? p->P : g.P;  // cut rows are within it (fft_geom)
   ra.n_events = d.n_events;
   ra.n_channels = d.n_channels;
   ra.norms = p->norms;
   if (p->traces) {
     ra.traces = p->traces;
-    ra.tr_stride = g.P;
-    ra.tr_len = g.P;
+    ra.tr_stride = ra.period;
+    ra.tr_len = g.n_seg ? std::max(in_len, d.trace_len) : g.P;
   } else {
     ra.traces = d_traces;
     ra.tr_stride = trace_stride;
@@ -972,7 +1035,7 @@ int sxc::fft_plan_execute(sxc_plan* p, const float* d_traces, const float* d_rev
   const FftGeom g = fft_geom(p, in_len, d_rev != nullptr);
   int rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[0], st));
-  if ((rc = fft_stage_forward(p, g, d_traces, d_rev, trace_stride, in_len, st))) return rc;
+  if ((rc = fft_stage_forward(p, g, 0, p->d.n_events, d_traces, d_rev, trace_stride, in_len, p->tie_count, st))) return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[1], st));
   if ((rc = fft_stage_pairs(p, g, d_rev != nullptr, p->work, p->n_work, d_vals_pos, d_lags_pos, d_vals_neg,
                             d_lags_neg, st)))
@@ -1034,39 +1097,8 @@ int sxc::fft_plan_blocks(sxc_plan* p, int B) {
 // Forward (and reversed-row) R2C of the rows of events [e0, e1).
 int sxc::fft_plan_forward_events(sxc_plan* p, int e0, int e1, const float* d_traces, const float* d_rev,
                                  long long trace_stride, int in_len, hipStream_t st) {
-  const sxc_plan_desc& d = p->d;
-  const FftGeom g = fft_geom(p, in_len, d_rev != nullptr);
-  const long long r0 = (long long)e0 * d.n_channels;
-  ForwardArgs fa{};
-  fa.in = d_traces + r0 * trace_stride;
-  fa.in_stride = trace_stride;
-  fa.in_len = in_len;
-  fa.L = d.trace_len;
-  fa.n_rows = (e1 - e0) * d.n_channels;
-  fa.n_channels = d.n_channels;
-  fa.demean = d.demean;
-  fa.norms = p->norms + r0;
-  fa.out_traces = p->traces ? p->traces + r0 * g.P : nullptr;
-  fa.out_stride = g.P;
-  fa.spec = p->spec + r0 * g.spec_stride;
-  fa.spec_stride = g.spec_stride;
-  fa.tw = g.fwd2;
-  fa.post_tw = g.post;
-  if (fa.n_rows <= 0) return SXC_OK;
-  HIP_CHECK(launch_forward(g.R, fa, st));
-  if (d_rev) {
-    ForwardArgs ra = fa;
-    ra.in = d_rev + r0 * trace_stride;
-    ra.demean = 0;
-    ra.norms = nullptr;
-    ra.out_traces = nullptr;
-    ra.spec = p->col_spec + r0 * g.spec_stride;
-    ra.reversed = 1;
-    ra.rev_shift = d.trace_len - 1;
-    ra.norms_in = p->norms + r0;
-    HIP_CHECK(launch_forward(g.R, ra, st));
-  }
-  return SXC_OK;
+  return fft_stage_forward(p, fft_geom(p, in_len, d_rev != nullptr), e0, e1, d_traces, d_rev, trace_stride, in_len,
+                           nullptr, st);
 }
 
 // Launch group g of a blocked execute: its pairs, then the resolver over the

@@ -33,6 +33,15 @@ struct ForwardArgs {
   int rev_shift;
   const double* norms_in;
   unsigned* zero;         // optional: set to 0 (the near-tie counter of the execute this launch begins)
+  // Segment mode (n_seg > 0): every row gives n_seg row spectra and n_seg
+  // column spectra of the launch's period P.  Segment s is the samples
+  // [s seg_len, (s + 1) seg_len) for the row side and, for the column side, those
+  // and the seg_back before and seg_ahead after them, sample n at element
+  // (n - s seg_len) mod P (seg_len + seg_back + seg_ahead <= P), all with the
+  // whole row's mean and energy.  Row r's spectra: spec and seg_cols, from row
+  // r n_seg on.  out_traces takes the row side's samples.
+  int n_seg, seg_len, seg_back, seg_ahead;
+  float2* seg_cols;
 };
 
 struct PairArgs {
@@ -71,6 +80,8 @@ struct ResolveArgs {
   long long rev_stride;
   int rev_len;
   int rev_shift;
+  int n_spec;             // spectra of an event: n_channels, or as many per segment
+  int period;             // of the FP64 sums: lags are circular mod this
   int n_events;
   int n_channels;
   const double* norms;    // [n_events * n_channels]
@@ -181,6 +192,23 @@ inline PairShape pair_shape_for(int R, int n_channels) {
   int i = 0;
   while (!pair_shape_fits(R, n_channels, pair_shape(R, i)) && pair_shape(R, i + 1).waves > 0) ++i;
   return pair_shape(R, i);
+}
+
+// Measured time of the pair kernel at period 128 R with 1 .. 8 channels (ms,
+// N = 1500; the mean of the full lag range and +-P/5): what the choice between
+// periods compares.
+inline double pair_cost(int R, int n_channels) {
+  struct Row { int R; double ms[8]; };
+  static constexpr Row rows[] = {{8, {0.90, 1.04, 1.26, 1.49, 1.75, 2.15, 2.44, 2.72}},
+                                 {16, {1.56, 1.90, 2.27, 2.66, 3.41, 4.03, 4.64, 5.17}},
+                                 {24, {2.34, 2.81, 3.35, 4.30, 5.20, 6.11, 6.87, 7.73}},
+                                 {32, {3.08, 3.72, 4.72, 5.60, 6.72, 8.40, 9.08, 11.9}},
+                                 {40, {4.26, 5.09, 6.06, 7.25, 8.80, 11.4, 14.4, 17.4}},
+                                 {48, {4.81, 5.97, 7.09, 8.47, 12.0, 15.6, 18.9, 22.5}},
+                                 {64, {7.46, 9.09, 11.2, 14.3, 18.8, 23.7, 28.3, 33.1}}};
+  for (const Row& r : rows)
+    if (r.R == R) return r.ms[n_channels - 1];
+  return 0.0;
 }
 
 // Columns per work item: 64 keep one chunk's column spectra in an XCD's L2 over

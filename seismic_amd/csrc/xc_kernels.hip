@@ -120,6 +120,63 @@ constexpr int fwd_waves() {
   return w > 8 ? 8 : (w < 1 ? 1 : w);
 }
 
+// The row's samples in registers -> its scaled half spectrum in memory.
+template <int R>
+__device__ __forceinline__ void forward_finish(const ForwardArgs& a, cf (&d)[R], float scale, float2* out,
+                                               const float2* twl, float2* wl, float2* zl, int lane) {
+  constexpr int M = 64 * R;
+  constexpr int P = 2 * M;
+  wave_fft<R, -1>(d, twl, wl, lane);
+#pragma unroll
+  for (int r = 0; r < R; ++r) zl[wave_out_index<R>(lane, r)] = c2f(d[r]);
+  wave_lds_fence();
+
+  auto emit = [&](int k, cf X) {
+    if (a.reversed) {
+      // X * exp(+2 pi i q / P), q = k * rev_shift mod P, from the table of
+      // exp(-2 pi i k / P), k <= M: conj(post[q]) for q <= M, post[P - q] above
+      const int q = (int)(((long long)k * a.rev_shift) % P);
+      const cf pq = f2c(a.post_tw[q <= M ? q : P - q]);
+      const cf ph = cmk(pq.x, q <= M ? -pq.y : pq.y);
+      X = cmul(X, ph);
+      X.y = -X.y;  // stored conjugated: the pair kernel conjugates its column operand
+    }
+    if (k == 0 || k == M) X.y = 0.f;
+    out[k] = make_float2(X.x * scale, X.y * scale);
+  };
+  // X[k] = E + O e^{-2 pi i k/P} and, E and O of the mirrored bin being
+  // conjugates, X[M-k] = conj(E - O e^{-2 pi i k/P}), with
+  // E = (Z[k] + conj Z[M-k])/2, O = -i/2 (Z[k] - conj Z[M-k]), Z[M] = Z[0]
+  auto convert = [&](int k, float2 t) {
+    const cf z = f2c(zl[k]);
+    cf zm = f2c(zl[k > 0 ? M - k : 0]);
+    zm.y = -zm.y;
+    const cf e = cmk(0.5f * (z.x + zm.x), 0.5f * (z.y + zm.y));
+    const cf dd = csub(z, zm);
+    const cf od = cmul(cmk(0.5f * dd.y, -0.5f * dd.x), f2c(t));
+    emit(k, cadd(e, od));
+    if (2 * k != M) emit(M - k, cmk(e.x - od.x, od.y - e.y));
+  };
+  // the post-twiddles of the next four steps are requested before the stores of
+  // this four (which the compiler cannot move loads across)
+  constexpr int kStep = 4;
+  static_assert((R / 2) % kStep == 0, "whole steps");
+  float2 tw[kStep];
+#pragma unroll
+  for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[lane + 64 * u];
+#pragma unroll 1
+  for (int k0 = lane; k0 < M / 2; k0 += 64 * kStep) {
+    float2 t[kStep];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) t[u] = tw[u];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[min(k0 + 64 * (kStep + u), M)];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) convert(k0 + 64 * u, t[u]);
+  }
+  if (lane == 0) convert(M / 2, a.post_tw[M / 2]);
+}
+
 template <int R>
 __device__ __forceinline__ void forward_row(const ForwardArgs& a, int row, const float2* twl, float2* wl,
                                             float2* zl, int lane) {
@@ -187,60 +244,77 @@ __device__ __forceinline__ void forward_row(const ForwardArgs& a, int row, const
   if (lane == 0 && !a.reversed) a.norms[row] = sqrt(E);
   const float scale = E > 0.0 ? (float)(1.0 / sqrt(E * (double)a.n_channels * (double)P)) : 0.f;
 
-  wave_fft<R, -1>(d, twl, wl, lane);
-#pragma unroll
-  for (int r = 0; r < R; ++r) zl[wave_out_index<R>(lane, r)] = c2f(d[r]);
-  wave_lds_fence();
-
-  float2* out = a.spec + (long long)row * a.spec_stride;
-  auto emit = [&](int k, cf X) {
-    if (a.reversed) {
-      // X * exp(+2 pi i q / P), q = k * rev_shift mod P, from the table of
-      // exp(-2 pi i k / P), k <= M: conj(post[q]) for q <= M, post[P - q] above
-      const int q = (int)(((long long)k * a.rev_shift) % P);
-      const cf pq = f2c(a.post_tw[q <= M ? q : P - q]);
-      const cf ph = cmk(pq.x, q <= M ? -pq.y : pq.y);
-      X = cmul(X, ph);
-      X.y = -X.y;  // stored conjugated: the pair kernel conjugates its column operand
-    }
-    if (k == 0 || k == M) X.y = 0.f;
-    out[k] = make_float2(X.x * scale, X.y * scale);
-  };
-  // X[k] = E + O e^{-2 pi i k/P} and, E and O of the mirrored bin being
-  // conjugates, X[M-k] = conj(E - O e^{-2 pi i k/P}), with
-  // E = (Z[k] + conj Z[M-k])/2, O = -i/2 (Z[k] - conj Z[M-k]), Z[M] = Z[0]
-  auto convert = [&](int k, float2 t) {
-    const cf z = f2c(zl[k]);
-    cf zm = f2c(zl[k > 0 ? M - k : 0]);
-    zm.y = -zm.y;
-    const cf e = cmk(0.5f * (z.x + zm.x), 0.5f * (z.y + zm.y));
-    const cf dd = csub(z, zm);
-    const cf od = cmul(cmk(0.5f * dd.y, -0.5f * dd.x), f2c(t));
-    emit(k, cadd(e, od));
-    if (2 * k != M) emit(M - k, cmk(e.x - od.x, od.y - e.y));
-  };
-  // the post-twiddles of the next four steps are requested before the stores of
-  // this four (which the compiler cannot move loads across)
-  constexpr int kStep = 4;
-  static_assert((R / 2) % kStep == 0, "whole steps");
-  float2 tw[kStep];
-#pragma unroll
-  for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[lane + 64 * u];
-#pragma unroll 1
-  for (int k0 = lane; k0 < M / 2; k0 += 64 * kStep) {
-    float2 t[kStep];
-#pragma unroll
-    for (int u = 0; u < kStep; ++u) t[u] = tw[u];
-#pragma unroll
-    for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[min(k0 + 64 * (kStep + u), M)];
-#pragma unroll
-    for (int u = 0; u < kStep; ++u) convert(k0 + 64 * u, t[u]);
-  }
-  if (lane == 0) convert(M / 2, a.post_tw[M / 2]);
+  forward_finish<R>(a, d, scale, a.spec + (long long)row * a.spec_stride, twl, wl, zl, lane);
 }
 
-
+// Item v of a segment-mode launch: row v / (2 n_seg), segment v / 2 % n_seg, row
+// side (v even) or column side.  Every wave sums its row's mean and energy
+// itself: a row is at most 8192 samples, which its 2 n_seg waves read from L2,
+// and a launch of its own would cost a small job more.
 template <int R>
+__device__ __forceinline__ void forward_segment(const ForwardArgs& a, int v, const float2* twl, float2* wl,
+                                                float2* zl, int lane) {
+  constexpr int P = 128 * R;
+  wave_lds_fence();  // the previous item's reads of this wave's buffer come first
+  const bool col = v & 1;
+  const int row = (v >> 1) / a.n_seg, seg = (v >> 1) - row * a.n_seg, s0 = seg * a.seg_len;
+  const float* x = a.in + (long long)row * a.in_stride;
+  const int last = a.in_len - 1;
+  constexpr int U = 8;  // 64-sample steps whose loads are in flight together
+  auto sum = [&](auto&& term) {
+    double s = 0.0;
+    for (int n0 = lane; n0 < a.L; n0 += 64 * U) {
+      float u[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) u[k] = x[min(n0 + 64 * k, last)];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int n = n0 + 64 * k;
+        s += n < a.L ? term(n < a.in_len ? u[k] : 0.f) : 0.0;
+      }
+    }
+    return wave_sum_f64(s);
+  };
+  const double mean = a.demean ? sum([](float u) { return (double)u; }) / (double)a.L : 0.0;
+  const double E = sum([&](float u) {
+    const double w = (double)(a.demean ? (float)((double)u - mean) : u);
+    return w * w;
+  });
+  // element m: sample n = s0 + m, or s0 + m - P before the segment (column side)
+  const int end = s0 + a.seg_len + (col ? a.seg_ahead : 0), begin = s0 - (col ? a.seg_back : 0);
+  auto sample = [&](int m) {
+    int n = s0 + m;
+    n -= n >= end ? P : 0;
+    const float u = x[min(max(n, 0), last)], w = n < a.in_len ? u : 0.f;
+    const float z = a.demean && n < a.L ? (float)((double)w - mean) : w;
+    return n >= max(begin, 0) && n < end ? z : 0.f;
+  };
+  cf d[R];
+#pragma unroll
+  for (int m = 0; m < R; ++m) {
+    const int n = 2 * (lane + 64 * m);
+    d[m].x = sample(n);
+    d[m].y = sample(n + 1);
+  }
+  if (!col) {
+    if (a.out_traces) {
+      float* o = a.out_traces + (long long)row * a.out_stride + s0;
+      const int n_out = min(a.seg_len, (int)a.out_stride - s0);
+#pragma unroll
+      for (int m = 0; m < R; ++m) {
+        const int n = 2 * (lane + 64 * m);
+        if (n < n_out) o[n] = d[m].x;
+        if (n + 1 < n_out) o[n + 1] = d[m].y;
+      }
+    }
+    if (lane == 0 && seg == 0) a.norms[row] = sqrt(E);
+  }
+  const float scale = E > 0.0 ? (float)(1.0 / sqrt(E * (double)a.n_channels * (double)P)) : 0.f;
+  float2* out = (col ? a.seg_cols : a.spec) + ((long long)row * a.n_seg + seg) * a.spec_stride;
+  forward_finish<R>(a, d, scale, out, twl, wl, zl, lane);
+}
+
+template <int R, bool SEG>
 __global__ __launch_bounds__(64 * fwd_waves<R>()) void k_forward(ForwardArgs a) {
   constexpr int M = 64 * R;
   constexpr int P = 2 * M;
@@ -254,8 +328,10 @@ __global__ __launch_bounds__(64 * fwd_waves<R>()) void k_forward(ForwardArgs a) 
   if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0u;
   stage_twiddles<TwLayout<R>::kFft, 64 * W>(twl, a.tw, threadIdx.x);
   __syncthreads();
-  for (int row = blockIdx.x * W + wv; row < a.n_rows; row += gridDim.x * W) {
-    forward_row<R>(a, row, twl, wl, zl, lane);
+  const int n = SEG ? a.n_rows * 2 * a.n_seg : a.n_rows;
+  for (int row = blockIdx.x * W + wv; row < n; row += gridDim.x * W) {
+    if constexpr (SEG) forward_segment<R>(a, row, twl, wl, zl, lane);
+    else forward_row<R>(a, row, twl, wl, zl, lane);
   }
 }
 
@@ -758,7 +834,6 @@ __device__ __forceinline__ void corrn_f64(const float* __restrict__ ti, int len_
 template <int R>
 __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
   constexpr int M = 64 * R;
-  constexpr int P = 2 * M;
   extern __shared__ __align__(16) float2 smem[];
   const int lane = threadIdx.x;
   // records [begin, end): tie_begin, when set, holds the count before the
@@ -785,8 +860,8 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
     wave_lds_fence();
     cf y[R];
     const float2* cols = a.col_spec ? a.col_spec : a.spec;
-    pair_inverse<R, RowFrom::kMemory>(y, nullptr, 0, a.spec + (long long)i * a.n_channels * a.spec_stride,
-                                      cols + (long long)j * a.n_channels * a.spec_stride, a.spec_stride, a.n_channels, twl,
+    pair_inverse<R, RowFrom::kMemory>(y, nullptr, 0, a.spec + (long long)i * a.n_spec * a.spec_stride,
+                                      cols + (long long)j * a.n_spec * a.spec_stride, a.spec_stride, a.n_spec, twl,
                                       wl, lane);
     {
       WinBits<R, 4> wb;
@@ -839,8 +914,8 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
         int shift[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          int t = a.rev_traces ? (batch[q] + a.rev_shift) % P : batch[q];
-          shift[q] = t < 0 ? t + P : t;
+          int t = a.rev_traces ? (batch[q] + a.rev_shift) % a.period : batch[q];
+          shift[q] = t < 0 ? t + a.period : t;
         }
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
         for (int c = 0; c < a.n_channels; ++c) {
@@ -852,12 +927,12 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
           // a side's usual two candidates in a two-lag pass
           if (a.rev_traces) {
             const float* rj = a.rev_traces + ((long long)j * a.n_channels + c) * a.rev_stride;
-            if (nb <= 2) corrn_f64<2>(ti, a.tr_len, rj, a.rev_len, P, shift, true, lane, sum);
-            else corrn_f64<4>(ti, a.tr_len, rj, a.rev_len, P, shift, true, lane, sum);
+            if (nb <= 2) corrn_f64<2>(ti, a.tr_len, rj, a.rev_len, a.period, shift, true, lane, sum);
+            else corrn_f64<4>(ti, a.tr_len, rj, a.rev_len, a.period, shift, true, lane, sum);
           } else {
             const float* tj = a.traces + ((long long)j * a.n_channels + c) * a.tr_stride;
-            if (nb <= 2) corrn_f64<2>(ti, a.tr_len, tj, a.tr_len, P, shift, false, lane, sum);
-            else corrn_f64<4>(ti, a.tr_len, tj, a.tr_len, P, shift, false, lane, sum);
+            if (nb <= 2) corrn_f64<2>(ti, a.tr_len, tj, a.tr_len, a.period, shift, false, lane, sum);
+            else corrn_f64<4>(ti, a.tr_len, tj, a.tr_len, a.period, shift, false, lane, sum);
           }
           const double w = ni * nj * (double)a.n_channels;
 #pragma unroll
@@ -918,10 +993,11 @@ hipError_t launch_forward_r(const ForwardArgs& a, hipStream_t st) {
   if (a.n_rows <= 0) return hipSuccess;
   constexpr int W = fwd_waves<R>();
   const size_t lds = (size_t)(TwLayout<R>::kFft + W * fwd_wave_buf<R>()) * sizeof(float2);
-  hipError_t e = hipFuncSetAttribute((const void*)k_forward<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  auto kernel = a.n_seg > 0 ? k_forward<R, true> : k_forward<R, false>;
+  hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  const int groups = (a.n_rows + W - 1) / W;
-  hipLaunchKernelGGL(k_forward<R>, dim3(groups < 1024 ? groups : 1024), dim3(64 * W), lds, st, a);
+  const long long groups = ((long long)a.n_rows * (a.n_seg > 0 ? 2 * a.n_seg : 1) + W - 1) / W;
+  hipLaunchKernelGGL(kernel, dim3(groups < 1024 ? (int)groups : 1024), dim3(64 * W), lds, st, a);
   return hipGetLastError();
 }
 
@@ -948,13 +1024,14 @@ static hipError_t launch_pairs_rw(int groups, const PairArgs& a, int grid, hipSt
   return launch_pairs_rfw<R, 4, W, S, kRow>(a, grid, st);
 }
 
-// Narrow-window builds go with the shapes of up to four channels;
+// Narrow-window builds go with the shapes of up to four channels (eight at the
+// periods that cut rows use, P <= 2048);
 // as many channels in LDS as the last shape holds when none holds all.
 template <int R, int I>
 static hipError_t launch_pairs_fit(int groups, const PairArgs& a, int grid, hipStream_t st) {
   constexpr PairShape k = pair_shape(R, I);
   if constexpr (k.waves > 0) {
-    constexpr bool kNarrow = I == 0 || !pair_shape_fits(R, 4, pair_shape(R, I - (I > 0)));
+    constexpr bool kNarrow = I == 0 || !pair_shape_fits(R, R <= 16 ? 8 : 4, pair_shape(R, I - (I > 0)));
     if (pair_shape_fits(R, a.n_channels, k))
       return launch_pairs_rw<R, k.waves, k.per_simd, RowFrom::kLds, kNarrow>(groups, a, grid, st);
     return launch_pairs_fit<R, I + 1>(groups, a, grid, st);

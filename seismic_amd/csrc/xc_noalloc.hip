@@ -118,14 +118,14 @@ int scratch_for_device(int dev, DeviceScratch** out) {
 
 using namespace sxc;
 
-// chunk: columns per work item, 0: the plan's choice.
-static int execute_noalloc(const sxc_plan_desc* desc, int chunk, const float* d_traces, long long trace_stride,
+// small: rows kept whole and the longest column chunks.
+static int execute_noalloc(const sxc_plan_desc* desc, bool small, const float* d_traces, long long trace_stride,
                            int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg,
                            void* stream) {
   int rc;
   sxc_plan p;
-  p.chunk = chunk;
-  fft_plan_geometry(*desc, kNoallocTieCap, &p);
+  p.chunk = small ? 64 : 0;
+  fft_plan_geometry(*desc, kNoallocTieCap, !small, &p);
   if (in_len < 1 || in_len > p.P || trace_stride < in_len) {
     set_error("in_len %d must be in [1, P=%d] and <= trace_stride %lld", in_len, p.P, trace_stride);
     return SXC_ERR_INVALID;
@@ -141,7 +141,7 @@ static int execute_noalloc(const sxc_plan_desc* desc, int chunk, const float* d_
   const long long rows = (long long)desc->n_events * desc->n_channels;
   size_t off = ds->tables_end;
   const size_t o_spec = off;
-  off = align256(off + (size_t)rows * p.spec_stride * sizeof(float2));
+  off = align256(off + p.spec_elems * sizeof(float2));
   const size_t o_norms = off;
   off = align256(off + (size_t)rows * sizeof(double));
   const size_t o_traces = off;
@@ -152,9 +152,9 @@ static int execute_noalloc(const sxc_plan_desc* desc, int chunk, const float* d_
   off = align256(off + (size_t)p.tie_cap * sizeof(int4));
   const size_t o_count = off;
   off = align256(off + sizeof(unsigned));
-  // a job at the limit keeps the shortest work list
-  if (off > kScratchBytes && p.chunk < 64)
-    return execute_noalloc(desc, 64, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
+  // a job at the limit keeps the fewest spectra and the shortest work list
+  if (off > kScratchBytes && !small)
+    return execute_noalloc(desc, true, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
                            stream);
   if (off > kScratchBytes) {
     set_error("this job needs %zu bytes of workspace; the no-allocation entry point holds at most %zu "
@@ -172,11 +172,12 @@ static int execute_noalloc(const sxc_plan_desc* desc, int chunk, const float* d_
   p.fwd2 = (float2*)(b + ds->tab[p.R].fwd);
   p.inv2 = (float2*)(b + ds->tab[p.R].inv);
   p.post = (float2*)(b + ds->tab[p.R].post);
-  if (p.narrow.P) {
-    p.narrow.fwd2 = (float2*)(b + ds->tab[p.narrow.R].fwd);
-    p.narrow.inv2 = (float2*)(b + ds->tab[p.narrow.R].inv);
-    p.narrow.post = (float2*)(b + ds->tab[p.narrow.R].post);
-  }
+  for (FftGeom* g : {&p.narrow, &p.cut})
+    if (g->P) {
+      g->fwd2 = (float2*)(b + ds->tab[g->R].fwd);
+      g->inv2 = (float2*)(b + ds->tab[g->R].inv);
+      g->post = (float2*)(b + ds->tab[g->R].post);
+    }
   p.device = dev;
   hipStream_t st = (hipStream_t)stream;
   p.last_stream = st;
@@ -207,6 +208,6 @@ extern "C" int sxc_plan_execute_noalloc(const sxc_plan_desc* desc, const float* 
     set_error("the no-allocation entry point runs the FFT form only");
     return SXC_ERR_INVALID;
   }
-  return execute_noalloc(desc, 0, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
+  return execute_noalloc(desc, false, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
                          stream);
 }

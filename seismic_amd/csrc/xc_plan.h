@@ -39,6 +39,7 @@ struct FftGeom {
   long long spec_stride = 0;  // float2 per (event, channel) row
   float2 *fwd2 = nullptr, *inv2 = nullptr, *post = nullptr;
   bool full = false;          // the pair kernel scans every lag unmasked
+  int n_seg = 0, seg_len = 0; // segments of a row (ForwardArgs), 0: whole rows
 };
 }  // namespace sxc
 
@@ -50,11 +51,14 @@ struct sxc_plan {
   // FFT form: the period of executes on traces short enough that it gives the
   // same correlations over the window (fft_geom); P = 0: none below P
   sxc::FftGeom narrow;
+  // FFT form: rows cut in segments at a period shorter still; P = 0: not worth it
+  sxc::FftGeom cut;
   long long n_pairs = 0;
   int n_work = 0, chunk = 0, tie_cap = 0;  // chunk: columns per work item (0: chosen by fft_plan_geometry)
   float tie_tol = 1e-5f;
   // device workspace
-  float2* spec = nullptr;
+  float2* spec = nullptr;      // spec_elems
+  size_t spec_elems = 0;
   float2* col_spec = nullptr;  // reversed-row executes: column spectra (allocated on first use)
   double* norms = nullptr;
   float* traces = nullptr;     // demeaned copy for the FP64 resolver (demean only)
@@ -90,8 +94,9 @@ struct sxc_plan {
 
 void plan_free(sxc_plan* p);
 namespace sxc {
-// FFT form: fills the plan's geometry (no device memory).
-void fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, sxc_plan* p);
+// FFT form: fills the plan's geometry (no device memory); may_cut: with rows cut
+// in segments where that is faster, which takes more memory for spectra.
+void fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bool may_cut, sxc_plan* p);
 // FFT form: the period an execute on rows of in_len samples runs at, and
 // whether it scans every lag.
 FftGeom fft_geom(const sxc_plan* p, int in_len, bool reversed);

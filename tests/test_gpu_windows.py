@@ -9,6 +9,8 @@ matters, against FP64 direct sums.
 
 Bars, as for the other FFT-form tests: coefficients within 1e-5, lags equal
 wherever the FP64 gap of the two best lags is at least 1e-12."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -114,3 +116,53 @@ def test_period_follows_rows_and_window(P, L, in_len, lo, hi, C, demean):
         assert not v[none].any() and not lag[none].any()
         sure = ~none & (gap >= 1e-12)
         assert np.array_equal(lag[sure], lo + np.argmax(sign * c, axis=-1)[sure])
+
+
+@pytest.mark.parametrize("P,L,in_len,lo,hi,C,demean", [
+    (8192, 4096, 4096, -50, 50, 1, False),     # segments of 924 samples at period 1024
+    (8192, 4095, 4095, -50, 50, 1, True),
+    (8192, 4096, 4096, -512, 512, 1, False),   # 1024 samples at 2048
+    (8192, 4096, 4096, -511, 500, 2, True),
+    (8192, 4095, 3000, -50, 50, 1, False),     # rows shorter than L: fewer segments
+    (8192, 4095, 3000, -50, 50, 1, True),      # demeaned up to L, beyond the rows
+    (8192, 4000, 4300, -20, 20, 1, True),      # rows longer than L, still within the segments
+    (8192, 4096, 8192, -50, 50, 1, False),     # rows of P samples: whole rows, wrap at 8192
+    (8192, 4096, 700, -50, 50, 1, False),      # rows of less than one segment
+    (8192, 4000, 4000, 100, 400, 1, False),    # one-sided windows
+    (8192, 4000, 4000, -400, -100, 1, False),
+    (8192, 4000, 4000, -1023, 1024, 1, False),
+    (4096, 2048, 2048, -100, 100, 1, False),
+    (4096, 1999, 1999, -37, 36, 3, True),
+    (4096, 2049, 2049, 0, 1, 2, False),
+    (2048, 1100, 1100, 5, 6, 4, False),
+    (3072, 2900, 2900, -1, 170, 2, False),
+])
+def test_rows_in_segments(P, L, in_len, lo, hi, C, demean):
+    """Windows far shorter than the traces: the rows are cut in segments at a
+    shorter period, whose products are summed before one transform."""
+    test_period_follows_rows_and_window(P, L, in_len, lo, hi, C, demean)
+
+
+@pytest.mark.parametrize("demean", [False, True])
+def test_segments_host_call_and_no_allocation(demean):
+    """A job big enough for event bands, and the entry point without
+    allocations, against the plan's own execute: bitwise equal."""
+    n, C, L, P, lo, hi = 1100, 1, 3001, 8192, -60, 45
+    x, _ = synth.make_events(n, C, L, seed=9)
+    x += np.float32(0.25 * demean)
+    d = DeviceArray.from_numpy(x)
+    plan = engine.AllPairsPlan(n, C, L, P, lo, hi, demean=demean)
+    print(f"case segments host and noalloc demean={demean}", flush=True)
+    out = plan.execute(d)
+    synchronize()
+    want = [o.numpy() for o in out]
+    host = engine.allpairs_host(x, P, lo, hi, demean=demean)
+    for o in out:
+        o.zero_()
+    rc = plan.lib.sxc_plan_execute_noalloc(ctypes.byref(plan.desc), ctypes.c_void_p(d.ptr), L, L,
+                                           *(ctypes.c_void_p(o.ptr) for o in out), ctypes.c_void_p(0))
+    assert rc == 0
+    synchronize()
+    for w, h, o in zip(want, host, out):
+        assert np.array_equal(w, h) and np.array_equal(w, o.numpy())
+    plan.close()

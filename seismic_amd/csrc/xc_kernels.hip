@@ -1089,122 +1089,126 @@ hipError_t launch_copy_f4(float4* dst, const float4* src, long long n, hipStream
   return hipGetLastError();
 }
 
-// One workgroup (256 threads) per (row, column slice): each thread keeps a
-// sorted list of its K best (K >= k, a compile-time capacity) over a strided
-// share of the slice in registers -- a candidate not better than the thread's
-// K-th best is rejected with one comparison -- then wave 0 merges the 256
-// lists with k rounds of a wave-wide argmax.  Order: larger value, then
-// smaller index (idx_in[c] when given, else the column c).  The k winners
-// (value, lag, index) of slice s go to out[(row * slices + s) * k ...];
-// fewer than k candidates pad with (-inf, 0, -1).
+// Top k of a row (or of a slice of its columns), larger value first, then the
+// smaller column -> out[(row * slices + slice) * k ...] as (value, lag, idx_in[c]
+// when given, else the column c), padded with (-inf, 0, -1).
+//
+// A latency chain, so nothing waits on a barrier until the end: every wave walks
+// its own share of the columns, 64 kV at a time in registers (each lane's sorted,
+// so that its best is at hand), with its k best in lanes 0 .. k-1, best first; a
+// round takes the largest of what is left (one DPP reduction over values, one
+// over columns), shifts it into the list and stops at the first that is no better
+// than the k-th.  The first wave then absorbs the others' lists the same way.
+// 4096 columns, k = 10, one row 8.5 us (two launches of 20.7 with a sorted list per
+// thread and k rounds of shuffles before; 16 waves of 4 values and 4 of 16, unsorted
+// and shifted by shuffles, 18.9 and 23.5).
 constexpr int kTopkMax = 32;
-__device__ __forceinline__ bool better(float v, int c, float bv, int bc) {
-  return v > bv || (v == bv && c < bc);
+constexpr int kTopkWaves = 8;
+typedef unsigned long long u64;
+// A candidate: its value's bits in unsigned order (-0 as +0), then ~column; 0: none,
+// which is what a NaN gives.
+__device__ __forceinline__ u64 topk_cand(float v, int c) {
+  const unsigned u = __float_as_uint(v + 0.f);
+  const unsigned key = (u >> 31) ? ~u : u | 0x80000000u;
+  return v != v ? 0ull : (u64)key << 32 | ~(unsigned)c;
 }
-template <int K>
-__global__ __launch_bounds__(256) void k_topk(const float* __restrict__ v, const int* __restrict__ l,
-                                              const int* __restrict__ idx_in, long long row_stride,
-                                              int n_cols, int k, float* out_v, int* out_l, int* out_idx) {
-  __shared__ float cv[256 * K];
-  __shared__ int cc[256 * K];
-  __shared__ int cp[256 * K];
+__device__ __forceinline__ float topk_value(u64 c) {
+  const unsigned key = (unsigned)(c >> 32);
+  return __uint_as_float((key >> 31) ? key & 0x7fffffffu : ~key);
+}
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+#pragma unroll
+  for (int k = 0; k < 6; ++k) v = max(v, (unsigned)dpp_i((int)v, k));
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+// A lane's V candidates in descending order (Batcher's odd-even merge network).
+template <int V>
+__device__ __forceinline__ void topk_sort(u64 (&c)[V]) {
+#pragma unroll
+  for (int p = 1; p < V; p *= 2)
+#pragma unroll
+    for (int q = p; q >= 1; q /= 2)
+#pragma unroll
+      for (int a = 0; a + q < V; ++a)
+        if (a >= q % p && (a - q % p) / q % 2 == 0 && a / (2 * p) == (a + q) / (2 * p)) {
+          const u64 x = c[a], y = c[a + q];
+          c[a] = x > y ? x : y;
+          c[a + q] = x > y ? y : x;
+        }
+}
+// Every lane's candidates (sorted; used up) into the list t.
+template <int V>
+__device__ __forceinline__ void topk_absorb(u64& t, int k, int lane, u64 (&c)[V]) {
+  for (;;) {
+    const unsigned hi = (unsigned)(c[0] >> 32), m = wave_max_u32(hi);
+    if (m == 0u) return;
+    const unsigned w = wave_max_u32(hi == m ? (unsigned)c[0] : 0u);
+    const u64 best = (u64)m << 32 | w;
+    const u64 last = (u64)(unsigned)__builtin_amdgcn_readlane((int)(t >> 32), k - 1) << 32 |
+                     (unsigned)__builtin_amdgcn_readlane((int)t, k - 1);
+    if (best <= last) return;
+    const int rank = __popcll(__ballot(t > best));
+    // the lane before's entry (wave shift right by one)
+    const u64 before = (u64)(unsigned)__builtin_amdgcn_update_dpp(0, (int)(t >> 32), 0x138, 0xF, 0xF, true) << 32 |
+                       (unsigned)__builtin_amdgcn_update_dpp(0, (int)t, 0x138, 0xF, 0xF, true);
+    t = lane == rank ? best : (lane > rank ? before : t);
+    const bool owner = c[0] == best;
+#pragma unroll
+    for (int u = 0; u < V; ++u) c[u] = owner ? (u + 1 < V ? c[u + 1 < V ? u + 1 : u] : 0ull) : c[u];
+  }
+}
+__global__ __launch_bounds__(64 * kTopkWaves) void k_topk(const float* __restrict__ v, const int* __restrict__ l,
+                                                          const int* __restrict__ idx_in, long long row_stride,
+                                                          int n_cols, int k, float* out_v, int* out_l, int* out_idx) {
+  constexpr int kV = 8;
+  __shared__ u64 lists[kTopkWaves * kTopkMax];
   const int row = blockIdx.x, slice = blockIdx.y, n_slices = gridDim.y;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int width = (n_cols + n_slices - 1) / n_slices;
   const int cb = slice * width, ce = min(n_cols, cb + width);
   const long long base = (long long)row * row_stride;
-  const float* rv = v + base;
-  float tv[K];
-  int tc[K], tp[K];
+  u64 t = 0ull;
+  for (int c0 = cb + wv * 64 * kV; c0 < ce; c0 += kTopkWaves * 64 * kV) {
+    float x[kV];
+    u64 c[kV];
 #pragma unroll
-  for (int q = 0; q < K; ++q) { tv[q] = -INFINITY; tc[q] = 0x7fffffff; tp[q] = 0; }
-  // eight loads in flight per thread, then the eight candidates in order
-  constexpr int kBatch = 8;
-  for (int c0 = cb + threadIdx.x; c0 < ce; c0 += 256 * kBatch) {
-    float xb[kBatch];
+    for (int u = 0; u < kV; ++u) x[u] = v[base + min(c0 + 64 * u + lane, ce - 1)];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int c = c0 + 256 * u;
-      xb[u] = c < ce ? rv[c] : -INFINITY;
+    for (int u = 0; u < kV; ++u) {
+      const int col = c0 + 64 * u + lane;
+      c[u] = col < ce ? topk_cand(x[u], col) : 0ull;
     }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int c = c0 + 256 * u;
-      if (c >= ce) continue;
-      float x = xb[u];
-      int xc = idx_in ? idx_in[base + c] : c;
-      int xp = c;
-      if (!better(x, xc, tv[K - 1], tc[K - 1])) continue;
-#pragma unroll
-      for (int q = 0; q < K; ++q) {  // insertion, keeps tv sorted descending
-        if (better(x, xc, tv[q], tc[q])) {
-          const float sv = tv[q];
-          const int sc = tc[q], sp = tp[q];
-          tv[q] = x; tc[q] = xc; tp[q] = xp;
-          x = sv; xc = sc; xp = sp;
-        }
-      }
-    }
+    topk_sort<kV>(c);
+    topk_absorb<kV>(t, k, lane, c);
   }
-#pragma unroll
-  for (int q = 0; q < K; ++q) {
-    cv[threadIdx.x * K + q] = tv[q];
-    cc[threadIdx.x * K + q] = tc[q];
-    cp[threadIdx.x * K + q] = tp[q];
-  }
+  if (lane < kTopkMax) lists[wv * kTopkMax + lane] = t;
   __syncthreads();
-  if (threadIdx.x >= 64) return;
-  const int lane = threadIdx.x;
-  int head[4] = {0, 0, 0, 0};  // next unused candidate of the 4 lists this lane owns
-  for (int r = 0; r < k; ++r) {
-    float bv = -INFINITY;
-    int bc = 0x7fffffff, bp = 0, bl = -1;
+  if (wv != 0) return;
+  constexpr int kL = kTopkWaves * kTopkMax / 64;
+  u64 c[kL];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int t = lane + 64 * u;
-      if (head[u] < K) {
-        const float x = cv[t * K + head[u]];
-        const int xc = cc[t * K + head[u]];
-        if (better(x, xc, bv, bc)) { bv = x; bc = xc; bp = cp[t * K + head[u]]; bl = u; }
-      }
-    }
-    // wave argmax over (bv, bc), carrying the winner's position
-    float wv = bv;
-    int wc = bc, wp = bp;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(wv, o, 64);
-      const int oc = __shfl_xor(wc, o, 64);
-      const int op = __shfl_xor(wp, o, 64);
-      if (better(ov, oc, wv, wc)) { wv = ov; wc = oc; wp = op; }
-    }
-    if (bl >= 0 && bc == wc && bv == wv) head[bl]++;  // the owner advances its list
-    if (lane == 0) {
-      const long long o = ((long long)row * n_slices + slice) * k + r;
-      const bool ok = wc != 0x7fffffff;
-      out_v[o] = ok ? wv : -INFINITY;
-      out_idx[o] = ok ? wc : -1;
-      out_l[o] = ok ? l[base + wp] : 0;
-    }
+  for (int u = 0; u < kL; ++u) {
+    const int e = lane + 64 * u;  // list 0 is this wave's own
+    c[u] = e >= kTopkMax && e % kTopkMax < k ? lists[e] : 0ull;
   }
-}
-
-template <int K>
-static void launch_topk_k(const float* v, const int* l, const int* idx_in, long long row_stride, int n_rows,
-                          int n_slices, int n_cols, int k, float* out_v, int* out_l, int* out_idx,
-                          hipStream_t st) {
-  hipLaunchKernelGGL(k_topk<K>, dim3(n_rows, n_slices), dim3(256), 0, st, v, l, idx_in, row_stride, n_cols, k,
-                     out_v, out_l, out_idx);
+  topk_sort<kL>(c);
+  topk_absorb<kL>(t, k, lane, c);
+  if (lane < k) {
+    const long long o = ((long long)row * n_slices + slice) * k + lane;
+    const bool ok = t != 0ull;
+    const int col = (int)~(unsigned)t;
+    out_v[o] = ok ? topk_value(t) : -INFINITY;
+    out_idx[o] = ok ? (idx_in ? idx_in[base + col] : col) : -1;
+    out_l[o] = ok ? l[base + col] : 0;
+  }
 }
 
 static void launch_topk_any(const float* v, const int* l, const int* idx_in, long long row_stride, int n_rows,
                             int n_slices, int n_cols, int k, float* out_v, int* out_l, int* out_idx,
                             hipStream_t st) {
-  if (k <= 8)
-    launch_topk_k<8>(v, l, idx_in, row_stride, n_rows, n_slices, n_cols, k, out_v, out_l, out_idx, st);
-  else if (k <= 16)
-    launch_topk_k<16>(v, l, idx_in, row_stride, n_rows, n_slices, n_cols, k, out_v, out_l, out_idx, st);
-  else
-    launch_topk_k<32>(v, l, idx_in, row_stride, n_rows, n_slices, n_cols, k, out_v, out_l, out_idx, st);
+  hipLaunchKernelGGL(k_topk, dim3(n_rows, n_slices), dim3(64 * kTopkWaves), 0, st, v, l, idx_in, row_stride, n_cols,
+                     k, out_v, out_l, out_idx);
 }
 
 hipError_t launch_topk(const float* v, const int* l, int n_rows, int n_cols, int k, float* out_v,

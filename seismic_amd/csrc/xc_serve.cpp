@@ -38,7 +38,7 @@
 // n - P, whichever lies in (-P/2, P/2]; a reported lag outside
 // -(Lc-1) .. Lq-1 is moved back by P when the results are assembled
 // (period_for, wrap_lag).  Events of one batch are grouped by P and each group
-// runs its own forward / pair / top-k launches.
+// runs its own forward and pair launches; one top-k launch serves the batch.
 #include <hip/hip_runtime_api.h>
 #include <math.h>
 #include <string.h>
@@ -174,23 +174,21 @@ struct Request {
 
 struct Slot {
   hipStream_t stream = nullptr;
+  int* d_len = nullptr;        // [B], padded (len_bytes); one buffer with
   float* d_traces = nullptr;   // [B][C][Lq]
-  int* d_len = nullptr;        // [B]
   float2* d_spec = nullptr;    // [B][C][Mmax + 32]
   double* d_norms = nullptr;   // [B][C]
   float* d_sv = nullptr;       // [B][ncat] scores
   int* d_sl = nullptr;         // [B][ncat] lags
-  float* d_tv = nullptr;       // [B][k]
-  int* d_tl = nullptr;
-  int* d_ti = nullptr;
+  float* d_tv = nullptr;       // [3][rows of the batch][k]: values, lags, indices
   float* d_kv = nullptr;       // [B][kTopkMaxSlices * k] top-k candidates per column slice
   int* d_kl = nullptr;
   int* d_ki = nullptr;
   unsigned* d_tie = nullptr;
-  float* h_traces = nullptr;   // pinned staging
-  int* h_len = nullptr;
+  int* h_len = nullptr;        // pinned staging, laid out as on the device
+  float* h_traces = nullptr;
   float* h_tv = nullptr;
-  int* h_tl = nullptr;
+  int* h_tl = nullptr;         // into h_tv (run_batch)
   int* h_ti = nullptr;
 };
 
@@ -235,20 +233,22 @@ struct sxc_server {
 namespace {
 
 void slot_free(Slot* s) {
-  void* dev[] = {s->d_traces, s->d_len, s->d_spec, s->d_norms, s->d_sv, s->d_sl,
-                 s->d_tv, s->d_tl, s->d_ti, s->d_kv, s->d_kl, s->d_ki, s->d_tie};
+  void* dev[] = {s->d_len, s->d_spec, s->d_norms, s->d_sv, s->d_sl, s->d_tv, s->d_kv, s->d_kl, s->d_ki, s->d_tie};
   for (void* p : dev)
     if (p) (void)hipFree(p);
-  void* host[] = {s->h_traces, s->h_len, s->h_tv, s->h_tl, s->h_ti};
+  void* host[] = {s->h_len, s->h_tv};
   for (void* p : host)
     if (p) (void)hipHostFree(p);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   *s = Slot{};
 }
 
+// The lengths of a batch, in front of its traces in one buffer.
+size_t len_bytes(const sxc_server_desc& d) { return ((size_t)d.max_batch_events * sizeof(int) + 255) / 256 * 256; }
+
 unsigned long long slot_bytes(const sxc_server_desc& d, long long spec_stride_max) {
   const unsigned long long B = d.max_batch_events, C = d.n_channels;
-  return B * C * (unsigned long long)d.max_query_len * 4 + B * 4 + B * C * spec_stride_max * 8 +
+  return B * C * (unsigned long long)d.max_query_len * 4 + len_bytes(d) + B * C * spec_stride_max * 8 +
          B * C * 8 + B * (unsigned long long)d.n_catalog * 8 + B * d.top_k * 12 +
          B * kTopkMaxSlices * d.top_k * 12 + 64;
 }
@@ -257,24 +257,21 @@ int slot_create(sxc_server* S, Slot* s) {
   const sxc_server_desc& d = S->d;
   const size_t B = d.max_batch_events, C = d.n_channels;
   SRV_CHECK(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
-  SRV_CHECK(hipMalloc((void**)&s->d_traces, B * C * d.max_query_len * sizeof(float)));
-  SRV_CHECK(hipMalloc((void**)&s->d_len, B * sizeof(int)));
+  const size_t in_bytes = len_bytes(d) + B * C * d.max_query_len * sizeof(float);
+  SRV_CHECK(hipMalloc((void**)&s->d_len, in_bytes));
+  s->d_traces = reinterpret_cast<float*>(s->d_len) + len_bytes(d) / sizeof(float);
   SRV_CHECK(hipMalloc((void**)&s->d_spec, B * C * S->spec_stride_max * sizeof(float2)));
   SRV_CHECK(hipMalloc((void**)&s->d_norms, B * C * sizeof(double)));
   SRV_CHECK(hipMalloc((void**)&s->d_sv, B * d.n_catalog * sizeof(float)));
   SRV_CHECK(hipMalloc((void**)&s->d_sl, B * d.n_catalog * sizeof(int)));
-  SRV_CHECK(hipMalloc((void**)&s->d_tv, B * d.top_k * sizeof(float)));
-  SRV_CHECK(hipMalloc((void**)&s->d_tl, B * d.top_k * sizeof(int)));
-  SRV_CHECK(hipMalloc((void**)&s->d_ti, B * d.top_k * sizeof(int)));
+  SRV_CHECK(hipMalloc((void**)&s->d_tv, 3 * B * d.top_k * sizeof(float)));
   SRV_CHECK(hipMalloc((void**)&s->d_kv, B * kTopkMaxSlices * d.top_k * sizeof(float)));
   SRV_CHECK(hipMalloc((void**)&s->d_kl, B * kTopkMaxSlices * d.top_k * sizeof(int)));
   SRV_CHECK(hipMalloc((void**)&s->d_ki, B * kTopkMaxSlices * d.top_k * sizeof(int)));
   SRV_CHECK(hipMalloc((void**)&s->d_tie, sizeof(unsigned)));
-  SRV_CHECK(hipHostMalloc((void**)&s->h_traces, B * C * d.max_query_len * sizeof(float), hipHostMallocDefault));
-  SRV_CHECK(hipHostMalloc((void**)&s->h_len, B * sizeof(int), hipHostMallocDefault));
-  SRV_CHECK(hipHostMalloc((void**)&s->h_tv, B * d.top_k * sizeof(float), hipHostMallocDefault));
-  SRV_CHECK(hipHostMalloc((void**)&s->h_tl, B * d.top_k * sizeof(int), hipHostMallocDefault));
-  SRV_CHECK(hipHostMalloc((void**)&s->h_ti, B * d.top_k * sizeof(int), hipHostMallocDefault));
+  SRV_CHECK(hipHostMalloc((void**)&s->h_len, in_bytes, hipHostMallocDefault));
+  s->h_traces = reinterpret_cast<float*>(s->h_len) + len_bytes(d) / sizeof(float);
+  SRV_CHECK(hipHostMalloc((void**)&s->h_tv, 3 * B * d.top_k * sizeof(float), hipHostMallocDefault));
   return SXC_OK;
 }
 
@@ -286,9 +283,10 @@ int run_batch(sxc_server* S, Slot* s, const std::vector<std::pair<int, int>>& gr
   // groups: (first row, row count) per period; the period is recomputed
   int n_total = 0;
   for (auto& g : groups) n_total = std::max(n_total, g.first + g.second);
-  SRV_CHECK(hipMemcpyAsync(s->d_traces, s->h_traces, (size_t)n_total * C * Lq * sizeof(float),
+  if (n_total == 0) return SXC_OK;
+  // lengths and traces, one copy
+  SRV_CHECK(hipMemcpyAsync(s->d_len, s->h_len, len_bytes(d) + (size_t)n_total * C * Lq * sizeof(float),
                            hipMemcpyHostToDevice, s->stream));
-  SRV_CHECK(hipMemcpyAsync(s->d_len, s->h_len, (size_t)n_total * sizeof(int), hipMemcpyHostToDevice, s->stream));
   for (size_t gi = 0; gi < groups.size(); ++gi) {
     const int first = groups[gi].first, cnt = groups[gi].second;
     if (cnt == 0) continue;
@@ -334,17 +332,18 @@ int run_batch(sxc_server* S, Slot* s, const std::vector<std::pair<int, int>>& gr
     pa.tie_count = s->d_tie;
     pa.tie_cap = 0;  // serving ranks by FP32 values; no FP64 tie records
     SRV_CHECK(launch_pairs(T.R, true, pa, pair_grid(pa.n_work), s->stream));
-    // top-k: a few rows would leave most CUs idle, so each row's columns are
-    // split over slices (about 512 workgroups, at least 2048 columns each)
-    const int slices = std::max(1, std::min({kTopkMaxSlices, (512 + cnt - 1) / cnt, d.n_catalog / 2048}));
-    const size_t kt = (size_t)first * kTopkMaxSlices * d.top_k;
-    SRV_CHECK(launch_topk_split(pa.vpos, pa.lpos, cnt, d.n_catalog, d.top_k, slices, s->d_kv + kt, s->d_kl + kt,
-                                s->d_ki + kt, s->d_tv + (size_t)first * d.top_k,
-                                s->d_tl + (size_t)first * d.top_k, s->d_ti + (size_t)first * d.top_k, s->stream));
   }
-  SRV_CHECK(hipMemcpyAsync(s->h_tv, s->d_tv, (size_t)n_total * d.top_k * sizeof(float), hipMemcpyDeviceToHost, s->stream));
-  SRV_CHECK(hipMemcpyAsync(s->h_tl, s->d_tl, (size_t)n_total * d.top_k * sizeof(int), hipMemcpyDeviceToHost, s->stream));
-  SRV_CHECK(hipMemcpyAsync(s->h_ti, s->d_ti, (size_t)n_total * d.top_k * sizeof(int), hipMemcpyDeviceToHost, s->stream));
+  // top-k of every row at once; a few rows of a large catalog would leave most
+  // CUs idle, so their columns are split over slices (about 512 workgroups, at
+  // least 16384 columns each)
+  const int slices = std::max(1, std::min({kTopkMaxSlices, (512 + n_total - 1) / n_total, d.n_catalog / 16384}));
+  const size_t nk = (size_t)n_total * d.top_k;
+  int* d_out = reinterpret_cast<int*>(s->d_tv);  // values, lags and indices of the batch, one copy
+  SRV_CHECK(launch_topk_split(s->d_sv, s->d_sl, n_total, d.n_catalog, d.top_k, slices, s->d_kv, s->d_kl, s->d_ki,
+                              s->d_tv, d_out + nk, d_out + 2 * nk, s->stream));
+  SRV_CHECK(hipMemcpyAsync(s->h_tv, s->d_tv, 3 * nk * sizeof(float), hipMemcpyDeviceToHost, s->stream));
+  s->h_tl = reinterpret_cast<int*>(s->h_tv) + nk;
+  s->h_ti = s->h_tl + nk;
   SRV_CHECK(hipStreamSynchronize(s->stream));
   return SXC_OK;
 }

@@ -589,8 +589,13 @@ static int prepare_execute_reversed(sxc_plan* p, const float* d_traces, const fl
 // pairs of column band b - 1 compute, and once the last band is in, row band
 // a's outputs are copied out while row band a + 1 completes.  Only the first
 // band's input copy and the last row band's output copy are not hidden.
-static constexpr int kBands = 8;
 static constexpr int kBandMinEvents = 1024;
+// More bands hide more of the copies, but each is two launch groups of serial,
+// partly filled kernels (15 groups of 125 us pairs and 26 us resolver at N = 1024).
+// Drop-in call with 8 bands -> these: N = 1024, L = 2048 5.16 -> 4.77 ms, L = 1000 2.51
+// -> 2.05, N = 1400 6.35 -> 5.15 (4 bands 5.45), N = 2048 15.5 -> 15.0 (3 bands the
+// same); N = 4096 25.8-26.3 with 4 as with 8.
+static int band_count(int n_events) { return n_events < 2048 ? 3 : (n_events < 4096 ? 4 : 8); }
 
 // SEISMIC_XCORR_BLOCKED=0 runs every host-buffer call unblocked (read per call).
 static bool blocking_enabled() {
@@ -606,10 +611,11 @@ static int run_blocked(HostJob* j, const float* traces, const float* reversed, l
                        const HistArgs* hist = nullptr) {
   sxc_plan* p = j->p;
   int rc;
-  if ((rc = fft_plan_blocks(p, kBands))) return rc;
+  const int n_bands = band_count(p->d.n_events);
+  if ((rc = fft_plan_blocks(p, n_bands))) return rc;
   if (!j->cs) HIP_CHECK(hipStreamCreateWithFlags(&j->cs, hipStreamNonBlocking));
   if (!j->xs) HIP_CHECK(hipStreamCreateWithFlags(&j->xs, hipStreamNonBlocking));
-  while ((int)j->band_ev.size() < 2 * kBands) {
+  while ((int)j->band_ev.size() < 2 * n_bands) {
     hipEvent_t e;
     HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     j->band_ev.push_back(e);
@@ -618,7 +624,7 @@ static int run_blocked(HostJob* j, const float* traces, const float* reversed, l
   const float* d_rev = reversed ? j->rev : nullptr;
   const int C = p->d.n_channels;
   HIP_CHECK(launch_fill_u32(p->tie_count, 0u, 1, j->cs));
-  for (int b = 0; b < kBands; ++b) {
+  for (int b = 0; b < n_bands; ++b) {
     // event band b in (copy stream), then its transforms and pairs (compute stream)
     const int e0 = p->band_ev[b], e1 = p->band_ev[b + 1];
     const size_t off = (size_t)e0 * C * trace_stride, cnt = (size_t)(e1 - e0) * C * trace_stride;
@@ -629,11 +635,11 @@ static int run_blocked(HostJob* j, const float* traces, const float* reversed, l
     HIP_CHECK(hipEventRecord(j->band_ev[b], j->xs));
     HIP_CHECK(hipStreamWaitEvent(j->cs, j->band_ev[b], 0));
     if ((rc = fft_plan_forward_events(p, e0, e1, j->in, d_rev, trace_stride, in_len, j->cs))) break;
-    if (b < kBands - 1) {
+    if (b < n_bands - 1) {
       rc = fft_plan_group(p, b, j->in, d_rev, trace_stride, in_len, j->vp, j->lp, j->vn, j->ln, j->cs);
     } else {
-      for (int a = 0; a < kBands && !rc; ++a) {
-        rc = fft_plan_group(p, kBands - 1 + a, j->in, d_rev, trace_stride, in_len, j->vp, j->lp, j->vn, j->ln,
+      for (int a = 0; a < n_bands && !rc; ++a) {
+        rc = fft_plan_group(p, n_bands - 1 + a, j->in, d_rev, trace_stride, in_len, j->vp, j->lp, j->vn, j->ln,
                             j->cs);
         if (!rc && hist) {
           const long long n = p->d.n_events, r0 = p->band_ev[a], r1 = p->band_ev[a + 1];
@@ -646,16 +652,16 @@ static int run_blocked(HostJob* j, const float* traces, const float* reversed, l
           ha.n = c;
           HIP_CHECK(launch_hist_threshold(ha, j->cs));
         }
-        if (!rc) HIP_CHECK(hipEventRecord(j->band_ev[kBands + a], j->cs));
+        if (!rc) HIP_CHECK(hipEventRecord(j->band_ev[n_bands + a], j->cs));
       }
     }
     if (rc) break;
   }
   const long long n = p->d.n_events;
   auto packed = [n](long long r) { return r * n - r * (r - 1) / 2; };  // first index of row r
-  for (int a = 0; a < kBands && !rc; ++a) {
+  for (int a = 0; a < n_bands && !rc; ++a) {
     const size_t o = (size_t)packed(p->band_ev[a]), c = (size_t)packed(p->band_ev[a + 1]) - o;
-    HIP_CHECK(hipStreamWaitEvent(j->xs, j->band_ev[kBands + a], 0));
+    HIP_CHECK(hipStreamWaitEvent(j->xs, j->band_ev[n_bands + a], 0));
     const HostSeg out[4] = {{vals_pos + o, j->vp + o, c * sizeof(float)},
                             {lags_pos + o, j->lp + o, c * sizeof(int)},
                             {vals_neg + o, j->vn + o, c * sizeof(float)},

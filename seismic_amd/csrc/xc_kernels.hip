@@ -371,7 +371,8 @@ __device__ __forceinline__ float2 spec_load(__amdgpu_buffer_rsrc_t r, int voff, 
 // Channels [0, n_lds) of row i are read from xi_lds (stride M + 1), the others from
 // xi in memory (stride xj_stride).
 enum class RowFrom { kLds, kMemory, kBoth };
-template <int R, RowFrom kRow, int kLoadGroup = 32>
+// kChannels: channels loaded together.
+template <int R, RowFrom kRow, int kChannels, int kLoadGroup = 32>
 __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restrict__ xi_lds, int n_lds,
                                              const float2* __restrict__ xi, const float2* __restrict__ xj,
                                              long long xj_stride, int nch, const float2* tw,
@@ -380,49 +381,90 @@ __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restric
   float yN = 0.f;
   const __amdgpu_buffer_rsrc_t rj = spec_rsrc(xj, xj_stride, nch, M);
   const __amdgpu_buffer_rsrc_t ri = spec_rsrc(xi, xj_stride, nch, M);
-  // channel 0 initialises the accumulators, channels 1.. add to them
-  auto channel = [&](int c, auto first_c, auto memory_c) {
+  // Channels [c, c + kN): channel 0 initialises the accumulators, the others add to
+  // them.
+  auto channels = [&](int c, auto count_c, auto first_c, auto memory_c) {
+    constexpr int kN = decltype(count_c)::value;
     constexpr bool kFirst = decltype(first_c)::value;
     constexpr bool XI_GLOBAL = decltype(memory_c)::value;
-    const float2* ai = XI_GLOBAL ? xi + c * xj_stride : xi_lds + c * (M + 1);
-    const int soff_j = (int)(8 * c * xj_stride);
     // per-lane byte offset, redefined per channel (in the loads' block, with
     // a known range) so the bin offsets stay instruction immediates instead
     // of one hoisted offset register per load
     int lv = lane;
     asm volatile("" : "+v"(lv));
     const int vb = 8 * (lv & 63);
+    float2 aN[kN], bN[kN];
     // All of a group's global loads are issued before the compiler fence so
     // they are in flight together (one L2 round trip per group, not per row).
+    // Two channels at a time at P = 1024, where registers allow, and the Nyquist
+    // bins with them: N = 1500, P = 1024, C = 6 .. 8 5%
+    // faster, N = 16, C = 1, L = 4096, +-50 (5 segments) 37.4 -> 35.5 us.  At P = 2048
+    // and 3072 the Nyquist bin's registers alone cost 1-3%.
+    constexpr bool kEarly = kChannels > 1;
     constexpr int kGroup = load_group(R, kLoadGroup);
     static_assert(R % kGroup == 0, "load groups must tile the lane's bins");
 #pragma unroll
     for (int m0 = 0; m0 < R; m0 += kGroup) {
-      float2 Bv[kGroup];
-      float2 Av[XI_GLOBAL ? kGroup : 1];
+      float2 Bv[kN][kGroup];
+      float2 Av[kN][XI_GLOBAL ? kGroup : 1];
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) Bv[u] = spec_load(rj, vb + 512 * (m0 + u), soff_j);
-      if constexpr (XI_GLOBAL) {
+      for (int n = 0; n < kN; ++n) {
+        const int soff = (int)(8 * (c + n) * xj_stride);
 #pragma unroll
-        for (int u = 0; u < kGroup; ++u) Av[u] = spec_load(ri, vb + 512 * (m0 + u), soff_j);
+        for (int u = 0; u < kGroup; ++u) Bv[n][u] = spec_load(rj, vb + 512 * (m0 + u), soff);
+        if constexpr (XI_GLOBAL) {
+#pragma unroll
+          for (int u = 0; u < kGroup; ++u) Av[n][u] = spec_load(ri, vb + 512 * (m0 + u), soff);
+        }
+        if (kEarly && m0 == 0) {
+          bN[n] = spec_load(rj, 8 * M, soff);
+          if constexpr (XI_GLOBAL) aN[n] = spec_load(ri, 8 * M, soff);
+        }
       }
       asm volatile("" ::: "memory");
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) {
-        const int m = m0 + u;
-        cf A = f2c(XI_GLOBAL ? Av[XI_GLOBAL ? u : 0] : ai[lane + 64 * m]);
-        cf B = f2c(Bv[u]);
-        if constexpr (kFirst) {
-          y[m].x = __builtin_fmaf(A.x, B.x, A.y * B.y);
-          y[m].y = __builtin_fmaf(A.y, B.x, -A.x * B.y);
-        } else {
-          y[m].x = __builtin_fmaf(A.x, B.x, __builtin_fmaf(A.y, B.y, y[m].x));
-          y[m].y = __builtin_fmaf(A.y, B.x, __builtin_fmaf(-A.x, B.y, y[m].y));
+      for (int n = 0; n < kN; ++n) {
+        const float2* ai = xi_lds + (c + n) * (M + 1);
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+          const int m = m0 + u;
+          cf A = f2c(XI_GLOBAL ? Av[n][XI_GLOBAL ? u : 0] : ai[lane + 64 * m]);
+          cf B = f2c(Bv[n][u]);
+          if (kFirst && n == 0) {
+            y[m].x = __builtin_fmaf(A.x, B.x, A.y * B.y);
+            y[m].y = __builtin_fmaf(A.y, B.x, -A.x * B.y);
+          } else {
+            y[m].x = __builtin_fmaf(A.x, B.x, __builtin_fmaf(A.y, B.y, y[m].x));
+            y[m].y = __builtin_fmaf(A.y, B.x, __builtin_fmaf(-A.x, B.y, y[m].y));
+          }
         }
       }
     }
-    const float2 aN = ai[M], bN = xj[c * xj_stride + M];
-    yN = kFirst ? __builtin_fmaf(aN.x, bN.x, aN.y * bN.y) : __builtin_fmaf(aN.x, bN.x, __builtin_fmaf(aN.y, bN.y, yN));
+#pragma unroll
+    for (int n = 0; n < kN; ++n) {
+      if constexpr (!XI_GLOBAL) aN[n] = xi_lds[(c + n) * (M + 1) + M];
+      else if (!kEarly) aN[n] = xi[(c + n) * xj_stride + M];
+      if (!kEarly) bN[n] = xj[(c + n) * xj_stride + M];
+      yN = kFirst && n == 0 ? __builtin_fmaf(aN[n].x, bN[n].x, aN[n].y * bN[n].y)
+                            : __builtin_fmaf(aN[n].x, bN[n].x, __builtin_fmaf(aN[n].y, bN[n].y, yN));
+    }
+  };
+  constexpr std::integral_constant<int, 1> one{};
+  // channels [0, n), kChannels at a time
+  auto run = [&](int n, auto memory_c) {
+    int c = 1;
+    if constexpr (kChannels > 1) {
+      constexpr std::integral_constant<int, kChannels> some{};
+      if (n >= kChannels) {
+        channels(0, some, std::true_type{}, memory_c);
+        for (c = kChannels; c + kChannels <= n; c += kChannels) channels(c, some, std::false_type{}, memory_c);
+      } else {
+        channels(0, one, std::true_type{}, memory_c);
+      }
+    } else {
+      channels(0, one, std::true_type{}, memory_c);
+    }
+    for (; c < n; ++c) channels(c, one, std::false_type{}, memory_c);
   };
   // Wave priority by phase (s_setprio; the arbiter issues from the waves of
   // a SIMD in priority order): 2 while the column spectra are loaded and
@@ -431,15 +473,10 @@ __device__ __forceinline__ void pair_inverse(cf (&y)[R], const float2* __restric
   // which keeps the SIMD's waves staggered over the phases instead of all
   // waiting on memory or LDS at once (pair kernel 6% faster at P = 4096).
   __builtin_amdgcn_s_setprio(2);
-  if constexpr (kRow == RowFrom::kMemory) {
-    channel(0, std::true_type{}, std::true_type{});
-    for (int c = 1; c < nch; ++c) channel(c, std::false_type{}, std::true_type{});
-  } else {
-    channel(0, std::true_type{}, std::false_type{});
-    for (int c = 1; c < (kRow == RowFrom::kLds ? nch : n_lds); ++c) channel(c, std::false_type{}, std::false_type{});
-    if constexpr (kRow == RowFrom::kBoth)
-      for (int c = n_lds; c < nch; ++c) channel(c, std::false_type{}, std::true_type{});
-  }
+  if constexpr (kRow == RowFrom::kMemory) run(nch, std::true_type{});
+  else run(kRow == RowFrom::kLds ? nch : n_lds, std::false_type{});
+  if constexpr (kRow == RowFrom::kBoth)
+    for (int c = n_lds; c < nch; ++c) channels(c, one, std::false_type{}, std::true_type{});
   __builtin_amdgcn_s_setprio(1);
   // c2r ignores the imaginary parts of the DC and Nyquist bins
   if (lane == 0) y[0].y = 0.f;
@@ -747,7 +784,7 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
       // smaller load groups where registers are short: the budget of 4 waves
       // per SIMD (128 VGPRs), and at P >= 6144 channels from memory (twice
       // the loads in flight) and the budget of 3
-      pair_inverse<R, kRow, (kPerSimd >= 4 || (R >= 48 && (kRow != RowFrom::kLds || kPerSimd == 3))) ? 16 : 32>(
+      pair_inverse<R, kRow, R == 8 ? 2 : 1, (kPerSimd >= 4 || (R >= 48 && (kRow != RowFrom::kLds || kPerSimd == 3))) ? 16 : 32>(
           y, xi_lds, n_lds, src, xj, a.spec_stride, a.n_channels, twl, wl, lane);
       if constexpr (G > 0) apply_window<R, G>(y, wb);
       Best pos, neg;
@@ -860,7 +897,7 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
     wave_lds_fence();
     cf y[R];
     const float2* cols = a.col_spec ? a.col_spec : a.spec;
-    pair_inverse<R, RowFrom::kMemory>(y, nullptr, 0, a.spec + (long long)i * a.n_spec * a.spec_stride,
+    pair_inverse<R, RowFrom::kMemory, R == 8 ? 2 : 1>(y, nullptr, 0, a.spec + (long long)i * a.n_spec * a.spec_stride,
                                       cols + (long long)j * a.n_spec * a.spec_stride, a.spec_stride, a.n_spec, twl,
                                       wl, lane);
     {

@@ -126,6 +126,18 @@ __device__ __forceinline__ void forward_finish(const ForwardArgs& a, cf (&d)[R],
                                                const float2* twl, float2* wl, float2* zl, int lane) {
   constexpr int M = 64 * R;
   constexpr int P = 2 * M;
+  // the first post-twiddles are requested before the transform where registers
+  // allow (N = 16, P = 4096 spilled: 49 -> 56 us), those of the next four steps
+  // before the stores of this four (which the compiler cannot move loads across)
+  constexpr int kStep = 4;
+  static_assert((R / 2) % kStep == 0, "whole steps");
+  float2 tw[kStep];
+  auto first_tw = [&] {
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[lane + 64 * u];
+  };
+  if constexpr (R <= 24) first_tw();
+
   wave_fft<R, -1>(d, twl, wl, lane);
 #pragma unroll
   for (int r = 0; r < R; ++r) zl[wave_out_index<R>(lane, r)] = c2f(d[r]);
@@ -157,13 +169,7 @@ __device__ __forceinline__ void forward_finish(const ForwardArgs& a, cf (&d)[R],
     emit(k, cadd(e, od));
     if (2 * k != M) emit(M - k, cmk(e.x - od.x, od.y - e.y));
   };
-  // the post-twiddles of the next four steps are requested before the stores of
-  // this four (which the compiler cannot move loads across)
-  constexpr int kStep = 4;
-  static_assert((R / 2) % kStep == 0, "whole steps");
-  float2 tw[kStep];
-#pragma unroll
-  for (int u = 0; u < kStep; ++u) tw[u] = a.post_tw[lane + 64 * u];
+  if constexpr (R > 24) first_tw();
 #pragma unroll 1
   for (int k0 = lane; k0 < M / 2; k0 += 64 * kStep) {
     float2 t[kStep];
@@ -761,17 +767,31 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
     const bool dense = a.dense_cols > 0;
     const float2* src = a.spec + (long long)i * a.n_channels * a.spec_stride;
     {
-      // a channel's loads are all in flight before its first store
-      constexpr int T = 64 * kWaves, kPer = (M + T - 1) / T;
+      // a channel's loads, or four channels' at short periods, are all in flight
+      // before their first store
+      constexpr int T = 64 * kWaves, kPer = (M + T - 1) / T, kCh = kPer > 3 ? 1 : 4;
+      auto stage = [&](int c, auto count_c) {
+        constexpr int kN = decltype(count_c)::value;
+        float2 v[kN][kPer];
+#pragma unroll
+        for (int n = 0; n < kN; ++n)
+#pragma unroll
+          for (int u = 0; u < kPer; ++u) v[n][u] = src[(c + n) * a.spec_stride + min((int)threadIdx.x + u * T, M)];
+#pragma unroll
+        for (int n = 0; n < kN; ++n)
+#pragma unroll
+          for (int u = 0; u < kPer; ++u)
+            if (M % T == 0 || (int)threadIdx.x + u * T < M) xi_lds[(c + n) * (M + 1) + threadIdx.x + u * T] = v[n][u];
+      };
       __syncthreads();
-      for (int c = 0; c < n_lds; ++c) {
-        const float2* sc = src + c * a.spec_stride;
-        float2 v[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) v[u] = sc[min((int)threadIdx.x + u * T, M)];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u)
-          if (M % T == 0 || (int)threadIdx.x + u * T < M) xi_lds[c * (M + 1) + threadIdx.x + u * T] = v[u];
+      int c = 0;
+      for (; c + kCh <= n_lds; c += kCh) stage(c, std::integral_constant<int, kCh>{});
+      if constexpr (kCh > 1) {
+        if (c + 2 <= n_lds) {
+          stage(c, std::integral_constant<int, 2>{});
+          c += 2;
+        }
+        if (c < n_lds) stage(c, std::integral_constant<int, 1>{});
       }
       if ((int)threadIdx.x < n_lds) xi_lds[threadIdx.x * (M + 1) + M] = src[threadIdx.x * a.spec_stride + M];
       __syncthreads();
@@ -890,10 +910,12 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
   // compact tables (as the pair kernel): 11.8 KB of LDS at P = 4096
   float2* twl = smem;
   float2* wl = smem + TwLayoutCT<R>::kInv;
+  int4 t = a.ties[begin + rec0];  // its load runs beside the tables'
   stage_twiddles<TwLayoutCT<R>::kInv, 64>(twl, a.tw + TwLayout<R>::kInv, lane);
   for (unsigned rec = rec0; rec < seg_end; rec += n_local) {
-    const int4 t = a.ties[begin + rec];
-    const int i = t.x, j = t.y, side = t.z;
+    if (rec != rec0) t = a.ties[begin + rec];
+    const int i = __builtin_amdgcn_readfirstlane(t.x), j = __builtin_amdgcn_readfirstlane(t.y);
+    const int side = __builtin_amdgcn_readfirstlane(t.z);
     wave_lds_fence();
     cf y[R];
     const float2* cols = a.col_spec ? a.col_spec : a.spec;
@@ -934,6 +956,9 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
       });
     }
     wave_lds_fence();
+    // lane c: the norms of channel c
+    const int nc = min(lane, a.n_channels - 1);
+    const double norm_i = a.norms[(long long)i * a.n_channels + nc], norm_j = a.norms[(long long)j * a.n_channels + nc];
     for (int sd = 0; sd < 2; ++sd) {
       if (!(side & (1 << sd))) continue;
       const double sg = sd == 0 ? 1.0 : -1.0;
@@ -956,8 +981,7 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
         }
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
         for (int c = 0; c < a.n_channels; ++c) {
-          const double ni = a.norms[(long long)i * a.n_channels + c];
-          const double nj = a.norms[(long long)j * a.n_channels + c];
+          const double ni = __shfl(norm_i, c, 64), nj = __shfl(norm_j, c, 64);
           if (!(ni > 0.0 && nj > 0.0)) continue;
           const float* ti = a.traces + ((long long)i * a.n_channels + c) * a.tr_stride;
           double sum[4] = {0.0, 0.0, 0.0, 0.0};

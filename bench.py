@@ -157,6 +157,25 @@ def time_plan(plan, tr, outs, stream, steps, warmup):
     return ms, plan.timing(), plan.stats()
 
 
+def lag_issued_flops(n, c, length, lo, hi, products):
+    """MFMA flops k_lag_pairs issues over all pairs: 32-lag blocks in ranges of
+    at most 7 (bf16x3, 3 products) or 8 (fp16), each over the 16-sample chunks
+    its lags use, for every row of the upper triangle's 32 x 32 tiles."""
+    blocks = -(-(hi - lo + 1) // 32)
+    ranges = -(-blocks // (7 if products == 3 else 8))
+    nb = -(-blocks // ranges)
+    n_long = blocks - ranges * (nb - 1)
+    steps = b0 = 0
+    for r in range(ranges):
+        k = nb if r < n_long else nb - 1
+        l0 = lo + 32 * b0
+        l1 = min(l0 + 32 * k - 1, hi)
+        steps += k * ((min(length, length - l0) + 15) // 16 - max(0, -l1) // 16)
+        b0 += k
+    t = -(-n // 32)
+    return 2.0 * 32 * 32 * 16 * products * steps * c * 32 * (t * (t + 1) // 2)
+
+
 def lag_forms(ev, tr, stream, steps, warmup, f64=None):
     """MFMA lag-window forms and the FFT form on the same +-LAG_WINDOW window;
     f64 = (packed indices, FP64 reference on that window) adds each form's
@@ -170,14 +189,7 @@ def lag_forms(ev, tr, stream, steps, warmup, f64=None):
         outs = plan.alloc_outputs()
         ms, tm, st = time_plan(plan, tr, outs, stream, steps, warmup)
         k = 3 if name == "bf16x3" else 1
-        T = (N + 31) // 32
-        n_tiles = T * (T + 1) // 2
-        lag_first = -w
-        while (lag_first - 1) % 8:
-            lag_first -= 1
-        n_lags_issued = 8 * ((w - lag_first + 1 + 7) // 8)
-        l16 = (L + 15) // 16 * 16
-        issued = n_tiles * 1024 * k * 2.0 * n_lags_issued * l16 * C
+        issued = lag_issued_flops(N, C, L, -w, w, k)
         useful = N * (N - 1) / 2 * 2.0 * ((2 * w + 1) * L - w * (w + 1)) * C
         kern_s = tm["ms_pairs"] / 1e3
         out[name] = {
@@ -397,7 +409,7 @@ def tiled_leg(n_events: int, block: int, fp64_pairs: int):
     tr.free()
     pairs = n_events * (n_events + 1) // 2
     rate = pairs / wall
-    issued = 3 * 2 * (2 * w + 1) * L  # bf16x3 MFMA flops per pair
+    issued = lag_issued_flops(n_events, 1, L, -w, w, 3) / pairs  # bf16x3 MFMA flops per pair
     sure = ref_gap >= 1e-12
     live = ref_v > 1e-3
     out = {"n_events": n_events, "samples": L, "lags": [-w, w], "form": "bf16x3", "block": block,

@@ -128,33 +128,25 @@ void plan_free(sxc_plan* p) {
 
 namespace sxc {
 
-// Twiddle tables in the device layout of TwLayout<R> (xc_fft.hpp):
-//   [k2*64 + t] = W_M^(t*k2), k2 < R;  [64R + k*8 + t1] = W_64^(t1*k);
-//   inverse only: [64R + 64 + m*64 + t] = exp(+2 pi i (t + 64 m) / P).
+// Twiddle tables in the device layouts of xc_fft.hpp: TwLayout<R> (sign -1, the
+// forward transform) or TwLayoutCT<R> (sign +1, the inverse one).
 std::vector<float2> wave_tables(int R, int sign) {
   const int M = 64 * R, P = 2 * M;
-  const int kW = 64 * R, kPre = 64 * R + 64;
-  std::vector<float2> t(sign > 0 ? kPre + 64 * R : kPre);
-  for (int k = 0; k < R; ++k)
-    for (int l = 0; l < 64; ++l) twiddle((long)l * k, M, sign, &t[k * 64 + l].x, &t[k * 64 + l].y);
-  for (int k = 0; k < 8; ++k)
-    for (int l = 0; l < 8; ++l) twiddle((long)l * k, 64, sign, &t[kW + k * 8 + l].x, &t[kW + k * 8 + l].y);
-  if (sign > 0) {
-    for (int m = 0; m < R; ++m)
-      for (int l = 0; l < 64; ++l) twiddle(l + 64L * m, P, +1, &t[kPre + m * 64 + l].x, &t[kPre + m * 64 + l].y);
-    // compact inverse tables (TwLayoutCT) follow the full ones
-    const size_t b = t.size();
-    t.resize(b + 640 + 8 * R);
-    for (int k = 0; k < 8; ++k)
-      for (int l = 0; l < 64; ++l) twiddle((long)l * k, M, +1, &t[b + k * 64 + l].x, &t[b + k * 64 + l].y);
+  std::vector<float2> t;
+  t.reserve(64 * R + 640);
+  auto add = [&](long num, long den) {
+    t.emplace_back();
+    twiddle(num, den, sign, &t.back().x, &t.back().y);
+  };
+  for (int k = 0; k < (sign > 0 ? 8 : R); ++k)
+    for (int l = 0; l < 64; ++l) add((long)l * k, M);
+  if (sign > 0)
     for (int a = 0; a < R / 8; ++a)
-      for (int l = 0; l < 64; ++l)
-        twiddle(8L * l * a, M, +1, &t[b + 512 + a * 64 + l].x, &t[b + 512 + a * 64 + l].y);
-    for (int k = 0; k < 8; ++k)
-      for (int l = 0; l < 8; ++l)
-        twiddle((long)l * k, 64, +1, &t[b + 512 + 8 * R + k * 8 + l].x, &t[b + 512 + 8 * R + k * 8 + l].y);
-    for (int l = 0; l < 64; ++l) twiddle(l, P, +1, &t[b + 576 + 8 * R + l].x, &t[b + 576 + 8 * R + l].y);
-  }
+      for (int l = 0; l < 64; ++l) add(8L * l * a, M);
+  for (int k = 0; k < 8; ++k)
+    for (int l = 0; l < 8; ++l) add((long)l * k, 64);
+  if (sign > 0)
+    for (int l = 0; l < 64; ++l) add(l, P);
   return t;
 }
 

@@ -291,19 +291,16 @@ constexpr int kWaveLds = 576;  // float2 per wave for the chunked transposes
 // (float2, FP64 generated on the host and rounded once):
 //   step 2:  tw[k2*64 + t] = W_M^(t*k2), k2 < R           (R*64 entries)
 //   w64:     tw[kW64 + k*8 + t1] = W_64^(t1*k), k, t1 < 8  (64 entries)
-//   pre:     tw[kPre + m*64 + t] = exp(+2 pi i (t + 64 m) / P), m < R
-//            (half-length C2R packing; inverse tables only)
+// for the forward transform.
 template <int R>
 struct TwLayout {
   static constexpr int kS2 = 0;
   static constexpr int kW64 = 64 * R;
-  static constexpr int kPre = 64 * R + 64;
-  static constexpr int kFft = kPre;          // entries a wave FFT needs
-  static constexpr int kInv = kPre + 64 * R; // entries the pair kernels need
+  static constexpr int kFft = 64 * R + 64;
 };
 
-// Compact inverse tables, for pair kernels whose staged row spectra leave no
-// room for the full ones (stored right after them, at offset kInv):
+// Compact tables of the inverse transform, which leave the pair kernels room for
+// the row spectra (and need fewer LDS reads):
 //   step 2:  A[b][t] = W_M^(t*b), b < 8, and B[a][t] = W_M^(8*t*a), a < R/8,
 //            so W_M^(t*k2) = A[k2 % 8] * B[k2 / 8]            (512 + 8R entries)
 //   w64:     as in the full tables                          (64 entries)

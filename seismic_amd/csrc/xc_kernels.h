@@ -61,7 +61,7 @@ struct PairArgs {
   int lag_lo, lag_hi;     // scanned lags, inclusive
   float threshold;
   float tie_tol;
-  const float2* tw;       // inverse twiddle tables (TwLayout, then TwLayoutCT)
+  const float2* tw;       // inverse twiddle tables (TwLayoutCT)
   float* vpos;
   int* lpos;
   float* vneg;

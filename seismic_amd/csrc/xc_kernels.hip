@@ -743,7 +743,7 @@ __global__ __launch_bounds__(kWaves * 64, kPerSimd) void k_pairs(PairArgs a) {
   float2* xi_lds = smem + kTab;
   float2* wl = xi_lds + n_lds * (M + 1) + wv * kWaveLds;
 
-  stage_twiddles<kTab, 64 * kWaves>(twl, a.tw + TwLayout<R>::kInv, threadIdx.x);
+  stage_twiddles<kTab, 64 * kWaves>(twl, a.tw, threadIdx.x);
   WinBits<R, G> wb;
   if constexpr (G > 0) win_bits<R, G>(wb, lane, a.lag_lo, a.lag_hi);
 
@@ -911,7 +911,7 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
   float2* twl = smem;
   float2* wl = smem + TwLayoutCT<R>::kInv;
   int4 t = a.ties[begin + rec0];  // its load runs beside the tables'
-  stage_twiddles<TwLayoutCT<R>::kInv, 64>(twl, a.tw + TwLayout<R>::kInv, lane);
+  stage_twiddles<TwLayoutCT<R>::kInv, 64>(twl, a.tw, lane);
   for (unsigned rec = rec0; rec < seg_end; rec += n_local) {
     if (rec != rec0) t = a.ties[begin + rec];
     const int i = __builtin_amdgcn_readfirstlane(t.x), j = __builtin_amdgcn_readfirstlane(t.y);

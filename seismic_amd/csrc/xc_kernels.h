@@ -168,7 +168,9 @@ constexpr size_t pair_lds_bytes(int R, int n_channels, int waves) {
 // 3.97 -> 3.90; one 12-wave workgroup -> 3 of 4: P = 5120, C = 1 4.26 -> 4.20,
 // P = 6144 5.11 -> 5.00.  W is a multiple of 4: 6, 10 or 14 waves load the four
 // SIMDs unevenly and the next workgroup no longer fits (P = 1024 with 14: 1.12).
-// P = 8192 runs 8 waves: its 128 spectrum registers per lane need 256 VGPRs.
+// P = 8192 runs 8 waves per CU: its 128 spectrum registers per lane need 256 VGPRs;
+// two workgroups of 4 where one channel leaves the LDS for them: N = 1500, C = 1
+// 7.14 -> 6.83 ms, +-2730 8.55 -> 7.79, N = 200 233 -> 221 us.
 struct PairShape {
   int waves, per_simd;  // W, S; 0: no further shape
 };
@@ -178,7 +180,7 @@ constexpr PairShape pair_shape(int R, int i) {
   constexpr PairShape k24[] = {{8, 4}, {16, 4}, {12, 3}, {0, 0}, {0, 0}};
   constexpr PairShape k32[] = {{8, 4}, {16, 4}, {12, 3}, {8, 2}, {0, 0}};
   constexpr PairShape k48[] = {{4, 3}, {12, 3}, {8, 2}, {0, 0}, {0, 0}};  // and R = 40
-  constexpr PairShape k64[] = {{8, 2}, {0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  constexpr PairShape k64[] = {{4, 2}, {8, 2}, {0, 0}, {0, 0}, {0, 0}};
   return R == 8 ? k8[i] : R == 16 ? k16[i] : R == 24 ? k24[i] : R == 32 ? k32[i] : R == 64 ? k64[i] : k48[i];
 }
 constexpr bool pair_shape_fits(int R, int n_channels, PairShape k) {
@@ -225,9 +227,9 @@ template <typename Items>
 inline int pair_chunk(int R, int n_channels, Items items) {
   const PairShape k = pair_shape_for(R, n_channels);
   const long long slots = 256 * 4 * k.per_simd / k.waves;
-  int best = 64;
+  int best = 64;  // 4 columns only ever pay for workgroups of 4 waves
   double cost = 0.0;
-  for (int c : {64, 32, 16, 8}) {
+  for (int c : {64, 32, 16, 8, 4}) {
     const double t = (double)((items(c) + slots - 1) / slots) * ((c + k.waves - 1) / k.waves + 0.5);
     if (c == 64 || t < 0.97 * cost) {
       best = c;

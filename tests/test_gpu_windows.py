@@ -166,3 +166,20 @@ def test_segments_host_call_and_no_allocation(demean):
     for w, h, o in zip(want, host, out):
         assert np.array_equal(w, h) and np.array_equal(w, o.numpy())
     plan.close()
+
+
+@pytest.mark.parametrize("P", [5120, 6144, 8192])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 11, 32, 66])
+def test_small_jobs_of_four_wave_workgroups(P, n):
+    """One channel at the periods whose workgroups have four waves: items of 4
+    columns in the smallest jobs."""
+    L, lo, hi = P // 2 + 100, -P // 2 + 1, P // 2
+    ev, _ = synth.make_events(n, 1, L, seed=P + n)
+    print(f"case four-wave job N={n} P={P}", flush=True)
+    vp, lp, vn, ln = engine.allpairs_host(ev, P, lo, hi)
+    c = _ncc_f64(ev, L, P, lo, hi, False)
+    for v, lag, sign in ((vp, lp, 1.0), (-vn, ln, -1.0)):
+        w = np.partition(sign * c, -2, axis=-1)[:, -2:]  # the two best
+        assert np.abs(v - np.maximum(w[:, 1], 0.0)).max() <= 1e-5
+        sure = (w[:, 1] > 1e-12) & (w[:, 1] - w[:, 0] >= 1e-12)
+        assert np.array_equal(lag[sure], lo + np.argmax(sign * c, axis=-1)[sure])

@@ -195,8 +195,7 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   p->l16 = (L + 15) / 16 * 16;
   p->lag_first = desc->lag_lo;
   p->n_blocks = (desc->lag_hi - desc->lag_lo + 1 + kLagBlock - 1) / kLagBlock;
-  // samples lag_first .. l16 + the last block's last lag; operand loads past a
-  // row's end return 0
+  // samples lag_first .. l16 + the last block's last lag
   p->hs = p->l16 + kLagBlock * p->n_blocks;
   p->n_pairs = (long long)desc->n_events * (desc->n_events + 1) / 2;
   // default bands: at least twice the largest coefficient error against FP64
@@ -208,16 +207,15 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   const long long rows = (long long)desc->n_events * desc->n_channels;
   auto fail = [&](int code) { plan_free(p); return code; };
   int rc;
-  const size_t h_elems = (size_t)rows * 2 * p->hs;
-  const size_t b_elems = (size_t)((desc->n_events + 31) / 32 * 32) * desc->n_channels * p->l16;
-  // one allocation (h_hi): row operands, then column operands, 256-byte aligned
-  const size_t h_size = (h_elems + 127) / 128 * 128, b_size = (b_elems + 127) / 128 * 128;
+  // one allocation (h_hi) for the operands
+  const LagOperands ops =
+      lag_operands(rows, (desc->n_events + 31LL) / 32 * 32 * desc->n_channels, p->hs, p->l16);
   const bool two = desc->form == SXC_FORM_LAG_BF16X3;
-  if ((rc = dev_alloc(&p->h_hi, (h_size + b_size) * (two ? 2 : 1), "trace operands"))) return fail(rc);
-  p->b_hi = p->h_hi + h_size;
+  if ((rc = dev_alloc(&p->h_hi, (size_t)(ops.h + ops.b) * (two ? 2 : 1), "trace operands"))) return fail(rc);
+  p->b_hi = p->h_hi + ops.h;
   if (two) {
-    p->h_lo = p->b_hi + b_size;
-    p->b_lo = p->h_lo + h_size;
+    p->h_lo = p->b_hi + ops.b;
+    p->b_lo = p->h_lo + ops.h;
   }
   if ((rc = dev_alloc(&p->norms, (size_t)rows, "norms"))) return fail(rc);
   if ((rc = dev_alloc(&p->lag_traces, (size_t)(rows * L), "FP32 traces"))) return fail(rc);

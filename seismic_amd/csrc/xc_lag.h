@@ -9,6 +9,20 @@ constexpr int kLagBlock = 32;  // lags per block (one accumulator tile each)
 // from the last lag at or below its first that is 1 modulo 8.
 constexpr int kLagMaxSpan = 65536;
 
+// Elements past a row's or a column tile's operand that the product's loads may
+// reach (their values are not used).
+constexpr int kLagAhead = 8192;
+// Parts of the operands' allocation, in elements (256-byte aligned): row operands
+// of `rows` rows, then column operands of `cols` rows (a multiple of 32 events),
+// which with what follows them are the room past the row operands.
+struct LagOperands {
+  long long h, b;  // elements of each part
+};
+inline LagOperands lag_operands(long long rows, long long cols, int hs, int l16) {
+  auto up = [](long long n) { return (n + 127) / 128 * 128; };
+  return {up(rows * 2 * hs), up(cols * l16 + kLagAhead)};
+}
+
 struct LagPrepArgs {
   const float* in;          // [n_rows][in_stride]
   long long in_stride;

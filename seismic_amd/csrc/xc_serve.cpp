@@ -188,7 +188,7 @@ struct Slot {
   int* h_len = nullptr;        // pinned staging, laid out as on the device
   float* h_traces = nullptr;
   float* h_tv = nullptr;
-  int* h_tl = nullptr;         // into h_tv (run_batch)
+  int* h_tl = nullptr;         // into h_tv, set by a batch that succeeds (run_batch)
   int* h_ti = nullptr;
 };
 
@@ -405,7 +405,7 @@ void worker_loop(sxc_server* S, int slot_index) {
       for (size_t r = 0; r < batch.size(); ++r) {
         Request& q = *batch[r];
         q.result.resize((size_t)q.n * d.top_k);
-        for (int e = 0; e < q.n; ++e) {
+        for (int e = 0; rc == SXC_OK && e < q.n; ++e) {  // a failed batch has no results to read
           const int P = period_for(q.lengths[e], d.catalog_len);
           for (int k = 0; k < d.top_k; ++k) {
             const size_t src = (size_t)row_of[r][e] * d.top_k + k;

@@ -183,3 +183,23 @@ def test_small_jobs_of_four_wave_workgroups(P, n):
         assert np.abs(v - np.maximum(w[:, 1], 0.0)).max() <= 1e-5
         sure = (w[:, 1] > 1e-12) & (w[:, 1] - w[:, 0] >= 1e-12)
         assert np.array_equal(lag[sure], lo + np.argmax(sign * c, axis=-1)[sure])
+
+
+def test_loud_rows_past_the_trace_length_stay_in_the_window():
+    """Rows longer than L with loud samples past it: coefficients far above 1,
+    whose rounding at lags outside the window is no near tie of 0.  Positive
+    traces have no negative side; no reported lag may leave the window."""
+    n, L, in_len, P = 12, 500, 1400, 3072
+    lo, hi = 1 - in_len, in_len - 1
+    x = np.random.default_rng(3).uniform(1.0, 2.0, (n, 1, in_len)).astype(np.float32)
+    x[..., :L] *= np.float32(0.01)
+    print(f"case loud rows P={P} L={L} in_len={in_len} [{lo}, {hi}]", flush=True)
+    plan = engine.AllPairsPlan(n, 1, L, P, lo, hi)
+    out = plan.execute(DeviceArray.from_numpy(x))
+    synchronize()
+    vp, lp, vn, ln = [o.numpy() for o in out]
+    plan.close()
+    c = _ncc_f64(x, L, P, lo, hi, False)
+    assert (c > 0.05).all() and np.abs(vp / c.max(-1) - 1.0).max() <= 1e-5
+    assert ((lp >= lo) & (lp <= hi)).all()
+    assert not vn.any() and not ln.any()

@@ -872,13 +872,14 @@ sxc::FftGeom sxc::fft_geom(const sxc_plan* p, int in_len, bool reversed) {
   }
   // A window over every lag at which two rows can overlap is scanned without
   // masks (N = 1111, C = 2, P = 3072: 1.66 -> 1.56 ms): the other lags hold
-  // rounding around an exact 0, below 5e-7 where every sample enters the energy and
-  // coefficients are at most 1 (rows no longer than L).  Where such a value is the
-  // extremum it is within the band of 0, so the pair is recorded and the
-  // resolver, which looks at the window alone, settles it; hence the default
-  // band at least and room for every record.
-  if (ext <= p->d.trace_len && ext + reach <= g.P && p->d.lag_lo <= 1 - ext && p->d.lag_hi >= ext - 1 && p->tie_tol >= 2e-6f &&
-      p->tie_cap >= p->n_pairs)
+  // rounding around an exact 0, below kScanNoise where every sample enters the
+  // energy and coefficients are at most 1 (rows no longer than L).  Where such a
+  // value is the extremum it is within the band of 0, so the pair is recorded and
+  // the resolver, which looks at the window alone, settles it; hence the default
+  // band at least and room for every record.  A threshold below the rounding
+  // would have the masked scan record fewer pairs.
+  if (ext <= p->d.trace_len && ext + reach <= g.P && p->d.lag_lo <= 1 - ext && p->d.lag_hi >= ext - 1 &&
+      (p->d.threshold <= 0.f || p->d.threshold >= kScanNoise) && p->tie_tol >= 2e-6f && p->tie_cap >= p->n_pairs)
     g.full = true;
   return g;
 }

@@ -44,6 +44,9 @@ struct ForwardArgs {
   float2* seg_cols;
 };
 
+// Bound of the FP32 rounding of a coefficient (at most 1) that is exactly 0.
+constexpr float kScanNoise = 5e-7f;
+
 struct PairArgs {
   const float2* spec;     // row spectra [n_rows][n_channels][spec_stride]
   long long spec_stride;

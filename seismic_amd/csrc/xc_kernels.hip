@@ -711,8 +711,10 @@ __device__ __forceinline__ void scan_wave(const cf (&y)[R], int lane, float tol,
   pos.lag = (want_p && slot_p >= 0) ? slot_lag<R>(__ffsll((long long)msk_p) - 1, slot_p) : 0;
   neg.v = want_n ? mn : (mn < 0.f ? mn : 0.f);
   neg.lag = (want_n && slot_n >= 0) ? slot_lag<R>(__ffsll((long long)msk_n) - 1, slot_n) : 0;
-  tie_p = want_p && (cnt_p > 1 || cp <= 0.f);
-  tie_n = want_n && (cnt_n > 1 || cn >= 0.f);
+  // also near 0, the scan's starting state; with kScanNoise, no value outside the
+  // window of an unmasked scan decides whether a pair is recorded
+  tie_p = want_p && (cnt_p > 1 || cp <= kScanNoise);
+  tie_n = want_n && (cnt_n > 1 || cn >= -kScanNoise);
 }
 
 __device__ __forceinline__ long long packed_index(int i, int j, int n) {

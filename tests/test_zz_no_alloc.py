@@ -70,3 +70,34 @@ def test_noalloc_rejects_oversize():
                                       ctypes.c_void_p(tiny.ptr), ctypes.c_void_p(tiny.ptr),
                                       ctypes.c_void_p(stream.handle))
     assert rc == -1 and "FFT form only" in _lib.last_error(lib)
+
+
+@pytest.mark.parametrize("thr", [0.0, 3e-7])
+def test_noalloc_equals_the_unmasked_scan(thr):
+    """Every overlapping lag in the window, more pairs than the entry point holds
+    records: it scans with masks what a plan scans without.  Event 0 is positive,
+    events 1 .. 399 negative but for a first sample whose size makes the pair's
+    largest coefficient, at its last lag, from just below the near-tie band of 0 to
+    just above it."""
+    lib = _lib.load_engine()
+    n, few, L, P, lo, hi = 1500, 400, 500, 1024, -499, 499
+    x, _ = synth.make_events(n, 1, L, seed=11)
+    rng = np.random.default_rng(12)
+    y = rng.uniform(0.5, 1.0, (few, L))
+    y[1:] *= -1.0
+    y[1:, 0] = 0.0
+    y[1:, 0] = np.linspace(1.9e-6, 2.3e-6, few - 1) * np.linalg.norm(y[0]) * np.linalg.norm(y[1:], axis=-1) / y[0, -1]
+    x[:few, 0] = y
+    print(f"case noalloc unmasked N={n} P={P} [{lo}, {hi}] thr={thr}", flush=True)
+    d = DeviceArray.from_numpy(x)
+    plan = engine.AllPairsPlan(n, 1, L, P, lo, hi, threshold=thr)
+    stream = Stream()
+    ref = plan.execute(d, in_len=L, stream=stream)
+    stream.synchronize()
+    ref = [o.numpy() for o in ref]
+    outs = plan.alloc_outputs()
+    assert _noalloc(lib, plan.desc, d, L, L, outs, stream) == 0, _lib.last_error(lib)
+    stream.synchronize()
+    for a, o, name in zip(ref, outs, ("vals_pos", "lags_pos", "vals_neg", "lags_neg")):
+        assert np.array_equal(a, o.numpy()), name
+    plan.close()

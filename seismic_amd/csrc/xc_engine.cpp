@@ -8,6 +8,7 @@
 #include <hip/hip_runtime_api.h>
 #include <math.h>
 #include <stdarg.h>
+#include <stdint.h>
 #include <stdio.h>
 #include <string.h>
 
@@ -734,13 +735,6 @@ const char* seismic_last_error(void) { return last_error(); }
 
 }  // extern "C"
 
-// Work items (row, column chunk) of the packed triangle, chunk-major: chunk c
-// holds min(N, chunk (c + 1)) rows.
-static long long triangle_items(long long n, long long chunk) {
-  const long long q = n / chunk, r = n % chunk;
-  return chunk * (q * (q + 1) / 2) + (r ? n : 0);
-}
-
 // Geometry of an FFT-form plan (no device memory): period, strides, pair and
 // work-item counts, near-tie band and record capacity.
 void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bool may_cut, sxc_plan* p) {
@@ -887,16 +881,23 @@ sxc::FftGeom sxc::fft_geom(const sxc_plan* p, int in_len, bool reversed) {
 namespace {
 using namespace sxc;
 
-// The three stages of an FFT-form execute, asynchronous on st.
-// Column spectra of an execute with cut rows: after its row spectra.
-float2* seg_cols(const sxc_plan* p, const FftGeom& g) {
-  return p->spec + (long long)p->d.n_events * p->d.n_channels * g.n_seg * g.spec_stride;
+// Spectra of a launch: where event 0's row spectra and, with cut rows, its column
+// spectra lie (or would, when the memory holds later events only).
+struct Spectra {
+  float2 *rows, *cols;
+};
+// A plan's own: with cut rows, the column spectra after the row spectra.
+Spectra plan_spectra(const sxc_plan* p, const FftGeom& g) {
+  return {p->spec,
+          g.n_seg ? p->spec + (long long)p->d.n_events * p->d.n_channels * g.n_seg * g.spec_stride : nullptr};
 }
 
+// The three stages of an FFT-form execute, asynchronous on st.
 // Forward (and reversed-row) R2C of the rows of events [e0, e1); zero: a counter
-// to clear.
-int fft_stage_forward(sxc_plan* p, const FftGeom& g, int e0, int e1, const float* d_traces, const float* d_rev,
-                      long long trace_stride, int in_len, unsigned* zero, hipStream_t st) {
+// to clear; sides: ForwardArgs::seg_sides.
+int fft_stage_forward(sxc_plan* p, const FftGeom& g, const Spectra& sp, int sides, int e0, int e1,
+                      const float* d_traces, const float* d_rev, long long trace_stride, int in_len, unsigned* zero,
+                      hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   const long long r0 = (long long)e0 * d.n_channels, s0 = r0 * std::max(1, g.n_seg) * g.spec_stride;
   const long long tr_stride = g.n_seg ? p->P : g.P;
@@ -911,7 +912,7 @@ int fft_stage_forward(sxc_plan* p, const FftGeom& g, int e0, int e1, const float
   fa.norms = p->norms + r0;
   fa.out_traces = p->traces ? p->traces + r0 * tr_stride : nullptr;
   fa.out_stride = tr_stride;
-  fa.spec = p->spec + s0;
+  fa.spec = sp.rows + s0;
   fa.spec_stride = g.spec_stride;
   fa.tw = g.fwd2;
   fa.post_tw = g.post;
@@ -921,7 +922,8 @@ int fft_stage_forward(sxc_plan* p, const FftGeom& g, int e0, int e1, const float
     fa.seg_len = g.seg_len;
     fa.seg_back = std::max(0, d.lag_hi);
     fa.seg_ahead = std::max(0, -d.lag_lo);
-    fa.seg_cols = seg_cols(p, g) + s0;
+    fa.seg_cols = sp.cols + s0;
+    fa.seg_sides = sides;
   }
   if (fa.n_rows <= 0) return SXC_OK;
   HIP_CHECK(launch_forward(g.R, fa, st));
@@ -941,12 +943,12 @@ int fft_stage_forward(sxc_plan* p, const FftGeom& g, int e0, int e1, const float
 }
 
 // The pair kernel over work items [work, work + n_work).
-int fft_stage_pairs(sxc_plan* p, const FftGeom& g, bool reversed, const int2* work, int n_work, float* d_vals_pos, int* d_lags_pos,
-                    float* d_vals_neg, int* d_lags_neg, hipStream_t st) {
+int fft_stage_pairs(sxc_plan* p, const FftGeom& g, const Spectra& sp, bool reversed, const int2* work, int n_work,
+                    float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   PairArgs pa{};
-  pa.spec = p->spec;
-  pa.col_spec = reversed ? p->col_spec : (g.n_seg ? seg_cols(p, g) : nullptr);
+  pa.spec = sp.rows;
+  pa.col_spec = reversed ? p->col_spec : sp.cols;
   pa.spec_stride = g.spec_stride;
   pa.n_events = d.n_events;
   pa.n_channels = d.n_channels * std::max(1, g.n_seg);
@@ -971,12 +973,12 @@ int fft_stage_pairs(sxc_plan* p, const FftGeom& g, bool reversed, const int2* wo
 
 // The FP64 resolver over the near-tie records from *tie_begin (null: all) of
 // up to n_pairs pairs.
-int fft_stage_resolve(sxc_plan* p, const FftGeom& g, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
-                      long long n_pairs, const unsigned* tie_begin, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
-                      int* d_lags_neg, hipStream_t st) {
+int fft_stage_resolve(sxc_plan* p, const FftGeom& g, const Spectra& sp, const float* d_traces, const float* d_rev,
+                      long long trace_stride, int in_len, long long n_pairs, const unsigned* tie_begin,
+                      float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
   ResolveArgs ra{};
-  ra.spec = p->spec;
+  ra.spec = sp.rows;
   ra.spec_stride = g.spec_stride;
   if (d_rev) {
     ra.col_spec = p->col_spec;
@@ -984,8 +986,8 @@ int fft_stage_resolve(sxc_plan* p, const FftGeom& g, const float* d_traces, cons
     ra.rev_stride = trace_stride;
     ra.rev_len = in_len;
     ra.rev_shift = d.trace_len - 1;
-  } else if (g.n_seg) {
-    ra.col_spec = seg_cols(p, g);
+  } else {
+    ra.col_spec = sp.cols;
   }
   ra.n_spec = d.n_channels * std::max(1, g.n_seg);
   ra.period = g.n_seg ? p->P : g.P;  // cut rows are within it (fft_geom)
@@ -1031,18 +1033,52 @@ int sxc::fft_plan_execute(sxc_plan* p, const float* d_traces, const float* d_rev
   hipEvent_t* ev = nullptr;
   if (p->timing && p->timed < (int)p->events.size() / 4) ev = &p->events[4 * p->timed++];
   const FftGeom g = fft_geom(p, in_len, d_rev != nullptr);
+  const Spectra sp = plan_spectra(p, g);
   int rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[0], st));
-  if ((rc = fft_stage_forward(p, g, 0, p->d.n_events, d_traces, d_rev, trace_stride, in_len, p->tie_count, st))) return rc;
+  if ((rc = fft_stage_forward(p, g, sp, 0, 0, p->d.n_events, d_traces, d_rev, trace_stride, in_len, p->tie_count, st)))
+    return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[1], st));
-  if ((rc = fft_stage_pairs(p, g, d_rev != nullptr, p->work, p->n_work, d_vals_pos, d_lags_pos, d_vals_neg,
+  if ((rc = fft_stage_pairs(p, g, sp, d_rev != nullptr, p->work, p->n_work, d_vals_pos, d_lags_pos, d_vals_neg,
                             d_lags_neg, st)))
     return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[2], st));
-  if ((rc = fft_stage_resolve(p, g, d_traces, d_rev, trace_stride, in_len, p->n_pairs, nullptr, d_vals_pos, d_lags_pos,
-                              d_vals_neg, d_lags_neg, st)))
+  if ((rc = fft_stage_resolve(p, g, sp, d_traces, d_rev, trace_stride, in_len, p->n_pairs, nullptr, d_vals_pos,
+                              d_lags_pos, d_vals_neg, d_lags_neg, st)))
     return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[3], st));
+  return SXC_OK;
+}
+
+// Column band b's spectra stay while its row bands come and go; the row side of
+// band b itself comes first, as it leaves the norms (and demeaned traces) that
+// the resolver reads for b's columns.
+int sxc::fft_plan_execute_bands(sxc_plan* p, const FftGeom& g, int band, float2* rows, float2* cols,
+                                const float* d_traces, long long trace_stride, int in_len, float* d_vals_pos,
+                                int* d_lags_pos, float* d_vals_neg, int* d_lags_neg,
+                                const std::function<int(int, int, int, int)>& fill, hipStream_t st) {
+  const int n = p->d.n_events, n_bands = (n + band - 1) / band;
+  const size_t event_bytes = (size_t)p->d.n_channels * g.n_seg * g.spec_stride * sizeof(float2);
+  auto event0 = [&](float2* first, int e) { return (float2*)((uintptr_t)first - (size_t)e * event_bytes); };
+  int rc;
+  for (int b = 0; b < n_bands; ++b) {
+    const int c0 = b * band, c1 = std::min(n, c0 + band);
+    for (int k = 0; k <= b; ++k) {
+      const int r0 = (k == 0 ? b : k - 1) * band, r1 = std::min(n, r0 + band);
+      const Spectra sp{event0(rows, r0), event0(cols, c0)};
+      if (k == 0 && (rc = fft_stage_forward(p, g, sp, 2, c0, c1, d_traces, nullptr, trace_stride, in_len, nullptr, st)))
+        return rc;
+      if ((rc = fft_stage_forward(p, g, sp, 1, r0, r1, d_traces, nullptr, trace_stride, in_len, p->tie_count, st)))
+        return rc;
+      const int n_work = fill(r0, r1 - r0, c0, c1 - c0);
+      if (n_work < 0) return n_work;
+      if ((rc = fft_stage_pairs(p, g, sp, false, p->work, n_work, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg, st)))
+        return rc;
+      if ((rc = fft_stage_resolve(p, g, sp, d_traces, nullptr, trace_stride, in_len, (long long)(r1 - r0) * (c1 - c0),
+                                  nullptr, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg, st)))
+        return rc;
+    }
+  }
   return SXC_OK;
 }
 
@@ -1095,8 +1131,8 @@ int sxc::fft_plan_blocks(sxc_plan* p, int B) {
 // Forward (and reversed-row) R2C of the rows of events [e0, e1).
 int sxc::fft_plan_forward_events(sxc_plan* p, int e0, int e1, const float* d_traces, const float* d_rev,
                                  long long trace_stride, int in_len, hipStream_t st) {
-  return fft_stage_forward(p, fft_geom(p, in_len, d_rev != nullptr), e0, e1, d_traces, d_rev, trace_stride, in_len,
-                           nullptr, st);
+  const FftGeom g = fft_geom(p, in_len, d_rev != nullptr);
+  return fft_stage_forward(p, g, plan_spectra(p, g), 0, e0, e1, d_traces, d_rev, trace_stride, in_len, nullptr, st);
 }
 
 // Launch group g of a blocked execute: its pairs, then the resolver over the
@@ -1107,12 +1143,13 @@ int sxc::fft_plan_group(sxc_plan* p, int g, const float* d_traces, const float* 
   HIP_CHECK(hipMemcpyAsync(p->grp_count + g, p->tie_count, sizeof(unsigned), hipMemcpyDeviceToDevice, st));
   const int i0 = p->grp_item[g], i1 = p->grp_item[g + 1];
   const FftGeom geom = fft_geom(p, in_len, d_rev != nullptr);
+  const Spectra sp = plan_spectra(p, geom);
   int rc;
-  if ((rc = fft_stage_pairs(p, geom, d_rev != nullptr, p->blk_work + i0, i1 - i0, d_vals_pos, d_lags_pos, d_vals_neg,
-                            d_lags_neg, st)))
+  if ((rc = fft_stage_pairs(p, geom, sp, d_rev != nullptr, p->blk_work + i0, i1 - i0, d_vals_pos, d_lags_pos,
+                            d_vals_neg, d_lags_neg, st)))
     return rc;
-  return fft_stage_resolve(p, geom, d_traces, d_rev, trace_stride, in_len, (long long)(i1 - i0) * p->chunk, p->grp_count + g, d_vals_pos, d_lags_pos,
-                           d_vals_neg, d_lags_neg, st);
+  return fft_stage_resolve(p, geom, sp, d_traces, d_rev, trace_stride, in_len, (long long)(i1 - i0) * p->chunk,
+                           p->grp_count + g, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg, st);
 }
 
 extern "C" {

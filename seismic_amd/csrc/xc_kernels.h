@@ -42,6 +42,7 @@ struct ForwardArgs {
   // r n_seg on.  out_traces takes the row side's samples.
   int n_seg, seg_len, seg_back, seg_ahead;
   float2* seg_cols;
+  int seg_sides;          // 0: both sides' spectra, 1: the row side's only (with norms and out_traces), 2: the column side's
 };
 
 // Bound of the FP32 rounding of a coefficient (at most 1) that is exactly 0.
@@ -240,6 +241,12 @@ inline int pair_chunk(int R, int n_channels, Items items) {
     }
   }
   return best;
+}
+// Work items (row, column chunk) of the packed triangle, chunk-major: chunk c
+// holds min(N, chunk (c + 1)) rows.
+inline long long triangle_items(long long n, long long chunk) {
+  const long long q = n / chunk, r = n % chunk;
+  return chunk * (q * (q + 1) / 2) + (r ? n : 0);
 }
 // Workgroups of a pair launch: a multiple of 8 (one share per XCD).
 inline int pair_grid(int n_work) { return n_work >= 4096 ? 4096 : (n_work + 7) / 8 * 8; }

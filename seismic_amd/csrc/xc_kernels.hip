@@ -254,7 +254,7 @@ __device__ __forceinline__ void forward_row(const ForwardArgs& a, int row, const
 }
 
 // Item v of a segment-mode launch: row v / (2 n_seg), segment v / 2 % n_seg, row
-// side (v even) or column side.  Every wave sums its row's mean and energy
+// side (v even) or column side; with one side, row v / n_seg, segment v % n_seg.  Every wave sums its row's mean and energy
 // itself: a row is at most 8192 samples, which its 2 n_seg waves read from L2,
 // and a launch of its own would cost a small job more.
 template <int R>
@@ -262,8 +262,8 @@ __device__ __forceinline__ void forward_segment(const ForwardArgs& a, int v, con
                                                 float2* zl, int lane) {
   constexpr int P = 128 * R;
   wave_lds_fence();  // the previous item's reads of this wave's buffer come first
-  const bool col = v & 1;
-  const int row = (v >> 1) / a.n_seg, seg = (v >> 1) - row * a.n_seg, s0 = seg * a.seg_len;
+  const bool col = a.seg_sides ? a.seg_sides == 2 : (v & 1) != 0;
+  const int u = a.seg_sides ? v : v >> 1, row = u / a.n_seg, seg = u - row * a.n_seg, s0 = seg * a.seg_len;
   const float* x = a.in + (long long)row * a.in_stride;
   const int last = a.in_len - 1;
   constexpr int U = 8;  // 64-sample steps whose loads are in flight together
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(64 * fwd_waves<R>()) void k_forward(ForwardArgs a) 
   if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0u;
   stage_twiddles<TwLayout<R>::kFft, 64 * W>(twl, a.tw, threadIdx.x);
   __syncthreads();
-  const int n = SEG ? a.n_rows * 2 * a.n_seg : a.n_rows;
+  const int n = SEG ? a.n_rows * a.n_seg * (a.seg_sides ? 1 : 2) : a.n_rows;
   for (int row = blockIdx.x * W + wv; row < n; row += gridDim.x * W) {
     if constexpr (SEG) forward_segment<R>(a, row, twl, wl, zl, lane);
     else forward_row<R>(a, row, twl, wl, zl, lane);
@@ -1059,7 +1059,7 @@ hipError_t launch_forward_r(const ForwardArgs& a, hipStream_t st) {
   auto kernel = a.n_seg > 0 ? k_forward<R, true> : k_forward<R, false>;
   hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  const long long groups = ((long long)a.n_rows * (a.n_seg > 0 ? 2 * a.n_seg : 1) + W - 1) / W;
+  const long long groups = ((long long)a.n_rows * (a.n_seg > 0 ? a.n_seg * (a.seg_sides ? 1 : 2) : 1) + W - 1) / W;
   hipLaunchKernelGGL(kernel, dim3(groups < 1024 ? (int)groups : 1024), dim3(64 * W), lds, st, a);
   return hipGetLastError();
 }

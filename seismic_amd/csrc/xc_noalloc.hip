@@ -3,8 +3,10 @@
 //
 // No counterpart in the reference.  It serves callers that cannot call
 // hipMalloc -- code under HIP graph capture, tight serving loops, harnesses
-// that forbid allocation -- and runs exactly the kernels of sxc_plan_execute
-// with the same launch shapes.  Their workspace (spectra, norms, demeaned
+// that forbid allocation -- and runs the kernels of sxc_plan_execute at the same
+// period and on the same segments of the rows, so that the results are the same bit
+// for bit.  A job whose rows are cut and whose spectra do not fit runs in pairs of
+// event bands.  The workspace (spectra, norms, demeaned
 // traces, work list, near-tie records and counter, and the
 // twiddle tables of every FFT period) lives in one file-scope device array,
 // `scratch`, of kScratchBytes per GPU, held until the process ends.
@@ -36,19 +38,24 @@ constexpr long long kNoallocTieCap = 1LL << 20;  // near-tie records (16 B each)
 constexpr int kMaxDevices = 64;
 constexpr int kRadices[] = {8, 16, 24, 32, 40, 48, 64};
 
-// Work items (row i, first column) of column chunk c = blockIdx.x, in the
-// chunk-major order of the plan's host-built list: with K columns per chunk,
-// chunk c holds rows 0 .. min(N, K (c + 1)) - 1, and chunks before it
-// min(N, K (c' + 1)) each, i.e. K/2 c (c + 1) items while K (c' + 1) <= N, then
-// N per chunk.
-__global__ __launch_bounds__(256) void k_fill_work(int2* work, int n, int chunk) {
+// Work items (row i, first column) of column chunk c = blockIdx.x of the columns
+// [col0, col0 + n), in the chunk-major order of the plan's host-built list.
+// Rows before the columns: every one of them per chunk.  The columns' own
+// triangle (row0 == col0): with K columns per chunk, chunk c holds its rows 0 ..
+// min(N, K (c + 1)) - 1, and chunks before it min(N, K (c' + 1)) each, i.e. K/2 c
+// (c + 1) items while K (c' + 1) <= N, then N per chunk.
+__global__ __launch_bounds__(256) void k_fill_work(int2* work, int row0, int rows, int col0, int n, int chunk) {
   const long long c = blockIdx.x;
+  const int j0 = (int)(c * chunk);
+  if (row0 != col0) {
+    for (int i = threadIdx.x; i < rows; i += blockDim.x) work[c * rows + i] = make_int2(row0 + i, col0 + j0);
+    return;
+  }
   const long long q = n / chunk;  // chunks whose K (c' + 1) <= N
   const long long half = chunk / 2;
   const long long off = c <= q ? half * c * (c + 1) : half * q * (q + 1) + (c - q) * n;
-  const int j0 = (int)(c * chunk);
   const int j1 = min(n, j0 + chunk);
-  for (int i = threadIdx.x; i < j1; i += blockDim.x) work[off + i] = make_int2(i, max(i, j0));
+  for (int i = threadIdx.x; i < j1; i += blockDim.x) work[off + i] = make_int2(row0 + i, col0 + max(i, j0));
 }
 
 struct TableOffsets {
@@ -118,6 +125,34 @@ int scratch_for_device(int dev, DeviceScratch** out) {
 
 using namespace sxc;
 
+namespace {
+// Byte offsets of a call's workspace after the tables.
+struct Layout {
+  size_t norms, traces, ties, count, work, spec, end;
+};
+Layout layout(const sxc_plan& p, size_t begin, long long n_work, size_t spec_elems) {
+  const long long rows = (long long)p.d.n_events * p.d.n_channels;
+  Layout l;
+  size_t off = begin;
+  auto part = [&](size_t bytes) {
+    const size_t at = off;
+    off = align256(off + bytes);
+    return at;
+  };
+  l.norms = part((size_t)rows * sizeof(double));
+  l.traces = part(p.d.demean ? (size_t)rows * p.P * sizeof(float) : 0);
+  l.ties = part((size_t)p.tie_cap * sizeof(int4));
+  l.count = part(sizeof(unsigned));
+  l.work = part((size_t)n_work * sizeof(int2));
+  l.spec = part(spec_elems * sizeof(float2));
+  l.end = off;
+  return l;
+}
+// Work items of n columns' own triangle, or of as many rows before them: the
+// larger of the two.
+long long band_items(int n, int chunk) { return (long long)n * ((n + chunk - 1) / chunk); }
+}  // namespace
+
 // small: rows kept whole and the longest column chunks.
 static int execute_noalloc(const sxc_plan_desc* desc, bool small, const float* d_traces, long long trace_stride,
                            int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg,
@@ -137,38 +172,38 @@ static int execute_noalloc(const sxc_plan_desc* desc, bool small, const float* d
   }
   DeviceScratch* ds = nullptr;
   if ((rc = scratch_for_device(dev, &ds))) return rc;
-  // per-call layout after the tables
-  const long long rows = (long long)desc->n_events * desc->n_channels;
-  size_t off = ds->tables_end;
-  const size_t o_spec = off;
-  off = align256(off + p.spec_elems * sizeof(float2));
-  const size_t o_norms = off;
-  off = align256(off + (size_t)rows * sizeof(double));
-  const size_t o_traces = off;
-  if (desc->demean) off = align256(off + (size_t)rows * p.P * sizeof(float));
-  const size_t o_work = off;
-  off = align256(off + (size_t)p.n_work * sizeof(int2));
-  const size_t o_ties = off;
-  off = align256(off + (size_t)p.tie_cap * sizeof(int4));
-  const size_t o_count = off;
-  off = align256(off + sizeof(unsigned));
-  // a job at the limit keeps the fewest spectra and the shortest work list
-  if (off > kScratchBytes && !small)
-    return execute_noalloc(desc, true, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg, d_lags_neg,
-                           stream);
-  if (off > kScratchBytes) {
+  Layout l = layout(p, ds->tables_end, p.n_work, p.spec_elems);
+  int band = 0;  // events of a band, 0: the whole job at once
+  if (l.end > kScratchBytes && !small) {
+    // a job at the limit keeps the fewest spectra and the shortest work list; where
+    // a plan's execute cuts these rows, so do the bands
+    sxc_plan whole;
+    whole.chunk = 64;
+    fft_plan_geometry(*desc, kNoallocTieCap, false, &whole);
+    const bool fits = layout(whole, ds->tables_end, whole.n_work, whole.spec_elems).end <= kScratchBytes;
+    const int n_seg = fft_geom(&p, in_len, false).n_seg;
+    if (!fits || !n_seg)
+      return execute_noalloc(desc, true, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg,
+                             d_lags_neg, stream);
+    const size_t event_elems = (size_t)desc->n_channels * n_seg * p.cut.spec_stride;
+    for (int k = 2; l.end > kScratchBytes && band != p.chunk; ++k) {
+      band = ((desc->n_events + k - 1) / k + p.chunk - 1) / p.chunk * p.chunk;
+      l = layout(p, ds->tables_end, band_items(band, p.chunk), 2 * band * event_elems);
+    }
+  }
+  if (l.end > kScratchBytes) {
     set_error("this job needs %zu bytes of workspace; the no-allocation entry point holds at most %zu "
               "(%zu after the twiddle tables): use sxc_plan_execute",
-              off, kScratchBytes, kScratchBytes - ds->tables_end);
+              l.end, kScratchBytes, kScratchBytes - ds->tables_end);
     return SXC_ERR_INVALID;
   }
   unsigned char* b = ds->base;
-  p.spec = (float2*)(b + o_spec);
-  p.norms = (double*)(b + o_norms);
-  p.traces = desc->demean ? (float*)(b + o_traces) : nullptr;
-  p.work = (int2*)(b + o_work);
-  p.ties = (int4*)(b + o_ties);
-  p.tie_count = (unsigned*)(b + o_count);
+  p.spec = (float2*)(b + l.spec);
+  p.norms = (double*)(b + l.norms);
+  p.traces = desc->demean ? (float*)(b + l.traces) : nullptr;
+  p.work = (int2*)(b + l.work);
+  p.ties = (int4*)(b + l.ties);
+  p.tie_count = (unsigned*)(b + l.count);
   p.fwd2 = (float2*)(b + ds->tab[p.R].fwd);
   p.inv2 = (float2*)(b + ds->tab[p.R].inv);
   p.post = (float2*)(b + ds->tab[p.R].post);
@@ -181,15 +216,26 @@ static int execute_noalloc(const sxc_plan_desc* desc, bool small, const float* d
   p.device = dev;
   hipStream_t st = (hipStream_t)stream;
   p.last_stream = st;
-  // the work list of this call (the previous call's contents are stale); the
-  // tie counter is cleared by the execute itself
-  const int n_chunks = (desc->n_events + p.chunk - 1) / p.chunk;
-  hipLaunchKernelGGL(k_fill_work, dim3(n_chunks), dim3(256), 0, st, p.work, desc->n_events, p.chunk);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    set_error("scratch set-up launches failed: %s", hipGetErrorString(e));
-    return SXC_ERR_HIP;
+  // the work list of these rows and columns (the previous call's contents are
+  // stale); the tie counter is cleared by the execute itself
+  auto fill = [&](int row0, int rows, int col0, int cols) -> int {
+    const int n_chunks = (cols + p.chunk - 1) / p.chunk;
+    hipLaunchKernelGGL(k_fill_work, dim3(n_chunks), dim3(256), 0, st, p.work, row0, rows, col0, cols, p.chunk);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      set_error("scratch set-up launches failed: %s", hipGetErrorString(e));
+      return SXC_ERR_HIP;
+    }
+    return (int)(row0 == col0 ? triangle_items(cols, p.chunk) : (long long)rows * n_chunks);
+  };
+  if (band) {
+    const FftGeom g = fft_geom(&p, in_len, false);
+    float2* cols = p.spec + (size_t)band * desc->n_channels * g.n_seg * g.spec_stride;
+    return fft_plan_execute_bands(&p, g, band, p.spec, cols, d_traces, trace_stride, in_len, d_vals_pos, d_lags_pos,
+                                  d_vals_neg, d_lags_neg, fill, st);
   }
+  const int n_work = fill(0, desc->n_events, 0, desc->n_events);
+  if (n_work < 0) return n_work;
   return fft_plan_execute(&p, d_traces, nullptr, trace_stride, in_len, d_vals_pos, d_lags_pos, d_vals_neg,
                           d_lags_neg, st);
 }

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <functional>
 #include <vector>
 
 #include "../../include/seismic_xcorr.h"
@@ -104,6 +105,14 @@ FftGeom fft_geom(const sxc_plan* p, int in_len, bool reversed);
 // FP64 resolver on the plan's workspace (asynchronous on st).
 int fft_plan_execute(sxc_plan* p, const float* d_traces, const float* d_rev, long long trace_stride, int in_len,
                      float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg, hipStream_t st);
+// FFT form: the same with cut rows in the memory of two bands of `band` events (a
+// multiple of the column chunk): `rows` and `cols` take one band's row and column
+// spectra, every pair of bands is run in turn, and fill(row0, rows, col0, cols)
+// enqueues the pair's work items into p->work and returns their number.  The
+// outputs equal fft_plan_execute's.
+int fft_plan_execute_bands(sxc_plan* p, const FftGeom& g, int band, float2* rows, float2* cols, const float* d_traces,
+                           long long trace_stride, int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg,
+                           int* d_lags_neg, const std::function<int(int, int, int, int)>& fill, hipStream_t st);
 // FFT form, blocked (host-buffer calls): fft_plan_blocks prepares B event
 // bands and the 2B - 1 launch groups; with event band b's traces on the
 // device, fft_plan_forward_events transforms them and fft_plan_group(b) (b <

@@ -101,3 +101,33 @@ def test_noalloc_equals_the_unmasked_scan(thr):
     for a, o, name in zip(ref, outs, ("vals_pos", "lags_pos", "vals_neg", "lags_neg")):
         assert np.array_equal(a, o.numpy()), name
     plan.close()
+
+
+@pytest.mark.parametrize("n,C,L,P,lo,hi,in_len,demean", [
+    (3000, 1, 4096, 8192, -50, 50, 4096, False),   # two bands of whole segments, the last one shorter
+    (1600, 1, 4096, 8192, -50, 50, 4096, True),
+    (3000, 2, 2048, 4096, -100, 100, 2048, False),
+    (3000, 1, 4096, 8192, -50, 50, 2000, False),   # rows of fewer segments
+    (3000, 1, 4096, 8192, -50, 50, 6000, False),   # rows too long to be cut: whole rows
+])
+def test_noalloc_beyond_the_array_with_cut_rows(n, C, L, P, lo, hi, in_len, demean):
+    """Jobs whose rows a plan cuts in segments and whose segment spectra exceed
+    the array (whole rows at P would fit): pairs of event bands, the same bits."""
+    lib = _lib.load_engine()
+    x, _ = synth.make_events(n, C, in_len, seed=n + L)
+    x += np.float32(0.25 * demean)
+    print(f"case noalloc bands N={n} C={C} L={L} P={P} [{lo},{hi}] in_len={in_len} demean={demean}", flush=True)
+    d = DeviceArray.from_numpy(x)
+    plan = engine.AllPairsPlan(n, C, L, P, lo, hi, demean=demean)
+    stream = Stream()
+    ref = plan.execute(d, in_len=in_len, stream=stream)
+    stream.synchronize()
+    ref = [o.numpy() for o in ref]
+    outs = plan.alloc_outputs()
+    for o in outs:
+        o.zero_()
+    assert _noalloc(lib, plan.desc, d, in_len, in_len, outs, stream) == 0, _lib.last_error(lib)
+    stream.synchronize()
+    for a, o, name in zip(ref, outs, ("vals_pos", "lags_pos", "vals_neg", "lags_neg")):
+        assert np.array_equal(a, o.numpy()), name
+    plan.close()

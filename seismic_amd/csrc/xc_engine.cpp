@@ -737,7 +737,7 @@ const char* seismic_last_error(void) { return last_error(); }
 
 // Geometry of an FFT-form plan (no device memory): period, strides, pair and
 // work-item counts, near-tie band and record capacity.
-void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bool may_cut, sxc_plan* p) {
+void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Rows how, sxc_plan* p) {
   p->d = desc;
   p->P = desc.padded_size;
   p->M = p->P / 2;
@@ -776,7 +776,7 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bo
   // L = 2048, +-100 3.67 -> 1.17; C = 3, L = 2500, +-60 7.23 -> 3.21; N = 16, C = 1,
   // L = 4096, +-50 114 -> 37 us.
   const int P1 = p->narrow.P ? p->narrow.P : p->P;  // the period of executes on whole rows
-  if (may_cut && desc.trace_len + reach <= p->P) {
+  if (how == Rows::kCut && desc.trace_len + reach <= p->P) {
     double best = 0.95 * pair_cost(P1 / 128, desc.n_channels);
     for (int P : {1024, 2048, 3072, 4096, 5120}) {
       const int len = P - std::max(0, desc.lag_hi) - std::max(0, -desc.lag_lo);
@@ -804,17 +804,10 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bo
   p->n_work = (int)triangle_items(desc.n_events, p->chunk);
 }
 
-extern "C" {
-
-int sxc_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
-  clear_error();
-  if (!desc || !out) { set_error("null argument"); return SXC_ERR_INVALID; }
-  *out = nullptr;
-  int rc = validate_desc(*desc);
-  if (rc) return rc;
-  if (is_lag_form(desc->form)) return lag_plan_create(desc, out);
+static int fft_plan_create(const sxc_plan_desc* desc, Rows how, sxc_plan** out) {
+  int rc;
   sxc_plan* p = new sxc_plan();
-  fft_plan_geometry(*desc, 1LL << 24, true, p);
+  fft_plan_geometry(*desc, 1LL << 24, how, p);
   HIP_CHECK(hipGetDevice(&p->device));
   const long long rows = (long long)desc->n_events * desc->n_channels;
   auto fail = [&](int code) { plan_free(p); return code; };
@@ -835,6 +828,23 @@ int sxc_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
     if (g->P && (rc = upload_tables(g->R, &g->fwd2, &g->inv2, &g->post))) return fail(rc);
   *out = p;
   return SXC_OK;
+}
+
+extern "C" {
+
+int sxc_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
+  clear_error();
+  if (!desc || !out) { set_error("null argument"); return SXC_ERR_INVALID; }
+  *out = nullptr;
+  int rc = validate_desc(*desc);
+  if (rc) return rc;
+  if (is_lag_form(desc->form)) return lag_plan_create(desc, out);
+  rc = fft_plan_create(desc, Rows::kCut, out);
+  if (rc == SXC_ERR_MEMORY) {  // the spectra of cut rows may not fit where whole rows' do
+    clear_error();
+    rc = fft_plan_create(desc, Rows::kWhole, out);
+  }
+  return rc;
 }
 
 int sxc_plan_destroy(sxc_plan* plan) {

@@ -160,7 +160,7 @@ static int execute_noalloc(const sxc_plan_desc* desc, bool small, const float* d
   int rc;
   sxc_plan p;
   p.chunk = small ? 64 : 0;
-  fft_plan_geometry(*desc, kNoallocTieCap, !small, &p);
+  fft_plan_geometry(*desc, kNoallocTieCap, small ? Rows::kWhole : Rows::kCut, &p);
   if (in_len < 1 || in_len > p.P || trace_stride < in_len) {
     set_error("in_len %d must be in [1, P=%d] and <= trace_stride %lld", in_len, p.P, trace_stride);
     return SXC_ERR_INVALID;
@@ -179,7 +179,7 @@ static int execute_noalloc(const sxc_plan_desc* desc, bool small, const float* d
     // a plan's execute cuts these rows, so do the bands
     sxc_plan whole;
     whole.chunk = 64;
-    fft_plan_geometry(*desc, kNoallocTieCap, false, &whole);
+    fft_plan_geometry(*desc, kNoallocTieCap, Rows::kWhole, &whole);
     const bool fits = layout(whole, ds->tables_end, whole.n_work, whole.spec_elems).end <= kScratchBytes;
     const int n_seg = fft_geom(&p, in_len, false).n_seg;
     if (!fits || !n_seg)

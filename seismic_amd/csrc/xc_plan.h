@@ -25,6 +25,7 @@ inline int dev_alloc(T** p, size_t count, const char* what) {
   if (count == 0) count = 1;
   hipError_t e = hipMalloc((void**)p, count * sizeof(T));
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch would report it
     set_error("device allocation of %s (%zu bytes) failed: %s", what, count * sizeof(T), hipGetErrorString(e));
     *p = nullptr;
     return SXC_ERR_MEMORY;
@@ -95,9 +96,12 @@ struct sxc_plan {
 
 void plan_free(sxc_plan* p);
 namespace sxc {
-// FFT form: fills the plan's geometry (no device memory); may_cut: with rows cut
-// in segments where that is faster, which takes more memory for spectra.
-void fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, bool may_cut, sxc_plan* p);
+// Rows of an FFT-form plan's executes: cut in segments where that is faster, which
+// takes more memory for spectra; or whole, at the smallest period that gives the
+// window.
+enum class Rows { kCut, kWhole };
+// FFT form: fills the plan's geometry (no device memory).
+void fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Rows how, sxc_plan* p);
 // FFT form: the period an execute on rows of in_len samples runs at, and
 // whether it scans every lag.
 FftGeom fft_geom(const sxc_plan* p, int in_len, bool reversed);

@@ -12,6 +12,7 @@ size_t limit = (size_t)1 << 40;
 static std::mutex mu;
 static std::map<const char*, size_t> blocks;
 static size_t in_use = 0;
+static hipError_t last = hipSuccess;  // as hipGetLastError would return it
 
 size_t used() {
   std::lock_guard<std::mutex> lk(mu);
@@ -38,7 +39,7 @@ extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
   std::lock_guard<std::mutex> lk(mu);
   *p = nullptr;
-  if (n > limit || in_use > limit - n) return hipErrorOutOfMemory;
+  if (n > limit || in_use > limit - n) return last = hipErrorOutOfMemory;
   *p = calloc(n ? n : 1, 1);
   blocks[(const char*)*p] = n;
   in_use += n;
@@ -53,6 +54,11 @@ hipError_t hipFree(void* p) {
     free(p);
   }
   return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = last;
+  last = hipSuccess;
+  return e;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   *p = malloc(n ? n : 1);
@@ -112,7 +118,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
 namespace sxc {
 template <typename F, typename... A>
 static hipError_t call(const F& f, const A&... a) {
-  return f && f(a...) ? hipErrorLaunchFailure : hipSuccess;
+  return f && f(a...) ? hipErrorLaunchFailure : hipGetLastError();  // the launchers report it
 }
 hipError_t launch_forward(int R, const ForwardArgs& a, hipStream_t) {
   if (a.zero) *a.zero = 0u;

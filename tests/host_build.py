@@ -11,8 +11,9 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 CLANG = os.path.join(ROCM, "llvm", "bin", "clang++")
 
 
-def run_host(tmp_path, program, sources):
-    """Builds HOST/program with the named engine sources; returns (status, output)."""
+def run_host(tmp_path, program, sources, *args):
+    """Builds HOST/program with the named engine sources and runs it with args;
+    returns (status, output)."""
     srcs = [os.path.join(HOST, program), os.path.join(HOST, "standin.cpp")] + [os.path.join(CSRC, s) for s in sources]
     objs = [str(tmp_path / (os.path.basename(s) + ".o")) for s in srcs]
 
@@ -24,5 +25,5 @@ def run_host(tmp_path, program, sources):
         list(pool.map(compile_one, zip(srcs, objs)))
     exe = str(tmp_path / "program")
     subprocess.run([CLANG, *objs, "-lpthread", "-o", exe], check=True)
-    r = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    r = subprocess.run([exe, *args], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     return r.returncode, r.stdout

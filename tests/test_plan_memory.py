@@ -1,0 +1,11 @@
+"""Device memory of plans, on the CPU (the engine's host code with a stand-in HIP
+runtime that counts allocations against a limit): a plan that can be made in
+less memory is made where its first choice does not fit."""
+from host_build import run_host
+
+SOURCES = ["xc_engine.cpp", "xc_hostio.cpp"]
+
+
+def test_fft_plan_keeps_rows_whole_where_segments_do_not_fit(tmp_path):
+    rc, out = run_host(tmp_path, "plan_memory.cpp", SOURCES, "fft")
+    assert rc == 0, f"status {rc}: {out}"

@@ -477,6 +477,8 @@ static size_t job_cache_budget() {
   return mb > 0 ? (size_t)mb << 20 : 0;
 }
 
+static int fft_plan_create(const sxc_plan_desc* desc, Rows how, sxc_plan** out);
+
 static int job_acquire(const sxc_plan_desc& d, long long stride, bool reversed, int n_classes, HostJob** out) {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
@@ -498,7 +500,7 @@ static int job_acquire(const sxc_plan_desc& d, long long stride, bool reversed, 
   j->reversed = reversed;
   j->n_classes = n_classes;
   j->device = dev;
-  int rc = sxc_plan_create(&d, &j->p);
+  int rc = reversed && !is_lag_form(d.form) ? fft_plan_create(&d, Rows::kPeriod, &j->p) : sxc_plan_create(&d, &j->p);
   const long long rows = (long long)d.n_events * d.n_channels;
   const size_t in = (size_t)(rows * stride), np = (size_t)d.n_events * (d.n_events + 1) / 2;
   if (!rc) rc = dev_alloc(&j->in, in, "input traces");
@@ -758,7 +760,7 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Ro
   // C = 3, L = 2048, P = 4096, +-512 runs at 3072: 17.7 -> 13.4 ms.
   const int reach = std::max(std::abs(desc.lag_lo), std::abs(desc.lag_hi));
   for (int P : {1024, 2048, 3072, 4096, 5120, 6144})
-    if (P < p->P && P >= desc.trace_len + reach && desc.lag_lo > -P / 2 && desc.lag_hi <= P / 2) {
+    if (how != Rows::kPeriod && P < p->P && P >= desc.trace_len + reach && desc.lag_lo > -P / 2 && desc.lag_hi <= P / 2) {
       p->narrow.P = P;
       p->narrow.M = P / 2;
       p->narrow.R = P / 128;

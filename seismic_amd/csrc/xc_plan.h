@@ -98,8 +98,8 @@ void plan_free(sxc_plan* p);
 namespace sxc {
 // Rows of an FFT-form plan's executes: cut in segments where that is faster, which
 // takes more memory for spectra; or whole, at the smallest period that gives the
-// window.
-enum class Rows { kCut, kWhole };
+// window; or whole, at the caller's period, as reversed-row executes run.
+enum class Rows { kCut, kWhole, kPeriod };
 // FFT form: fills the plan's geometry (no device memory).
 void fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Rows how, sxc_plan* p);
 // FFT form: the period an execute on rows of in_len samples runs at, and

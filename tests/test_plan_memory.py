@@ -9,3 +9,8 @@ SOURCES = ["xc_engine.cpp", "xc_hostio.cpp"]
 def test_fft_plan_keeps_rows_whole_where_segments_do_not_fit(tmp_path):
     rc, out = run_host(tmp_path, "plan_memory.cpp", SOURCES, "fft")
     assert rc == 0, f"status {rc}: {out}"
+
+
+def test_reversed_row_jobs_hold_one_period(tmp_path):
+    rc, out = run_host(tmp_path, "reversed_job.cpp", SOURCES)
+    assert rc == 0, f"status {rc}: {out}"

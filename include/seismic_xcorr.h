@@ -58,7 +58,8 @@ typedef struct {
   int lag_hi;        /* last scanned lag >= lag_lo: FFT form <= P/2, lag forms < L */
   float threshold;   /* pos kept if > threshold, neg if < -threshold */
   float tie_tol;     /* near-tie band in coefficient units; <= 0 selects the form's default
-                        (FFT 2e-6, bf16x3 2e-5, fp16 2.5e-4) */
+                        (FFT 2e-6, bf16x3 2e-5, fp16 2.5e-4); the lag forms widen it by 4e-6, as
+                        they rank lags by all but the last four bits of their FP32 values */
   int demean;        /* 1: subtract the FP64 mean of the first L samples of each trace */
   int form;          /* SXC_FORM_* */
 } sxc_plan_desc;

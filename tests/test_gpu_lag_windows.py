@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from seismic_amd import engine
+from seismic_amd.device import DeviceArray, synchronize
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +60,36 @@ def test_nonfinite_rows(oracle, name, lo, hi, at, bad):
     hit = (pi == e) | (pj == e)
     assert not vp[hit].any() and not lp[hit].any() and not vn[hit].any() and not ln[hit].any()
     assert np.abs(vp - ref["pos"])[~hit].max() <= tol and np.abs(vn - ref["neg"])[~hit].max() <= tol
+
+
+def test_lags_beyond_the_record_capacity():
+    """More near ties than records (a band of every value): the pairs beyond the
+    capacity keep the lag of their FP32 extremum, also where another lag is within
+    16 units in the last place.  Single spikes against events with two spikes of
+    0.6875 + 3 and + 6 such units: every product is exact."""
+    n, L, w = 5800, 64, 30
+    rng = np.random.default_rng(5)
+    at = rng.integers(20, 45, n)
+    x = np.zeros((n, 1, L), np.float32)
+    e = np.arange(n)
+    one, two = e[::2], e[1::2]
+    x[one, 0, at[one]] = 1.0
+    a, b = 0.6875 + 3 * 2.0**-24, 0.6875 + 6 * 2.0**-24
+    x[two, 0, at[two]] = a
+    x[two, 0, at[two] - 1] = b
+    x[two, 0, at[two] + 12] = np.sqrt(1.0 - a * a - b * b)
+    print(f"case records beyond the capacity N={n} L={L} +-{w}", flush=True)
+    plan = engine.AllPairsPlan(n, 1, L, 0, -w, w, tie_tol=10.0, form=engine.FORM_LAG_BF16X3)
+    out = plan.execute(DeviceArray.from_numpy(x))
+    synchronize()
+    vp, lp, vn, ln = [o.numpy() for o in out]
+    stats = plan.stats()
+    plan.close()
+    assert stats["tie_overflow"] > 10000
+    i, j = np.triu_indices(n)
+    k = (i % 2 == 0) & (j % 2 == 1)
+    assert np.array_equal(lp[k], at[i[k]] - (at[j[k]] - 1)) and np.abs(vp[k] - b).max() <= 2e-7
+    k = (i % 2 == 1) & (j % 2 == 0)
+    assert np.array_equal(lp[k], at[i[k]] - 1 - at[j[k]])
+    k = (i % 2 == 0) & (j % 2 == 0)
+    assert np.array_equal(lp[k], at[i[k]] - at[j[k]]) and (vp[k] == 1.0).all()

@@ -121,7 +121,7 @@ void plan_free(sxc_plan* p) {
   for (hipEvent_t e : p->events) (void)hipEventDestroy(e);
   void* bufs[] = {p->spec, p->col_spec, p->norms, p->traces, p->work, p->ties, p->tie_count,
                   p->fwd2, p->narrow.fwd2, p->cut.fwd2, p->h_hi, p->lag_traces, p->tiles,
-                  p->fnorms, p->wide, p->wide_count, p->blk_work, p->grp_count};
+                  p->fnorms, p->wide, p->wide_count, p->blk_work, p->grp_count, p->energy};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   delete p;
@@ -188,10 +188,25 @@ static std::vector<int2> build_work(int n, int chunk) {
 
 // Lag-window form: the row and column operands of every trace as bf16 (hi, lo)
 // or fp16, 32 x 32 pair tiles of the upper triangle, blocks of kLagBlock lags.
+// The row operands are two copies of every trace: where they do not fit, they are
+// held for a band of events at a time and made again for each.
+int lag_smaller_band(int band) { return band > 32 ? (band / 2 + 31) / 32 * 32 : 0; }
+
 int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
+  int rc = SXC_ERR_MEMORY;
+  for (int band = desc->n_events; rc == SXC_ERR_MEMORY && band > 0; band = lag_smaller_band(band)) {
+    clear_error();
+    rc = sxc_lag_plan_create_band(desc, band, out);
+  }
+  return rc;
+}
+
+int sxc_lag_plan_create_band(const sxc_plan_desc* desc, int band, sxc_plan** out) {
+  if (!desc || !out || band < 1 || (band < desc->n_events && band % 32)) { set_error("band must be a multiple of 32"); return SXC_ERR_INVALID; }
   sxc_plan* p = new sxc_plan();
   p->d = *desc;
   p->lag = true;
+  p->row_band = std::min(band, desc->n_events);
   const int L = desc->trace_len;
   p->l16 = (L + 15) / 16 * 16;
   p->lag_first = desc->lag_lo;
@@ -210,7 +225,8 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
   int rc;
   // one allocation (h_hi) for the operands
   const LagOperands ops =
-      lag_operands(rows, (desc->n_events + 31LL) / 32 * 32 * desc->n_channels, p->hs, p->l16);
+      lag_operands((long long)p->row_band * desc->n_channels, (desc->n_events + 31LL) / 32 * 32 * desc->n_channels,
+                   p->hs, p->l16);
   const bool two = desc->form == SXC_FORM_LAG_BF16X3;
   if ((rc = dev_alloc(&p->h_hi, (size_t)(ops.h + ops.b) * (two ? 2 : 1), "trace operands"))) return fail(rc);
   p->b_hi = p->h_hi + ops.h;
@@ -219,6 +235,7 @@ int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out) {
     p->b_lo = p->h_lo + ops.h;
   }
   if ((rc = dev_alloc(&p->norms, (size_t)rows, "norms"))) return fail(rc);
+  if (p->row_band < desc->n_events && (rc = dev_alloc(&p->energy, (size_t)rows, "energies"))) return fail(rc);
   if ((rc = dev_alloc(&p->lag_traces, (size_t)(rows * L), "FP32 traces"))) return fail(rc);
   const int T = (desc->n_events + 31) / 32;
   std::vector<int2> tiles;
@@ -305,37 +322,64 @@ int sxc::lag_plan_resolve_wide(sxc_plan* p, long long n_pairs, float* vp, int* l
   return SXC_OK;
 }
 
-int lag_plan_prep(sxc_plan* p, const float* d_traces, long long trace_stride, int in_len, hipStream_t st) {
+// Arguments of a launch over the rows of events [e0, e1).
+static LagPrepArgs lag_prep_args(const sxc_plan* p, int e0, int e1) {
   const sxc_plan_desc& d = p->d;
-  const int rows = d.n_events * d.n_channels;
+  const long long r0 = (long long)e0 * d.n_channels;
   LagPrepArgs pa{};
-  pa.in = d_traces;
-  pa.in_stride = trace_stride;
-  pa.in_len = in_len;
   pa.L = d.trace_len;
-  pa.n_rows = rows;
+  pa.n_rows = (e1 - e0) * d.n_channels;
   pa.n_channels = d.n_channels;
-  pa.demean = d.demean;
   pa.fp16 = d.form == SXC_FORM_LAG_FP16;
   pa.lag_first = p->lag_first;
   pa.hs = p->hs;
   pa.l16 = p->l16;
   pa.h_hi = p->h_hi;
   pa.h_lo = p->h_lo;
-  pa.b_hi = p->b_hi;
-  pa.b_lo = p->b_lo;
-  pa.zero0 = p->tie_count;
-  pa.zero1 = p->wide_count;
-  pa.norms = p->norms;
-  pa.traces_out = p->lag_traces;
-  HIP_CHECK(launch_lag_prep(pa, st));
+  pa.b_hi = p->b_hi + r0 * p->l16;  // e0 is a multiple of 32: whole column tiles
+  pa.b_lo = p->b_lo ? p->b_lo + r0 * p->l16 : nullptr;
+  pa.norms = p->norms + r0;
+  return pa;
+}
+
+int lag_plan_prep(sxc_plan* p, const float* d_traces, long long trace_stride, int in_len, hipStream_t st) {
+  const sxc_plan_desc& d = p->d;
+  for (int e0 = 0; e0 < d.n_events; e0 += p->row_band) {
+    const long long r0 = (long long)e0 * d.n_channels;
+    LagPrepArgs pa = lag_prep_args(p, e0, std::min(d.n_events, e0 + p->row_band));
+    pa.in = d_traces + r0 * trace_stride;
+    pa.in_stride = trace_stride;
+    pa.in_len = in_len;
+    pa.demean = d.demean;
+    pa.zero0 = e0 ? nullptr : p->tie_count;
+    pa.zero1 = e0 ? nullptr : p->wide_count;
+    pa.energy = p->energy ? p->energy + r0 : nullptr;
+    pa.traces_out = p->lag_traces + r0 * d.trace_len;
+    HIP_CHECK(launch_lag_prep(pa, st));
+    p->row_first = e0;
+  }
   return SXC_OK;
 }
 
-sxc::LagPairArgs sxc::lag_pair_args(const sxc_plan* p) {
-  LagPairArgs ka{};
-  ka.h_hi = p->h_hi;
-  ka.h_lo = p->h_lo;
+// The row operands of the band from event e0 on, unless they are the ones held.
+static int lag_plan_rows(sxc_plan* p, int e0, hipStream_t st) {
+  if (p->row_first == e0) return SXC_OK;
+  const long long r0 = (long long)e0 * p->d.n_channels;
+  LagPrepArgs pa = lag_prep_args(p, e0, std::min(p->d.n_events, e0 + p->row_band));
+  pa.in = p->lag_traces + r0 * p->d.trace_len;
+  pa.in_stride = pa.in_len = p->d.trace_len;
+  pa.energy_in = p->energy + r0;
+  HIP_CHECK(launch_lag_prep(pa, st));
+  p->row_first = e0;
+  return SXC_OK;
+}
+
+static LagPairArgs lag_pair_args(const sxc_plan* p, const LagPairArgs& base) {
+  LagPairArgs ka = base;
+  // the pair kernel finds event i's row operand i events from these
+  const size_t held = (size_t)p->row_first * p->d.n_channels * 2 * p->hs * sizeof(unsigned short);
+  ka.h_hi = (const unsigned short*)((uintptr_t)p->h_hi - held);
+  ka.h_lo = p->h_lo ? (const unsigned short*)((uintptr_t)p->h_lo - held) : nullptr;
   ka.b_hi = p->b_hi;
   ka.b_lo = p->b_lo;
   ka.hs = p->hs;
@@ -354,6 +398,23 @@ sxc::LagPairArgs sxc::lag_pair_args(const sxc_plan* p) {
   return ka;
 }
 
+int sxc::lag_plan_pairs(sxc_plan* p, const LagPairArgs& base, int row0, int rows,
+                        const std::function<long long(int)>& tiles, hipStream_t st) {
+  const int band = p->row_band, last = (row0 + rows - 1) / band;
+  // from the last band back: the preparation of all rows leaves its operands
+  for (int k = last; k >= row0 / band; --k) {
+    const int e0 = std::max(row0, k * band), e1 = std::min(row0 + rows, (k + 1) * band);
+    int rc = lag_plan_rows(p, k * band, st);
+    if (rc) return rc;
+    LagPairArgs ka = lag_pair_args(p, base);
+    const long long t0 = tiles((e0 - row0) / 32), t1 = tiles((e1 - row0 + 31) / 32);
+    ka.tiles = base.tiles + t0;
+    ka.n_tiles = (int)(t1 - t0);
+    HIP_CHECK(launch_lag_pairs(p->d.form == SXC_FORM_LAG_BF16X3, ka, st));
+  }
+  return SXC_OK;
+}
+
 static int lag_plan_execute(sxc_plan* p, const float* d_traces, long long trace_stride, int in_len,
                             float* vp, int* lp, float* vn, int* ln, hipStream_t st) {
   const sxc_plan_desc& d = p->d;
@@ -364,14 +425,14 @@ static int lag_plan_execute(sxc_plan* p, const float* d_traces, long long trace_
   if (rc) return rc;
   if ((rc = lag_plan_spectra(p, st))) return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[1], st));
-  LagPairArgs ka = lag_pair_args(p);
+  LagPairArgs ka{};
   ka.tiles = p->tiles;
-  ka.n_tiles = p->n_tiles;
   ka.vpos = vp;
   ka.lpos = lp;
   ka.vneg = vn;
   ka.lneg = ln;
-  HIP_CHECK(launch_lag_pairs(d.form == SXC_FORM_LAG_BF16X3, ka, st));
+  const long long T = (d.n_events + 31) / 32;
+  if ((rc = lag_plan_pairs(p, ka, 0, d.n_events, [T](long long r) { return r * T - r * (r - 1) / 2; }, st))) return rc;
   if (ev) HIP_CHECK(hipEventRecord(ev[2], st));
   LagResolveArgs ra{};
   ra.traces = p->lag_traces;
@@ -449,7 +510,8 @@ static size_t plan_device_bytes(const sxc_plan* p) {
   b += (size_t)p->n_work * sizeof(int2) * (p->blk_work ? 2 : 1) +
        (size_t)p->tie_cap * sizeof(int4) * (p->lag ? 3 : 1);
   if (p->lag)
-    b += rows * ((size_t)p->hs * 2 + p->l16) * 2 * (p->h_lo ? 2 : 1) + rows * (size_t)p->d.trace_len * sizeof(float);
+    b += ((size_t)p->row_band * p->d.n_channels * p->hs * 2 + rows * p->l16) * 2 * (p->h_lo ? 2 : 1) +
+         rows * (size_t)p->d.trace_len * sizeof(float) + (p->energy ? rows * sizeof(double) : 0);
   return b;
 }
 
@@ -479,6 +541,24 @@ static size_t job_cache_budget() {
 
 static int fft_plan_create(const sxc_plan_desc* desc, Rows how, sxc_plan** out);
 
+// A job's plan (FFT form: with these rows; lag forms: row operands for `band` events
+// at a time) and buffers.
+static int job_make(HostJob* j, Rows how, int band) {
+  const sxc_plan_desc& d = j->d;
+  int rc = validate_desc(d);
+  if (!rc) rc = is_lag_form(d.form) ? sxc_lag_plan_create_band(&d, band, &j->p) : fft_plan_create(&d, how, &j->p);
+  const size_t in = (size_t)d.n_events * d.n_channels * j->stride, np = (size_t)d.n_events * (d.n_events + 1) / 2;
+  if (!rc) rc = dev_alloc(&j->in, in, "input traces");
+  if (!rc && j->reversed) rc = dev_alloc(&j->rev, in, "reversed traces");
+  if (!rc) rc = dev_alloc(&j->vp, np, "output values");
+  if (!rc) rc = dev_alloc(&j->vn, np, "output values");
+  if (!rc) rc = dev_alloc(&j->lp, np, "output lags");
+  if (!rc) rc = dev_alloc(&j->ln, np, "output lags");
+  if (!rc && j->n_classes > 0) rc = dev_alloc(&j->hist, 2 * (size_t)j->n_classes, "histograms");
+  j->buf_bytes = (in * (j->reversed ? 2 : 1) + 4 * np + 2 * (size_t)j->n_classes) * 4;
+  return rc;
+}
+
 static int job_acquire(const sxc_plan_desc& d, long long stride, bool reversed, int n_classes, HostJob** out) {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
@@ -494,29 +574,29 @@ static int job_acquire(const sxc_plan_desc& d, long long stride, bool reversed, 
       }
     }
   }
-  HostJob* j = new HostJob();
-  j->d = d;
-  j->stride = stride;
-  j->reversed = reversed;
-  j->n_classes = n_classes;
-  j->device = dev;
-  int rc = reversed && !is_lag_form(d.form) ? fft_plan_create(&d, Rows::kPeriod, &j->p) : sxc_plan_create(&d, &j->p);
-  const long long rows = (long long)d.n_events * d.n_channels;
-  const size_t in = (size_t)(rows * stride), np = (size_t)d.n_events * (d.n_events + 1) / 2;
-  if (!rc) rc = dev_alloc(&j->in, in, "input traces");
-  if (!rc && reversed) rc = dev_alloc(&j->rev, in, "reversed traces");
-  if (!rc) rc = dev_alloc(&j->vp, np, "output values");
-  if (!rc) rc = dev_alloc(&j->vn, np, "output values");
-  if (!rc) rc = dev_alloc(&j->lp, np, "output lags");
-  if (!rc) rc = dev_alloc(&j->ln, np, "output lags");
-  if (!rc && n_classes > 0) rc = dev_alloc(&j->hist, 2 * (size_t)n_classes, "histograms");
-  if (rc) {
+  Rows how = reversed ? Rows::kPeriod : Rows::kCut;
+  for (int band = d.n_events;;) {
+    HostJob* j = new HostJob();
+    j->d = d;
+    j->stride = stride;
+    j->reversed = reversed;
+    j->n_classes = n_classes;
+    j->device = dev;
+    const int rc = job_make(j, how, band);
+    if (rc == SXC_OK) {
+      *out = j;
+      return SXC_OK;
+    }
     job_free(j);
-    return rc;
+    if (rc != SXC_ERR_MEMORY) return rc;
+    if (is_lag_form(d.form)) {
+      if ((band = lag_smaller_band(band)) == 0) return rc;
+    } else {
+      if (how != Rows::kCut) return rc;
+      how = Rows::kWhole;
+    }
+    clear_error();
   }
-  j->buf_bytes = (in * (reversed ? 2 : 1) + 4 * np + 2 * (size_t)n_classes) * 4;
-  *out = j;
-  return SXC_OK;
 }
 
 // Back to the cache (or freed); evicts the least recently used idle jobs

@@ -42,6 +42,10 @@ struct LagPrepArgs {
   unsigned* zero0;          // optional counters to clear
   unsigned* zero1;
   double* norms;            // [n_rows]
+  double* energy;           // optional [n_rows]
+  // Row operands alone, of traces demeaned before, with the energies an earlier
+  // launch left.
+  const double* energy_in;
   float* traces_out;        // [n_rows][L] FP32 copy (demeaned) for the FP64 resolver
 };
 

@@ -84,30 +84,38 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
   }
   const float* x = a.in + (long long)row * a.in_stride;
   __shared__ double red[256];
-  double s1 = 0.0;
-  for (int n = threadIdx.x; n < a.L; n += 256) s1 += (double)(n < a.in_len ? x[n] : 0.f);
-  red[threadIdx.x] = s1;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+  double mean = 0.0, E;
+  if (a.energy_in) {
+    E = a.energy_in[row];
+  } else {
+    double s1 = 0.0;
+    for (int n = threadIdx.x; n < a.L; n += 256) s1 += (double)(n < a.in_len ? x[n] : 0.f);
+    red[threadIdx.x] = s1;
     __syncthreads();
-  }
-  const double mean = a.demean ? red[0] / (double)a.L : 0.0;
-  __syncthreads();
-  double s2 = 0.0;
-  for (int n = threadIdx.x; n < a.L; n += 256) {
-    const float v = n < a.in_len ? x[n] : 0.f;
-    const float u = a.demean ? (float)((double)v - mean) : v;
-    s2 += (double)u * (double)u;
-  }
-  red[threadIdx.x] = s2;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    for (int o = 128; o > 0; o >>= 1) {
+      if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+      __syncthreads();
+    }
+    mean = a.demean ? red[0] / (double)a.L : 0.0;
     __syncthreads();
+    double s2 = 0.0;
+    for (int n = threadIdx.x; n < a.L; n += 256) {
+      const float v = n < a.in_len ? x[n] : 0.f;
+      const float u = a.demean ? (float)((double)v - mean) : v;
+      s2 += (double)u * (double)u;
+    }
+    red[threadIdx.x] = s2;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+      __syncthreads();
+    }
+    E = red[0];
+    if (threadIdx.x == 0) {
+      a.norms[row] = sqrt(E);
+      if (a.energy) a.energy[row] = E;
+    }
   }
-  const double E = red[0];
-  if (threadIdx.x == 0) a.norms[row] = sqrt(E);
   const double scale = E > 0.0 ? 1.0 / sqrt(E * (double)a.n_channels) : 0.0;
   // A row with a NaN or infinite sample has no coefficients: NaN throughout, so
   // that every lag of its pairs is NaN whatever samples a range of lags skips,
@@ -142,6 +150,7 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
       l0[a.hs / 2 + q] = l[1] | (unsigned)l[2] << 16;
     }
   }
+  if (a.energy_in) return;
   store_columns(a, row, part);
   if (a.traces_out) {
     float* tr = a.traces_out + (long long)row * a.L;
@@ -776,7 +785,8 @@ __global__ __launch_bounds__(256) void k_pack_block(PackBlockArgs a) {
 // ----------------------------------------------------------------------------
 hipError_t launch_lag_prep(const LagPrepArgs& a, hipStream_t st) {
   if (a.n_rows <= 0) return hipSuccess;
-  const int events = a.n_rows / a.n_channels, rows = (events + 31) / 32 * 32 * a.n_channels;
+  const int events = a.n_rows / a.n_channels;
+  const int rows = a.energy_in ? a.n_rows : (events + 31) / 32 * 32 * a.n_channels;  // with the last column tile's empty ones
   hipLaunchKernelGGL(k_lag_prep, dim3(rows), dim3(256), 0, st, a);
   return hipGetLastError();
 }

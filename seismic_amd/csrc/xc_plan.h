@@ -73,6 +73,10 @@ struct sxc_plan {
   // lag-window form
   bool lag = false;
   int l16 = 0, hs = 0, lag_first = 0, n_blocks = 0, n_tiles = 0;
+  // row operands are held for row_band events at a time (a multiple of 32, or all):
+  // those from row_first on
+  int row_band = 0, row_first = 0;
+  double* energy = nullptr;  // row_band < n_events
   unsigned short *h_hi = nullptr, *h_lo = nullptr, *b_hi = nullptr, *b_lo = nullptr;  // LagPrepArgs
   float* lag_traces = nullptr;
   int2* tiles = nullptr;
@@ -131,11 +135,20 @@ int fft_plan_group(sxc_plan* p, int g, const float* d_traces, const float* d_rev
                    int in_len, float* d_vals_pos, int* d_lags_pos, float* d_vals_neg, int* d_lags_neg,
                    hipStream_t st);
 }  // namespace sxc
-// lag-window forms: planes, norms, FP32 traces, triangle tile list, tie records
+// lag-window forms: operands, norms, FP32 traces, triangle tile list, tie records;
+// row operands for as many events at a time as fit, or (_band) for `band`
 int lag_plan_create(const sxc_plan_desc* desc, sxc_plan** out);
+extern "C" int sxc_lag_plan_create_band(const sxc_plan_desc* desc, int band, sxc_plan** out);
+// the next smaller band to try when memory does not suffice, 0: none
+int lag_smaller_band(int band);
 namespace sxc {
-// lag-window forms: the pair kernel's arguments but for tiles and outputs
-LagPairArgs lag_pair_args(const sxc_plan* p);
+// lag-window forms: the pair kernel over the tiles of a list that is ordered by
+// row, `base` holding everything but the operands and n_tiles; tiles(r) is the
+// number of tiles in the list's first r rows of tiles, of which the first is of
+// event row0 and the rows of `rows` events are run.  Row operands that are not
+// held are made as it goes.
+int lag_plan_pairs(sxc_plan* p, const LagPairArgs& base, int row0, int rows,
+                   const std::function<long long(int)>& tiles, hipStream_t st);
 // lag-window forms: spectra of the FP32 traces at the plan's period P (when it has one)
 int lag_plan_spectra(sxc_plan* p, hipStream_t st);
 // lag-window forms: FP64 resolution of the wide near ties (the FFT form's resolver)

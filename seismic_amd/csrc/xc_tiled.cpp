@@ -39,7 +39,6 @@ struct sxc_tiled {
   std::vector<int2> blocks;  // (I, J), J >= I, row-major
   int2* d_tiles_diag = nullptr;
   int2* d_tiles_full = nullptr;
-  int n_diag = 0, n_full = 0;
   float *d_vp = nullptr, *d_vn = nullptr;  // [block][block] FP32 values
   int *d_lp = nullptr, *d_ln = nullptr;
   unsigned short* d_coef[2][2] = {};       // [slot][pos, neg]
@@ -100,10 +99,9 @@ int enqueue_block(sxc_tiled* t, int b) {
   hipStream_t st = t->s_comp;
   HIP_CHECK(launch_fill_u32(p->tie_count, 0u, 1, st));
   if (p->wide_count) HIP_CHECK(launch_fill_u32(p->wide_count, 0u, 1, st));
-  LagPairArgs ka = lag_pair_args(p);
+  LagPairArgs ka{};
   const bool diag = bk.x == bk.y;
   ka.tiles = diag ? t->d_tiles_diag : t->d_tiles_full;
-  ka.n_tiles = diag ? t->n_diag : t->n_full;
   ka.tile_row0 = row0 / 32;
   ka.tile_col0 = col0 / 32;
   ka.out_ld = t->block;
@@ -113,7 +111,9 @@ int enqueue_block(sxc_tiled* t, int b) {
   ka.lpos = t->d_lp;
   ka.vneg = t->d_vn;
   ka.lneg = t->d_ln;
-  HIP_CHECK(launch_lag_pairs(d.form == SXC_FORM_LAG_BF16X3, ka, st));
+  const long long T = t->block / 32;
+  int rc = lag_plan_pairs(p, ka, row0, rows, [=](long long r) { return diag ? r * T - r * (r - 1) / 2 : r * T; }, st);
+  if (rc) return rc;
   LagResolveArgs ra{};
   ra.traces = p->lag_traces;
   ra.tr_stride = d.trace_len;
@@ -139,7 +139,7 @@ int enqueue_block(sxc_tiled* t, int b) {
   ra.wide_cap = p->tie_cap;
   const long long n_pairs = (long long)rows * cols;
   HIP_CHECK(launch_lag_resolve(ra, resolve_grid(n_pairs), st));
-  int rc = lag_plan_resolve_wide(p, n_pairs, t->d_vp, t->d_lp, t->d_vn, t->d_ln, t->block, row0, col0, st);
+  rc = lag_plan_resolve_wide(p, n_pairs, t->d_vp, t->d_lp, t->d_vn, t->d_ln, t->block, row0, col0, st);
   if (rc) return rc;
   HIP_CHECK(hipMemcpyAsync(t->h_ties + slot, p->tie_count, sizeof(unsigned), hipMemcpyDeviceToHost, st));
   // slot reuse: block b - 2's copy out of this slot must be complete
@@ -173,7 +173,8 @@ int enqueue_block(sxc_tiled* t, int b) {
 
 extern "C" {
 
-int sxc_tiled_create(const sxc_plan_desc* desc, int block, int want_neg, sxc_tiled** out) {
+// With row operands for `band` events at a time.
+int sxc_tiled_create_band(const sxc_plan_desc* desc, int block, int want_neg, int band, sxc_tiled** out) {
   clear_error();
   if (!desc || !out) { set_error("null argument"); return SXC_ERR_INVALID; }
   *out = nullptr;
@@ -195,7 +196,7 @@ int sxc_tiled_create(const sxc_plan_desc* desc, int block, int want_neg, sxc_til
   t->block = block;
   t->want_neg = want_neg != 0;
   auto fail = [&](int code) { tiled_free(t); return code; };
-  if ((rc = lag_plan_create(desc, &t->plan))) { t->plan = nullptr; return fail(rc); }
+  if ((rc = sxc_lag_plan_create_band(desc, band, &t->plan))) { t->plan = nullptr; return fail(rc); }
   const int N = desc->n_events;
   t->nb = (N + block - 1) / block;
   for (int I = 0; I < t->nb; ++I)
@@ -207,8 +208,6 @@ int sxc_tiled_create(const sxc_plan_desc* desc, int block, int want_neg, sxc_til
       full.push_back(make_int2(a, c));
       if (c >= a) diag.push_back(make_int2(a, c));
     }
-  t->n_diag = (int)diag.size();
-  t->n_full = (int)full.size();
   const size_t bb = (size_t)block * block;
   if ((rc = dev_alloc(&t->d_tiles_diag, diag.size(), "tile list")) ||
       (rc = dev_alloc(&t->d_tiles_full, full.size(), "tile list")) ||
@@ -245,6 +244,13 @@ int sxc_tiled_create(const sxc_plan_desc* desc, int block, int want_neg, sxc_til
     }
   *out = t;
   return SXC_OK;
+}
+
+int sxc_tiled_create(const sxc_plan_desc* desc, int block, int want_neg, sxc_tiled** out) {
+  int rc = SXC_ERR_MEMORY;
+  for (int band = desc ? std::max(1, desc->n_events) : 1; rc == SXC_ERR_MEMORY && band > 0; band = lag_smaller_band(band))
+    rc = sxc_tiled_create_band(desc, block, want_neg, band, out);
+  return rc;
 }
 
 int sxc_tiled_start(sxc_tiled* t, const float* d_traces, long long trace_stride, int in_len) {

@@ -1,9 +1,14 @@
-// Plans on a device with little memory left.  Argument "fft": a window far
-// shorter than the traces, in just the memory that whole rows need: the plan is made
-// and runs on whole rows; with more it runs on segments.
+// Plans, host-buffer jobs and tiled runs on a device with little memory left.
+// fft: a window far shorter than the traces, in just the memory that whole rows
+// need: the plan is made and runs on whole rows; with more it runs on segments.
+// lag: less memory than the row operands of all events take: they are held for a
+// band of events at a time, and every launch finds its rows' operands.
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <map>
+#include <set>
 #include <vector>
 
 #include "../../include/seismic_xcorr.h"
@@ -43,8 +48,109 @@ static int fft() {
   return standin::used() != 0;
 }
 
+
+// Follows the row operands: which event each place of the allocation holds.
+struct Rows {
+  const double* norms0 = nullptr;             // of event 0 (the first launch)
+  std::map<const unsigned short*, int> held;  // place -> event
+  std::set<std::pair<int, int>> pairs;        // tiles run
+  int launches = 0, bad = 0;
+  void watch() {
+    standin::on_lag_prep = [this](const sxc::LagPrepArgs& a) {
+      if (!a.energy_in && !norms0) norms0 = a.norms;
+      const int e0 = (int)(a.norms - norms0) / a.n_channels;
+      for (int e = 0; e < a.n_rows / a.n_channels; ++e) {
+        const unsigned short* at = a.h_hi + (size_t)e * a.n_channels * 2 * a.hs;
+        held[at] = e0 + e;
+        bad += !standin::size_of(at + (size_t)a.n_channels * 2 * a.hs - 1);
+      }
+      return 0;
+    };
+    standin::on_lag_pairs = [this](bool, const sxc::LagPairArgs& a) {
+      ++launches;
+      for (int t = 0; t < a.n_tiles; ++t) {
+        const int ti = a.tiles[t].x + a.tile_row0, tj = a.tiles[t].y + a.tile_col0;
+        if (32 * ti >= a.n_events || 32 * tj >= a.n_events) continue;
+        bad += !pairs.insert({ti, tj}).second;
+        for (int i = 32 * ti; i < std::min(32 * ti + 32, a.n_events); ++i) {
+          auto it = held.find((const unsigned short*)((size_t)a.h_hi + (size_t)i * a.n_channels * 4 * a.hs));
+          bad += it == held.end() || it->second != i;
+        }
+      }
+      return 0;
+    };
+  }
+  bool all(int n) {
+    const int T = (n + 31) / 32;
+    const bool ok = !bad && (int)pairs.size() == T * (T + 1) / 2;
+    if (!ok) printf("%d bad, %zu of %d tiles\n", bad, pairs.size(), T * (T + 1) / 2);
+    pairs.clear();
+    return ok;
+  }
+};
+
+static int lag() {
+  const int n = 203, C = 2, L = 1000, w = 40, block = 96;
+  const size_t np = (size_t)n * (n + 1) / 2;
+  std::vector<float> x((size_t)n * C * L, 1.f), v(np);
+  std::vector<int> l(np);
+  for (int form : {SXC_FORM_LAG_BF16X3, SXC_FORM_LAG_FP16}) {
+    sxc_plan_desc d{n, C, L, 0, -w, w, 0.f, 0.f, 1, form};
+    // 0: a plan, 1: a host-buffer job, 2: a tiled run; with all the memory, then with
+    // what zero-padded planes of l16 + 2 (w + 16) samples in place of the operands take
+    for (int what = 0; what < 3; ++what) {
+      size_t full = 0;
+      for (int low = 0; low < 2; ++low) {
+        // and one band of 32 events, energies and the room past the operands
+        const size_t sample = C * 2 * (form == SXC_FORM_LAG_BF16X3 ? 2 : 1);  // bytes of every event
+        const size_t l16 = 1008, hs = l16 + 32 * 3, operands = n * sample * (2 * hs + l16);
+        standin::limit = low ? full - operands + n * sample * (l16 + 2 * (w + 16)) + 32 * sample * 2 * hs + (1 << 16)
+                             : (size_t)1 << 40;
+        Rows r;
+        r.watch();
+        sxc_plan* p = nullptr;
+        sxc_tiled* t = nullptr;
+        int rc = 0;
+        if (what == 0) {
+          rc = sxc_plan_create(&d, &p);
+          full = rc || low ? full : standin::used();
+          for (int k = 0; k < 2 && !rc; ++k) {
+            rc = sxc_plan_execute(p, x.data(), L, L, v.data(), l.data(), v.data(), l.data(), nullptr);
+            if (!rc && !r.all(n)) rc = -100;
+          }
+          sxc_plan_destroy(p);
+        } else if (what == 1) {
+          setenv("SEISMIC_XCORR_CACHE_MB", "0", 1);
+          standin::on_resolve = [&](int, const sxc::ResolveArgs&) {
+            full = low ? full : standin::used();
+            return 0;
+          };
+          rc = sxc_allpairs_host(&d, x.data(), L, L, v.data(), l.data(), v.data(), l.data());
+          if (!rc && !r.all(n)) rc = -100;
+        } else {
+          rc = sxc_tiled_create(&d, block, 1, &t);
+          full = rc || low ? full : standin::used();
+          for (int k = 0; k < 2 && !rc; ++k) {
+            sxc_block_info b{};
+            rc = sxc_tiled_start(t, x.data(), L, L);
+            while (!rc && !(rc = sxc_tiled_next(t, &b, nullptr, nullptr, nullptr, nullptr, 0)) && b.index >= 0) {}
+            if (!rc && !r.all(n)) rc = -100;
+          }
+          sxc_tiled_destroy(t);
+        }
+        if (rc || standin::used())
+          return printf("form %d, case %d, low %d: %d (%s), %zu bytes left\n", form, what, low, rc, seismic_last_error(),
+                        standin::used()), 1;
+        if (low && standin::limit >= full) return printf("the limit does not tell\n"), 1;
+        printf("form %d case %d low %d: %d launches, limit %zu of %zu\n", form, what, low, r.launches, standin::limit, full);
+      }
+    }
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
-  const int rc = !strcmp(argv[1], "fft") ? fft() : 2;
+  const int rc = !strcmp(argv[1], "fft") ? fft() : lag();
   if (!rc) printf("ok\n");
   return rc;
 }

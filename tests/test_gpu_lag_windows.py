@@ -8,10 +8,12 @@ large enough that a wave takes two rows.  Every pair against FP64 direct sums.
 Bars as for the other lag-form tests: coefficients within 1e-5 (bf16x3) and
 2e-3 (fp16), lags equal wherever the FP64 gap of the two best lags is at least
 1e-12 (values above 1e-3)."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from seismic_amd import engine
+from seismic_amd import engine, tiled
 from seismic_amd.device import DeviceArray, synchronize
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +95,36 @@ def test_lags_beyond_the_record_capacity():
     assert np.array_equal(lp[k], at[i[k]] - 1 - at[j[k]])
     k = (i % 2 == 0) & (j % 2 == 0)
     assert np.array_equal(lp[k], at[i[k]] - at[j[k]]) and (vp[k] == 1.0).all()
+
+
+@pytest.mark.parametrize("name", ["bf16x3", "fp16"])
+@pytest.mark.parametrize("band,block", [(32, 32), (96, 64), (128, 224)])
+def test_row_operands_in_bands(name, band, block):
+    """Row operands held for some events at a time, as where memory is short: the
+    same bits as with all of them, for plans and tiled runs; rows shorter than L,
+    demeaned, one of them with a NaN; two executes."""
+    n, C, L, in_len, lo, hi = 203, 2, 700, 650, -70, 333
+    form, _ = FORMS[name]
+    x = np.random.default_rng(band).standard_normal((n, C, in_len)).astype(np.float32) + np.float32(0.5)
+    x[70, 1, 5] = np.nan
+    print(f"case row bands {name} N={n} C={C} L={L} [{lo}, {hi}] band={band} block={block}", flush=True)
+    d = DeviceArray.from_numpy(x)
+    plan = engine.AllPairsPlan(n, C, L, 0, lo, hi, demean=True, form=form)
+    want = [o.numpy() for o in plan.execute(d)]
+    plan.lib.sxc_plan_destroy(plan.handle)
+    assert plan.lib.sxc_lag_plan_create_band(ctypes.byref(plan.desc), band, ctypes.byref(plan.handle)) == 0
+    for _ in range(2):
+        out = plan.execute(d)
+        synchronize()
+        assert all(np.array_equal(w, o.numpy()) for w, o in zip(want, out))
+    plan.close()
+    run = tiled.TiledRun(n, C, L, lo, hi, form=form, block=block, demean=True)
+    run.lib.sxc_tiled_destroy(run.handle)
+    assert run.lib.sxc_tiled_create_band(ctypes.byref(plan.desc), block, 0, band, ctypes.byref(run.handle)) == 0
+    coef, lag = np.zeros((n, n), np.float16), np.zeros((n, n), np.int16)
+    i, j = np.triu_indices(n)
+    for _ in range(2):
+        run.start(d)
+        tiled.assemble(run, coef, lag)
+        assert np.array_equal(coef[i, j], want[0].astype(np.float16)) and np.array_equal(lag[i, j], want[1])
+    run.close()

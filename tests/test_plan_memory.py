@@ -6,8 +6,13 @@ from host_build import run_host
 SOURCES = ["xc_engine.cpp", "xc_hostio.cpp"]
 
 
+def test_lag_plans_hold_row_operands_in_bands(tmp_path):
+    rc, out = run_host(tmp_path, "plan_memory.cpp", SOURCES + ["xc_tiled.cpp"], "lag")
+    assert rc == 0, f"status {rc}: {out}"
+
+
 def test_fft_plan_keeps_rows_whole_where_segments_do_not_fit(tmp_path):
-    rc, out = run_host(tmp_path, "plan_memory.cpp", SOURCES, "fft")
+    rc, out = run_host(tmp_path, "plan_memory.cpp", SOURCES + ["xc_tiled.cpp"], "fft")
     assert rc == 0, f"status {rc}: {out}"
 
 

@@ -57,7 +57,7 @@ def prepare(events):
     max_pad = 1 << max_len.bit_length()
     padded = np.zeros((n_events, max_pad), dtype=np.float32)
     padded_rev = np.zeros((n_events, max_pad), dtype=np.float32)
-    if type(events) is np.ndarray and events.ndim == 2 and events.dtype in _PLAIN:
+    if n_events and type(events) is np.ndarray and events.ndim == 2 and events.dtype in _PLAIN:
         # rows of one length: two block copies (N = 1024, L = 2048: 15.5 ms of
         # np.pad calls -> 1.2 ms)
         padded[:, :max_len] = events

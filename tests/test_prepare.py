@@ -42,3 +42,16 @@ def test_prepare_refuses_rows_longer_than_the_period():
     ev[0], ev[1] = np.zeros(100, np.float32), np.zeros(200, np.float32)  # P = 128
     with pytest.raises(ValueError):
         correlation_lib.prepare(ev)
+
+
+@pytest.mark.parametrize("shape", [(0, 0), (0, 5), (3, 0)])
+def test_prepare_without_events_or_samples(shape):
+    """Left to the library, whose message reaches the caller."""
+    n, L, P, padded, rev, outs = correlation_lib.prepare(np.zeros(shape, np.float32))
+    assert (n, L, P) == (shape[0], 0, 1) and padded.shape == rev.shape == (n, 1)
+    assert not padded.any() and not rev.any() and all(o.shape == (n * (n + 1) // 2,) for o in outs)
+
+
+def test_no_events_reach_the_library():
+    with pytest.raises(RuntimeError, match="n_events must be >= 1"):
+        correlation_lib.compute_correlation(np.zeros((0, 5), np.float32), 1, 1, 0.0)

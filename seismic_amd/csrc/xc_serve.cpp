@@ -246,9 +246,10 @@ void slot_free(Slot* s) {
 // The lengths of a batch, in front of its traces in one buffer.
 size_t len_bytes(const sxc_server_desc& d) { return ((size_t)d.max_batch_events * sizeof(int) + 255) / 256 * 256; }
 
+// What a slot counts against the memory budget (not the rounding of its parts).
 unsigned long long slot_bytes(const sxc_server_desc& d, long long spec_stride_max) {
   const unsigned long long B = d.max_batch_events, C = d.n_channels;
-  return B * C * (unsigned long long)d.max_query_len * 4 + len_bytes(d) + B * C * spec_stride_max * 8 +
+  return B * C * (unsigned long long)d.max_query_len * 4 + B * 4 + B * C * spec_stride_max * 8 +
          B * C * 8 + B * (unsigned long long)d.n_catalog * 8 + B * d.top_k * 12 +
          B * kTopkMaxSlices * d.top_k * 12 + 64;
 }

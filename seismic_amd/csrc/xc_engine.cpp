@@ -859,14 +859,23 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Ro
   // L = 4096, +-50 114 -> 37 us.
   const int P1 = p->narrow.P ? p->narrow.P : p->P;  // the period of executes on whole rows
   if (how == Rows::kCut && desc.trace_len + reach <= p->P) {
-    double best = 0.95 * pair_cost(P1 / 128, desc.n_channels);
+    const double whole = pair_cost(P1 / 128, desc.n_channels);
+    double best = whole;
     for (int P : {1024, 2048, 3072, 4096, 5120}) {
+      // The transforms, 2 n_seg of P' for one of P1, are not in the costs: in a job of a
+      // few turns of workgroups they decide.  Segments at 4096 against whole rows at
+      // 5120 (C = 1, L = 4096, +-1000): N = 3..64 6-11% slower, 128 11%, 200 1%, 400 the
+      // same, 500 12% faster; at 2048 against 3072 (C = 2, L = 2048, +-200): N = 16 5%
+      // faster, 64 the same, 100..300 1-5% slower, 700 the same, 1000 3% faster.
+      const bool few = p->n_pairs < 65536, some = few && p->n_pairs >= 4096;
+      if (few && P >= 4096) continue;
+      const double most = (some && P >= 2048 ? 0.94 : 0.95) * whole;
       const int len = P - std::max(0, desc.lag_hi) - std::max(0, -desc.lag_lo);
       if (P >= P1 || len < 1 || desc.lag_lo <= -P / 2 || desc.lag_hi > P / 2) continue;
       const int n_seg = (desc.trace_len + len - 1) / len;
       if (n_seg < 2 || desc.n_channels * n_seg > 8) continue;  // (n_seg < 2: a lag window that no shorter period holds)
       const double cost = pair_cost(P / 128, desc.n_channels * n_seg);
-      if (cost >= best) continue;
+      if (cost >= best || cost >= most) continue;
       best = cost;
       FftGeom& g = p->cut;
       g.P = P;

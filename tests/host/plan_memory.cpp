@@ -149,8 +149,23 @@ static int lag() {
   return 0;
 }
 
+// Whole rows or segments, by the size of the job.
+static int rule() {
+  struct Case { int n, C, L, P, w, n_seg; };
+  for (const Case& c : {Case{64, 1, 4096, 8192, 1000, 0}, {200, 1, 4096, 8192, 1000, 0}, {500, 1, 4096, 8192, 1000, 2},
+                        {64, 2, 2048, 4096, 200, 2}, {200, 2, 2048, 4096, 200, 0}, {1000, 2, 2048, 4096, 200, 2},
+                        {64, 1, 4096, 8192, 50, 5}, {200, 1, 4096, 8192, 50, 5}}) {
+    sxc_plan_desc d{c.n, c.C, c.L, c.P, -c.w, c.w, 0.f, 0.f, 0, SXC_FORM_FFT_F32};
+    sxc_plan* p = nullptr;
+    if (sxc_plan_create(&d, &p) || execute(p, c.n, c.C, c.L) || g_seg != c.n_seg)
+      return printf("N=%d C=%d L=%d +-%d: %d segments\n", c.n, c.C, c.L, c.w, g_seg), 1;
+    sxc_plan_destroy(p);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
-  const int rc = !strcmp(argv[1], "fft") ? fft() : lag();
+  const int rc = !strcmp(argv[1], "fft") ? fft() : !strcmp(argv[1], "rule") ? rule() : lag();
   if (!rc) printf("ok\n");
   return rc;
 }

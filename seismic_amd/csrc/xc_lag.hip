@@ -217,18 +217,14 @@ __device__ __forceinline__ unsigned med3_u(unsigned a, unsigned b, unsigned c) {
 // negative side as unsigned ones (the most negative first, positive ones
 // last).  A key differs from its value by less than 16 units in the last place,
 // at most kKeySlack for |value| <= 1.  The best key's lag is the extremum's unless
-// the two best keys differ in their lag bits alone (`close`): the block that makes
-// them so, or brings a new extremum then, is searched for it (N = 2001, L = 4096,
-// +-512 fp16 12.73 -> 12.83 ms; +-1024 bf16x3 and three channels within 0.5%).
+// another key differs from it in the lag bits alone; such a pair is a near tie, which
+// FP64 settles, and one beyond the record capacity is searched again (seek_lags).
 constexpr float kKeySlack = 2e-6f;
 template <typename T>
 struct Best3 {
   T e, k1, k2, k3;
   int b1, b2;
-  int at;  // while k1 and k2 are close, the extremum's lag: 16 block + (15 - lag_order)
 };
-template <typename T>
-__device__ __forceinline__ bool close(T k1, T k2) { return (unsigned)(k1 ^ k2) < 16u; }
 __device__ __forceinline__ int top(int a, int b) { return a > b ? a : b; }
 __device__ __forceinline__ unsigned top(unsigned a, unsigned b) { return a > b ? a : b; }
 __device__ __forceinline__ int mid(int a, int b, int c) { return med3_i(a, b, c); }
@@ -236,7 +232,7 @@ __device__ __forceinline__ unsigned mid(unsigned a, unsigned b, unsigned c) { re
 
 template <typename T>
 __device__ __forceinline__ void insert16(Best3<T>& s, const T (&bits)[16], const T (&key)[16], int block) {
-  const T o1 = s.k1, o2 = s.k2, e0 = s.e;
+  const T o1 = s.k1, o2 = s.k2;
 #pragma unroll
   for (int r = 0; r < 16; r += 2) s.e = top(top(s.e, bits[r]), bits[r + 1]);
 #pragma unroll
@@ -245,14 +241,7 @@ __device__ __forceinline__ void insert16(Best3<T>& s, const T (&bits)[16], const
     s.k2 = mid(s.k1, s.k2, key[r]);
     s.k1 = top(s.k1, key[r]);
   }
-  const bool c1 = s.k1 != o1, now = close(s.k1, s.k2) && (s.e != e0 || c1 || s.k2 != o2);
-  if (__ballot(now)) {
-    int code = 0;  // the first lag has the largest
-#pragma unroll
-    for (int r = 0; r < 16; ++r) code = max(code, bits[r] == s.e ? 15 - lag_order(r) : 0);
-    const int before = close(o1, o2) ? s.at : 16 * s.b1 + ((int)o1 & 15);
-    s.at = now ? (s.e != e0 ? 16 * block + code : before) : s.at;
-  }
+  const bool c1 = s.k1 != o1;
   s.b2 = s.k2 == o2 ? s.b2 : ((c1 && s.k2 == o1) ? s.b1 : block);
   s.b1 = c1 ? block : s.b1;
 }
@@ -260,22 +249,20 @@ __device__ __forceinline__ void insert16(Best3<T>& s, const T (&bits)[16], const
 // A pair's state on one side with the keys in one (signed) order and the lags
 // as offsets from the first: what lanes and waves merge.
 struct Side {
-  int e, oe, k1, k2, k3, o1, o2;
+  int e, k1, k2, k3, o1, o2;
 };
 __device__ __forceinline__ int key_row(int key, int h) { return order_lag(h, 15 - (key & 15)); }
-template <typename T>
-__device__ __forceinline__ Side side_of(const Best3<T>& s, int h) {
-  constexpr T f = T(-1) < T(0) ? T(0) : (T)0x80000000u;  // unsigned order to signed order
-  const int o1 = 32 * s.b1 + key_row((int)s.k1, h), o2 = 32 * s.b2 + key_row((int)s.k2, h);
-  const int oe = close(s.k1, s.k2) ? 32 * (s.at >> 4) + key_row(s.at, h) : o1;
-  return Side{(int)(s.e ^ f), oe, (int)(s.k1 ^ f), (int)(s.k2 ^ f), (int)(s.k3 ^ f), o1, o2};
+__device__ __forceinline__ Side side_of(const Best3<int>& s, int h) {
+  return Side{s.e, s.k1, s.k2, s.k3, 32 * s.b1 + key_row(s.k1, h), 32 * s.b2 + key_row(s.k2, h)};
 }
-// Merge of two lists over disjoint lags; equal extrema and equal first keys go to
-// the smaller lag.
+__device__ __forceinline__ Side side_of(const Best3<unsigned>& s, int h) {
+  constexpr unsigned f = 0x80000000u;  // unsigned order to signed order
+  return Side{(int)(s.e ^ f), (int)(s.k1 ^ f), (int)(s.k2 ^ f), (int)(s.k3 ^ f),
+              32 * s.b1 + key_row((int)s.k1, h), 32 * s.b2 + key_row((int)s.k2, h)};
+}
+// Merge of two lists over disjoint lags; equal first keys go to the smaller lag.
 __device__ __forceinline__ void merge_side(Side& a, const Side& b) {
-  const int ea = a.e, eb = b.e, la = a.oe, lb = b.oe, first = la < lb ? la : lb;
-  a.oe = eb > ea ? lb : (eb == ea ? first : la);
-  a.e = top(ea, eb);
+  a.e = top(a.e, b.e);
   const bool tb = b.k1 > a.k1 || (b.k1 == a.k1 && b.o1 < a.o1);
   // W: the list whose head wins, O: the other
   const int w1 = tb ? b.k1 : a.k1, w2 = tb ? b.k2 : a.k2, w3 = tb ? b.k3 : a.k3;
@@ -289,9 +276,8 @@ __device__ __forceinline__ void merge_side(Side& a, const Side& b) {
   a.k3 = v_second ? top(w2, v2) : top(w3, v1);
 }
 __device__ __forceinline__ Side shfl_side(const Side& s, int mask) {
-  return Side{__shfl_xor(s.e, mask, 64),  __shfl_xor(s.oe, mask, 64), __shfl_xor(s.k1, mask, 64),
-              __shfl_xor(s.k2, mask, 64), __shfl_xor(s.k3, mask, 64), __shfl_xor(s.o1, mask, 64),
-              __shfl_xor(s.o2, mask, 64)};
+  return Side{__shfl_xor(s.e, mask, 64),  __shfl_xor(s.k1, mask, 64), __shfl_xor(s.k2, mask, 64),
+              __shfl_xor(s.k3, mask, 64), __shfl_xor(s.o1, mask, 64), __shfl_xor(s.o2, mask, 64)};
 }
 
 template <bool BF16X3>
@@ -429,9 +415,39 @@ __device__ __forceinline__ void scan_range(f32x16 (&acc)[NI * NB], int ni, Best3
   }
 }
 
+// First lags at which this row has the values p and n, block by block (the bits are
+// those of the ranges, whose products differ by zeros alone).  Every lane takes its
+// column's values.  Values past the window's last lag come after the first.
+template <bool BF16X3>
+__device__ __forceinline__ void seek_lags(const PlaneRows<BF16X3>& row, const PlaneRows<BF16X3>& cols, int vh, int vb,
+                                       const LagPairArgs& a, int h, float p, float n, int& fp, int& fn) {
+  const PlaneRows<BF16X3> rows[1] = {row};
+  int lp = a.lag_hi, ln = a.lag_hi;
+  for (int b = a.n_blocks - 1; b >= 0; --b) {
+    const int l0 = a.lag_first + 32 * b, l1 = min(l0 + 31, a.lag_hi);
+    f32x16 acc[1];
+    lag_range<BF16X3, 1, 1, 1>(acc, rows, cols, vh, vb, a, b, max(0, -l1) >> 4, (min(a.L, a.L - l0) + 15) >> 4);
+#pragma unroll
+    for (int o = 15; o >= 0; --o) {
+      const float v = acc[0][(o >> 1) + 8 * (o & 1)];
+      const int lag = l0 + order_lag(h, o);
+      lp = v == p ? lag : lp;
+      ln = v == n ? lag : ln;
+    }
+  }
+  fp = min(lp, __shfl_xor(lp, 32, 64));
+  fn = min(ln, __shfl_xor(ln, 32, 64));
+}
+
+// Place of pair (i, j) in the outputs.
+__device__ __forceinline__ long long out_index(const LagPairArgs& a, int i, int j) {
+  return a.out_ld ? (long long)(i - a.out_row0) * a.out_ld + (j - a.out_col0)
+                  : (long long)i * a.n_events - (long long)i * (i - 1) / 2 + (j - i);
+}
+
 constexpr int kLagWaves = 8;  // per workgroup, two per SIMD
 struct LagMerge {
-  int v[kLagWaves][14][64];
+  int v[kLagWaves][12][64];
 };
 
 // Bound by the matrix cores at the clock the power limit leaves: 0.82-0.86 busy
@@ -487,8 +503,8 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
     Best3<unsigned> neg[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      pos[i] = Best3<int>{0, 0, (int)0x80000000, (int)0x80000000, 0, 0, 0};
-      neg[i] = Best3<unsigned>{0x80000000u, 0x80000000u, 0u, 0u, 0, 0, 0};
+      pos[i] = Best3<int>{0, 0, (int)0x80000000, (int)0x80000000, 0, 0};
+      neg[i] = Best3<unsigned>{0x80000000u, 0x80000000u, 0u, 0u, 0, 0};
     }
     if (live)
       for (int rg = part; rg < a.n_ranges; rg += split) {
@@ -516,17 +532,17 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
       merge_side(n, shfl_side(n, 32));
       if (split > 1) {
         __syncthreads();  // the previous merge has been read
-        const int w[14] = {p.e, p.oe, p.k1, p.k2, p.k3, p.o1, p.o2, n.e, n.oe, n.k1, n.k2, n.k3, n.o1, n.o2};
+        const int w[12] = {p.e, p.k1, p.k2, p.k3, p.o1, p.o2, n.e, n.k1, n.k2, n.k3, n.o1, n.o2};
 #pragma unroll
-        for (int q = 0; q < 14; ++q) mg.v[wv][q][lane] = w[q];
+        for (int q = 0; q < 12; ++q) mg.v[wv][q][lane] = w[q];
         __syncthreads();
         if (part == 0)
           for (int o = 1; o < split; ++o) {
-            int u[14];
+            int u[12];
 #pragma unroll
-            for (int q = 0; q < 14; ++q) u[q] = mg.v[wv + o][q][lane];
-            merge_side(p, Side{u[0], u[1], u[2], u[3], u[4], u[5], u[6]});
-            merge_side(n, Side{u[7], u[8], u[9], u[10], u[11], u[12], u[13]});
+            for (int q = 0; q < 12; ++q) u[q] = mg.v[wv + o][q][lane];
+            merge_side(p, Side{u[0], u[1], u[2], u[3], u[4], u[5]});
+            merge_side(n, Side{u[6], u[7], u[8], u[9], u[10], u[11]});
           }
       }
       const int ii = i0 + i, j = j0 + r32;
@@ -536,6 +552,7 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
       const float p1 = __int_as_float(p.e), n1 = -mag(n.e);
       const bool kp = p1 > a.threshold && p1 > 0.f;
       const bool kn = n1 < -a.threshold && n1 < 0.f;
+      const int glp1 = a.lag_first + p.o1, gln1 = a.lag_first + n.o1;
       const float tol = a.tie_tol + 2.f * kKeySlack;
       const float q1 = __int_as_float(p.k1), m1 = mag(n.k1);
       // near ties; wide ones (a third lag in the band): every in-window lag is a candidate
@@ -544,12 +561,11 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
       const bool wp = tp && (q1 - __int_as_float(p.k3) < tol || q1 < tol);
       const bool wn = tn && (m1 - mag(n.k3) < tol || m1 < tol);
       if (out) {
-        const long long idx = a.out_ld ? (long long)(ii - a.out_row0) * a.out_ld + (j - a.out_col0)
-                                       : (long long)ii * a.n_events - (long long)ii * (ii - 1) / 2 + (j - ii);
+        const long long idx = out_index(a, ii, j);
         a.vpos[idx] = kp ? p1 : 0.f;
-        a.lpos[idx] = kp ? a.lag_first + p.oe : 0;
+        a.lpos[idx] = kp ? glp1 : 0;
         a.vneg[idx] = kn ? n1 : 0.f;
-        a.lneg[idx] = kn ? a.lag_first + n.oe : 0;
+        a.lneg[idx] = kn ? gln1 : 0;
       }
       const unsigned long long ties = __ballot(tp || tn);  // one counter update per wave
       if (ties) {
@@ -559,7 +575,18 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
         const unsigned slot = base + (unsigned)__popcll(ties & ((1ull << lane) - 1ull));
         if ((tp || tn) && slot < (unsigned)a.tie_cap) {
           a.ties[2 * slot] = make_int4(ii, j, (tp ? 1 : 0) | (tn ? 2 : 0) | (wp ? 4 : 0) | (wn ? 8 : 0), 0);
-          a.ties[2 * slot + 1] = make_int4(a.lag_first + p.o1, a.lag_first + p.o2, a.lag_first + n.o1, a.lag_first + n.o2);
+          a.ties[2 * slot + 1] = make_int4(glp1, a.lag_first + p.o2, gln1, a.lag_first + n.o2);
+        }
+        // beyond the capacity the extrema keep their own first lags
+        const bool lost = (tp || tn) && slot >= (unsigned)a.tie_cap;
+        if (__ballot(lost)) {
+          int fp, fn;
+          seek_lags<BF16X3>(rows[i], cols, vh, vb, a, h, p1, n1, fp, fn);
+          if (lost) {
+            const long long idx = out_index(a, ii, j);
+            a.lpos[idx] = kp ? fp : 0;
+            a.lneg[idx] = kn ? fn : 0;
+          }
         }
       }
     }

@@ -64,7 +64,8 @@ def test_nonfinite_rows(oracle, name, lo, hi, at, bad):
     assert np.abs(vp - ref["pos"])[~hit].max() <= tol and np.abs(vn - ref["neg"])[~hit].max() <= tol
 
 
-def test_lags_beyond_the_record_capacity():
+@pytest.mark.parametrize("sign", [1, -1])
+def test_lags_beyond_the_record_capacity(sign):
     """More near ties than records (a band of every value): the pairs beyond the
     capacity keep the lag of their FP32 extremum, also where another lag is within
     16 units in the last place.  Single spikes against events with two spikes of
@@ -80,7 +81,8 @@ def test_lags_beyond_the_record_capacity():
     x[two, 0, at[two]] = a
     x[two, 0, at[two] - 1] = b
     x[two, 0, at[two] + 12] = np.sqrt(1.0 - a * a - b * b)
-    print(f"case records beyond the capacity N={n} L={L} +-{w}", flush=True)
+    x[two] *= sign
+    print(f"case records beyond the capacity N={n} L={L} +-{w} sign={sign}", flush=True)
     plan = engine.AllPairsPlan(n, 1, L, 0, -w, w, tie_tol=10.0, form=engine.FORM_LAG_BF16X3)
     out = plan.execute(DeviceArray.from_numpy(x))
     synchronize()
@@ -89,10 +91,11 @@ def test_lags_beyond_the_record_capacity():
     plan.close()
     assert stats["tie_overflow"] > 10000
     i, j = np.triu_indices(n)
+    v, lag = (vp, lp) if sign > 0 else (-vn, ln)
     k = (i % 2 == 0) & (j % 2 == 1)
-    assert np.array_equal(lp[k], at[i[k]] - (at[j[k]] - 1)) and np.abs(vp[k] - b).max() <= 2e-7
+    assert np.array_equal(lag[k], at[i[k]] - (at[j[k]] - 1)) and np.abs(v[k] - b).max() <= 2e-7
     k = (i % 2 == 1) & (j % 2 == 0)
-    assert np.array_equal(lp[k], at[i[k]] - 1 - at[j[k]])
+    assert np.array_equal(lag[k], at[i[k]] - 1 - at[j[k]]) and np.abs(v[k] - b).max() <= 2e-7
     k = (i % 2 == 0) & (j % 2 == 0)
     assert np.array_equal(lp[k], at[i[k]] - at[j[k]]) and (vp[k] == 1.0).all()
 

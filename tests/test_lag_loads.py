@@ -5,8 +5,7 @@ Addresses of the product's operand loads: every lane of every range of lags over
 trace lengths from one sample on, both forms and several channels.  No load of the last row or column tile may leave
 the operands' allocation.
 
-The scan's running state: the extremum at its first lag among values that differ
-in their last bits."""
+The scan's running state among values that differ in their last bits."""
 import os
 import subprocess
 
@@ -26,5 +25,5 @@ def test_operand_loads_stay_in_the_allocation(tmp_path):
     _run(tmp_path, "lag_loads.cpp")
 
 
-def test_scan_keeps_the_extremum_at_its_first_lag(tmp_path):
+def test_scan_state(tmp_path):
     _run(tmp_path, "lag_scan.cpp")

@@ -68,7 +68,7 @@ def build(force: bool = False, verbose: bool = True, jobs: int | None = None) ->
         kobjs.append(out)
         if force or _stale(out, [src] + hdrs):
             steps.append([HIPCC] + HIP_FLAGS + [f"-DSXC_R={r}", "-c", src, "-o", out])
-    for name in ("xc_lag.hip", "xc_noalloc.hip"):
+    for name in ("xc_lag.hip", "xc_lag_tile.hip", "xc_noalloc.hip"):
         src = os.path.join(CSRC, name)
         out = os.path.join(OBJ, name.replace(".hip", ".o"))
         kobjs.append(out)

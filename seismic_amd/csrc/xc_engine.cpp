@@ -80,9 +80,7 @@ int validate_desc(const sxc_plan_desc& d) {
       return SXC_ERR_INVALID;
     }
     if (!(d.threshold == d.threshold)) { set_error("threshold is NaN"); return SXC_ERR_INVALID; }
-    long long lf = d.lag_lo;
-    while (((lf - 1) % 8 + 8) % 8 != 0) --lf;
-    const long long span = (d.lag_hi - lf + 1 + 15) / 16 * 16;
+    const long long span = (d.lag_hi - (long long)tile_first_lag(d.lag_lo) + 1 + 15) / 16 * 16;
     if (span > kLagMaxSpan) {
       set_error("lag window [%d, %d] spans more than %d lags (the lag forms' limit)", d.lag_lo, d.lag_hi,
                 kLagMaxSpan - 16);
@@ -224,10 +222,21 @@ int sxc_lag_plan_create_band(const sxc_plan_desc* desc, int band, sxc_plan** out
   auto fail = [&](int code) { plan_free(p); return code; };
   int rc;
   // one allocation (h_hi) for the operands
-  const LagOperands ops =
+  const bool two = desc->form == SXC_FORM_LAG_BF16X3;
+  LagOperands ops =
       lag_operands((long long)p->row_band * desc->n_channels, (desc->n_events + 31LL) / 32 * 32 * desc->n_channels,
                    p->hs, p->l16);
-  const bool two = desc->form == SXC_FORM_LAG_BF16X3;
+  if (lag_tiles(two, desc->n_events, desc->n_channels, L, desc->lag_lo, desc->lag_hi)) {
+    p->tile = true;
+    p->row_band = desc->n_events;
+    p->lag_first = tile_first_lag(desc->lag_lo);
+    p->n_blocks = (desc->lag_hi - p->lag_first + 1 + kTileLags - 1) / kTileLags;
+    // the window of block lb starts at element p0 + n0 + 8h - lb - 15 and takes 24
+    p->p0 = std::max(0, (p->lag_first + kTileLags * p->n_blocks - 1 + 7) / 8 * 8);
+    p->ls = (std::max(p->p0 + p->l16, p->p0 + p->l16 - p->lag_first + 9) + 7) / 8 * 8;
+    p->hs = 0;
+    ops = {(rows * p->ls + 127) / 128 * 128, 0};
+  }
   if ((rc = dev_alloc(&p->h_hi, (size_t)(ops.h + ops.b) * (two ? 2 : 1), "trace operands"))) return fail(rc);
   p->b_hi = p->h_hi + ops.h;
   if (two) {
@@ -338,6 +347,12 @@ static LagPrepArgs lag_prep_args(const sxc_plan* p, int e0, int e1) {
   pa.h_lo = p->h_lo;
   pa.b_hi = p->b_hi + r0 * p->l16;  // e0 is a multiple of 32: whole column tiles
   pa.b_lo = p->b_lo ? p->b_lo + r0 * p->l16 : nullptr;
+  if (p->tile) {
+    pa.p_hi = p->h_hi;
+    pa.p_lo = p->h_lo;
+    pa.p0 = p->p0;
+    pa.ls = p->ls;
+  }
   pa.norms = p->norms + r0;
   return pa;
 }
@@ -390,6 +405,11 @@ static LagPairArgs lag_pair_args(const sxc_plan* p, const LagPairArgs& base) {
   ka.lag_hi = p->d.lag_hi;
   ka.lag_first = p->lag_first;
   ka.n_blocks = p->n_blocks;
+  ka.p_hi = p->h_hi;
+  ka.p_lo = p->h_lo;
+  ka.ls = p->ls;
+  ka.p0 = p->p0;
+  ka.lag_lo = p->d.lag_lo;
   ka.threshold = p->d.threshold;
   ka.tie_tol = p->tie_tol;
   ka.ties = p->ties;
@@ -410,7 +430,8 @@ int sxc::lag_plan_pairs(sxc_plan* p, const LagPairArgs& base, int row0, int rows
     const long long t0 = tiles((e0 - row0) / 32), t1 = tiles((e1 - row0 + 31) / 32);
     ka.tiles = base.tiles + t0;
     ka.n_tiles = (int)(t1 - t0);
-    HIP_CHECK(launch_lag_pairs(p->d.form == SXC_FORM_LAG_BF16X3, ka, st));
+    const bool two = p->d.form == SXC_FORM_LAG_BF16X3;
+    HIP_CHECK(p->tile ? launch_lag_tiles(two, ka, st) : launch_lag_pairs(two, ka, st));
   }
   return SXC_OK;
 }
@@ -510,7 +531,8 @@ static size_t plan_device_bytes(const sxc_plan* p) {
   b += (size_t)p->n_work * sizeof(int2) * (p->blk_work ? 2 : 1) +
        (size_t)p->tie_cap * sizeof(int4) * (p->lag ? 3 : 1);
   if (p->lag)
-    b += ((size_t)p->row_band * p->d.n_channels * p->hs * 2 + rows * p->l16) * 2 * (p->h_lo ? 2 : 1) +
+    b += (p->tile ? rows * p->ls : (size_t)p->row_band * p->d.n_channels * p->hs * 2 + rows * p->l16) * 2 *
+             (p->h_lo ? 2 : 1) +
          rows * (size_t)p->d.trace_len * sizeof(float) + (p->energy ? rows * sizeof(double) : 0);
   return b;
 }

@@ -72,20 +72,24 @@ __device__ __forceinline__ void store_columns(const LagPrepArgs& a, int row, Par
   }
 }
 
+// What a launch makes: the operands, the row operands alone (LagPrepArgs::energy_in)
+// or planes (p_hi).
+enum class Prep { kOperands, kRows, kPlanes };
+template <Prep kWhat>
 __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
   const int row = blockIdx.x;
   if (row == 0 && threadIdx.x == 0) {
     if (a.zero0) *a.zero0 = 0u;
     if (a.zero1) *a.zero1 = 0u;
   }
-  if (row >= a.n_rows) {  // the last column tile's empty events
+  if (kWhat == Prep::kOperands && row >= a.n_rows) {  // the last column tile's empty events
     store_columns(a, row, [](int, unsigned short& h, unsigned short& l) { h = l = 0; });
     return;
   }
   const float* x = a.in + (long long)row * a.in_stride;
   __shared__ double red[256];
   double mean = 0.0, E;
-  if (a.energy_in) {
+  if constexpr (kWhat == Prep::kRows) {
     E = a.energy_in[row];
   } else {
     double s1 = 0.0;
@@ -121,6 +125,14 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
   // that every lag of its pairs is NaN whatever samples a range of lags skips,
   // and the pairs come out as (0, lag 0) as in the FFT form.
   const float outside = E <= 1.7e308 ? 0.f : __int_as_float(0x7fc00000);
+  auto store_trace = [&] {
+    if (!a.traces_out) return;
+    float* tr = a.traces_out + (long long)row * a.L;
+    for (int n = threadIdx.x; n < a.L; n += 256) {
+      const float v = n < a.in_len ? x[n] : 0.f;
+      tr[n] = a.demean && n < a.in_len ? (float)((double)v - mean) : v;
+    }
+  };
   // sample n of the scaled trace as its 16-bit hi and lo parts
   auto part = [&](int n, unsigned short& h, unsigned short& l) {
     float v = outside;
@@ -136,6 +148,16 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
       l = f32_to_bf16_rne(v - bf16_to_f32(h));
     }
   };
+  if constexpr (kWhat == Prep::kPlanes) {
+    for (int s = threadIdx.x; s < a.ls; s += 256) {
+      unsigned short h, l;
+      part(s - a.p0, h, l);
+      a.p_hi[(long long)row * a.ls + s] = h;
+      if (a.p_lo) a.p_lo[(long long)row * a.ls + s] = l;
+    }
+    store_trace();
+    return;
+  }
   // row operand: element q of copy 0 is sample q + lag_first, of copy 1 the next
   unsigned* h0 = reinterpret_cast<unsigned*>(a.h_hi + (long long)row * 2 * a.hs);
   unsigned* l0 = a.h_lo ? reinterpret_cast<unsigned*>(a.h_lo + (long long)row * 2 * a.hs) : nullptr;
@@ -150,15 +172,9 @@ __global__ __launch_bounds__(256) void k_lag_prep(LagPrepArgs a) {
       l0[a.hs / 2 + q] = l[1] | (unsigned)l[2] << 16;
     }
   }
-  if (a.energy_in) return;
+  if constexpr (kWhat == Prep::kRows) return;
   store_columns(a, row, part);
-  if (a.traces_out) {
-    float* tr = a.traces_out + (long long)row * a.L;
-    for (int n = threadIdx.x; n < a.L; n += 256) {
-      const float v = n < a.in_len ? x[n] : 0.f;
-      tr[n] = a.demean && n < a.in_len ? (float)((double)v - mean) : v;
-    }
-  }
+  store_trace();
 }
 
 // ----------------------------------------------------------------------------
@@ -415,13 +431,39 @@ __device__ __forceinline__ void scan_range(f32x16 (&acc)[NI * NB], int ni, Best3
   }
 }
 
+template <bool BF16X3>
+__device__ __forceinline__ PlaneRows<BF16X3> row_operand(const LagPairArgs& a, int i) {
+  const long long o = (long long)min(i, a.n_events - 1) * a.n_channels * 2 * a.hs;
+  PlaneRows<BF16X3> r;
+  r.hi = plane_rsrc(a.h_hi + o, 2ll * a.n_channels * a.hs);
+  if constexpr (BF16X3) r.lo = plane_rsrc(a.h_lo + o, 2ll * a.n_channels * a.hs);
+  return r;
+}
+template <bool BF16X3>
+__device__ __forceinline__ PlaneRows<BF16X3> column_operand(const LagPairArgs& a, int j0) {
+  const long long o = (long long)(j0 / 32) * a.n_channels * a.l16 * 32;
+  PlaneRows<BF16X3> c;
+  c.hi = plane_rsrc(a.b_hi + o, 32ll * a.n_channels * a.l16);
+  if constexpr (BF16X3) c.lo = plane_rsrc(a.b_lo + o, 32ll * a.n_channels * a.l16);
+  return c;
+}
+// Lane offsets in bytes: A row r starts lag(r) samples in, at an even element of the
+// copy of its parity; B column r of the chunk's two groups of 8 samples.
+__device__ __forceinline__ int row_offset(const LagPairArgs& a, int lane) {
+  const int r = lane & 31;
+  return 2 * ((r >> 4) * a.hs + 8 * (lane >> 5) + 2 * (r & 15));
+}
+__device__ __forceinline__ int column_offset(int lane) { return 16 * lane; }
+
 // First lags at which this row has the values p and n, block by block (the bits are
 // those of the ranges, whose products differ by zeros alone).  Every lane takes its
 // column's values.  Values past the window's last lag come after the first.
 template <bool BF16X3>
-__device__ __forceinline__ void seek_lags(const PlaneRows<BF16X3>& row, const PlaneRows<BF16X3>& cols, int vh, int vb,
-                                       const LagPairArgs& a, int h, float p, float n, int& fp, int& fn) {
-  const PlaneRows<BF16X3> rows[1] = {row};
+__device__ __forceinline__ void seek_lags(const LagPairArgs& a, int i, int j0, int lane, float p, float n, int& fp,
+                                          int& fn) {
+  const int h = lane >> 5;
+  const PlaneRows<BF16X3> rows[1] = {row_operand<BF16X3>(a, i)}, cols = column_operand<BF16X3>(a, j0);
+  const int vh = row_offset(a, lane), vb = column_offset(lane);
   int lp = a.lag_hi, ln = a.lag_hi;
   for (int b = a.n_blocks - 1; b >= 0; --b) {
     const int l0 = a.lag_first + 32 * b, l1 = min(l0 + 31, a.lag_hi);
@@ -437,12 +479,6 @@ __device__ __forceinline__ void seek_lags(const PlaneRows<BF16X3>& row, const Pl
   }
   fp = min(lp, __shfl_xor(lp, 32, 64));
   fn = min(ln, __shfl_xor(ln, 32, 64));
-}
-
-// Place of pair (i, j) in the outputs.
-__device__ __forceinline__ long long out_index(const LagPairArgs& a, int i, int j) {
-  return a.out_ld ? (long long)(i - a.out_row0) * a.out_ld + (j - a.out_col0)
-                  : (long long)i * a.n_events - (long long)i * (i - 1) / 2 + (j - i);
 }
 
 constexpr int kLagWaves = 8;  // per workgroup, two per SIMD
@@ -474,10 +510,7 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
   const int split = a.split, part = wv % split;
   const int rows_per_wg = kLagWaves / split * NI, groups = 32 / rows_per_wg;
   const int n_items = a.n_tiles * groups;
-  // lane offsets in bytes: A row r starts lag(r) samples in, at an even element
-  // of the copy of its parity; B column r32 of the chunk's two groups of 8 samples
-  const int vh = 2 * ((r32 >> 4) * a.hs + 8 * h + 2 * (r32 & 15));
-  const int vb = 16 * (32 * h + r32);
+  const int vh = row_offset(a, lane), vb = column_offset(lane);
   // XCD-aware walk: XCD blockIdx % 8 takes its own contiguous eighth of the
   // items, so the tiles of a row of tiles share their rows' operands in its L2
   const int n_xcd = (gridDim.x % 8 == 0) ? 8 : 1;
@@ -489,16 +522,10 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
     if (ib >= a.n_events || j0 >= a.n_events) continue;  // ragged last block (workgroup-uniform)
     const int i0 = ib + wv / split * NI;  // this wave's first row
     const bool live = i0 < a.n_events;
-    PlaneRows<BF16X3> rows[NI], cols;
+    PlaneRows<BF16X3> rows[NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const long long o = (long long)min(i0 + i, a.n_events - 1) * a.n_channels * 2 * a.hs;
-      rows[i].hi = plane_rsrc(a.h_hi + o, 2ll * a.n_channels * a.hs);
-      if constexpr (BF16X3) rows[i].lo = plane_rsrc(a.h_lo + o, 2ll * a.n_channels * a.hs);
-    }
-    const long long bo = (long long)(j0 / 32) * a.n_channels * a.l16 * 32;
-    cols.hi = plane_rsrc(a.b_hi + bo, 32ll * a.n_channels * a.l16);
-    if constexpr (BF16X3) cols.lo = plane_rsrc(a.b_lo + bo, 32ll * a.n_channels * a.l16);
+    for (int i = 0; i < NI; ++i) rows[i] = row_operand<BF16X3>(a, i0 + i);
+    const PlaneRows<BF16X3> cols = column_operand<BF16X3>(a, j0);
     Best3<int> pos[NI];
     Best3<unsigned> neg[NI];
 #pragma unroll
@@ -561,7 +588,7 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
       const bool wp = tp && (q1 - __int_as_float(p.k3) < tol || q1 < tol);
       const bool wn = tn && (m1 - mag(n.k3) < tol || m1 < tol);
       if (out) {
-        const long long idx = out_index(a, ii, j);
+        const long long idx = lag_out_index(a, ii, j);
         a.vpos[idx] = kp ? p1 : 0.f;
         a.lpos[idx] = kp ? glp1 : 0;
         a.vneg[idx] = kn ? n1 : 0.f;
@@ -581,9 +608,9 @@ __global__ __launch_bounds__(64 * kLagWaves, 2) void k_lag_pairs(LagPairArgs a) 
         const bool lost = (tp || tn) && slot >= (unsigned)a.tie_cap;
         if (__ballot(lost)) {
           int fp, fn;
-          seek_lags<BF16X3>(rows[i], cols, vh, vb, a, h, p1, n1, fp, fn);
+          seek_lags<BF16X3>(a, ii, j0, lane, p1, n1, fp, fn);
           if (lost) {
-            const long long idx = out_index(a, ii, j);
+            const long long idx = lag_out_index(a, ii, j);
             a.lpos[idx] = kp ? fp : 0;
             a.lneg[idx] = kn ? fn : 0;
           }
@@ -813,8 +840,13 @@ __global__ __launch_bounds__(256) void k_pack_block(PackBlockArgs a) {
 hipError_t launch_lag_prep(const LagPrepArgs& a, hipStream_t st) {
   if (a.n_rows <= 0) return hipSuccess;
   const int events = a.n_rows / a.n_channels;
-  const int rows = a.energy_in ? a.n_rows : (events + 31) / 32 * 32 * a.n_channels;  // with the last column tile's empty ones
-  hipLaunchKernelGGL(k_lag_prep, dim3(rows), dim3(256), 0, st, a);
+  const int rows = (events + 31) / 32 * 32 * a.n_channels;  // with the last column tile's empty ones
+  if (a.energy_in)
+    hipLaunchKernelGGL(k_lag_prep<Prep::kRows>, dim3(a.n_rows), dim3(256), 0, st, a);
+  else if (a.p_hi)
+    hipLaunchKernelGGL(k_lag_prep<Prep::kPlanes>, dim3(a.n_rows), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_lag_prep<Prep::kOperands>, dim3(rows), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

@@ -77,6 +77,9 @@ struct sxc_plan {
   // those from row_first on
   int row_band = 0, row_first = 0;
   double* energy = nullptr;  // row_band < n_events
+  // few lags (lag_tiles): planes at h_hi (and h_lo) instead of the operands
+  bool tile = false;
+  int p0 = 0, ls = 0;
   unsigned short *h_hi = nullptr, *h_lo = nullptr, *b_hi = nullptr, *b_lo = nullptr;  // LagPrepArgs
   float* lag_traces = nullptr;
   int2* tiles = nullptr;

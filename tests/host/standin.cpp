@@ -128,6 +128,7 @@ hipError_t launch_pairs(int R, bool full, const PairArgs& a, int, hipStream_t) {
 hipError_t launch_resolve(int R, const ResolveArgs& a, int, hipStream_t) { return call(on_resolve, R, a); }
 hipError_t launch_lag_prep(const LagPrepArgs& a, hipStream_t) { return call(on_lag_prep, a); }
 hipError_t launch_lag_pairs(bool bf16x3, LagPairArgs a, hipStream_t) { return call(on_lag_pairs, bf16x3, a); }
+hipError_t launch_lag_tiles(bool bf16x3, const LagPairArgs& a, hipStream_t) { return call(on_lag_pairs, bf16x3, a); }
 hipError_t launch_fill_u32(unsigned* p, unsigned v, int n, hipStream_t) {
   for (int k = 0; k < n; ++k) p[k] = v;
   return hipSuccess;

@@ -131,3 +131,42 @@ def test_row_operands_in_bands(name, band, block):
         tiled.assemble(run, coef, lag)
         assert np.array_equal(coef[i, j], want[0].astype(np.float16)) and np.array_equal(lag[i, j], want[1])
     run.close()
+
+
+@pytest.mark.parametrize("name,n,C,L,lo,hi", [
+    ("bf16x3", 512, 3, 1400, -20, 20), ("bf16x3", 520, 3, 1397, -15, 17), ("bf16x3", 512, 3, 1400, -7, 40),
+    ("bf16x3", 512, 1, 4100, 100, 140), ("bf16x3", 512, 3, 1400, -1399, -1360), ("bf16x3", 600, 3, 2500, 60, 95),
+    ("bf16x3", 1200, 3, 4096, -31, 31), ("bf16x3", 1200, 3, 4096, -50, 50), ("bf16x3", 1200, 3, 4096, 0, 0),
+    ("bf16x3", 1200, 3, 4096, -4095, -4080), ("fp16", 1200, 1, 4096, -3, -3), ("fp16", 1200, 3, 2500, -10, 11),
+    ("fp16", 1200, 3, 4096, -23, 20), ("fp16", 1200, 3, 4096, -24, 25)])
+def test_few_lags_on_many_samples(oracle, name, n, C, L, lo, hi):
+    """Windows that run on the tile kernel (jobs that fill the CUs, one to seven
+    blocks of 16 lags from a first lag that is 1 modulo 8 on): a sample of the
+    pairs against FP64 direct sums, a row with a NaN, and a tiled run against the
+    packed execute."""
+    form, tol = FORMS[name]
+    rng = np.random.default_rng(n + L + hi)
+    x = rng.standard_normal((n, C, L + 2)).astype(np.float32)
+    x = (x[..., 2:] + x[..., 1:-1] + x[..., :-2]) * np.float32(0.5)
+    bad = x.copy()
+    bad[7, 0, L // 2] = np.nan
+    print(f"case few lags {name} n={n} C={C} L={L} [{lo}, {hi}]", flush=True)
+    plan = engine.AllPairsPlan(n, C, L, 0, lo, hi, form=form)
+    d = DeviceArray.from_numpy(bad)
+    vp, lp, vn, ln = [o.numpy() for o in plan.execute(d)]
+    plan.close()
+    pi, pj = oracle.packed_pairs(n)
+    hit = (pi == 7) | (pj == 7)
+    assert not vp[hit].any() and not lp[hit].any() and not vn[hit].any() and not ln[hit].any()
+    k = np.unique(np.concatenate([np.flatnonzero(~hit)[-40:], rng.choice(np.flatnonzero(~hit), 3000)]))
+    ref = oracle.pairs_f64(x, pi[k], pj[k], lo, hi, circular=False)
+    assert np.abs(vp[k] - ref["pos"]).max() <= tol and np.abs(vn[k] - ref["neg"]).max() <= tol
+    sp = (ref["pos"] > 1e-3) & (ref["gap_pos"] >= 1e-12)
+    sn = (ref["neg"] < -1e-3) & (ref["gap_neg"] >= 1e-12)
+    assert np.array_equal(lp[k][sp], ref["lag_pos"][sp]) and np.array_equal(ln[k][sn], ref["lag_neg"][sn])
+    run = tiled.TiledRun(n, C, L, lo, hi, form=form, block=256)
+    coef, lag = np.zeros((n, n), np.float16), np.zeros((n, n), np.int16)
+    run.start(d)
+    tiled.assemble(run, coef, lag)
+    run.close()
+    assert np.array_equal(coef[pi, pj], vp.astype(np.float16)) and np.array_equal(lag[pi, pj], lp)

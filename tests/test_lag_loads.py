@@ -27,3 +27,7 @@ def test_operand_loads_stay_in_the_allocation(tmp_path):
 
 def test_scan_state(tmp_path):
     _run(tmp_path, "lag_scan.cpp")
+
+
+def test_tile_kernel_loads_stay_in_the_planes(tmp_path):
+    _run(tmp_path, "lag_tile_loads.cpp")

@@ -50,6 +50,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -137,7 +138,11 @@ struct Buffers {
   std::vector<float*> idle;
   void make(size_t floats, int count) {
     count = (int)std::min<size_t>(count, kBufferBytes / (floats * sizeof(float)));
-    mem.assign(floats * count, 0.f);
+    try {
+      mem.assign(floats * count, 0.f);
+    } catch (const std::bad_alloc&) {
+      return;  // requests allocate their own
+    }
     for (int k = 0; k < count; ++k) idle.push_back(mem.data() + k * floats);
   }
   float* take() {

@@ -18,6 +18,8 @@
  *   - "pos" is the largest coefficient above 0 and its first lag, "neg" the
  *     smallest below 0 (Correlation_in_OMP/correlation_c.cpp:102-111); a
  *     value not beyond the threshold is stored as (0, 0) (:119-136);
+ *   - an event with a NaN or infinite sample has no coefficients: its pairs are
+ *     (0, lag 0), at whatever lags the sample would be reached;
  *   - near ties (another lag within tie_tol of the winner) are settled by an
  *     FP64 re-evaluation of the candidate lags, ties to the smaller lag;
  *   - return value 0 on success, negative on error (see seismic_last_error).

@@ -864,7 +864,6 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Ro
   for (int P : {1024, 2048, 3072, 4096, 5120, 6144})
     if (how != Rows::kPeriod && P < p->P && P >= desc.trace_len + reach && desc.lag_lo > -P / 2 && desc.lag_hi <= P / 2) {
       p->narrow.P = P;
-      p->narrow.M = P / 2;
       p->narrow.R = P / 128;
       p->narrow.spec_stride = P / 2 + 32;
       break;
@@ -901,7 +900,6 @@ void sxc::fft_plan_geometry(const sxc_plan_desc& desc, long long tie_cap_max, Ro
       best = cost;
       FftGeom& g = p->cut;
       g.P = P;
-      g.M = P / 2;
       g.R = P / 128;
       g.spec_stride = P / 2 + 32;
       g.n_seg = n_seg;
@@ -970,7 +968,6 @@ int sxc_plan_destroy(sxc_plan* plan) {
 sxc::FftGeom sxc::fft_geom(const sxc_plan* p, int in_len, bool reversed) {
   FftGeom g;
   g.R = p->R;
-  g.M = p->M;
   g.P = p->P;
   g.spec_stride = p->spec_stride;
   g.fwd2 = p->fwd2;

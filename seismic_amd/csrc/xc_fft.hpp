@@ -30,10 +30,6 @@ __device__ __forceinline__ cf csub(cf a, cf b) { return cf{a.x - b.x, a.y - b.y}
 __device__ __forceinline__ cf cmul(cf a, cf b) {
   return cf{__builtin_fmaf(a.x, b.x, -a.y * b.y), __builtin_fmaf(a.x, b.y, a.y * b.x)};
 }
-// a * conj(b)
-__device__ __forceinline__ cf cmulc(cf a, cf b) {
-  return cf{__builtin_fmaf(a.x, b.x, a.y * b.y), __builtin_fmaf(a.y, b.x, -a.x * b.y)};
-}
 __device__ __forceinline__ cf f2c(float2 v) { return cf{v.x, v.y}; }
 __device__ __forceinline__ float2 c2f(cf v) { return make_float2(v.x, v.y); }
 

@@ -5,8 +5,8 @@
 namespace sxc {
 
 constexpr int kLagBlock = 32;  // lags per block (one accumulator tile each)
-// A plan's window spans at most this many lags, counted in whole blocks of 16
-// from the last lag at or below its first that is 1 modulo 8.
+// The widest window a plan takes, in whole blocks of kTileLags from tile_first_lag on (a
+// limit of the interface: the product over lags needs none).
 constexpr int kLagMaxSpan = 65536;
 
 // Elements past a row's or a column tile's operand that the product's loads may

@@ -1,5 +1,6 @@
 // Lag-window form on MFMA (gfx950): the correlation over a bounded window of
-// lags as dense products.
+// lags as dense products.  (Some windows of few lags run tile by tile instead:
+// xc_lag_tile.hip.)
 //
 // The coefficient c_ij(l) = sum_c sum_n xh_ic[n] xh_jc[n - l]
 // (xh = x / (|x| sqrt(C)), linear correlation, zero outside [0, L)) is, with
@@ -489,13 +490,15 @@ struct LagMerge {
 // Bound by the matrix cores at the clock the power limit leaves: 0.82-0.86 busy
 // at 1.6-1.8 GHz, 1.6 PFLOP/s of bf16 and 1.3 of fp16 issued (a 16384-cubed
 // library matmul reaches 1.31 and 1.25 on the same card); deeper or shallower
-// operand rings, one to three steps ahead, change it by less than 1%.  A kernel
-// whose products were 32 x 32 pairs at one lag, with 24-sample column windows
-// shifted into 16 operands per step (3-4 vector instructions per product, one
-// wave per SIMD) and every range run over all samples, took N = 1500, C = 3,
-// L = 2048, +-512 bf16x3 32.0 ms against 25.2 here, N = 2001, L = 4096, +-512 fp16
-// 17.2 against 12.7, and N = 40..491 up to 16 times as long: its unit of work was
-// a whole 32 x 32 tile.
+// operand rings, one to three steps ahead, change it by less than 1%.  The tile kernel
+// (xc_lag_tile.hip: 32 x 32 pairs at one lag, 24-sample column windows
+// shifted into 16 operands per step, 3-4 vector instructions per product, one
+// wave per SIMD, every lag over all samples) takes N = 1500, C = 3,
+// L = 2048, +-512 bf16x3 32.1 ms against 25.3 here, N = 2001, L = 4096, +-512 fp16
+// 17.2 against 12.7, and N = 40..491 up to 16 times as long: its unit of work is
+// a whole 32 x 32 tile.  Windows of one or two blocks are bound by the operand loads,
+// which take the CU's load path about 22 cycles each: N = 2000, C = 3, L = 4096, +-20
+// bf16x3 7.48 ms, 0.8 of the rate above (the tile kernel 5.9).
 //
 // One workgroup per (tile of 32 columns, group of rows of the tile's 32).  Its
 // waves take NI consecutive rows each; when a job has too few rows to fill the

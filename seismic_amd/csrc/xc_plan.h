@@ -37,7 +37,7 @@ inline int dev_alloc(T** p, size_t count, const char* what) {
 namespace sxc {
 // An FFT period and its device tables.
 struct FftGeom {
-  int R = 0, M = 0, P = 0;
+  int R = 0, P = 0;
   long long spec_stride = 0;  // float2 per (event, channel) row
   float2 *fwd2 = nullptr, *inv2 = nullptr, *post = nullptr;
   bool full = false;          // the pair kernel scans every lag unmasked

@@ -37,7 +37,8 @@ enum {
   SXC_ERR_HIP = -2,       /* a HIP runtime call failed */
   SXC_ERR_MEMORY = -3,    /* device allocation failed */
   SXC_ERR_TIES = -4,      /* results written, but near ties overflowed the FP64 resolver's
-                             record capacity: those pairs keep their FP32 argmax lag */
+                             record capacity: those pairs keep an FP32 lag, in the lag forms the
+                             argmax, in the FFT form that of a value within the band */
   SXC_ERR_OVERLOAD = -5,  /* serving: request shed by admission (latency budget or queue bound) */
 };
 

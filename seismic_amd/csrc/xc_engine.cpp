@@ -488,8 +488,8 @@ static int check_tie_overflow(sxc_plan* p) {
   int rc = sxc_plan_stats(p, &stt);
   if (rc) return rc;
   if (stt.tie_overflow) {
-    set_error("%llu near ties exceeded the FP64 resolver's record capacity (%d): their lags are the FP32 "
-              "argmax, not the FP64 one",
+    set_error("%llu near ties exceeded the FP64 resolver's record capacity (%d): their lags are FP32 "
+              "ones, not the FP64 argmax",
               stt.tie_overflow, p->tie_cap);
     return SXC_ERR_TIES;
   }
